@@ -114,7 +114,7 @@ static void free_all(mhpc_ctx *c) {
                     c->mlp_grad, c->mlp_norm, c->mlp_x, c->mlp_t, c->mlp_hprev, c->mlp_idx,
                     c->mlp_partial, c->mlp_loss_partial, c->mlp_loss, c->mlp_io_x, c->mlp_io_y,
                     c->hlist[0], c->hlist[1], c->hlist[2], c->sdirty,
-                    c->h0slot, c->olist, c->ocount, c->hcnt, c->nn_start, c->nn_start_rng, c->hhard,
+                    c->h0slot, c->olist, c->ocount, c->seglist, c->hcnt, c->nn_start, c->nn_start_rng, c->hhard,
                     c->xyzm, c->ppar, c->cpar};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
@@ -187,6 +187,7 @@ static int create_impl(mhpc_ctx *c, int64_t cap, int64_t cap_cells) {
     HIPC(dalloc(&c->hhard, cap));
     HIPC(dalloc(&c->olist, cap));
     HIPC(dalloc(&c->ocount, 4));
+    HIPC(dalloc(&c->seglist, nn_parts_max(cap)));
     HIPC(dalloc(&c->hcnt, cap));
     // start table levels: the smallest K with 8^K >= cap (one geometric cell per particle on
     // average at the deepest level), 1 <= K <= MHPC_NN_KMAX

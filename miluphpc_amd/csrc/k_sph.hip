@@ -25,6 +25,10 @@
 static_assert(NN_LEAF_GROUP < NN_CWIN, "a clipped range crosses at most one end of the window");
 #define NN_OUTLIER 4.0       // group-mode outlier: h above this factor x the group's smallest
 #define NN_OUTLIER_MAX 32    // at most this many outliers per group are split off
+#define NN_SPLIT_VOL 8.0     // group walks: a box of more than this many search cubes (2 h)^3 ...
+#define NN_SPLIT_CAND 4096   // ... whose start cells hold more than this many particles is split
+#define NN_SPLIT_MIN 16      // split-off parts of fewer particles go to the per-particle mode
+static_assert(64 / NN_SPLIT_MIN <= MHPC_NN_PARTS_PER_GROUP, "the part list holds every group's parts");
 #define NN_SPARSE 64         // re-lists: groups with at most this many flagged particles go per particle
 #define NN_DRANGES 256       // direct form: candidate ranges per wavefront
 #define NN_DSPAN 5           // direct form: start cells per axis - 1 (<= 216 cells)
@@ -96,9 +100,12 @@ struct NNArgs {
                               // (slot of list_out); read by the dirty marking
     int32_t *out_list;        // group mode: outlier particles deferred to the per-particle mode
     uint32_t *out_count;
+    ulonglong2 *seg_list;     // group mode: {group, lanes} of the parts split off (see nn_split_group)
+    uint32_t *seg_count;
     uint32_t *err;
     unsigned long long *counters;
     const double *chmax;      // per cell: an upper bound of its particles' h
+    const uint8_t *lcp;       // key levels sorted particles k and k + 1 share (group splits)
     // h-iteration passes: the bounds the new h of the particles still iterating raise
     double *chmax_raise;
     const int32_t *ppar, *cpar;
@@ -228,6 +235,36 @@ __device__ __forceinline__ bool nn_win_clip(int w0, int w1, int &rs, int &rc, in
     return true;
 }
 
+// Lebesgue prefix of the level-K cell with the per-axis indices (ix, iy, iz) (the lower half of
+// an axis sets its key bit, so the indices' bits enter inverted).
+__device__ __forceinline__ uint64_t nn_cell_prefix(int ix, int iy, int iz, int K) {
+    uint64_t P = 0;
+    for (int l = K - 1; l >= 0; l--) {
+        const uint64_t d = (uint64_t)(((ix >> l) & 1) ^ 1) | ((uint64_t)(((iy >> l) & 1) ^ 1) << 1) |
+                           ((uint64_t)(((iz >> l) & 1) ^ 1) << 2);
+        P = (P << 3) | d;
+    }
+    return P;
+}
+
+// Particles in the start cells a walk for the box [lo, hi] would begin from (see nn_start_push):
+// the candidates it has to stream, short of what the distance bounds prune.
+__device__ __forceinline__ int nn_box_particles(const NNArgs &A, double lox, double hix, double loy, double hiy,
+                                                double loz, double hiz) {
+    const NNStart S = nn_start_level(A, lox, hix, loy, hiy, loz, hiz);
+    if (S.K < 1) return (int)A.n;
+    const int bx = S.ilx >> S.s, by = S.ily >> S.s, bz = S.ilz >> S.s;
+    const int nx = (S.ihx >> S.s) - bx + 1, ny = (S.ihy >> S.s) - by + 1, nz = (S.ihz >> S.s) - bz + 1;
+    const int lane = wave_lane();
+    int cnt = 0;
+    if (lane < nx * ny * nz) {
+        const int64_t e = nn_tab_off(S.K) +
+                          (int64_t)nn_cell_prefix(bx + lane % nx, by + (lane / nx) % ny, bz + lane / (nx * ny), S.K);
+        if (A.stab[e] >= 0) cnt = A.srng[e].y;
+    }
+    return wave_sum(cnt);
+}
+
 // Start a walk for the box [lo, hi]: the deepest table level K <= kmax at which the box
 // spans at most 4 cells per axis, and the table's node for every such cell (a cell of level
 // K, a particle alone in it, or none).  Every particle inside the box lies in one of these
@@ -256,12 +293,7 @@ __device__ __forceinline__ int nn_start_push(LdsT &L, const NNArgs &A, double lo
         const int nx = (ihx >> s) - bx + 1, ny = (ihy >> s) - by + 1, nz = (ihz >> s) - bz + 1;
         if (lane < nx * ny * nz && lane % nparts == part) {
             const int ix = bx + lane % nx, iy = by + (lane / nx) % ny, iz = bz + lane / (nx * ny);
-            uint64_t P = 0;
-            for (int l = K - 1; l >= 0; l--) {
-                const uint64_t d = (uint64_t)(((ix >> l) & 1) ^ 1) | ((uint64_t)(((iy >> l) & 1) ^ 1) << 1) |
-                                   ((uint64_t)(((iz >> l) & 1) ^ 1) << 2);
-                P = (P << 3) | d;
-            }
+            const uint64_t P = nn_cell_prefix(ix, iy, iz, K);
             node = A.stab[nn_tab_off(K) + (int64_t)P];
             if (node >= 0) rng = A.srng[nn_tab_off(K) + (int64_t)P];
         }
@@ -328,12 +360,7 @@ __device__ __forceinline__ bool nn_direct(LdsT &L, const NNArgs &A, double lox, 
         int first = 0, num = 0;
         if (idx < ncell) {
             const int ix = bx + idx % nx, iy = by + (idx / nx) % ny, iz = bz + idx / (nx * ny);
-            uint64_t P = 0;
-            for (int l = K - 1; l >= 0; l--) {
-                const uint64_t d = (uint64_t)(((ix >> l) & 1) ^ 1) | ((uint64_t)(((iy >> l) & 1) ^ 1) << 1) |
-                                   ((uint64_t)(((iz >> l) & 1) ^ 1) << 2);
-                P = (P << 3) | d;
-            }
+            const uint64_t P = nn_cell_prefix(ix, iy, iz, K);
             const int64_t e = nn_tab_off(K) + (int64_t)P;
             const int node = A.stab[e];
             if (node >= 0 && (node < A.n || nn_cell_reaches(A, q, node - A.n))) {
@@ -604,32 +631,91 @@ __device__ __forceinline__ bool h_update(const NNArgs &A, int N, double hi, doub
     return fin;
 }
 
+// bounding box of the active lanes' positions and their largest h
+struct NNBox {
+    double x0, x1, y0, y1, z0, z1, h;
+};
+__device__ __forceinline__ NNBox nn_box(bool active, double x, double y, double z, double h) {
+    NNBox B;
+    B.h = wave_max(active ? h : 0.0);
+    B.x0 = wave_min(active ? x : 1e300); B.x1 = wave_max(active ? x : -1e300);
+    B.y0 = wave_min(active ? y : 1e300); B.y1 = wave_max(active ? y : -1e300);
+    B.z0 = wave_min(active ? z : 1e300); B.z1 = wave_max(active ? z : -1e300);
+    return B;
+}
+
+// A run of 64 keys can cross a boundary of a large cell.  The Lebesgue curve jumps there, so the
+// run's box may hold a good part of the domain although each particle's surroundings are small:
+// on a 47^3 lattice the worst such group streamed all 103,823 particles as candidates, and its
+// one wavefront was the walk's whole time (1.75 ms; split, see nn_split_group, SPLIT_NOW ms).  The box is worth splitting when it is
+// both large against the search radius and crowded; a group whose box is small against h, or
+// holds few particles, gains nothing from a second walk.
+__device__ __forceinline__ bool nn_split_wanted(const NNArgs &A, const NNBox &B, uint64_t m) {
+    if ((m & (m - 1)) == 0) return false;   // one particle
+    const double w = 2.0 * B.h, ex = B.x1 - B.x0, ey = B.y1 - B.y0, ez = B.z1 - B.z0;
+    if (!((w + ex) * (w + ey) * (w + ez) > NN_SPLIT_VOL * (w * w * w))) return false;
+    return nn_box_particles(A, B.x0 - B.h, B.x1 + B.h, B.y0 - B.h, B.y1 + B.h, B.z0 - B.h, B.z1 + B.h) > NN_SPLIT_CAND;
+}
+
+// Splits a group's active particles into runs that need no further split, cutting at the
+// boundaries of the largest cells first (the smallest shared key prefix between consecutive
+// particles; of several, the last).  Runs of at least NN_SPLIT_MIN particles are listed for
+// k_nn_walk_parts, one wavefront each; the others go to the per-particle mode, where lanes are
+// candidates.  Every active particle ends up in exactly one of the two lists.
+__device__ __forceinline__ void nn_split_group(const NNArgs &A, int64_t group, int64_t k, bool active, double x,
+                                               double y, double z, double h) {
+    const int lane = wave_lane();
+    uint64_t todo = wave_ballot(active);
+    while (todo != 0) {
+        uint64_t m = todo;
+        for (;;) {
+            const NNBox B = nn_box((m >> lane) & 1ull, x, y, z, h);
+            if (!nn_split_wanted(A, B, m)) break;
+            // lanes first .. last - 1 of the run own the boundary to their successor
+            const int first = __builtin_ctzll(m), last = 63 - __builtin_clzll(m);
+            const int cut = lane >= first && lane < last ? (int)A.lcp[k] * 64 + (63 - lane) : 0x7fffffff;
+            const int at = 63 - (wave_min(cut) & 63);   // first <= at < last
+            m &= (2ull << at) - 1ull;
+        }
+        todo &= ~m;
+        const int num = popc64(m);
+        const bool part = num >= NN_SPLIT_MIN;
+        uint32_t b = 0;
+        if (lane == 0) b = part ? atomicAdd(A.seg_count, 1u) : atomicAdd(A.out_count, (uint32_t)num);
+        b = __shfl(b, 0);
+        if (part) {
+            if (lane == 0) A.seg_list[b] = make_ulonglong2((unsigned long long)group, m);
+        } else if ((m >> lane) & 1ull) {
+            A.out_list[b + popc64(m & lanemask_lt())] = (int32_t)k;
+        }
+    }
+}
+
 // Group mode: one wavefront owns 64 consecutive sorted particles and walks once with the
-// bounding box of its active particles grown by their largest h.
+// bounding box of its active particles grown by their largest h, or once per part of the group
+// where the box would be far larger than its particles' surroundings.
 // MODE 0: build lists (only the particles flagged in `only` when it is set);
 // MODE 1: one Jacobi pass of the h-iteration (count only; with list_out set, the
 // unconverged particles are appended to it for the next pass);
 // MODE 2: MODE 1 that also writes every particle's list with the h of this pass
 // (speculative: kept for the particles whose list cannot change afterwards)
-template <int MODE>
-__global__ __launch_bounds__(64 * NN_WAVES) void k_nn_walk(NNArgs A) {
-    __shared__ NNWaveLdsF lds_all[NN_WAVES];
-    const int w = threadIdx.x / 64, lane = wave_lane();
-    NNWaveLdsF &L = lds_all[w];
-    const int64_t group = xcd_block(blockIdx.x, gridDim.x) * NN_WAVES + w;
+// SEG: `mSeg` lanes of the group only (a part that an earlier launch split off).
+template <int MODE, bool SEG>
+__device__ __forceinline__ void nn_group(NNWaveLdsF &L, const NNArgs &A, int64_t group, uint64_t mSeg) {
+    const int lane = wave_lane();
     const int64_t k = group * 64 + lane;
     const int64_t n = A.n;
-    if (group * 64 >= n) return;
     const bool valid = k < n;
     bool active = valid;
-    if (MODE >= 1 && valid) active = A.done[k] == 0;
-    if (MODE == 0 && valid && A.only) active = A.only[k] != 0;
+    if (SEG) active = valid && ((mSeg >> lane) & 1ull);
+    if (!SEG && MODE >= 1 && valid) active = A.done[k] == 0;
+    if (!SEG && MODE == 0 && valid && A.only) active = A.only[k] != 0;
     uint64_t mActive = wave_ballot(active);
     if (mActive == 0) {
-        if (MODE >= 1 && valid) A.h_next[k] = A.h[k];
+        if (MODE >= 1 && valid && !SEG) A.h_next[k] = A.h[k];
         return;
     }
-    if (MODE == 0 && A.only && A.out_list && popc64(mActive) <= NN_SPARSE) {
+    if (!SEG && MODE == 0 && A.only && A.out_list && popc64(mActive) <= NN_SPARSE) {
         // a re-list of a few flagged particles: 64 lanes testing candidates for one or two of
         // them is wasted, so they go to the per-particle mode (lanes = candidates)
         uint32_t b = 0;
@@ -644,8 +730,8 @@ __global__ __launch_bounds__(64 * NN_WAVES) void k_nn_walk(NNArgs A) {
     const double hi2 = hi * hi;
     // outliers: a few active particles with h above NN_OUTLIER x the group's smallest would
     // grow the search box of all 64; they go to the per-particle mode instead
-    bool outlier = false;
-    if (A.out_list) {
+    bool outlier = SEG && !active;   // a part's other lanes belong to other waves
+    if (!SEG && A.out_list) {
         const double hmin = wave_min(active ? hi : 1e300);
         const bool big = active && hi > NN_OUTLIER * hmin;
         const uint64_t mO = wave_ballot(big);
@@ -661,11 +747,14 @@ __global__ __launch_bounds__(64 * NN_WAVES) void k_nn_walk(NNArgs A) {
     }
     // search box: bounding box of the active lanes grown by their largest h (plus a
     // relative margin far above FP64 rounding, so pruning never drops a true pair)
-    const double hmax = wave_max(active ? hi : 0.0);
+    const NNBox B = nn_box(active, xi, yi, zi, hi);
+    if (!SEG && A.seg_list && nn_split_wanted(A, B, mActive)) {
+        nn_split_group(A, group, k, active, xi, yi, zi, hi);
+        if (MODE >= 1 && valid && !active && !outlier) A.h_next[k] = hi;
+        return;
+    }
+    const double hmax = B.h, bx0 = B.x0, bx1 = B.x1, by0 = B.y0, by1 = B.y1, bz0 = B.z0, bz1 = B.z1;
     const double grow = hmax * (1.0 + 1e-9);
-    const double bx0 = wave_min(active ? xi : 1e300), bx1 = wave_max(active ? xi : -1e300);
-    const double by0 = wave_min(active ? yi : 1e300), by1 = wave_max(active ? yi : -1e300);
-    const double bz0 = wave_min(active ? zi : 1e300), bz1 = wave_max(active ? zi : -1e300);
     const double lox = bx0 - grow, hix = bx1 + grow;
     const double loy = by0 - grow, hiy = by1 + grow;
     const double loz = bz0 - grow, hiz = bz1 + grow;
@@ -830,6 +919,28 @@ __global__ __launch_bounds__(64 * NN_WAVES) void k_nn_walk(NNArgs A) {
             }
         }
         if (lane == 0) atomicAdd(&cnt_slot(A.counters)[CNT_H_COUNTS], (unsigned long long)popc64(mActive));
+    }
+}
+
+template <int MODE>
+__global__ __launch_bounds__(64 * NN_WAVES) void k_nn_walk(NNArgs A) {
+    __shared__ NNWaveLdsF lds_all[NN_WAVES];
+    const int w = threadIdx.x / 64;
+    const int64_t group = xcd_block(blockIdx.x, gridDim.x) * NN_WAVES + w;
+    if (group * 64 >= A.n) return;
+    nn_group<MODE, false>(lds_all[w], A, group, 0ull);
+}
+
+// the parts of groups that k_nn_walk<MODE> split off, one wavefront each
+template <int MODE>
+__global__ __launch_bounds__(64 * NN_WAVES) void k_nn_walk_parts(NNArgs A) {
+    __shared__ NNWaveLdsF lds_all[NN_WAVES];
+    const int w = threadIdx.x / 64;
+    const uint32_t cnt = *A.seg_count;
+    for (int64_t t = (int64_t)blockIdx.x * NN_WAVES + w; t < cnt; t += (int64_t)gridDim.x * NN_WAVES) {
+        const ulonglong2 s = A.seg_list[t];
+        nn_group<MODE, true>(lds_all[w], A, (int64_t)s.x, s.y);
+        wave_sync();
     }
 }
 
@@ -1159,9 +1270,14 @@ static NNArgs nn_common(mhpc_ctx *c) {
     a.err = c->err;
     a.counters = c->counters;
     a.chmax = c->chmax;
+    a.lcp = c->lcp;
     return a;
 }
 
+// parts of split groups: at most about one resident round of wavefronts, looping over the list
+static unsigned nn_parts_grid(mhpc_ctx *c) {
+    return (unsigned)std::min<int64_t>(ceil_div(nn_parts_max(c->n), NN_WAVES), 2048);
+}
 static unsigned nn_grid(mhpc_ctx *c) { return (unsigned)ceil_div(ceil_div(c->n, 64), NN_WAVES); }
 
 // done flags, iteration counts and dirty flags to zero; the per-pass list counters, the
@@ -1178,7 +1294,7 @@ __global__ void k_h_init(int64_t n, uint8_t *done, int32_t *iters, uint8_t *dirt
         cnt_slot[k] = 0u;
     }
     if (k < nlc) list_counts[k] = 0;
-    if (k < 2) ocount[k] = 0;
+    if (k < 4) ocount[k] = 0;
 }
 
 // the raise for the listed particles (after pass 0: the particles still iterating are the ones
@@ -1228,13 +1344,18 @@ void launch_h_iterate(mhpc_ctx *c, int passes, bool speculative, hipEvent_t *wal
     const unsigned g1 = (unsigned)std::min<int64_t>(ceil_div(c->n, NN1_WAVES), NN1_MAX_BLOCKS);
     a.out_list = c->olist;
     a.out_count = c->ocount;   // zeroed by k_h_init
+    a.seg_list = c->seglist;
+    a.seg_count = c->ocount + 2;
+    const unsigned gs = nn_parts_grid(c);
     if (walk_events) (void)hipEventRecord(walk_events[0], c->stream);
     if (speculative) {
         a.nbr4 = reinterpret_cast<int4 *>(c->nbr);
         a.stride = c->cap_pad;
         hipLaunchKernelGGL(k_nn_walk<2>, dim3(nn_grid(c)), dim3(64 * NN_WAVES), 0, c->stream, a);
+        hipLaunchKernelGGL(k_nn_walk_parts<2>, dim3(gs), dim3(64 * NN_WAVES), 0, c->stream, a);
     } else {
         hipLaunchKernelGGL(k_nn_walk<1>, dim3(nn_grid(c)), dim3(64 * NN_WAVES), 0, c->stream, a);
+        hipLaunchKernelGGL(k_nn_walk_parts<1>, dim3(gs), dim3(64 * NN_WAVES), 0, c->stream, a);
     }
     if (walk_events) (void)hipEventRecord(walk_events[1], c->stream);
     // the group mode's outliers, same pass, per-particle mode
@@ -1305,7 +1426,10 @@ void launch_neighbours_fixup(mhpc_ctx *c) {
     b.only = c->sdirty;
     b.out_list = c->olist;
     b.out_count = c->ocount + 1;
+    b.seg_list = c->seglist;
+    b.seg_count = c->ocount + 3;
     hipLaunchKernelGGL(k_nn_walk<0>, dim3(nn_grid(c)), dim3(64 * NN_WAVES), 0, c->stream, b);
+    hipLaunchKernelGGL(k_nn_walk_parts<0>, dim3(nn_parts_grid(c)), dim3(64 * NN_WAVES), 0, c->stream, b);
     b.out_list = nullptr;
     b.list_in = c->olist;
     b.count_in = c->ocount + 1;
@@ -1327,10 +1451,13 @@ void launch_neighbours(mhpc_ctx *c) {
     a.sml_out = nullptr;
     a.siters = c->siters;
     a.iters_out = nullptr;
-    launch_fill_u32(c, c->ocount, 0u, 1);
+    launch_fill_u32(c, c->ocount, 0u, 4);
     a.out_list = c->olist;
     a.out_count = c->ocount;
+    a.seg_list = c->seglist;
+    a.seg_count = c->ocount + 2;
     hipLaunchKernelGGL(k_nn_walk<0>, dim3(nn_grid(c)), dim3(64 * NN_WAVES), 0, c->stream, a);
+    hipLaunchKernelGGL(k_nn_walk_parts<0>, dim3(nn_parts_grid(c)), dim3(64 * NN_WAVES), 0, c->stream, a);
     a.out_list = nullptr;
     a.list_in = c->olist;
     a.count_in = c->ocount;

@@ -142,7 +142,9 @@ struct mhpc_ctx {
     int32_t *hlist[3] = {nullptr, nullptr, nullptr};   // h-iteration: unconverged particles per pass
     uint8_t *sdirty = nullptr;                   // speculative lists: particles to re-list
     int32_t *olist = nullptr;                    // neighbour search: group-mode outliers
-    uint32_t *ocount = nullptr;
+    uint32_t *ocount = nullptr;                  // [4] outliers of pass 0 / of the list fix-up, then
+                                                 // the parts of the same two walks
+    ulonglong2 *seglist = nullptr;               // neighbour search: parts of split groups
     double *h0slot = nullptr;                    // pass-0 h of the unconverged particles (list slot)
     int32_t *hhard = nullptr;                    // tail passes: slots left to the split counts
     uint32_t *hlist_count = nullptr;             // = dstatus->hlist_count: list lengths of the
@@ -258,6 +260,10 @@ void launch_diagnostics(mhpc_ctx *c, double *partial, mhpc_diagnostics *out);
 #endif
 
 static inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// most parts a neighbour walk over n particles can split off (see nn_split_group)
+#define MHPC_NN_PARTS_PER_GROUP 4
+static inline int64_t nn_parts_max(int64_t n) { return MHPC_NN_PARTS_PER_GROUP * ceil_div(n, 64); }
 
 __device__ __forceinline__ int wave_lane() { return (int)__lane_id(); }
 
