@@ -26,10 +26,18 @@ static_assert(NN_LEAF_GROUP < NN_CWIN, "a clipped range crosses at most one end 
 #define NN_OUTLIER 4.0       // group-mode outlier: h above this factor x the group's smallest
 #define NN_OUTLIER_MAX 32    // at most this many outliers per group are split off
 #define NN_SPLIT_VOL 8.0     // group walks: a box of more than this many search cubes (2 h)^3 ...
-#define NN_SPLIT_CAND 4096   // ... whose start cells hold more than this many particles is split
+#define NN_SPLIT_CAND 3072   // ... whose start cells hold more than this many particles is split
 #define NN_SPLIT_MIN 16      // split-off parts of fewer particles go to the per-particle mode
 static_assert(64 / NN_SPLIT_MIN <= MHPC_NN_PARTS_PER_GROUP, "the part list holds every group's parts");
-#define NN_SPARSE 64         // re-lists: groups with at most this many flagged particles go per particle
+// Re-lists: groups with at most this many flagged particles go per particle (lanes are
+// candidates), the others are walked again.  A group walk costs as much as about ten
+// per-particle searches: with 64 / 32 / 16 / 8 / 4 a step of the 128^3 blast takes
+// 9.61 / 9.50 / 8.96 / 8.88 / 8.87 ms and the 1M cloud's RHS 7.45 / 7.41 / 6.91 / 6.68 / 6.63 ms.
+// With fewer groups than fill the chip the walk's latency counts instead: every flagged
+// particle gets its own wavefront (16^3: 446 us against 466).
+#define NN_SPARSE 8
+#define NN_SPARSE_FEW 64     // below NN_FEW_GROUPS groups
+#define NN_FEW_GROUPS 1024   // one wavefront per SIMD
 #define NN_DRANGES 256       // direct form: candidate ranges per wavefront
 #define NN_DSPAN 5           // direct form: start cells per axis - 1 (<= 216 cells)
 #define NN_DIRECT_MAX 32768  // direct form: candidates per wavefront
@@ -94,6 +102,8 @@ struct NNArgs {
     uint32_t *cnt_slot;       // split counting: neighbour count of list slot t
     const int32_t *slot_list; // split counting: the list slots it takes
     const uint32_t *slot_count;
+    int sparse;               // list mode with `only`: groups with at most this many flagged particles
+                              // go to the per-particle mode
     const uint8_t *only;      // list mode: when set, only particles with only[k] != 0
     uint8_t *dirty;           // dirty marking: particles whose list must be rebuilt
     double *h0_slot;          // pass 0 with lists: the pass-0 h of each unconverged particle
@@ -647,9 +657,12 @@ __device__ __forceinline__ NNBox nn_box(bool active, double x, double y, double 
 // A run of 64 keys can cross a boundary of a large cell.  The Lebesgue curve jumps there, so the
 // run's box may hold a good part of the domain although each particle's surroundings are small:
 // on a 47^3 lattice the worst such group streamed all 103,823 particles as candidates, and its
-// one wavefront was the walk's whole time (1.75 ms; split, see nn_split_group, SPLIT_NOW ms).  The box is worth splitting when it is
-// both large against the search radius and crowded; a group whose box is small against h, or
-// holds few particles, gains nothing from a second walk.
+// one wavefront was the walk's whole time (1.75 ms; 0.22 ms with such groups split, and their
+// parts take 0.09 ms).  The box is worth splitting when it is both large against the search
+// radius and crowded; a group whose box is small against h, or holds few particles, gains nothing
+// from a second walk.  Bounds measured: a volume of 6 / 8 / 12 search cubes gives 1052 / 1050 /
+// 1186 us for the 47^3 RHS in two walks, 2048 / 3072 / 4096 / 8192 candidates 995 / 1006 / 1058 /
+// 1234 us there and 9.80 / 9.60 / 9.61 / 9.62 ms for a step of the 128^3 blast.
 __device__ __forceinline__ bool nn_split_wanted(const NNArgs &A, const NNBox &B, uint64_t m) {
     if ((m & (m - 1)) == 0) return false;   // one particle
     const double w = 2.0 * B.h, ex = B.x1 - B.x0, ey = B.y1 - B.y0, ez = B.z1 - B.z0;
@@ -715,7 +728,7 @@ __device__ __forceinline__ void nn_group(NNWaveLdsF &L, const NNArgs &A, int64_t
         if (MODE >= 1 && valid && !SEG) A.h_next[k] = A.h[k];
         return;
     }
-    if (!SEG && MODE == 0 && A.only && A.out_list && popc64(mActive) <= NN_SPARSE) {
+    if (!SEG && MODE == 0 && A.only && A.out_list && popc64(mActive) <= A.sparse) {
         // a re-list of a few flagged particles: 64 lanes testing candidates for one or two of
         // them is wasted, so they go to the per-particle mode (lanes = candidates)
         uint32_t b = 0;
@@ -1424,6 +1437,7 @@ void launch_neighbours_fixup(mhpc_ctx *c) {
     b.stride = c->cap_pad;
     b.snoi = c->snoi;
     b.only = c->sdirty;
+    b.sparse = ceil_div(c->n, 64) < NN_FEW_GROUPS ? NN_SPARSE_FEW : NN_SPARSE;
     b.out_list = c->olist;
     b.out_count = c->ocount + 1;
     b.seg_list = c->seglist;
