@@ -122,6 +122,7 @@ static void free_all(mhpc_ctx *c) {
         if (c->f_own[f]) (void)hipFree(c->f_own[f]);
     if (c->h_status) (void)hipHostFree(c->h_status);
     if (c->h_status1) (void)hipHostFree(c->h_status1);
+    if (c->h_diag) (void)hipHostFree(c->h_diag);
     for (int e = 0; e < MHPC_NUM_EVENTS; e++)
         if (c->ev[e]) (void)hipEventDestroy(c->ev[e]);
     if (c->sync_ev) (void)hipEventDestroy(c->sync_ev);
@@ -139,6 +140,7 @@ static int create_impl(mhpc_ctx *c, int64_t cap, int64_t cap_cells) {
     memset(c->h_status, 0, sizeof(DevStatus));
     HIPC(hipHostMalloc((void **)&c->h_status1, sizeof(DevStatus), hipHostMallocDefault));
     memset(c->h_status1, 0, sizeof(DevStatus));
+    HIPC(hipHostMalloc((void **)&c->h_diag, sizeof(mhpc_diagnostics), hipHostMallocDefault));
     c->err = &c->dstatus->err;
     c->counters = c->dstatus->counters;
     c->sort_check = &c->dstatus->sort_check;
@@ -887,11 +889,11 @@ extern "C" int mhpc_leapfrog_update_v(mhpc_ctx *c, double dt) {
 
 extern "C" int mhpc_compute_diagnostics(mhpc_ctx *c, mhpc_diagnostics *out) {
     if (!c || !out) return MHPC_E_ARG;
-    mhpc_diagnostics *d = reinterpret_cast<mhpc_diagnostics *>(c->diag_out);
-    launch_diagnostics(c, c->diag_partial, d);
+    // the fold writes its record straight into pinned host memory: no copy behind it
+    launch_diagnostics(c, c->diag_partial, c->h_diag);
     HIPC(hipGetLastError());
-    HIPC(hipMemcpyAsync(out, d, sizeof(*out), hipMemcpyDeviceToHost, c->stream));
     HIPC(ctx_sync(c));
+    *out = *c->h_diag;
     return MHPC_OK;
 }
 

@@ -169,6 +169,7 @@ struct mhpc_ctx {
     DevStatus *h_status = nullptr;               // its pinned host mirror
     DevStatus *h_status1 = nullptr;              // a second pinned copy: the first RHS of a fused
                                                  // PC-Euler step
+    mhpc_diagnostics *h_diag = nullptr;          // pinned: the global sums' record
     uint32_t *err = nullptr;                     // = &dstatus->err
     unsigned long long *counters = nullptr;      // = dstatus->counters
     hipEvent_t ev[MHPC_NUM_EVENTS] = {};
