@@ -2,18 +2,19 @@
 //
 // The reference walks the tree once per particle (computeForces_v1, gravity.cu:252-396)
 // or once per warp of 32 sorted particles with a warp vote on the acceptance test
-// (computeForces_v2, gravity.cu:726-903).  Here one wavefront owns a GROUP of 64
-// consecutive key-sorted particles and walks the tree once for all of them:
-//   * the 64 lanes test up to 64 stacked nodes at a time (FP64, exact, the acceptance
-//     test the oracle restates), so the traversal itself is parallel across lanes.  Vote
-//     form (the reference v2's warp vote, gravity.cu:836, over the group of 64): a cell is
+// (computeForces_v2, gravity.cu:726-903).  Here one wavefront, or a workgroup of several, owns
+// a GROUP of 64 consecutive key-sorted particles and walks the tree once for all of them:
+//   * the 64 lanes of a wavefront test up to 64 stacked nodes at a time (FP64, exact, the
+//     acceptance test the oracle restates), so the traversal itself is parallel across lanes.
+//     Vote form (the reference v2's warp vote, gravity.cu:836, over the group of 64): a cell is
 //     accepted only if every member accepts it with its own distance.  A lane's cell that
 //     passes the test against the group's bounding box passes it for every member (the box
 //     distance is a lower bound of each member's, also after rounding), so only the other
-//     cells are put to the vote: for each, all 64 lanes test it against their own particle
-//     and one ballot decides.  Box form: the bounding-box test alone (one test per group);
-//     it opens more cells;
-//   * leaves and accepted cells go to two LDS interaction lists shared by the wave;
+//     cells are put to the vote: first the lane tests its cell against the member furthest out
+//     in the cell's direction, whose rejection already decides; for the cells left, all 64
+//     lanes test against their own particle and one ballot decides.  Box form: the
+//     bounding-box test alone (one test per group); it opens more cells;
+//   * leaves and accepted cells go to LDS interaction lists of the wavefront;
 //   * each time a list holds 64 entries all 64 lanes evaluate it, every lane reading
 //     the same LDS entry (broadcast) for its own particle.  FP32 mode: entries are
 //     staged as FP32 positions relative to the group's centre (each rounded once from the
@@ -21,45 +22,42 @@
 //     sums are added with Kahan compensation.  FP64 mode: plain FP64 throughout.
 // The stack lives in LDS; the number of nodes popped per round shrinks as the stack
 // fills so it cannot overflow (a hard bound still sets ERRF_STACK).
+//
+// Several wavefronts per group (MULTI) share the group's stack: each round pops up to 64 nodes
+// per wavefront, every wavefront keeps its own interaction lists and partial sums over its nodes,
+// and the partial sums are added in wavefront order at the end (same interactions, same counts).
+// With one wavefront per group, 65,536 particles are 1024 wavefronts, one per SIMD, and every
+// dependent FP64 operation and LDS read shows its latency (launch_bh chooses the width).
+#include <type_traits>
+
 #include "mhpc_internal.h"
 
-#define BH_WAVES 2                       // waves (groups) per block
+#define BH_WAVES 2                       // one wavefront per group: groups per block
+#define BH_MULTI_MAX 8                   // wavefronts per group at most
 static_assert(MHPC_BH_GROUP == 64, "one Barnes-Hut group per wavefront");
-#define BH_STACK 768                     // soft stack capacity per wave
+#define BH_STACK 768                     // soft stack capacity
 #define BH_STACK_PHYS (BH_STACK + 192)   // hard capacity
+// a group with several wavefronts pops up to 64 nodes per wavefront and round: its stack holds
+// as many more children
+__host__ __device__ constexpr int bh_stack_soft(int waves) { return BH_STACK + 448 * (waves - 1); }
+__host__ __device__ constexpr int bh_stack_phys(int waves) { return bh_stack_soft(waves) + 192; }
 #define BH_LIST 128
+#define BH_FILL_WAVES 16384              // see bh_waves_per_group
 
-// FP64 mode: list entries keep FP64 positions
-struct BHWaveLds64 {
-    int stack[BH_STACK_PHYS];
-    // particle list
-    double px[BH_LIST], py[BH_LIST], pz[BH_LIST];
-    double pm[BH_LIST];
-    int pid[BH_LIST];
-    // cell list
-    double cx[BH_LIST], cy[BH_LIST], cz[BH_LIST];
-    double cm[BH_LIST];
-    float4 q0[BH_LIST];
-    float2 q1[BH_LIST];
+// Interaction lists of one wavefront.  `p` holds the particles (id = sorted position) and,
+// without quadrupoles, the accepted cells too (id = -1): both are the same monopole term.
+// FP64 mode: {x, y, z, m}; FP32 mode: FP32 {x, y, z, m} relative to the group's centre (rounded
+// once per entry from the FP64 difference, instead of once per lane and interaction).
+template <bool FP64, bool QUAD>
+struct BHLists {
+    typedef typename std::conditional<FP64, double4, float4>::type rec;
+    rec p[BH_LIST];
+    int id[BH_LIST];
+    // cells with their quadrupole
+    rec c[QUAD ? BH_LIST : 1];
+    float4 q0[QUAD ? BH_LIST : 1];
+    float2 q1[QUAD ? BH_LIST : 1];
 };
-
-// FP32 mode: list entries are FP32 {x, y, z, m} relative to the group's centre (rounded
-// once per entry from the FP64 difference, instead of once per lane and interaction)
-struct BHWaveLds32 {
-    int stack[BH_STACK_PHYS];
-    float4 p[BH_LIST];
-    int pid[BH_LIST];
-    float4 c[BH_LIST];
-    float4 q0[BH_LIST];
-    float2 q1[BH_LIST];
-};
-
-template <bool FP64>
-struct BHLds;
-template <>
-struct BHLds<true> { typedef BHWaveLds64 type; };
-template <>
-struct BHLds<false> { typedef BHWaveLds32 type; };
 
 template <bool FP64>
 struct BHAcc;
@@ -74,31 +72,39 @@ struct BHAcc<true> {
     Plain64 x, y, z, phi;
 };
 
-// 1/sqrt(x) for x >= 0, 0 for x = 0, from the hardware reciprocal square root: for normal x
-// the same value rsqrtf gives, without the compiler's scaling for denormal inputs (four
-// instructions per interaction).  x = r^2 + eps^2 is normal unless eps = 0 and two particles
-// are closer than ~1e-19; such x are raised to the smallest normal float.
+// 1/sqrt(x) for normal x > 0.  SOFT: x is known to be at least the softening, a normal number.
+// Otherwise x = 0 (the particle itself, unsoftened) gives 0, and smaller x are raised to the
+// smallest normal number, so that the bare hardware estimates apply (no denormal scaling).
+template <bool SOFT>
 __device__ __forceinline__ float rsq_pos(float x) {
+    if (SOFT) return __builtin_amdgcn_rsqf(x);
     return x > 0.f ? __builtin_amdgcn_rsqf(fmaxf(x, 1.17549435e-38f)) : 0.f;
 }
+template <bool SOFT>
+__device__ __forceinline__ double rsq_pos(double x) {
+    const double y = rsq_f64(SOFT ? x : fmax(x, 2.2250738585072014e-308));
+    return SOFT || x > 0.0 ? y : 0.0;
+}
 
-// FP32 batches: plain FP32 sums over the (at most 64) entries of one batch, then one
-// compensated (Kahan) addition of each batch sum into the running total
-template <bool POT>
-__device__ __forceinline__ void eval_particles32(const BHWaveLds32 &L, int cnt, float px, float py, float pz,
-                                                 int self, float eps2, BHAcc<false> &acc) {
+// Monopole batch, FP32: plain FP32 sums over the (at most 64) entries, then one compensated
+// (Kahan) addition of each batch sum into the running total.  13 instructions and the
+// reciprocal square root per interaction.
+template <bool POT, bool SOFT, typename ListT>
+__device__ __forceinline__ void eval_mono(const ListT &L, int cnt, float px, float py, float pz, int self,
+                                          float eps2, BHAcc<false> &acc) {
     float bx = 0.f, by = 0.f, bz = 0.f, bp = 0.f;
+#pragma unroll 4
     for (int e = 0; e < cnt; e++) {
         const float4 q = L.p[e];
         const float dx = q.x - px, dy = q.y - py, dz = q.z - pz;
         const float r2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, __builtin_fmaf(dz, dz, eps2)));
-        const float rinv = rsq_pos(r2);
+        const float rinv = rsq_pos<SOFT>(r2);
         const float mr = q.w * rinv;
         const float mr3 = mr * rinv * rinv;
         bx = __builtin_fmaf(mr3, dx, bx);
         by = __builtin_fmaf(mr3, dy, by);
         bz = __builtin_fmaf(mr3, dz, bz);
-        if (POT && L.pid[e] != self) bp -= mr;
+        if (POT && L.id[e] != self) bp -= mr;
     }
     acc.x.add(bx);
     acc.y.add(by);
@@ -106,136 +112,58 @@ __device__ __forceinline__ void eval_particles32(const BHWaveLds32 &L, int cnt, 
     if (POT) acc.phi.add(bp);
 }
 
-template <bool POT, bool QUAD>
-__device__ __forceinline__ void eval_cells32(const BHWaveLds32 &L, int cnt, float px, float py, float pz,
-                                             float eps2, BHAcc<false> &acc) {
-    float bx = 0.f, by = 0.f, bz = 0.f, bp = 0.f;
+// The same in FP64, summed as it comes.
+template <bool POT, bool SOFT, typename ListT>
+__device__ __forceinline__ void eval_mono(const ListT &L, int cnt, double px, double py, double pz, int self,
+                                          double eps2, BHAcc<true> &acc) {
+#pragma unroll 4
     for (int e = 0; e < cnt; e++) {
-        const float4 q = L.c[e];
-        const float dx = q.x - px, dy = q.y - py, dz = q.z - pz;
-        const float r2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, __builtin_fmaf(dz, dz, eps2)));
-        const float rinv = rsq_pos(r2);
-        const float rinv2 = rinv * rinv;
-        const float mr = q.w * rinv;
-        const float mr3 = mr * rinv2;
-        bx = __builtin_fmaf(mr3, dx, bx);
-        by = __builtin_fmaf(mr3, dy, by);
-        bz = __builtin_fmaf(mr3, dz, bz);
-        if (POT) bp -= mr;
-        if (QUAD) {
-            const float4 a = L.q0[e];
-            const float2 b = L.q1[e];
-            const float qdx = __builtin_fmaf(a.x, dx, __builtin_fmaf(a.y, dy, a.z * dz));
-            const float qdy = __builtin_fmaf(a.y, dx, __builtin_fmaf(a.w, dy, b.x * dz));
-            const float qdz = __builtin_fmaf(a.z, dx, __builtin_fmaf(b.x, dy, b.y * dz));
-            const float dqd = __builtin_fmaf(dx, qdx, __builtin_fmaf(dy, qdy, dz * qdz));
-            const float rinv5 = rinv2 * rinv2 * rinv;
-            const float t = 2.5f * dqd * rinv5 * rinv2;
-            bx = __builtin_fmaf(t, dx, __builtin_fmaf(-qdx, rinv5, bx));
-            by = __builtin_fmaf(t, dy, __builtin_fmaf(-qdy, rinv5, by));
-            bz = __builtin_fmaf(t, dz, __builtin_fmaf(-qdz, rinv5, bz));
-            if (POT) bp = __builtin_fmaf(-0.5f * dqd, rinv5, bp);
-        }
+        const double4 q = L.p[e];
+        const double dx = q.x - px, dy = q.y - py, dz = q.z - pz;
+        const double r2 = fma(dx, dx, fma(dy, dy, fma(dz, dz, eps2)));
+        const double rinv = rsq_pos<SOFT>(r2);
+        const double mr = q.w * rinv;
+        const double mr3 = mr * (rinv * rinv);
+        acc.x.s = fma(mr3, dx, acc.x.s);
+        acc.y.s = fma(mr3, dy, acc.y.s);
+        acc.z.s = fma(mr3, dz, acc.z.s);
+        if (POT && L.id[e] != self) acc.phi.s -= mr;
+    }
+}
+
+// Cells with the traceless quadrupole: a = (m r^-3 + 5/2 (d.Qd) r^-7) d - r^-5 Qd, the two terms
+// along d taken together (33 instead of 39 instructions per interaction: the 16.7M Plummer walk
+// is bound by its instruction rate, 34.7 -> 32.6 ms).
+template <bool POT, bool SOFT, typename ListT, typename AccT, typename T>
+__device__ __forceinline__ void eval_quad(const ListT &L, int cnt, T px, T py, T pz, T eps2, AccT &acc) {
+    constexpr bool FP64 = sizeof(T) == 8;
+    T bx = 0, by = 0, bz = 0, bp = 0;
+#pragma unroll 2
+    for (int e = 0; e < cnt; e++) {
+        const auto q = L.c[e];
+        const float4 a = L.q0[e];
+        const float2 b = L.q1[e];
+        const T qxx = a.x, qxy = a.y, qxz = a.z, qyy = a.w, qyz = b.x, qzz = b.y;
+        const T dx = q.x - px, dy = q.y - py, dz = q.z - pz;
+        const T r2 = fma(dx, dx, fma(dy, dy, fma(dz, dz, eps2)));
+        const T rinv = rsq_pos<SOFT>(r2);
+        const T u = rinv * rinv;
+        const T r3 = rinv * u;
+        const T r5 = r3 * u;
+        const T qdx = fma(qxx, dx, fma(qxy, dy, qxz * dz));
+        const T qdy = fma(qxy, dx, fma(qyy, dy, qyz * dz));
+        const T qdz = fma(qxz, dx, fma(qyz, dy, qzz * dz));
+        const T dqd = fma(dx, qdx, fma(dy, qdy, dz * qdz));
+        const T k = r3 * fma(T(2.5), (dqd * u) * u, q.w);
+        bx = fma(k, dx, fma(-r5, qdx, bx));
+        by = fma(k, dy, fma(-r5, qdy, by));
+        bz = fma(k, dz, fma(-r5, qdz, bz));
+        if (POT) bp -= fma(T(0.5) * dqd, r5, q.w * rinv);
     }
     acc.x.add(bx);
     acc.y.add(by);
     acc.z.add(bz);
     if (POT) acc.phi.add(bp);
-}
-
-// particle-particle (monopole) batch, FP64 mode
-template <bool FP64, bool POT>
-__device__ __forceinline__ void eval_particles(const BHWaveLds64 &L, int cnt, double px, double py,
-                                               double pz, int self, double eps2, BHAcc<FP64> &acc) {
-    for (int e = 0; e < cnt; e++) {
-        if constexpr (FP64) {
-            const double dx = L.px[e] - px, dy = L.py[e] - py, dz = L.pz[e] - pz;
-            const double r2 = dx * dx + dy * dy + dz * dz + eps2;
-            const double rinv = r2 > 0.0 ? 1.0 / sqrt(r2) : 0.0;
-            const double mr3 = L.pm[e] * rinv * rinv * rinv;
-            acc.x.add(mr3 * dx);
-            acc.y.add(mr3 * dy);
-            acc.z.add(mr3 * dz);
-            if (POT && L.pid[e] != self) acc.phi.add(-L.pm[e] * rinv);
-        } else {
-            const float dx = (float)(L.px[e] - px), dy = (float)(L.py[e] - py),
-                        dz = (float)(L.pz[e] - pz);
-            const float r2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, __builtin_fmaf(dz, dz, (float)eps2)));
-            const float rinv = rsq_pos(r2);
-            const float mr = (float)L.pm[e] * rinv;
-            const float mr3 = mr * rinv * rinv;
-            acc.x.add(mr3 * dx);
-            acc.y.add(mr3 * dy);
-            acc.z.add(mr3 * dz);
-            if (POT && L.pid[e] != self) acc.phi.add(-mr);
-        }
-    }
-}
-
-// particle-cell batch: monopole (+ traceless quadrupole)
-template <bool FP64, bool POT, bool QUAD>
-__device__ __forceinline__ void eval_cells(const BHWaveLds64 &L, int cnt, double px, double py,
-                                           double pz, double eps2, BHAcc<FP64> &acc) {
-    for (int e = 0; e < cnt; e++) {
-        if constexpr (FP64) {
-            const double dx = L.cx[e] - px, dy = L.cy[e] - py, dz = L.cz[e] - pz;
-            const double r2 = dx * dx + dy * dy + dz * dz + eps2;
-            const double rinv = r2 > 0.0 ? 1.0 / sqrt(r2) : 0.0;
-            const double rinv2 = rinv * rinv;
-            const double m = L.cm[e];
-            const double mr3 = m * rinv * rinv2;
-            double fx = mr3 * dx, fy = mr3 * dy, fz = mr3 * dz;
-            double ph = -m * rinv;
-            if (QUAD) {
-                const float4 a = L.q0[e];
-                const float2 b = L.q1[e];
-                const double qxx = a.x, qxy = a.y, qxz = a.z, qyy = a.w, qyz = b.x, qzz = b.y;
-                const double qdx = qxx * dx + qxy * dy + qxz * dz;
-                const double qdy = qxy * dx + qyy * dy + qyz * dz;
-                const double qdz = qxz * dx + qyz * dy + qzz * dz;
-                const double dqd = dx * qdx + dy * qdy + dz * qdz;
-                const double rinv5 = rinv2 * rinv2 * rinv;
-                const double t = 2.5 * dqd * rinv5 * rinv2;
-                fx += -qdx * rinv5 + t * dx;
-                fy += -qdy * rinv5 + t * dy;
-                fz += -qdz * rinv5 + t * dz;
-                ph += -0.5 * dqd * rinv5;
-            }
-            acc.x.add(fx);
-            acc.y.add(fy);
-            acc.z.add(fz);
-            if (POT) acc.phi.add(ph);
-        } else {
-            const float dx = (float)(L.cx[e] - px), dy = (float)(L.cy[e] - py),
-                        dz = (float)(L.cz[e] - pz);
-            const float r2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, __builtin_fmaf(dz, dz, (float)eps2)));
-            const float rinv = rsq_pos(r2);
-            const float rinv2 = rinv * rinv;
-            const float m = (float)L.cm[e];
-            const float mr = m * rinv;
-            const float mr3 = mr * rinv2;
-            float fx = mr3 * dx, fy = mr3 * dy, fz = mr3 * dz;
-            float ph = -mr;
-            if (QUAD) {
-                const float4 a = L.q0[e];
-                const float2 b = L.q1[e];
-                const float qdx = __builtin_fmaf(a.x, dx, __builtin_fmaf(a.y, dy, a.z * dz));
-                const float qdy = __builtin_fmaf(a.y, dx, __builtin_fmaf(a.w, dy, b.x * dz));
-                const float qdz = __builtin_fmaf(a.z, dx, __builtin_fmaf(b.x, dy, b.y * dz));
-                const float dqd = __builtin_fmaf(dx, qdx, __builtin_fmaf(dy, qdy, dz * qdz));
-                const float rinv5 = rinv2 * rinv2 * rinv;
-                const float t = 2.5f * dqd * rinv5 * rinv2;
-                fx = __builtin_fmaf(t, dx, __builtin_fmaf(-qdx, rinv5, fx));
-                fy = __builtin_fmaf(t, dy, __builtin_fmaf(-qdy, rinv5, fy));
-                fz = __builtin_fmaf(t, dz, __builtin_fmaf(-qdz, rinv5, fz));
-                ph = __builtin_fmaf(-0.5f * dqd, rinv5, ph);
-            }
-            acc.x.add(fx);
-            acc.y.add(fy);
-            acc.z.add(fz);
-            if (POT) acc.phi.add(ph);
-        }
-    }
 }
 
 // a uniform lane's double (l must be the same in every lane)
@@ -261,16 +189,40 @@ struct BHArgs {
     unsigned long long *counters;
 };
 
-template <bool FP64, bool POT, bool QUAD, bool VOTE>
-__global__ __launch_bounds__(64 * BH_WAVES) void k_bh_walk(BHArgs A) {
-    typedef typename BHLds<FP64>::type Lds;
-    __shared__ Lds lds_all[BH_WAVES];
-    const int w = threadIdx.x / 64, lane = wave_lane();
-    Lds &L = lds_all[w];
-    const int64_t group = xcd_block(blockIdx.x, gridDim.x) * BH_WAVES + w;
+// LDS of a block: the stacks, the vote's outermost members, and the wavefronts' lists
+template <bool FP64, bool QUAD>
+struct BHBlock {
+    typedef BHLists<FP64, QUAD> Lists;
+    // MULTI: one stack; otherwise one per wavefront
+    static __host__ __device__ constexpr size_t stack_ints(bool multi, int waves) {
+        return multi ? (size_t)bh_stack_phys(waves) : (size_t)BH_STACK_PHYS * waves;
+    }
+    static constexpr size_t bytes(bool multi, int waves) {
+        return sizeof(Lists) * waves + (multi ? 1 : waves) * 8 * 3 * sizeof(double) + stack_ints(multi, waves) * 4 +
+               4 * BH_MULTI_MAX;
+    }
+};
+
+template <bool FP64, bool POT, bool QUAD, bool VOTE, bool MULTI>
+__global__ __launch_bounds__(64 * (MULTI ? BH_MULTI_MAX : BH_WAVES)) void k_bh_walk(BHArgs A) {
+    typedef BHBlock<FP64, QUAD> Blk;
+    typedef typename Blk::Lists Lists;
+    typedef typename std::conditional<FP64, double, float>::type T;
+    extern __shared__ __align__(32) unsigned char lds[];
+    const int nw = blockDim.x / 64, w = threadIdx.x / 64, lane = wave_lane();
+    Lists &L = reinterpret_cast<Lists *>(lds)[w];
+    double *const ends_all = reinterpret_cast<double *>(lds + sizeof(Lists) * nw);
+    double *const ends = ends_all + (MULTI ? 0 : w * 24);   // [axis][octant] outermost member
+    int *const stack0 = reinterpret_cast<int *>(ends_all + (MULTI ? 1 : nw) * 24);
+    int *const stack = stack0 + (MULTI ? 0 : w * BH_STACK_PHYS);
+    int *const wtot = stack0 + Blk::stack_ints(MULTI, nw);   // MULTI: children pushed per wavefront
+    const int stack_soft = MULTI ? bh_stack_soft(nw) : BH_STACK;
+    const int stack_phys = MULTI ? bh_stack_phys(nw) : BH_STACK_PHYS;
+    const int64_t block = xcd_block(blockIdx.x, gridDim.x);
+    const int64_t group = MULTI ? block : block * nw + w;
     const int64_t k = group * 64 + lane;
     const int64_t n = A.n;
-    if (group * 64 >= n) return;   // whole wave exits together
+    if (group * 64 >= n) return;   // MULTI: the whole block, else the whole wave
     const bool valid = k < n;
     const double4 own = valid ? A.sxm[k] : make_double4(0.0, 0.0, 0.0, 0.0);
     const double px = own.x, py = own.y, pz = own.z;
@@ -287,24 +239,59 @@ __global__ __launch_bounds__(64 * BH_WAVES) void k_bh_walk(BHArgs A) {
     const double eps2 = A.eps2;
     // FP32 mode: positions relative to the group's centre
     const double refx = 0.5 * (glo_x + ghi_x), refy = 0.5 * (glo_y + ghi_y), refz = 0.5 * (glo_z + ghi_z);
-    const float pxr = (float)(px - refx), pyr = (float)(py - refy), pzr = (float)(pz - refz);
-    const float eps2f = (float)eps2;
+    const T tx = FP64 ? (T)px : (T)(px - refx), ty = FP64 ? (T)py : (T)(py - refy),
+            tz = FP64 ? (T)pz : (T)(pz - refz);
+    const T teps2 = (T)eps2;
+    const bool soft = teps2 >= (FP64 ? (T)2.2250738585072014e-308 : (T)1.17549435e-38f);
+    auto flush_p = [&](int cnt, BHAcc<FP64> &acc) {
+        if (soft) eval_mono<POT, true>(L, cnt, tx, ty, tz, (int)k, teps2, acc);
+        else eval_mono<POT, false>(L, cnt, tx, ty, tz, (int)k, teps2, acc);
+    };
+    auto flush_c = [&](int cnt, BHAcc<FP64> &acc) {
+        if (soft) eval_quad<POT, true>(L, cnt, tx, ty, tz, teps2, acc);
+        else eval_quad<POT, false>(L, cnt, tx, ty, tz, teps2, acc);
+    };
+
+    if (VOTE) {
+        // the member furthest out in each octant direction: a cell in that direction is nearest
+        // to it or to a member beside it, so its rejection settles most votes.  (Any member
+        // would do: a choice that rejects nothing only leaves the cell to the ballot.)
+        const double ux = valid ? px - refx : 0.0, uy = valid ? py - refy : 0.0, uz = valid ? pz - refz : 0.0;
+        if (!MULTI || w == 0) {
+#pragma unroll
+            for (int o = 0; o < 8; o++) {
+                const float d = (float)((o & 1 ? ux : -ux) + (o & 2 ? uy : -uy) + (o & 4 ? uz : -uz));
+                const uint64_t m = wave_ballot(valid && d == wave_max(valid ? d : -3.0e38f));
+                if (m != 0 && lane == __builtin_ctzll(m)) {
+                    ends[o] = px;
+                    ends[8 + o] = py;
+                    ends[16 + o] = pz;
+                } else if (m == 0 && lane == 0) {   // non-finite positions: any member
+                    ends[o] = px;
+                    ends[8 + o] = py;
+                    ends[16 + o] = pz;
+                }
+            }
+        }
+    }
 
     BHAcc<FP64> acc;
     int top = 1, pl_n = 0, cl_n = 0;
     long long n_cells = 0, n_parts = 0;
-    if (lane == 0) L.stack[0] = (int)n;   // root
-    wave_sync();
+    if (lane == 0 && (!MULTI || w == 0)) stack[0] = (int)n;   // root
+    if (MULTI) __syncthreads(); else wave_sync();
     const uint64_t lt = lanemask_lt();
     bool overflow = false;
     while (top > 0) {
-        int kpop = (BH_STACK - top) / 7;
+        int kpop = (stack_soft - top) / 7;
         kpop = kpop < 1 ? 1 : kpop;
-        kpop = kpop > 64 ? 64 : kpop;
+        kpop = kpop > 64 * (MULTI ? nw : 1) ? 64 * (MULTI ? nw : 1) : kpop;
         kpop = kpop > top ? top : kpop;
-        const int node = lane < kpop ? L.stack[top - kpop + lane] : -1;
+        // MULTI: the popped nodes are dealt to the wavefronts in turn, each its share of lanes
+        const int slot = MULTI ? lane * nw + w : lane;
+        const int node = slot < kpop ? stack[top - kpop + slot] : -1;
         top -= kpop;
-        wave_sync();
+        if (!MULTI) wave_sync();
         const bool isPart = node >= 0 && node < n;
         const bool isCell = node >= n;
         bool accept = false, open = false;
@@ -346,8 +333,16 @@ __global__ __launch_bounds__(64 * BH_WAVES) void k_bh_walk(BHArgs A) {
             accept = mac_ok(dx * dx + dy * dy + dz * dz, lev);
         }
         if constexpr (VOTE) {
-            // cells the box test rejects: every member tests each with its own distance
-            uint64_t mAmb = wave_ballot(isCell && !accept);
+            // cells the box test rejects: one member's rejection settles the vote, and the
+            // outermost member towards the cell is the likeliest to reject
+            bool amb = isCell && !accept;
+            if (amb) {
+                const int o = (ccx > refx ? 1 : 0) | (ccy > refy ? 2 : 0) | (ccz > refz ? 4 : 0);
+                const double dx = ccx - ends[o], dy = ccy - ends[8 + o], dz = ccz - ends[16 + o];
+                amb = mac_ok(dx * dx + dy * dy + dz * dz, lev);
+            }
+            // the others: every member tests each with its own distance
+            uint64_t mAmb = wave_ballot(amb);
             uint64_t mVote = 0;
             while (mAmb) {
                 const int b = __builtin_ctzll(mAmb);
@@ -361,41 +356,7 @@ __global__ __launch_bounds__(64 * BH_WAVES) void k_bh_walk(BHArgs A) {
             accept = accept || ((mVote >> lane) & 1ull);
         }
         open = isCell && !accept;
-        const uint64_t mP = wave_ballot(isPart), mA = wave_ballot(accept);
-        if (isPart) {
-            const int pos = pl_n + popc64(mP & lt);
-            const double4 r = prec;
-            if constexpr (FP64) {
-                L.px[pos] = r.x;
-                L.py[pos] = r.y;
-                L.pz[pos] = r.z;
-                L.pm[pos] = r.w;
-            } else {
-                L.p[pos] = make_float4((float)(r.x - refx), (float)(r.y - refy), (float)(r.z - refz), (float)r.w);
-            }
-            L.pid[pos] = node;
-        }
-        if (accept) {
-            const int pos = cl_n + popc64(mA & lt);
-            if constexpr (FP64) {
-                L.cx[pos] = ccx;
-                L.cy[pos] = ccy;
-                L.cz[pos] = ccz;
-                L.cm[pos] = cmass;
-            } else {
-                L.c[pos] = make_float4((float)(ccx - refx), (float)(ccy - refy), (float)(ccz - refz),
-                                       (float)cmass);
-            }
-            if (QUAD) {
-                L.q0[pos] = qa;
-                L.q1[pos] = make_float2(qb.x, qb.y);
-            }
-        }
-        pl_n += popc64(mP);
-        cl_n += popc64(mA);
-        n_parts += popc64(mP);
-        n_cells += popc64(mA);
-        // push the children of opened cells
+        // children of opened cells
         int ch[8];
         int nc = 0;
         if (open) {
@@ -405,81 +366,125 @@ __global__ __launch_bounds__(64 * BH_WAVES) void k_bh_walk(BHArgs A) {
             for (int s = 0; s < 8; s++) nc += ch[s] != -1;
         }
         const int incl = wave_incl_scan(nc);
-        const int tot = __shfl(incl, 63);
-        if (top + tot > BH_STACK_PHYS) {
+        int tot = __shfl(incl, 63), before = 0;
+        if (MULTI) {
+            // every wavefront has read its nodes before any pushes
+            if (lane == 0) wtot[w] = tot;
+            __syncthreads();
+            tot = 0;
+            for (int v = 0; v < nw; v++) {
+                const int t = wtot[v];
+                before += v < w ? t : 0;
+                tot += t;
+            }
+        }
+        if (top + tot > stack_phys) {   // MULTI: the same decision in every wavefront
             overflow = true;
             break;
         }
         if (open) {
-            int pos = top + incl - nc;
+            int pos = top + before + incl - nc;
 #pragma unroll
             for (int s = 7; s >= 0; s--)
-                if (ch[s] != -1) L.stack[pos++] = ch[s];
+                if (ch[s] != -1) stack[pos++] = ch[s];
         }
         top += tot;
+        // list entries: particles, and cells (with quadrupole: a list of their own)
+        const uint64_t mP = wave_ballot(isPart), mA = wave_ballot(accept);
+        const uint64_t mL = QUAD ? mP : (mP | mA);
+        const bool toP = isPart || (!QUAD && accept);
+        if (toP) {
+            const int pos = pl_n + popc64(mL & lt);
+            const double ex = isPart ? prec.x : ccx, ey = isPart ? prec.y : ccy, ez = isPart ? prec.z : ccz;
+            const double em = isPart ? prec.w : cmass;
+            if constexpr (FP64) L.p[pos] = make_double4(ex, ey, ez, em);
+            else L.p[pos] = make_float4((float)(ex - refx), (float)(ey - refy), (float)(ez - refz), (float)em);
+            if (POT) L.id[pos] = isPart ? node : -1;
+        }
+        if constexpr (QUAD) {
+            if (accept) {
+                const int pos = cl_n + popc64(mA & lt);
+                if constexpr (FP64) L.c[pos] = make_double4(ccx, ccy, ccz, cmass);
+                else
+                    L.c[pos] = make_float4((float)(ccx - refx), (float)(ccy - refy), (float)(ccz - refz),
+                                           (float)cmass);
+                L.q0[pos] = qa;
+                L.q1[pos] = make_float2(qb.x, qb.y);
+            }
+            cl_n += popc64(mA);
+        }
+        pl_n += popc64(mL);
+        n_parts += popc64(mP);
+        n_cells += popc64(mA);
         wave_sync();
         if (pl_n >= 64) {
-            if constexpr (FP64) eval_particles<FP64, POT>(L, 64, px, py, pz, (int)k, eps2, acc);
-            else eval_particles32<POT>(L, 64, pxr, pyr, pzr, (int)k, eps2f, acc);
+            flush_p(64, acc);
             wave_sync();
             const int rest = pl_n - 64;
             if (lane < rest) {
-                if constexpr (FP64) {
-                    const double a = L.px[64 + lane], b = L.py[64 + lane], d = L.pz[64 + lane];
-                    const double m = L.pm[64 + lane];
-                    L.px[lane] = a; L.py[lane] = b; L.pz[lane] = d; L.pm[lane] = m;
-                } else {
-                    const float4 a = L.p[64 + lane];
-                    L.p[lane] = a;
+                const auto a = L.p[64 + lane];
+                L.p[lane] = a;
+                if (POT) {
+                    const int id = L.id[64 + lane];
+                    L.id[lane] = id;
                 }
-                const int id = L.pid[64 + lane];
-                L.pid[lane] = id;
             }
             pl_n = rest;
             wave_sync();
         }
-        if (cl_n >= 64) {
-            if constexpr (FP64) eval_cells<FP64, POT, QUAD>(L, 64, px, py, pz, eps2, acc);
-            else eval_cells32<POT, QUAD>(L, 64, pxr, pyr, pzr, eps2f, acc);
-            wave_sync();
-            const int rest = cl_n - 64;
-            if (lane < rest) {
-                if constexpr (FP64) {
-                    const double a = L.cx[64 + lane], b = L.cy[64 + lane], d = L.cz[64 + lane];
-                    const double m = L.cm[64 + lane];
-                    L.cx[lane] = a; L.cy[lane] = b; L.cz[lane] = d; L.cm[lane] = m;
-                } else {
-                    const float4 a = L.c[64 + lane];
-                    L.c[lane] = a;
-                }
-                if (QUAD) {
+        if constexpr (QUAD) {
+            if (cl_n >= 64) {
+                flush_c(64, acc);
+                wave_sync();
+                const int rest = cl_n - 64;
+                if (lane < rest) {
+                    const auto a = L.c[64 + lane];
                     const float4 q0 = L.q0[64 + lane];
                     const float2 q1 = L.q1[64 + lane];
+                    L.c[lane] = a;
                     L.q0[lane] = q0;
                     L.q1[lane] = q1;
                 }
+                cl_n = rest;
+                wave_sync();
             }
-            cl_n = rest;
-            wave_sync();
         }
+        if (MULTI) __syncthreads();   // the pushed children are on the stack
     }
     if (overflow) {
         if (lane == 0) set_err(A.err, ERRF_STACK);
         return;
     }
-    if constexpr (FP64) {
-        if (pl_n > 0) eval_particles<FP64, POT>(L, pl_n, px, py, pz, (int)k, eps2, acc);
-        if (cl_n > 0) eval_cells<FP64, POT, QUAD>(L, cl_n, px, py, pz, eps2, acc);
-    } else {
-        if (pl_n > 0) eval_particles32<POT>(L, pl_n, pxr, pyr, pzr, (int)k, eps2f, acc);
-        if (cl_n > 0) eval_cells32<POT, QUAD>(L, cl_n, pxr, pyr, pzr, eps2f, acc);
+    if (pl_n > 0) flush_p(pl_n, acc);
+    if constexpr (QUAD) {
+        if (cl_n > 0) flush_c(cl_n, acc);
     }
-    if (valid) {
+    double ax = acc.x.value(), ay = acc.y.value(), az = acc.z.value(), ph = POT ? acc.phi.value() : 0.0;
+    if (MULTI) {
+        // the wavefronts' partial sums, added in wavefront order (their lists are done with)
+        __syncthreads();
+        double *const part = reinterpret_cast<double *>(lds);
+        static_assert(sizeof(Lists) >= 4 * 64 * sizeof(double), "the lists hold the partial sums");
+        part[(w * 4 + 0) * 64 + lane] = ax;
+        part[(w * 4 + 1) * 64 + lane] = ay;
+        part[(w * 4 + 2) * 64 + lane] = az;
+        part[(w * 4 + 3) * 64 + lane] = ph;
+        __syncthreads();
+        if (w == 0) {
+            for (int v = 1; v < nw; v++) {
+                ax += part[(v * 4 + 0) * 64 + lane];
+                ay += part[(v * 4 + 1) * 64 + lane];
+                az += part[(v * 4 + 2) * 64 + lane];
+                ph += part[(v * 4 + 3) * 64 + lane];
+            }
+        }
+    }
+    if (valid && (!MULTI || w == 0)) {
         const int32_t i = A.perm[k];
-        A.gax[i] = A.G * acc.x.value();
-        A.gay[i] = A.G * acc.y.value();
-        A.gaz[i] = A.G * acc.z.value();
-        if (POT) A.u[i] = 0.5 * own.w * A.G * acc.phi.value();
+        A.gax[i] = A.G * ax;
+        A.gay[i] = A.G * ay;
+        A.gaz[i] = A.G * az;
+        if (POT) A.u[i] = 0.5 * own.w * A.G * ph;
     }
     if (lane == 0) {
         atomicAdd(&cnt_slot(A.counters)[CNT_CELL_INT], (unsigned long long)(n_cells * nvalid));
@@ -487,14 +492,37 @@ __global__ __launch_bounds__(64 * BH_WAVES) void k_bh_walk(BHArgs A) {
     }
 }
 
+// Wavefronts per group: enough groups fill the chip (256 CUs, 4 SIMDs each) by themselves; with
+// fewer, each group is shared by up to 4 wavefronts, and by up to 8 where even that leaves the
+// chip half empty (not with quadrupoles, whose lists take more LDS).  RHS times with 1 wavefront
+// per group and with this rule: 65,536 FP64 monopole 735 / 514 us (8 wavefronts: 528), 300,007
+// FP32 quadrupole 1018 / 955 us (2 wavefronts: 978), a leapfrog step of 2048 385 / 293 us; 1M FP32
+// monopole (16,384 groups, so one either way) is no faster with two (6.13 / 6.22 ms with SPH).
+static int bh_waves_per_group(int64_t groups, bool quad) {
+    const int most = !quad && groups < BH_FILL_WAVES / 32 ? BH_MULTI_MAX : 4;
+    int w = 1;
+    while (w < most && groups * w < BH_FILL_WAVES) w *= 2;
+    return w;
+}
+
 template <bool FP64, bool POT, bool QUAD>
 static void launch_bh(mhpc_ctx *c, const BHArgs &a) {
+    typedef BHBlock<FP64, QUAD> Blk;
     const int64_t groups = ceil_div(c->n, 64);
-    const dim3 grid((unsigned)ceil_div(groups, BH_WAVES)), block(64 * BH_WAVES);
-    if (c->p.bh_accept == MHPC_BH_VOTE)
-        hipLaunchKernelGGL((k_bh_walk<FP64, POT, QUAD, true>), grid, block, 0, c->stream, a);
-    else
-        hipLaunchKernelGGL((k_bh_walk<FP64, POT, QUAD, false>), grid, block, 0, c->stream, a);
+    const bool vote = c->p.bh_accept == MHPC_BH_VOTE;
+    const int waves = bh_waves_per_group(groups, QUAD);
+    if (waves == 1) {
+        const dim3 grid((unsigned)ceil_div(groups, BH_WAVES)), block(64 * BH_WAVES);
+        const size_t bytes = Blk::bytes(false, BH_WAVES);
+        if (vote) hipLaunchKernelGGL((k_bh_walk<FP64, POT, QUAD, true, false>), grid, block, bytes, c->stream, a);
+        else hipLaunchKernelGGL((k_bh_walk<FP64, POT, QUAD, false, false>), grid, block, bytes, c->stream, a);
+        return;
+    }
+    static_assert(Blk::bytes(true, QUAD ? 4 : BH_MULTI_MAX) <= 65536, "LDS of a block");
+    const dim3 grid((unsigned)groups), block(64 * waves);
+    const size_t bytes = Blk::bytes(true, waves);
+    if (vote) hipLaunchKernelGGL((k_bh_walk<FP64, POT, QUAD, true, true>), grid, block, bytes, c->stream, a);
+    else hipLaunchKernelGGL((k_bh_walk<FP64, POT, QUAD, false, true>), grid, block, bytes, c->stream, a);
 }
 
 // ------------------------------------------------------------------------------------
