@@ -111,8 +111,8 @@ static void free_all(mhpc_ctx *c) {
                     c->cmass, c->cx, c->cy, c->cz, c->cquad, c->cquadf, c->cbmin, c->cbmax, c->chmax,
                     c->nbr, c->htable, c->bbox_partial, c->box, c->dstatus,
                     c->diag_partial, c->diag_out, c->pc_backup, c->mlp_params, c->mlp_m1, c->mlp_m2,
-                    c->mlp_grad, c->mlp_norm, c->mlp_x, c->mlp_t, c->mlp_hprev, c->mlp_idx,
-                    c->mlp_partial, c->mlp_loss_partial, c->mlp_loss, c->mlp_io_x, c->mlp_io_y,
+                    c->mlp_grad, c->mlp_norm, c->mlp_x, c->mlp_t, c->mlp_hprev,
+                    c->mlp_partial, c->mlp_frag, c->mlp_loss, c->mlp_io_x, c->mlp_io_y,
                     c->hlist[0], c->hlist[1], c->hlist[2], c->sdirty,
                     c->h0slot, c->olist, c->ocount, c->seglist, c->hcnt, c->nn_start, c->nn_start_rng, c->hhard,
                     c->xyzm, c->ppar, c->cpar};
@@ -620,8 +620,6 @@ extern "C" int mhpc_time_step(mhpc_ctx *c, double courant_fact, double forces_fa
 static int ensure_mlp(mhpc_ctx *c) {
     if (c->mlp_params) return MHPC_OK;
     const int np = mlp_num_params();
-    const int64_t max_waves = ceil_div(MLP_MAX_SAMPLES, 64);
-    const int64_t max_chunks = ceil_div(max_waves, 32);   // stage-1 reduction sums
     HIPC(dalloc(&c->mlp_params, np));
     HIPC(dalloc(&c->mlp_m1, np));
     HIPC(dalloc(&c->mlp_m2, np));
@@ -630,10 +628,8 @@ static int ensure_mlp(mhpc_ctx *c) {
     HIPC(dalloc(&c->mlp_x, c->cap * 8));
     HIPC(dalloc(&c->mlp_t, c->cap));
     HIPC(dalloc(&c->mlp_hprev, c->cap));
-    HIPC(dalloc(&c->mlp_idx, MLP_MAX_SAMPLES));
-    HIPC(dalloc(&c->mlp_partial, (max_waves + max_chunks) * np));
-    HIPC(dalloc(&c->mlp_loss_partial, max_waves + max_chunks));
-    c->mlp_max_waves = max_waves;
+    HIPC(dalloc(&c->mlp_partial, mlp_partial_size()));
+    HIPC(dalloc(&c->mlp_frag, mlp_frag_size()));
     HIPC(dalloc(&c->mlp_loss, 1));
     float norm[18];
     for (int k = 0; k < 18; k++) norm[k] = (k >= 8 && k < 15) || k == 17 ? 1.f : 0.f;
@@ -784,10 +780,9 @@ extern "C" int mhpc_mlp_train(mhpc_ctx *c, int nsamples, int iters, float lr, ui
         if (st != MHPC_OK) return st;
     }
     launch_mlp_targets(c);
+    launch_mlp_frag(c);
     for (int it = 0; it < iters; it++) {
-        launch_mlp_sample(c, nsamples, seed + (uint64_t)it);
-        launch_mlp_gradient(c, nsamples, c->mlp_x, c->mlp_t, c->mlp_idx, c->mlp_grad, c->mlp_loss);
-        launch_mlp_adam(c, lr, ++c->mlp_adam_step);
+        launch_mlp_train_step(c, nsamples, seed + (uint64_t)it, lr, ++c->mlp_adam_step);
     }
     HIPC(hipGetLastError());
     float l = 0.f;
@@ -830,7 +825,8 @@ extern "C" int mhpc_mlp_gradient(mhpc_ctx *c, const float *X, const float *T, in
     if (st != MHPC_OK) return st;
     HIPC(hipMemcpyAsync(c->mlp_io_x, X, sizeof(float) * 8 * (size_t)n, hipMemcpyHostToDevice, c->stream));
     HIPC(hipMemcpyAsync(c->mlp_io_y, T, sizeof(float) * (size_t)n, hipMemcpyHostToDevice, c->stream));
-    launch_mlp_gradient(c, n, c->mlp_io_x, c->mlp_io_y, nullptr, c->mlp_grad, c->mlp_loss);
+    launch_mlp_frag(c);
+    launch_mlp_gradient(c, n, c->mlp_io_x, c->mlp_io_y, c->mlp_grad, c->mlp_loss);
     HIPC(hipGetLastError());
     HIPC(hipMemcpyAsync(grad, c->mlp_grad, sizeof(float) * (size_t)mlp_num_params(), hipMemcpyDeviceToHost,
                         c->stream));

@@ -4,11 +4,10 @@
 // particle's state; the plain h-iteration starts from the prediction and has the last word.
 // No counterpart in the reference.
 //
-// Work split, training: one wavefront owns 64 samples.  Per layer it computes a 64 x 64 tile
-// product as 4 x 4 output blocks of 16 x 16 with K in steps of 16; activations are staged in
-// LDS as BF16 row-major [sample][feature] (the backward pass reads them).  Training writes
-// per-wave gradient partials that one block folds in wave order (deterministic), then Adam
-// updates the weights.  Inference keeps the activations in registers (mlp_forward_16).
+// Inference and training both take 16 samples per step with the activations and, in training,
+// the gradients' accumulators in registers (mlp_forward_16, k_mlp_train_grad).  Training writes
+// one gradient partial per block; one kernel folds them in a fixed order (deterministic) and
+// updates the weights (Adam).
 #include <math.h>
 
 #include "mhpc_internal.h"
@@ -21,6 +20,16 @@ __device__ __forceinline__ unsigned short f2bf(float f) {
     u += 0x7FFFu + ((u >> 16) & 1u);   // round to nearest even (inputs are finite)
     return (unsigned short)(u >> 16);
 }
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bfl2 __attribute__((ext_vector_type(2)));
+// the same rounding by the hardware's packed conversion (v_cvt_pk_bf16_f32)
+__device__ __forceinline__ unsigned pack_bf16(float a, float b) {
+    return __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{a, b}, bfl2));
+}
+__device__ __forceinline__ bf16x4 pack_bf16x4(float a, float b, float c, float d) {
+    const uint2 v = make_uint2(pack_bf16(a, b), pack_bf16(c, d));
+    return __builtin_bit_cast(bf16x4, v);
+}
 __device__ __forceinline__ float bf2f(unsigned short b) { return __uint_as_float(((unsigned)b) << 16); }
 
 // D(16x16) += A(16x16) B(16x16).  Fragments: lane l holds A[l%16][4(l/16)..+3],
@@ -31,12 +40,6 @@ __device__ __forceinline__ f32x4 mfma16(bf16x4 a, bf16x4 b, f32x4 c) {
 
 #define MLP_IN 8      // 7 features + 1 zero pad
 #define MLP_H 64
-#define MLP_KPAD 16   // layer-1 K padded to one MFMA step
-// LDS row strides (BF16 elements): four more than the row length, so that the 16 rows one MFMA
-// operand read touches fall in different banks (with the bare length every row starts in the
-// same bank: 16-way conflicts)
-#define MLP_KLD (MLP_KPAD + 4)
-#define MLP_HLD (MLP_H + 4)
 #define MLP_NPARAM (MLP_H * MLP_IN + MLP_H + MLP_H * MLP_H + MLP_H + MLP_H + 1)   // 4801
 
 // parameter offsets in the flat FP32 vector
@@ -51,81 +54,12 @@ static_assert(MLP_NPARAM == MHPC_MLP_NPARAM, "parameter layout of include/mhpc.h
 
 int mlp_num_params() { return MLP_NPARAM; }
 
-// weights as the kernels stage them: W1 [64][16] bf16 (cols >= 8 zero), W2 [64][64] bf16
-struct alignas(16) MlpLds {
-    unsigned short w1[MLP_H][MLP_KLD];
-    unsigned short w2[MLP_H][MLP_HLD];
-    float b1[MLP_H], b2[MLP_H], w3[MLP_H];
-    float b3;
-};
-
-__device__ void load_weights(MlpLds &W, const float *__restrict__ p) {
-    for (int t = threadIdx.x; t < MLP_H * MLP_KPAD; t += blockDim.x) {
-        const int o = t / MLP_KPAD, k = t % MLP_KPAD;
-        W.w1[o][k] = k < MLP_IN ? f2bf(p[P_W1 + o * MLP_IN + k]) : 0;
-    }
-    for (int t = threadIdx.x; t < MLP_H * MLP_H; t += blockDim.x) W.w2[t / MLP_H][t % MLP_H] = f2bf(p[P_W2 + t]);
-    for (int t = threadIdx.x; t < MLP_H; t += blockDim.x) {
-        W.b1[t] = p[P_B1 + t];
-        W.b2[t] = p[P_B2 + t];
-        W.w3[t] = p[P_W3 + t];
-    }
-    if (threadIdx.x == 0) W.b3 = p[P_B3];
-}
-
-// per-wave activations
-struct alignas(16) MlpWave {
-    unsigned short x[64][MLP_KLD];
-    unsigned short a1[64][MLP_HLD];
-    unsigned short a2[64][MLP_HLD];
-};
-
 // tanh(x) = 1 - 2 / (exp(2x) + 1) from the hardware exp2 and reciprocal estimates: absolute
 // error ~1e-7, far below the BF16 rounding the activations are stored with; saturates to
 // +-1 for large |x|
 __device__ __forceinline__ float tanh_fast(float x) {
     const float e = __builtin_amdgcn_exp2f(x * 2.8853900817779268f);   // exp(2x) = 2^(2x log2 e)
     return 1.f - 2.f * __builtin_amdgcn_rcpf(e + 1.f);
-}
-
-// Z(64 x 64) = act(Ain(64 x K) Wt(K x 64) + b); Ain row-major [sample][k], W row-major
-// [out][k] (so B[k][n] = W[n][k]); writes tanh(Z) as BF16 into Aout.
-template <int K, int LDA>
-__device__ __forceinline__ void dense_tanh(const unsigned short (*Ain)[LDA],
-                                           const unsigned short (*Wt)[LDA], const float *bias,
-                                           unsigned short (*Aout)[MLP_HLD]) {
-    const int lane = wave_lane(), r16 = lane & 15, q = lane >> 4;
-    for (int mt = 0; mt < 4; mt++) {
-        for (int nt = 0; nt < 4; nt++) {
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int kt = 0; kt < K / 16; kt++) {
-                // four consecutive k of one row: one 8-byte LDS read per operand
-                const int k0 = kt * 16 + 4 * q;
-                const bf16x4 a = *reinterpret_cast<const bf16x4 *>(&Ain[mt * 16 + r16][k0]);
-                const bf16x4 b = *reinterpret_cast<const bf16x4 *>(&Wt[nt * 16 + r16][k0]);
-                acc = mfma16(a, b, acc);
-            }
-            const int n = nt * 16 + r16;
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int m = mt * 16 + 4 * q + r;
-                Aout[m][n] = f2bf(tanh_fast(acc[r] + bias[n]));
-            }
-        }
-    }
-}
-
-__device__ __forceinline__ float mlp_forward_wave(const MlpLds &W, MlpWave &S) {
-    dense_tanh<MLP_KPAD, MLP_KLD>(S.x, W.w1, W.b1, S.a1);
-    wave_sync();
-    dense_tanh<MLP_H, MLP_HLD>(S.a1, W.w2, W.b2, S.a2);
-    wave_sync();
-    const int lane = wave_lane();
-    float y = W.b3;
-#pragma unroll 8
-    for (int k = 0; k < MLP_H; k++) y += bf2f(S.a2[lane][k]) * W.w3[k];
-    return y;
 }
 
 // ------------------------------------------------------------------------------------
@@ -301,177 +235,328 @@ __global__ __launch_bounds__(64 * MLP_INF_WAVES) void k_mlp_forward_raw(int64_t 
 }
 
 // ------------------------------------------------------------------------------------
-// training: per wave 64 samples -> forward, loss, backward; gradient partials per wave
-#define MLP_TR_WAVES 2
-struct MlpTrainWave {
-    MlpWave f;
-    unsigned short dz2[64][MLP_HLD];
-    unsigned short dz1[64][MLP_HLD];
-    float dy[64];
-};
+// random sample of a training step: a hash of the seed and the slot
+__device__ __forceinline__ uint64_t mix64(uint64_t z) {
+    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+    return z ^ (z >> 31);
+}
 
-__global__ __launch_bounds__(64 * MLP_TR_WAVES) void k_mlp_train_grad(int64_t nb, const float *__restrict__ X,
-                                                                     const float *__restrict__ T,
-                                                                     const int32_t *__restrict__ idx,
-                                                                     const float *__restrict__ params,
-                                                                     float *__restrict__ partial,
-                                                                     float *__restrict__ loss_partial) {
-    __shared__ MlpLds W;
-    __shared__ MlpTrainWave Sw[MLP_TR_WAVES];
-    load_weights(W, params);
-    __syncthreads();
-    const int w = threadIdx.x / 64, lane = wave_lane(), r16 = lane & 15, q = lane >> 4;
-    MlpTrainWave &S = Sw[w];
-    const int64_t wid = (int64_t)blockIdx.x * MLP_TR_WAVES + w;
-    const int64_t base = wid * 64;
-    float *g = partial + wid * MLP_NPARAM;
-    if (base >= nb) return;
-    const int64_t s = base + lane;
-    const bool valid = s < nb;
-    const int64_t src = valid ? (idx ? (int64_t)idx[s] : s) : 0;
+// Training gradient: each wavefront takes 16 samples per step -> forward, loss, backward -- and
+// keeps the gradient in registers over all its steps (MFMA accumulators of dW2 and dW1, per-lane
+// sums of the rest).
+//
+// Two layouts, "T" (lane (q, c) holds hidden units 4q + r of sample c) and "N" (samples 4q + r
+// of hidden unit c).  An MFMA result in one is an operand of the next product without any
+// exchange between lanes, and swapping the two operands of a product gives its result in the
+// other layout, with the same value for every element; so the forward pass is computed in both:
+//   T feeds the products over hidden units (layer 2, dA1 = dz2 W2);
+//   N feeds the products over samples (dW2 = dz2^T a1, dW1 = dz1^T x).
+// No activation goes through LDS.  Bound by latency and the 64 tanh per lane and step: one wave
+// per 64 samples with the activations in LDS (two wavefronts per CU, transposed 2-byte reads)
+// took 52 us for 65,536 samples, this 20 us
+// (30 us with the weights converted by every block instead of by the Adam update).
+#define MLP_TR_WAVES 4
+#define MLP_TR_BLOCKS 256                // gradient partials at most
+// A partial is laid out as the lanes hold it, four floats (r) per lane: dW2 blocks, dW1 blocks,
+// then dW3, db2, db1 per hidden unit, db3 and the loss.
+#define G_W1 (MLP_H * MLP_H)
+#define G_W3 (G_W1 + 4 * 64 * 4)
+#define G_B2 (G_W3 + MLP_H)
+#define G_B1 (G_B2 + MLP_H)
+#define G_B3 (G_B1 + MLP_H)
+#define G_LOSS (G_B3 + 1)
+#define MLP_ROW 5376
+static_assert(MLP_ROW > G_LOSS && MLP_ROW % 64 == 0, "a partial holds the gradient and the loss");
+
+// the parameter that element i of a partial is the gradient of (-1: none)
+__device__ __forceinline__ int mlp_param_of(int i) {
+    const int r = i & 3, lane = (i >> 2) & 63, c = lane & 15, q = lane >> 4;
+    if (i < G_W1) {
+        const int t = i >> 8, mt = t >> 2, nt = t & 3;
+        return P_W2 + (mt * 16 + 4 * q + r) * MLP_H + nt * 16 + c;
+    }
+    if (i < G_W3) return c < MLP_IN ? P_W1 + (((i - G_W1) >> 8) * 16 + 4 * q + r) * MLP_IN + c : -1;
+    if (i < G_B2) return P_W3 + (i - G_W3);
+    if (i < G_B1) return P_B2 + (i - G_B2);
+    if (i < G_B3) return P_B1 + (i - G_B1);
+    return i == G_B3 ? P_B3 : -1;
+}
+
+// Weight fragments in BF16 as the training kernel's lanes hold them (lane-contiguous 8-byte
+// loads): W1 and W2 with K = inputs (fragments 0..3 and 4 + 4 mt + kt), W2 with K = its outputs
+// (20 + 4 mt + kt).  Written once per call by k_mlp_frag and kept up to date by the Adam update.
+#define MLP_NFRAG 36
+__device__ __forceinline__ void put_frag(unsigned short *__restrict__ frag, int p, float v) {
+    const unsigned short b = f2bf(v);
+    if (p < P_B1) {
+        const int o = p / MLP_IN, k = p % MLP_IN;
+        frag[(((o >> 4) * 64) + (k >> 2) * 16 + (o & 15)) * 4 + (k & 3)] = b;
+    } else if (p >= P_W2 && p < P_B2) {
+        const int j = (p - P_W2) / MLP_H, k = (p - P_W2) % MLP_H, t = (j >> 4) * 4 + (k >> 4);
+        frag[((4 + t) * 64 + ((k >> 2) & 3) * 16 + (j & 15)) * 4 + (k & 3)] = b;
+        frag[((20 + t) * 64 + ((j >> 2) & 3) * 16 + (k & 15)) * 4 + (j & 3)] = b;
+    }
+}
+
+__global__ __launch_bounds__(256) void k_mlp_frag(const float *__restrict__ params, unsigned short *__restrict__ frag) {
+    const int p = blockIdx.x * 256 + threadIdx.x;
+    if (p < 4 * 32 * 4) frag[((p >> 7) * 64 + 32) * 4 + (p & 127)] = 0;   // W1: inputs 8..15
+    if (p < MLP_NPARAM) put_frag(frag, p, params[p]);
+}
+
+int64_t mlp_frag_size() { return (int64_t)MLP_NFRAG * 64 * 4; }
+
+int64_t mlp_partial_size() { return (int64_t)MLP_TR_BLOCKS * MLP_ROW; }
+
+// SAMPLED: training slot i reads pair mix64(...) mod n of (X, T); otherwise pair i
+template <bool SAMPLED>
+__global__ __launch_bounds__(64 * MLP_TR_WAVES, 1) void k_mlp_train_grad(int64_t nb, int64_t n, uint64_t seed,
+                                                                        const float *__restrict__ X,
+                                                                        const float *__restrict__ T,
+                                                                        const float *__restrict__ params,
+                                                                        const bf16x4 *__restrict__ frag,
+                                                                        float *__restrict__ partial) {
+    __shared__ __align__(16) float sb1[MLP_H], sb2[MLP_H], sw3[MLP_H];
+    __shared__ __align__(16) float buf[2][MLP_ROW];
+    const int w = threadIdx.x / 64, lane = wave_lane(), c = lane & 15, q = lane >> 4;
+    const int64_t stride = (int64_t)gridDim.x * (16 * MLP_TR_WAVES);
+    int64_t s = ((int64_t)blockIdx.x * MLP_TR_WAVES + w) * 16 + c;
+    // sample c's features 4q .. 4q + 3 and target, requested a step ahead
+    float4 xv = make_float4(0.f, 0.f, 0.f, 0.f);
+    float tv = 0.f;
+    auto request = [&]() {
+        xv = make_float4(0.f, 0.f, 0.f, 0.f);
+        tv = 0.f;
+        if (s < nb) {
+            const int64_t src = SAMPLED ? (int64_t)(mix64(seed * 0x9E3779B97F4A7C15ull + (uint64_t)s) % (uint64_t)n) : s;
+            if (q < 2) xv = *reinterpret_cast<const float4 *>(X + src * MLP_IN + 4 * q);
+            tv = T[src];
+        }
+    };
+    // weight fragments: W1 and W2 with K = inputs (either operand), W2 with K = its outputs
+    bf16x4 w1[4], w2[4][4], w2t[4][4];
 #pragma unroll
-    for (int k = 0; k < MLP_KPAD; k++) S.f.x[lane][k] = (valid && k < MLP_IN) ? f2bf(X[src * MLP_IN + k]) : 0;
-    wave_sync();
-    const float y = mlp_forward_wave(W, S.f);
-    const float e = valid ? y - T[src] : 0.f;
-    const float dy = e / (float)nb;
-    S.dy[lane] = dy;
-    loss_partial[wid] = wave_sum(0.5f * e * e);
-    wave_sync();
-    // layer 3: gW3[k] = sum_i dy_i a2[i][k], gb3 = sum dy; dz2 = dy w3 (1 - a2^2)
-    {
-        float gw3 = 0.f;
-        for (int i = 0; i < 64; i++) gw3 += S.dy[i] * bf2f(S.f.a2[i][lane]);
-        g[P_W3 + lane] = gw3;
-        const float gb3 = wave_sum(dy);
-        if (lane == 0) g[P_B3] = gb3;
-        for (int k = 0; k < MLP_H; k++) {
-            const float a = bf2f(S.f.a2[lane][k]);
-            S.dz2[lane][k] = f2bf(dy * W.w3[k] * (1.f - a * a));
+    for (int mt = 0; mt < 4; mt++) {
+        w1[mt] = frag[mt * 64 + lane];
+#pragma unroll
+        for (int kt = 0; kt < 4; kt++) {
+            w2[mt][kt] = frag[(4 + 4 * mt + kt) * 64 + lane];
+            w2t[mt][kt] = frag[(20 + 4 * mt + kt) * 64 + lane];
         }
     }
-    wave_sync();
-    // gb2[j] = sum_i dz2[i][j]; gW2[j][k] = sum_i dz2[i][j] a1[i][k] (M = j, K = i, N = k)
-    {
-        float gb2 = 0.f;
-        for (int i = 0; i < 64; i++) gb2 += bf2f(S.dz2[i][lane]);
-        g[P_B2 + lane] = gb2;
-        for (int mt = 0; mt < 4; mt++)
-            for (int nt = 0; nt < 4; nt++) {
-                f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int kt = 0; kt < 4; kt++) {
-                    bf16x4 a, b;
-                    const int i0 = kt * 16 + 4 * q;
-#pragma unroll
-                    for (int u = 0; u < 4; u++) {
-                        a[u] = (short)S.dz2[i0 + u][mt * 16 + r16];
-                        b[u] = (short)S.f.a1[i0 + u][nt * 16 + r16];
-                    }
-                    acc = mfma16(a, b, acc);
-                }
-#pragma unroll
-                for (int r = 0; r < 4; r++) g[P_W2 + (mt * 16 + 4 * q + r) * MLP_H + nt * 16 + r16] = acc[r];
-            }
+    request();
+    if (threadIdx.x < MLP_H) {
+        sb1[threadIdx.x] = params[P_B1 + threadIdx.x];
+        sb2[threadIdx.x] = params[P_B2 + threadIdx.x];
+        sw3[threadIdx.x] = params[P_W3 + threadIdx.x];
     }
-    // dA1[i][k] = sum_j dz2[i][j] W2[j][k] (M = i, K = j, N = k); dz1 = dA1 (1 - a1^2)
-    for (int mt = 0; mt < 4; mt++)
-        for (int nt = 0; nt < 4; nt++) {
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    __syncthreads();
+    float b1n[4], b2n[4], w3n[4];
 #pragma unroll
-            for (int kt = 0; kt < 4; kt++) {
-                bf16x4 a, b;
-                const int j0 = kt * 16 + 4 * q;
-#pragma unroll
-                for (int u = 0; u < 4; u++) {
-                    a[u] = (short)S.dz2[mt * 16 + r16][j0 + u];
-                    b[u] = (short)W.w2[j0 + u][nt * 16 + r16];
-                }
-                acc = mfma16(a, b, acc);
-            }
+    for (int mt = 0; mt < 4; mt++) {
+        b1n[mt] = sb1[mt * 16 + c];
+        b2n[mt] = sb2[mt * 16 + c];
+        w3n[mt] = sw3[mt * 16 + c];
+    }
+    const float b3 = params[P_B3];
+    f32x4 gw2[4][4] = {}, gw1[4] = {};
+    float gw3[4] = {}, gb2[4] = {}, gb1[4] = {}, gb3 = 0.f, loss = 0.f;
+    const float inv_nb = 1.f / (float)nb;
+
+    while (wave_ballot(s < nb) != 0) {
+        const bool valid = s < nb;
+        const float t = tv;
+        const bf16x4 xb = pack_bf16x4(xv.x, xv.y, xv.z, xv.w);
+        s += stride;
+        request();
+        // x with K = samples: lane (q, c) takes feature c of samples 4q + r (c < 8; the other
+        // columns of dW1 are not used)
+        bf16x4 xn;
+        {
+            const uint2 xp = __builtin_bit_cast(uint2, xb);
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const int i = mt * 16 + 4 * q + r, k = nt * 16 + r16;
-                const float a1 = bf2f(S.f.a1[i][k]);
-                S.dz1[i][k] = f2bf(acc[r] * (1.f - a1 * a1));
+                const int from = 4 * q + r + ((c >> 2) & 1) * 16;
+                const unsigned lo = __shfl(xp.x, from), hi = __shfl(xp.y, from);
+                const unsigned v = (c & 2) ? hi : lo;
+                xn[r] = (short)((c & 1) ? (v >> 16) : v);
             }
         }
-    wave_sync();
-    // gb1[j] = sum_i dz1[i][j]; gW1[j][f] = sum_i dz1[i][j] x[i][f] (M = j, K = i, N = f)
-    {
-        float gb1 = 0.f;
-        for (int i = 0; i < 64; i++) gb1 += bf2f(S.dz1[i][lane]);
-        g[P_B1 + lane] = gb1;
+        // layer 1
+        bf16x4 a1t[4], a1n[4];
+#pragma unroll
         for (int mt = 0; mt < 4; mt++) {
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+            const float4 b = *reinterpret_cast<const float4 *>(&sb1[mt * 16 + 4 * q]);
+            const f32x4 dt = mfma16(w1[mt], xb, f32x4{0.f, 0.f, 0.f, 0.f});
+            const f32x4 dn = mfma16(xb, w1[mt], f32x4{0.f, 0.f, 0.f, 0.f});
+            const float bt[4] = {b.x, b.y, b.z, b.w};
+            a1t[mt] = pack_bf16x4(tanh_fast(dt[0] + bt[0]), tanh_fast(dt[1] + bt[1]), tanh_fast(dt[2] + bt[2]),
+                                  tanh_fast(dt[3] + bt[3]));
+            a1n[mt] = pack_bf16x4(tanh_fast(dn[0] + b1n[mt]), tanh_fast(dn[1] + b1n[mt]), tanh_fast(dn[2] + b1n[mt]),
+                                  tanh_fast(dn[3] + b1n[mt]));
+        }
+        // layer 2 (T): the output, then dz2 = dy w3 (1 - a2^2)
+        float a2t[4][4], w3t[4][4];
+        float y = 0.f;
 #pragma unroll
-            for (int kt = 0; kt < 4; kt++) {
-                bf16x4 a, b;
-                const int i0 = kt * 16 + 4 * q;
+        for (int mt = 0; mt < 4; mt++) {
+            f32x4 d = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int u = 0; u < 4; u++) {
-                    a[u] = (short)S.dz1[i0 + u][mt * 16 + r16];
-                    b[u] = (short)S.f.x[i0 + u][r16];
-                }
-                acc = mfma16(a, b, acc);
+            for (int kt = 0; kt < 4; kt++) d = mfma16(w2[mt][kt], a1t[kt], d);
+            const float4 b = *reinterpret_cast<const float4 *>(&sb2[mt * 16 + 4 * q]);
+            const float4 v = *reinterpret_cast<const float4 *>(&sw3[mt * 16 + 4 * q]);
+            const float bt[4] = {b.x, b.y, b.z, b.w}, vt[4] = {v.x, v.y, v.z, v.w};
+            const bf16x4 a2 = pack_bf16x4(tanh_fast(d[0] + bt[0]), tanh_fast(d[1] + bt[1]), tanh_fast(d[2] + bt[2]),
+                                          tanh_fast(d[3] + bt[3]));
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                a2t[mt][r] = bf2f((unsigned short)a2[r]);
+                w3t[mt][r] = vt[r];
+                y += a2t[mt][r] * vt[r];
             }
+        }
+        y += __shfl_xor(y, 16);
+        y += __shfl_xor(y, 32);
+        y += b3;
+        const float e = valid ? y - t : 0.f;
+        const float dy = e * inv_nb;
+        if (q == 0) {
+            loss += 0.5f * e * e;
+            gb3 += dy;
+        }
+        bf16x4 dz2t[4];
 #pragma unroll
-            for (int r = 0; r < 4; r++)
-                if (r16 < MLP_IN) g[P_W1 + (mt * 16 + 4 * q + r) * MLP_IN + r16] = acc[r];
+        for (int mt = 0; mt < 4; mt++) {
+            float z[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) z[r] = dy * w3t[mt][r] * (1.f - a2t[mt][r] * a2t[mt][r]);
+            dz2t[mt] = pack_bf16x4(z[0], z[1], z[2], z[3]);
+        }
+        float dyn[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) dyn[r] = __shfl(dy, 4 * q + r);
+        // layer 2 (N): dW3, db2, dW2
+#pragma unroll
+        for (int mt = 0; mt < 4; mt++) {
+            f32x4 d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int kt = 0; kt < 4; kt++) d = mfma16(a1t[kt], w2[mt][kt], d);
+            const bf16x4 a2 = pack_bf16x4(tanh_fast(d[0] + b2n[mt]), tanh_fast(d[1] + b2n[mt]),
+                                          tanh_fast(d[2] + b2n[mt]), tanh_fast(d[3] + b2n[mt]));
+            float z[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const float a = bf2f((unsigned short)a2[r]);
+                gw3[mt] += dyn[r] * a;
+                z[r] = dyn[r] * w3n[mt] * (1.f - a * a);
+            }
+            const bf16x4 dz = pack_bf16x4(z[0], z[1], z[2], z[3]);
+#pragma unroll
+            for (int r = 0; r < 4; r++) gb2[mt] += bf2f((unsigned short)dz[r]);
+#pragma unroll
+            for (int nt = 0; nt < 4; nt++) gw2[mt][nt] = mfma16(dz, a1n[nt], gw2[mt][nt]);
+        }
+        // dA1 = dz2 W2 (N), dz1 = dA1 (1 - a1^2): db1, dW1
+#pragma unroll
+        for (int nt = 0; nt < 4; nt++) {
+            f32x4 d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int kt = 0; kt < 4; kt++) d = mfma16(dz2t[kt], w2t[kt][nt], d);
+            float z[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const float a = bf2f((unsigned short)a1n[nt][r]);
+                z[r] = d[r] * (1.f - a * a);
+            }
+            const bf16x4 dz = pack_bf16x4(z[0], z[1], z[2], z[3]);
+#pragma unroll
+            for (int r = 0; r < 4; r++) gb1[nt] += bf2f((unsigned short)dz[r]);
+            gw1[nt] = mfma16(dz, xn, gw1[nt]);
         }
     }
+    // the per-lane sums over the wave
+#pragma unroll
+    for (int mt = 0; mt < 4; mt++) {
+        gw3[mt] += __shfl_xor(gw3[mt], 16);
+        gw3[mt] += __shfl_xor(gw3[mt], 32);
+        gb2[mt] += __shfl_xor(gb2[mt], 16);
+        gb2[mt] += __shfl_xor(gb2[mt], 32);
+        gb1[mt] += __shfl_xor(gb1[mt], 16);
+        gb1[mt] += __shfl_xor(gb1[mt], 32);
+    }
+    gb3 = wave_sum(gb3);
+    loss = wave_sum(loss);
+    // the block's sum (w0 + w2) + (w1 + w3), through LDS: waves 2 and 3 put their sums, waves 0
+    // and 1 add theirs (each only touches its own lanes' places)
+    auto put4 = [&](int i, const f32x4 &v) {
+        f32x4 &b = *reinterpret_cast<f32x4 *>(&buf[w & 1][i]);
+        b = w >= 2 ? v : v + b;
+    };
+    auto put1 = [&](int i, float v) { buf[w & 1][i] = w >= 2 ? v : v + buf[w & 1][i]; };
+    auto put_all = [&]() {
+#pragma unroll
+        for (int mt = 0; mt < 4; mt++) {
+#pragma unroll
+            for (int nt = 0; nt < 4; nt++) put4(((mt * 4 + nt) * 64 + lane) * 4, gw2[mt][nt]);
+            put4(G_W1 + (mt * 64 + lane) * 4, gw1[mt]);
+            if (q == 0) {
+                put1(G_W3 + mt * 16 + c, gw3[mt]);
+                put1(G_B2 + mt * 16 + c, gb2[mt]);
+                put1(G_B1 + mt * 16 + c, gb1[mt]);
+            }
+        }
+        if (lane == 0) {
+            put1(G_B3, gb3);
+            put1(G_LOSS, loss);
+        }
+    };
+    if (w >= 2) put_all();
+    __syncthreads();
+    if (w < 2) put_all();
+    __syncthreads();
+    f32x4 *g = reinterpret_cast<f32x4 *>(partial + (int64_t)blockIdx.x * MLP_ROW);
+    for (int i = threadIdx.x; i < (G_LOSS + 4) / 4; i += 64 * MLP_TR_WAVES)
+        g[i] = reinterpret_cast<const f32x4 *>(buf[0])[i] + reinterpret_cast<const f32x4 *>(buf[1])[i];
 }
 
-// fold per-wave partials in a fixed order (deterministic), in two levels: chunks of
-// MLP_RED_CHUNK waves in parallel (stage 1), then the chunk sums (stage 2);
-// loss = mean of 0.5 (y - t)^2
-#define MLP_RED_CHUNK 32
-__global__ __launch_bounds__(256) void k_mlp_reduce1(int nw, const float *__restrict__ partial,
-                                                     const float *__restrict__ loss_partial,
-                                                     float *__restrict__ part2, float *__restrict__ loss2) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    const int w0 = blockIdx.y * MLP_RED_CHUNK;
-    const int w1 = w0 + MLP_RED_CHUNK < nw ? w0 + MLP_RED_CHUNK : nw;
-    if (p < MLP_NPARAM) {
-        float s = 0.f;
-        for (int w = w0; w < w1; w++) s += partial[(int64_t)w * MLP_NPARAM + p];
-        part2[(int64_t)blockIdx.y * MLP_NPARAM + p] = s;
+// Folds the blocks' partials in a fixed order (deterministic) -- 16 wavefronts take every 16th
+// partial, then their sums in wavefront order -- and, with ADAM, updates the FP32 master weights
+// (beta1 0.9, beta2 0.999, eps 1e-8) in the same launch; loss = mean of 0.5 (y - t)^2.
+#define MLP_RED_WAVES 16
+template <bool ADAM>
+__global__ __launch_bounds__(64 * MLP_RED_WAVES) void k_mlp_reduce(int nblk, int64_t nb,
+                                                                  const float *__restrict__ partial,
+                                                                  float *__restrict__ grad, float *__restrict__ loss,
+                                                                  float *__restrict__ params, float *__restrict__ m1,
+                                                                  float *__restrict__ m2,
+                                                                  unsigned short *__restrict__ frag, float lr,
+                                                                  float bc1, float bc2) {
+    __shared__ float sum[MLP_RED_WAVES][64];
+    const int w = threadIdx.x / 64, lane = wave_lane();
+    const int i = blockIdx.x * 64 + lane;   // < MLP_ROW
+    float s = 0.f;
+#pragma unroll 8
+    for (int b = w; b < nblk; b += MLP_RED_WAVES) s += partial[(int64_t)b * MLP_ROW + i];
+    sum[w][lane] = s;
+    __syncthreads();
+    if (w != 0) return;
+    s = sum[0][lane];
+#pragma unroll
+    for (int v = 1; v < MLP_RED_WAVES; v++) s += sum[v][lane];
+    if (i == G_LOSS) *loss = s / (float)nb;
+    const int p = mlp_param_of(i);
+    if (p < 0) return;
+    grad[p] = s;
+    if (ADAM) {
+        const float a = 0.9f * m1[p] + 0.1f * s;
+        const float b = 0.999f * m2[p] + 0.001f * s * s;
+        m1[p] = a;
+        m2[p] = b;
+        const float v = params[p] - lr * (a / bc1) / (sqrtf(b / bc2) + 1e-8f);
+        params[p] = v;
+        put_frag(frag, p, v);
     }
-    if (p == 0) {
-        float s = 0.f;
-        for (int w = w0; w < w1; w++) s += loss_partial[w];
-        loss2[blockIdx.y] = s;
-    }
-}
-
-__global__ __launch_bounds__(256) void k_mlp_reduce2(int nchunks, int64_t nb, const float *__restrict__ part2,
-                                                     const float *__restrict__ loss2, float *__restrict__ grad,
-                                                     float *__restrict__ loss) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p < MLP_NPARAM) {
-        float s = 0.f;
-        for (int c = 0; c < nchunks; c++) s += part2[(int64_t)c * MLP_NPARAM + p];
-        grad[p] = s;
-    }
-    if (p == 0) {
-        float s = 0.f;
-        for (int c = 0; c < nchunks; c++) s += loss2[c];
-        *loss = s / (float)nb;
-    }
-}
-
-// Adam (beta1 0.9, beta2 0.999, eps 1e-8) on the FP32 master weights
-__global__ __launch_bounds__(256) void k_mlp_adam(float *__restrict__ params, float *__restrict__ m1,
-                                                  float *__restrict__ m2, const float *__restrict__ grad,
-                                                  float lr, float bc1, float bc2) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= MLP_NPARAM) return;
-    const float gg = grad[p];
-    const float a = 0.9f * m1[p] + 0.1f * gg;
-    const float b = 0.999f * m2[p] + 0.001f * gg * gg;
-    m1[p] = a;
-    m2[p] = b;
-    params[p] -= lr * (a / bc1) / (sqrtf(b / bc2) + 1e-8f);
 }
 
 // ------------------------------------------------------------------------------------
@@ -497,37 +582,38 @@ void launch_mlp_forward_raw(mhpc_ctx *c, int64_t n, const float *X, float *Y) {
                        c->mlp_params, Y);
 }
 
-// one gradient evaluation over nb samples (X, T or X[idx], T[idx]); grad and loss on the device
-void launch_mlp_gradient(mhpc_ctx *c, int64_t nb, const float *X, const float *T, const int32_t *idx,
-                         float *grad, float *loss) {
-    const int64_t nw = ceil_div(nb, 64);
-    hipLaunchKernelGGL(k_mlp_train_grad, dim3((unsigned)ceil_div(nw, MLP_TR_WAVES)), dim3(64 * MLP_TR_WAVES), 0,
-                       c->stream, nb, X, T, idx, c->mlp_params, c->mlp_partial, c->mlp_loss_partial);
-    // stage-1 sums go behind the per-wave partials in the same buffer (sized for the
-    // maximum wave count plus its chunk sums)
-    const int nchunks = (int)ceil_div(nw, MLP_RED_CHUNK);
-    float *part2 = c->mlp_partial + (int64_t)c->mlp_max_waves * MLP_NPARAM;
-    float *loss2 = c->mlp_loss_partial + c->mlp_max_waves;
-    hipLaunchKernelGGL(k_mlp_reduce1, dim3((unsigned)ceil_div(MLP_NPARAM, 256), (unsigned)nchunks), dim3(256), 0,
-                       c->stream, (int)nw, c->mlp_partial, c->mlp_loss_partial, part2, loss2);
-    hipLaunchKernelGGL(k_mlp_reduce2, dim3((unsigned)ceil_div(MLP_NPARAM, 256)), dim3(256), 0, c->stream, nchunks,
-                       nb, part2, loss2, grad, loss);
+static unsigned mlp_train_blocks(int64_t nb) {
+    return (unsigned)std::min<int64_t>(ceil_div(nb, 16 * MLP_TR_WAVES), MLP_TR_BLOCKS);
 }
 
-void launch_mlp_adam(mhpc_ctx *c, float lr, int step) {
+// the training kernel's weight fragments from the master weights
+void launch_mlp_frag(mhpc_ctx *c) {
+    hipLaunchKernelGGL(k_mlp_frag, dim3((unsigned)ceil_div(MLP_NPARAM, 256)), dim3(256), 0, c->stream,
+                       c->mlp_params, c->mlp_frag);
+}
+
+// one gradient evaluation over the nb pairs (X, T); grad and loss on the device
+void launch_mlp_gradient(mhpc_ctx *c, int64_t nb, const float *X, const float *T, float *grad, float *loss) {
+    const unsigned blocks = mlp_train_blocks(nb);
+    hipLaunchKernelGGL(k_mlp_train_grad<false>, dim3(blocks), dim3(64 * MLP_TR_WAVES), 0, c->stream, nb, nb,
+                       (uint64_t)0, X, T, c->mlp_params, reinterpret_cast<const bf16x4 *>(c->mlp_frag), c->mlp_partial);
+    hipLaunchKernelGGL(k_mlp_reduce<false>, dim3(MLP_ROW / 64), dim3(64 * MLP_RED_WAVES), 0, c->stream, (int)blocks,
+                       nb, c->mlp_partial, grad, loss, nullptr, nullptr, nullptr, nullptr, 0.f, 1.f, 1.f);
+}
+
+// one Adam step on nsamples random pairs of the context's features and targets
+void launch_mlp_train_step(mhpc_ctx *c, int64_t nsamples, uint64_t seed, float lr, int step) {
+    const unsigned blocks = mlp_train_blocks(nsamples);
     const float bc1 = 1.f - powf(0.9f, (float)step), bc2 = 1.f - powf(0.999f, (float)step);
-    hipLaunchKernelGGL(k_mlp_adam, dim3((unsigned)ceil_div(MLP_NPARAM, 256)), dim3(256), 0, c->stream,
-                       c->mlp_params, c->mlp_m1, c->mlp_m2, c->mlp_grad, lr, bc1, bc2);
+    hipLaunchKernelGGL(k_mlp_train_grad<true>, dim3(blocks), dim3(64 * MLP_TR_WAVES), 0, c->stream, nsamples, c->n,
+                       seed, c->mlp_x, c->mlp_t, c->mlp_params, reinterpret_cast<const bf16x4 *>(c->mlp_frag),
+                       c->mlp_partial);
+    hipLaunchKernelGGL(k_mlp_reduce<true>, dim3(MLP_ROW / 64), dim3(64 * MLP_RED_WAVES), 0, c->stream, (int)blocks,
+                       nsamples, c->mlp_partial, c->mlp_grad, c->mlp_loss, c->mlp_params, c->mlp_m1, c->mlp_m2,
+                       c->mlp_frag, lr, bc1, bc2);
 }
 
-// training targets: random sample indices (hash of seed and slot) and
-// T = (log(sml / h_previous) - mu_t) / sigma_t for every particle
-__device__ __forceinline__ uint64_t mix64(uint64_t z) {
-    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
-    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
-    return z ^ (z >> 31);
-}
-
+// training targets: T = (log(sml / h_previous) - mu_t) / sigma_t for every particle
 __global__ __launch_bounds__(256) void k_mlp_targets(int64_t n, const double *__restrict__ h,
                                                      const double *__restrict__ hprev,
                                                      const float *__restrict__ norm, float *__restrict__ T) {
@@ -535,18 +621,8 @@ __global__ __launch_bounds__(256) void k_mlp_targets(int64_t n, const double *__
     if (i < n) T[i] = (float)((log(h[i] / hprev[i]) - norm[16]) / norm[17]);
 }
 
-__global__ __launch_bounds__(256) void k_mlp_sample(int64_t n, int64_t ns, uint64_t seed, int32_t *__restrict__ idx) {
-    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (i < ns) idx[i] = (int32_t)(mix64(seed * 0x9E3779B97F4A7C15ull + (uint64_t)i) % (uint64_t)n);
-}
-
 void launch_mlp_targets(mhpc_ctx *c) {
     if (c->n <= 0) return;
     hipLaunchKernelGGL(k_mlp_targets, dim3((unsigned)ceil_div(c->n, 256)), dim3(256), 0, c->stream, c->n,
                        c->f[MHPC_F_SML], c->mlp_hprev, c->mlp_norm, c->mlp_t);
-}
-
-void launch_mlp_sample(mhpc_ctx *c, int64_t nsamples, uint64_t seed) {
-    hipLaunchKernelGGL(k_mlp_sample, dim3((unsigned)ceil_div(nsamples, 256)), dim3(256), 0, c->stream, c->n,
-                       nsamples, seed, c->mlp_idx);
 }

@@ -157,11 +157,10 @@ struct mhpc_ctx {
     float *mlp_x = nullptr;                      // [cap][8]
     float *mlp_t = nullptr;                      // [cap] targets
     double *mlp_hprev = nullptr;                 // [cap]
-    int32_t *mlp_idx = nullptr;                  // [max samples]
-    float *mlp_partial = nullptr, *mlp_loss_partial = nullptr, *mlp_loss = nullptr;
+    float *mlp_partial = nullptr, *mlp_loss = nullptr;   // per-block gradient partials; the loss
+    unsigned short *mlp_frag = nullptr;          // BF16 weights in the training kernel's lane order
     float *mlp_io_x = nullptr, *mlp_io_y = nullptr;   // test-hook staging
     int64_t mlp_io_cap = 0;
-    int64_t mlp_max_waves = 0;                   // per-wave gradient partials allocated
     int mlp_adam_step = 0;
     bool mlp_x_valid = false, mlp_norm_set = false;
     double *box = nullptr;                       // [6]
@@ -223,11 +222,12 @@ int mlp_num_params();
 void launch_mlp_features(mhpc_ctx *c, double dt);
 void launch_mlp_predict(mhpc_ctx *c);
 void launch_mlp_forward_raw(mhpc_ctx *c, int64_t n, const float *X, float *Y);
-void launch_mlp_gradient(mhpc_ctx *c, int64_t nb, const float *X, const float *T, const int32_t *idx,
-                         float *grad, float *loss);
-void launch_mlp_adam(mhpc_ctx *c, float lr, int step);
+int64_t mlp_partial_size();
+int64_t mlp_frag_size();
+void launch_mlp_frag(mhpc_ctx *c);
+void launch_mlp_gradient(mhpc_ctx *c, int64_t nb, const float *X, const float *T, float *grad, float *loss);
+void launch_mlp_train_step(mhpc_ctx *c, int64_t nsamples, uint64_t seed, float lr, int step);
 void launch_mlp_targets(mhpc_ctx *c);
-void launch_mlp_sample(mhpc_ctx *c, int64_t nsamples, uint64_t seed);
 void launch_mlp_renorm(mhpc_ctx *c);
 int pc_backup_fields();
 // The CFL time-step rule of setTimeStep (device_predictor_corrector_euler.cu:315-540) from the

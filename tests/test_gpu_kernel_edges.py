@@ -1,0 +1,167 @@
+"""Edges of the kernels that choose their work split by size: tile remainders, the smallest and the
+first size past each split, against the oracle or a plain restatement."""
+import numpy as np
+import pytest
+
+from miluphpc_amd import ics
+from conftest import print_case
+
+pytestmark = pytest.mark.gpu
+
+
+def load_ctx(lib, s, params):
+    ctx = lib.Context(len(s["x"]), params)
+    ctx.load(**{k: v for k, v in s.items() if k in lib.FIELD_ID})
+    return ctx
+
+
+def mlp_inputs(seed, n):
+    rng = np.random.default_rng(seed)
+    p = (rng.uniform(-1, 1, 4801) * 0.3).astype(np.float32)
+    X = rng.normal(size=(n, 8)).astype(np.float32)
+    X[:, 7] = 0.0
+    return p, X, rng.normal(size=n).astype(np.float32)
+
+
+@pytest.mark.parametrize("n", [1, 15, 17, 65, 16384, 16385, 40000])
+def test_mlp_gradient_is_the_sum_over_its_samples(gpu_lib, n):
+    """The gradient of n samples is the mean of the gradients of its parts: the first and the rest,
+    which split over wavefronts, blocks (256 x 64 samples fill one step) and steps differently.
+    Every sample's terms are the same BF16 products in both, scaled by a power of two at most
+    apart in dy before rounding; the sums are FP32, so parts and whole differ by BF16 roundings of
+    dz (2^-9 each, random) and FP32 sums."""
+    print_case(f"mlp gradient parts n={n}")
+    p, X, T = mlp_inputs(n, n)
+    with gpu_lib.Context(64) as ctx:
+        ctx.mlp_set_params(p)
+        g, loss = ctx.mlp_gradient(X, T)
+        g2, loss2 = ctx.mlp_gradient(X, T)
+        assert np.array_equal(g, g2) and loss == loss2   # deterministic
+        if n > 1:
+            k = max(1, n // 3)
+            ga, la = ctx.mlp_gradient(X[:k], T[:k])
+            gb, lb = ctx.mlp_gradient(X[k:], T[k:])
+            both = (k * ga.astype(np.float64) + (n - k) * gb) / n
+            assert loss == pytest.approx((k * la + (n - k) * lb) / n, rel=1e-4)
+            assert np.linalg.norm(g - both) <= 1e-2 * np.linalg.norm(both)
+    assert np.all(g[:512].reshape(64, 8)[:, 7] == 0.0)   # the padding input
+
+
+@pytest.mark.parametrize("nsamples", [1, 100, 16500])
+def test_mlp_train_step_is_adam_on_the_sampled_gradient(gpu_lib, nsamples):
+    """One training step equals Adam (its first step) on the gradient of the sampled pairs."""
+    print_case(f"mlp train step nsamples={nsamples}")
+    s = ics.sedov_lattice(12)
+    lr, seed = 1e-3, 5
+    flags = gpu_lib.RHS_SPH | gpu_lib.RHS_VARIABLE_SML | gpu_lib.RHS_FEATURES
+    with load_ctx(gpu_lib, s, ics.params_sedov()) as ctx:
+        n = ctx.n
+        ctx.mlp_init(3)
+        norm = np.zeros(18, np.float32)
+        norm[:7] = [-1.0, 1.0, 0.0, 0.0, 0.0, 0.0, 0.0]
+        norm[8:15] = 1.0
+        norm[17] = 0.1
+        ctx.mlp_set_norm(norm)
+        h0 = ctx.download("sml")
+        ctx.rhs(flags)
+        X, h1 = ctx.mlp_download_features(), ctx.download("sml")
+        T = (np.log(h1 / h0) / np.float64(norm[17])).astype(np.float32)
+        M = (1 << 64) - 1
+
+        def mix(z):
+            z = ((z ^ (z >> 30)) * 0xBF58476D1CE4E5B9) & M
+            z = ((z ^ (z >> 27)) * 0x94D049BB133111EB) & M
+            return z ^ (z >> 31)
+
+        idx = np.array([mix((seed * 0x9E3779B97F4A7C15 + i) & M) % n for i in range(nsamples)])
+        p0 = ctx.mlp_get_params()
+        g, loss_g = ctx.mlp_gradient(X[idx], T[idx])
+        loss = ctx.mlp_train(nsamples=nsamples, iters=1, lr=lr, seed=seed)
+        p1 = ctx.mlp_get_params()
+    assert loss == pytest.approx(loss_g, rel=1e-6)
+    g = g.astype(np.float64)
+    # the first step with the FP32 bias corrections; a dozen FP32 roundings of it, and one of p.
+    # Below |g| = 1e-6 the step is not saturated and follows the rounding of g itself
+    f32 = np.float32
+    bc1, bc2 = float(f32(1) - f32(0.9)), float(f32(1) - f32(0.999))
+    step = lr * (float(f32(0.1)) * g / bc1) / (np.sqrt(float(f32(0.001)) * g * g / bc2) + 1e-8)
+    sure = (np.abs(g) > 1e-6) | (g == 0.0)
+    assert sure.mean() > 0.5
+    assert np.abs((p1 - p0.astype(np.float64)) + step)[sure].max() <= 12 * 2.0 ** -24 * lr + 2.0 ** -24 * np.abs(p0).max()
+
+
+@pytest.mark.parametrize("n", [1000, 1025, 300000])
+def test_diagnostics_of_ragged_counts(gpu_lib, n):
+    """Global sums of counts around the block split (1024 per block; more than one particle per
+    thread above 262,144), every term's exact sum in extended precision to FP64 rounding."""
+    print_case(f"diagnostics n={n}")
+    rng = np.random.default_rng(n)
+    f = {k: rng.normal(size=n) + 0.5 for k in ("x", "y", "z", "vx", "vy", "vz")}
+    f.update(mass=rng.uniform(0.5, 1.5, n), e=rng.uniform(0, 1, n))
+    with gpu_lib.Context(n) as ctx:
+        ctx.load(**f)
+        ctx.upload("u", -f["mass"])
+        d = ctx.diagnostics()
+    L = {k: v.astype(np.longdouble) for k, v in f.items()}
+    m = L["mass"]
+    # each term takes at most 6 roundings before the compensated sum's one or two
+    checks = [("mass", d["mass"], m), ("potential", d["potential"], -m), ("internal", d["internal"], m * L["e"]),
+              ("kinetic", d["kinetic"], 0.5 * m * (L["vx"] ** 2 + L["vy"] ** 2 + L["vz"] ** 2))]
+    checks += [(f"momentum {a}", d["momentum"][a], m * L[t]) for a, t in enumerate(("vx", "vy", "vz"))]
+    for name, got, terms in checks:
+        assert abs(got - float(terms.sum())) <= 8 * 2.0 ** -53 * float(np.abs(terms).sum()), name
+
+
+@pytest.mark.parametrize("quad,precision", [(0, 0), (1, 0), (0, 1), (1, 1)])
+@pytest.mark.parametrize("vote", [0, 1])
+@pytest.mark.parametrize("n", [70, 2100, 33000])
+def test_barnes_hut_shared_groups(gpu_lib, orc, n, vote, quad, precision):
+    """Groups shared by several wavefronts (8 below 512 groups without quadrupole, else 4) give the
+    oracle walk's interactions and forces, with and without softening, with potential."""
+    print_case(f"shared groups n={n} vote={vote} quad={quad} precision={precision}")
+    s = ics.plummer(n, seed=n)
+    for eps2 in (1e-6, 0.0):
+        p = gpu_lib.default_params(theta=0.6, smoothing=eps2, curve=1, quadrupole=quad, bh_accept=vote,
+                                   precision=precision)
+        with load_ctx(gpu_lib, s, p) as ctx:
+            st = ctx.rhs(gpu_lib.RHS_GRAVITY | gpu_lib.RHS_POTENTIAL)
+            g = np.stack([ctx.download(k) for k in ("g_ax", "g_ay", "g_az")])
+            u = ctx.download("u")
+        o = orc.gravity_rhs(s, 0.6, eps2, curve=1, quad=bool(quad), vote=bool(vote), potential=True)
+        assert st["n_cell_interactions"] == o["n_cell"] and st["n_part_interactions"] == o["n_part"]
+        go = np.stack([o["ax"], o["ay"], o["az"]])
+        uo = 0.5 * s["mass"] * o["phi"]
+        size = np.sqrt((go ** 2).sum(0))
+        err = np.sqrt(((g - go) ** 2).sum(0)) / np.maximum(size, np.sqrt((size ** 2).mean()))
+        if precision == 0:
+            tol = 1e-12 if not quad else 2e-7   # quadrupoles are stored in FP32
+            assert err.max() <= tol
+            assert np.abs(u - uo).max() <= tol * np.abs(uo).max()
+        else:
+            assert np.percentile(err, 99) < 1e-5
+            assert np.percentile(np.abs(u / uo - 1.0), 99) < 1e-5
+
+
+@pytest.mark.parametrize("side", [25, 33])
+@pytest.mark.parametrize("curve", [0, 1])
+def test_neighbours_of_groups_that_straddle_a_curve_jump(gpu_lib, orc, side, curve):
+    """On lattices whose side is no power of two some runs of 64 Lebesgue keys span the domain; the
+    walks split them.  Lists, h and counts equal the oracle's, in both list structures."""
+    print_case(f"split groups side={side} curve={curve}")
+    s = ics.sedov_lattice(side)
+    rng = np.random.default_rng(side)
+    for k in "xyz":
+        s[k] = s[k] + rng.uniform(-0.02, 0.02, side ** 3) / side
+    s["sml"] = s["sml"] * rng.uniform(0.95, 1.05, side ** 3)   # some particles change h
+    p = ics.params_sedov(curve=curve, sml_max=4.0 * float(s["sml"].max()))
+    o = orc.sph_rhs(s, sml_max=p.sml_max)
+    for spec in (0, gpu_lib.RHS_SPECULATIVE_NN):
+        with load_ctx(gpu_lib, s, p) as ctx:
+            ctx.rhs(gpu_lib.RHS_SPH | gpu_lib.RHS_VARIABLE_SML | spec)
+            nnl, noi = ctx.neighbour_lists(180)
+            h, rho = ctx.download("sml"), ctx.download("rho")
+        assert np.array_equal(h, o["sml"])
+        assert np.array_equal(noi, o["noi"])
+        assert np.max(np.abs(rho / o["rho"] - 1.0)) <= 1e-12
+        used = np.arange(180) < noi[:, None]
+        assert np.array_equal(np.sort(np.where(used, nnl, -1), 1), np.sort(np.where(used, o["nnl"], -1), 1))
