@@ -8,6 +8,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <algorithm>
 #include <vector>
 
 #include "mhpc_internal.h"
@@ -198,7 +199,8 @@ static int create_impl(mhpc_ctx *c, int64_t cap, int64_t cap_cells) {
     HIPC(dalloc(&c->nn_start, nn_tab_off(c->nn_kmax + 1)));
     HIPC(dalloc(&c->nn_start_rng, nn_tab_off(c->nn_kmax + 1)));
     HIPC(dalloc(&c->lcp, cap));
-    c->tree_tiles_cap = ceil_div(cap, MHPC_TREE_TILE);
+    c->tree_tiles_cap = std::max<int64_t>(ceil_div(cap, MHPC_TREE_TILE),
+                                          std::min<int64_t>(ceil_div(cap, 256), MHPC_TREE_SMALL_TILES));
     HIPC(dalloc(&c->tcnt, (MHPC_LEVELS + 1) * c->tree_tiles_cap));
     HIPC(dalloc(&c->toff, (MHPC_LEVELS + 1) * c->tree_tiles_cap));
     HIPC(dalloc(&c->level_count, MHPC_LEVELS + 2));

@@ -10,6 +10,9 @@
 //              = lanes holding the same digit), the block stages the tile in LDS in
 //              digit order and writes each digit run contiguously.
 // HBM bytes per pass: count reads 8 B/key, scatter reads 12 and writes 12.
+//
+// Small sets are sorted by rank instead (k_sort_rank, k_sort_merge): a key's place is the number
+// of keys before it, counted directly, which is one or two launches and no host wait.
 #include <mutex>
 
 #include "mhpc_internal.h"
@@ -160,6 +163,109 @@ __global__ __launch_bounds__(SORT_BLOCK) void k_sort_scatter(const uint64_t *__r
     }
 }
 
+// ------------------------------------------------------------------------------------
+// Sort by rank.  A workgroup takes 64 keys of a tile of T keys (each lane one, the same in every
+// wavefront); its 16 wavefronts count, each over a sixteenth of the tile, the keys that come
+// before the lane's: smaller ones, and equal ones at smaller positions (a stable sort).  The
+// tile's keys are wave-uniform, so they come through scalar loads, and a comparison is two or
+// three instructions.  Writes each tile in sorted order.
+//
+// One tile (n <= SORT_RANK_MAX): the whole sort, one launch instead of 14 to 26 and the host's
+// check of a partial sort (2048 keys: 9 us, the radix passes 85 us with their launches).
+// Several tiles (n <= SORT_MERGE_MAX): k_sort_merge follows.  65,536 keys: 20 + 18 us against 121 us
+// of radix passes; at 103,823 keys 33 + 44 us against 75 us of partial passes, so the line lies there.
+#define SORT_RANK_WAVES 16
+#define SORT_RANK_MAX 8192
+#define SORT_RANK_TILE 2048
+#define SORT_MERGE_MAX 98304
+
+__global__ __launch_bounds__(64 * SORT_RANK_WAVES) void k_sort_rank(const uint64_t *__restrict__ keys, int n, int T,
+                                                                   uint64_t *__restrict__ kout,
+                                                                   int32_t *__restrict__ vout) {
+    __shared__ int part[SORT_RANK_WAVES][64];
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = wave_lane();
+    const int base = blockIdx.x * 64;              // T is a multiple of 64: one tile per workgroup
+    const int t0 = base / T * T, t1 = min(t0 + T, n);
+    const int i = base + lane;
+    const uint64_t key = i < n ? keys[i] : 0ull;
+    const int share = (t1 - t0 + SORT_RANK_WAVES - 1) / SORT_RANK_WAVES;
+    const int j0 = min(t0 + w * share, t1), j1 = min(j0 + share, t1);
+    int cnt = 0;
+    const int before = min(max(base, j0), j1);     // [j0, before): positions before the 64
+#pragma unroll 8
+    for (int j = j0; j < before; j++) cnt += keys[j] <= key ? 1 : 0;
+    const int own = min(max(base + 64, j0), j1);   // [before, own): among the 64
+    for (int j = before; j < own; j++) cnt += (keys[j] < key || (keys[j] == key && j < i)) ? 1 : 0;
+#pragma unroll 8
+    for (int j = own; j < j1; j++) cnt += keys[j] < key ? 1 : 0;
+    part[w][lane] = cnt;
+    __syncthreads();
+    if (w != 0 || i >= n) return;
+    int rank = t0;
+#pragma unroll
+    for (int v = 0; v < SORT_RANK_WAVES; v++) rank += part[v][lane];
+    kout[rank] = key;
+    vout[rank] = i;
+}
+
+// The tiles of k_sort_rank merged by rank: a key's place is its position in its own tile plus, by
+// binary search, the keys of every other tile that come before it (equal ones of earlier tiles).
+// A workgroup takes 64 keys, consecutive in their tile, so their searches share cache lines; its
+// 16 wavefronts share the other tiles, up to four each, whose searches are independent chains of
+// loads (one wavefront searching every tile was a chain of 96 load latencies, 64 us for 65,536
+// keys; 18 us).
+static_assert(SORT_MERGE_MAX <= 4 * SORT_RANK_WAVES * SORT_RANK_TILE, "four tiles per wavefront");
+__global__ __launch_bounds__(64 * SORT_RANK_WAVES) void k_sort_merge(const uint64_t *__restrict__ kin,
+                                                                    const int32_t *__restrict__ vin, int n,
+                                                                    uint64_t *__restrict__ kout,
+                                                                    int32_t *__restrict__ vout) {
+    __shared__ int part[SORT_RANK_WAVES][64];
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = wave_lane();
+    const int e = blockIdx.x * 64 + lane;
+    const uint64_t key = e < n ? kin[e] : 0ull;
+    const int own = blockIdx.x / (SORT_RANK_TILE / 64);
+    int cnt = 0;
+    int pos[4] = {0, 0, 0, 0};
+    // does the key at place `at` of this wavefront's tile u come before this one?
+    auto before = [&](int u, int at) {
+        const int t = w + u * SORT_RANK_WAVES, j = t * SORT_RANK_TILE + at;
+        if (t == own || at >= SORT_RANK_TILE || j >= n) return false;
+        const uint64_t k = kin[j];
+        return t < own ? k <= key : k < key;
+    };
+#pragma unroll
+    for (int step = SORT_RANK_TILE / 2; step >= 1; step >>= 1)
+#pragma unroll
+        for (int u = 0; u < 4; u++) pos[u] += before(u, pos[u] + step - 1) ? step : 0;
+    // the steps sum to T - 1: one last key decides whether the whole tile comes before
+#pragma unroll
+    for (int u = 0; u < 4; u++) cnt += pos[u] + (before(u, pos[u]) ? 1 : 0);
+    part[w][lane] = cnt;
+    __syncthreads();
+    if (w != 0 || e >= n) return;
+    int rank = e - own * SORT_RANK_TILE;
+#pragma unroll
+    for (int v = 0; v < SORT_RANK_WAVES; v++) rank += part[v][lane];
+    kout[rank] = key;
+    vout[rank] = vin[e];
+}
+
+// stable sort of n <= SORT_MERGE_MAX keys; keyB / valB: scratch of n elements.  in_place: the
+// outputs may overlap the keys, which the one-launch form would overwrite while they are read.
+static void sort_by_rank(hipStream_t stream, const uint64_t *keys, int64_t n, uint64_t *keyB, int32_t *valB,
+                         uint64_t *kout, int32_t *vout, bool in_place) {
+    const unsigned g = (unsigned)ceil_div(n, 64);
+    if (n <= SORT_RANK_MAX && !in_place) {
+        hipLaunchKernelGGL(k_sort_rank, dim3(g), dim3(64 * SORT_RANK_WAVES), 0, stream, keys, (int)n,
+                           (int)(ceil_div(n, 64) * 64), kout, vout);
+        return;
+    }
+    hipLaunchKernelGGL(k_sort_rank, dim3(g), dim3(64 * SORT_RANK_WAVES), 0, stream, keys, (int)n, SORT_RANK_TILE, keyB,
+                       valB);
+    hipLaunchKernelGGL(k_sort_merge, dim3(g), dim3(64 * SORT_RANK_WAVES), 0, stream, keyB, valB, (int)n, kout,
+                       vout);
+}
+
 // the buffers of the LSD passes: input keys (values = positions), the even passes' outputs,
 // the odd passes' outputs (the last pass's, so the result) and the per-pass tables
 struct SortBufs {
@@ -192,6 +298,10 @@ __global__ __launch_bounds__(256) void k_sort_check(const uint64_t *__restrict__
 void launch_sort(mhpc_ctx *c) {
     const int64_t n = c->n;
     if (n <= 0) return;
+    if (n <= SORT_MERGE_MAX) {
+        sort_by_rank(c->stream, c->key, n, c->keyB, c->valB, c->skey, c->perm, false);
+        return;
+    }
     const int64_t ntiles = ceil_div(n, MHPC_SORT_TILE);
     launch_fill_u32(c, c->digit_hist, 0u, MHPC_SORT_PASSES * MHPC_SORT_BUCKETS);
     int hb = (int)(ceil_div(n, SORT_BLOCK * 16) < 1024 ? ceil_div(n, SORT_BLOCK * 16) : 1024);
@@ -279,6 +389,17 @@ extern "C" int mhpc_sort_keys_noalloc(const uint64_t *keys, int64_t n, uint64_t 
     const int st = na_scratch(&ptr);
     if (st != MHPC_OK) return st;
     hipStream_t s = static_cast<hipStream_t>(stream);
+    if (n <= SORT_MERGE_MAX) {
+        const uintptr_t k0 = reinterpret_cast<uintptr_t>(keys), k1 = k0 + sizeof(uint64_t) * (size_t)n;
+        auto overlaps = [&](const void *p, size_t bytes) {
+            const uintptr_t a = reinterpret_cast<uintptr_t>(p);
+            return a < k1 && a + bytes > k0;
+        };
+        sort_by_rank(s, keys, n, reinterpret_cast<uint64_t *>(ptr + NA_KEYB),
+                     reinterpret_cast<int32_t *>(ptr + NA_VALB), sorted_keys, sorted,
+                     overlaps(sorted_keys, sizeof(uint64_t) * (size_t)n) || overlaps(sorted, sizeof(int32_t) * (size_t)n));
+        return hipGetLastError() == hipSuccess ? MHPC_OK : MHPC_E_HIP;
+    }
     uint32_t *digit_hist = reinterpret_cast<uint32_t *>(ptr + NA_DHIST);
     uint32_t *check = reinterpret_cast<uint32_t *>(ptr + NA_CHECK);
     // the digit histogram accumulates with atomics: cleared first (the previous call's counts

@@ -30,6 +30,7 @@
 #define MHPC_SORT_PASSES 8
 #define MHPC_SORT_TILE 2048    // keys per scatter block (256 threads x 8)
 #define MHPC_TREE_TILE 1024     // positions per tree block (256 threads x 4)
+#define MHPC_TREE_SMALL_TILES 1024   // up to this many tiles of 256 positions (256 threads x 1) instead
 #define MHPC_HTABLE_MAX 4096    // h-iteration factor table size
 #define MHPC_MAX_PASSES 64       // upper bound of max_counts
 #define MHPC_NUM_EVENTS 32   // two sets of 16: an RHS, and the second RHS of a fused PC-Euler step

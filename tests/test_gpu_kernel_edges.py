@@ -165,3 +165,74 @@ def test_neighbours_of_groups_that_straddle_a_curve_jump(gpu_lib, orc, side, cur
         assert np.max(np.abs(rho / o["rho"] - 1.0)) <= 1e-12
         used = np.arange(180) < noi[:, None]
         assert np.array_equal(np.sort(np.where(used, nnl, -1), 1), np.sort(np.where(used, o["nnl"], -1), 1))
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 2047, 8192, 8193, 20000, 98304, 98305])
+def test_key_sort_by_rank_edges(gpu_lib, n):
+    """The allocation-free key sort at the edges of its forms (one launch to 8,192 keys, tiles of
+    2,048 merged to 98,304, radix passes above) on full 64-bit keys with ties, the largest key among
+    them, and with the outputs over the inputs: numpy's stable sort."""
+    import ctypes as C
+    print_case(f"key sort n={n}")
+    rng = np.random.default_rng(n)
+    key = rng.integers(0, 1 << 64, n, dtype=np.uint64)
+    key[rng.random(n) < 0.5] &= np.uint64(7)
+    key[rng.random(n) < 0.1] = np.uint64(0xFFFFFFFFFFFFFFFF)
+    order = np.argsort(key, kind="stable")
+    with gpu_lib.Context(64) as ctx:
+        dk, ds, dv = ctx.device_alloc(8 * n), ctx.device_alloc(8 * n), ctx.device_alloc(4 * n)
+        for out in (ds, dk):   # separate, then in place
+            ctx.device_upload(dk, key)
+            st = gpu_lib.LIB.mhpc_sort_keys_noalloc(C.c_void_p(dk), n, C.c_void_p(out), C.c_void_p(dv), None)
+            assert st == gpu_lib.OK
+            assert np.array_equal(ctx.device_download(out, n, np.uint64), key[order])
+            assert np.array_equal(ctx.device_download(dv, n, np.int32), order)
+        for p in (dk, ds, dv):
+            ctx.device_free(p)
+
+
+@pytest.mark.parametrize("curve", [0, 1])
+def test_partial_radix_sort_falls_back(gpu_lib, orc, curve):
+    """Above the rank sort's range a context sorts only the levels its last tree needed, and in full
+    when two particles then share them: both orders are the stable sort's."""
+    print_case(f"partial radix sort, 47^3, curve {curve}")
+    s = ics.sedov_lattice(47)
+    with load_ctx(gpu_lib, s, gpu_lib.default_params(curve=curve)) as ctx:
+        for step in range(3):
+            if step == 2:
+                for c in "xyz":
+                    s[c][1] = s[c][0]
+                ctx.load(x=s["x"], y=s["y"], z=s["z"])
+            box = ctx.bbox()
+            ctx.keys()
+            ctx.sort()
+            perm = ctx.download("sorted")
+            if step < 2:
+                ctx.build_tree()
+                ctx.centres_of_mass()
+            assert np.array_equal(perm, orc.sort(orc.keys(s["x"], s["y"], s["z"], box, curve)))
+
+
+@pytest.mark.parametrize("n", [2, 257, 4096, 4097, 262144, 262145])
+def test_tree_and_com_at_the_tile_and_launch_splits(gpu_lib, orc, n):
+    """Octree and centres of mass bit-exact where the tree's tile (256 or 1024 positions) and the
+    bottom-up pass's launches (one to 4,096 particles) change."""
+    print_case(f"tree n={n}")
+    s = ics.plummer(n, seed=n)
+    with load_ctx(gpu_lib, s, gpu_lib.default_params(quadrupole=1)) as ctx:
+        box = ctx.bbox()
+        ctx.keys()
+        ctx.sort()
+        ctx.build_tree()
+        ctx.centres_of_mass()
+        t = ctx.tree()
+    o = orc.Tree(s["x"], s["y"], s["z"], box)
+    o.com(s["mass"])
+    assert len(t["mass"]) == o.ncells
+    lev = np.asarray(o.level[n:n + o.ncells])
+    assert np.array_equal(np.bincount(t["level"]), np.bincount(lev))
+    # the two number cells differently: compare as sets of (level, mass, centre)
+    nm, nx, ny, nz = (np.asarray(a)[n:n + o.ncells] for a in (o.nm, o.nx, o.ny, o.nz))
+    a = np.array(sorted(zip(t["level"], t["mass"], t["x"], t["y"], t["z"])))
+    b = np.array(sorted(zip(lev, nm, nx, ny, nz)))
+    assert np.array_equal(a, b)
