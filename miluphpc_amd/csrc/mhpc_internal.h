@@ -286,41 +286,88 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Wave reductions and scans on data-parallel-primitive moves and lane-row swaps: each step is one
+// or two VALU instructions, where a general shuffle goes through LDS (a round trip of about a
+// hundred cycles per step, which showed wherever a wavefront waits for its own reduction: the
+// walks' boxes and per-round scans).
+template <int CTRL>
+__device__ __forceinline__ int dpp_mov(int v) {
+    return __builtin_amdgcn_update_dpp(v, v, CTRL, 0xf, 0xf, false);
+}
+#define DPP_XOR1 0xB1          // quad_perm [1, 0, 3, 2]
+#define DPP_XOR2 0x4E          // quad_perm [2, 3, 0, 1]
+#define DPP_HALF_MIRROR 0x141  // lane i of each 8 <-> 7 - i
+#define DPP_MIRROR 0x140       // lane i of each 16 <-> 15 - i
+
+// the partner's value in step S of a butterfly over the wave (0: lane ^ 1, 1: lane ^ 2, 2 and 3:
+// mirrors, which pair the same halves once the smaller groups agree, 4: row ^ 1, 5: row ^ 2); for
+// 4 and 5 `a` and `b` receive both rows' values in every lane
+template <int S>
+__device__ __forceinline__ void wave_pair(unsigned v, unsigned &a, unsigned &b) {
+    if constexpr (S == 0) { a = v; b = (unsigned)dpp_mov<DPP_XOR1>((int)v); }
+    else if constexpr (S == 1) { a = v; b = (unsigned)dpp_mov<DPP_XOR2>((int)v); }
+    else if constexpr (S == 2) { a = v; b = (unsigned)dpp_mov<DPP_HALF_MIRROR>((int)v); }
+    else if constexpr (S == 3) { a = v; b = (unsigned)dpp_mov<DPP_MIRROR>((int)v); }
+    else if constexpr (S == 4) {
+        const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+        a = r[0];
+        b = r[1];
+    } else {
+        const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+        a = r[0];
+        b = r[1];
+    }
+}
+template <int S, typename T, typename Op>
+__device__ __forceinline__ T wave_step(T v, Op op) {
+    if constexpr (sizeof(T) == 4) {
+        unsigned a, b;
+        wave_pair<S>(__builtin_bit_cast(unsigned, v), a, b);
+        return op(__builtin_bit_cast(T, a), __builtin_bit_cast(T, b));
+    } else {
+        static_assert(sizeof(T) == 8, "32- or 64-bit values");
+        const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+        unsigned al, bl, ah, bh;
+        wave_pair<S>((unsigned)u, al, bl);
+        wave_pair<S>((unsigned)(u >> 32), ah, bh);
+        return op(__builtin_bit_cast(T, (unsigned long long)ah << 32 | al),
+                  __builtin_bit_cast(T, (unsigned long long)bh << 32 | bl));
+    }
+}
+// every lane receives the result; all lanes take part
+template <typename T, typename Op>
+__device__ __forceinline__ T wave_reduce(T v, Op op) {
+    v = wave_step<0>(v, op);
+    v = wave_step<1>(v, op);
+    v = wave_step<2>(v, op);
+    v = wave_step<3>(v, op);
+    v = wave_step<4>(v, op);
+    return wave_step<5>(v, op);
+}
+
 template <typename T>
 __device__ __forceinline__ T wave_min(T v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        T w = __shfl_xor(v, o);
-        v = w < v ? w : v;
-    }
-    return v;
+    return wave_reduce(v, [](T a, T b) { return b < a ? b : a; });
 }
 
 template <typename T>
 __device__ __forceinline__ T wave_max(T v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        T w = __shfl_xor(v, o);
-        v = w > v ? w : v;
-    }
-    return v;
+    return wave_reduce(v, [](T a, T b) { return b > a ? b : a; });
 }
 
 template <typename T>
 __device__ __forceinline__ T wave_sum(T v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    return v;
+    return wave_reduce(v, [](T a, T b) { return a + b; });
 }
 
-// inclusive prefix sum over the wave
+// inclusive prefix sum over the wave: within rows of 16 by shifts, then the rows' totals
 __device__ __forceinline__ int wave_incl_scan(int v) {
-    const int l = wave_lane();
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        int w = __shfl_up(v, o);
-        if (l >= o) v += w;
-    }
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);   // row_shr 1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);   // row_shr 2
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);   // row_shr 4
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);   // row_shr 8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // row 0 -> 1, 2 -> 3: last lane
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // rows 0-1 -> 2-3: lane 31
     return v;
 }
 
