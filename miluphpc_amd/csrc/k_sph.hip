@@ -352,6 +352,7 @@ __device__ __forceinline__ int nn_start_push(LdsT &L, const NNArgs &A, double lo
 // part (mod nparts).  Returns false, before any visit, when the box is too large for the
 // table, has more than NN_DRANGES non-empty cells or more than NN_DIRECT_MAX candidates
 // (counted over the whole box, so every part of a split search decides alike).
+static_assert(NN_DRANGES >= (NN_DSPAN + 1) * (NN_DSPAN + 1) * (NN_DSPAN + 1), "boxes are declined by candidates only");
 template <typename LdsT, typename VisitFn>
 __device__ __forceinline__ bool nn_direct(LdsT &L, const NNArgs &A, double lox, double hix, double loy,
                                           double hiy, double loz, double hiz, const NNCore &q, int part,
@@ -1215,6 +1216,100 @@ __global__ __launch_bounds__(256) void k_h_finish(NNArgs A) {
     }
 }
 
+// Particles that keep iterating, collected by one wavefront of a tail pass (lane i holds the i-th)
+// and appended to the next pass's list together: one atomic per 64 instead of one each (atomics
+// on one address serialise), and their cells' bounds raised by 64 lanes at once.
+struct HStay {
+    int32_t k = 0;
+    double h = 0.0;
+    bool raise = false;
+    int n = 0;
+    __device__ __forceinline__ void flush(const NNArgs &A) {
+        if (n == 0) return;
+        const int lane = wave_lane();
+        uint32_t b = 0;
+        if (lane == 0) b = atomicAdd(A.count_out, (uint32_t)n);
+        b = __shfl(b, 0);
+        if (lane < n) {
+            A.list_out[b + lane] = k;
+            if (raise) hmax_raise(A.chmax_raise, A.ppar, A.cpar, A.cap_cells, k, h);
+        }
+        n = 0;
+    }
+};
+
+// the h update of particle k after a count N in a tail pass (all lanes, the same values); the new
+// h goes to the other h array, so every count of the pass sees the h from its start
+__device__ __forceinline__ void h_tail_update(const NNArgs &A, int32_t k, int N, double hi, HStay &stay,
+                                              bool &changed) {
+    double hn;
+    const bool fin = h_update(A, N, hi, hn);
+    if (wave_lane() == 0) {
+        A.iters[k] = A.pass + 1;
+        A.snoi[k] = N;
+        A.h_next[k] = hn;
+        if (fin) A.done[k] = 1;
+    }
+    if (fin) return;
+    // the next pass counts with hn: the cell bounds must cover it (they cover hi)
+    if (wave_lane() == stay.n) {
+        stay.k = k;
+        stay.h = hn;
+        stay.raise = hn != hi;
+    }
+    changed = changed || hn != hi;
+    if (++stay.n == 64) stay.flush(A);
+}
+
+// A whole tail pass in one launch, for sets of at most NN_DIRECT_MAX particles (whose boxes the
+// direct form never declines): k_nn_count_direct's counts with the h update applied at once.  The
+// pass reads one h array and writes the other: a particle that finished holds the same h in both
+// (its last count left it unchanged), so only the listed ones are written.  On small sets the
+// launches are the time (16^3: RHS 397 us with three per pass, 378 us with this one).  On larger
+// ones every wavefront's append to the one list counter serialises with the others' (47^3: 26 us
+// per pass against 11 + 6 us of counts and their wave-aggregated update), and they keep three.
+__global__ __launch_bounds__(64 * NN1_WAVES) void k_h_pass(NNArgs A) {
+    __shared__ NNWaveLds lds_all[NN1_WAVES];
+    const int w = threadIdx.x / 64, lane = wave_lane();
+    NNWaveLds &L = lds_all[w];
+    const bool frozen = h_pass_frozen(A);
+    const uint32_t cnt = *A.count_in;
+    const int64_t nwaves = (int64_t)gridDim.x * NN1_WAVES;
+    HStay stay;
+    bool changed = false;
+    unsigned done = 0;
+    for (int64_t t = (int64_t)blockIdx.x * NN1_WAVES + w; t < cnt; t += nwaves) {
+        const int32_t k = A.list_in[t];
+        const double hi = A.h[k];
+        int count = 0;
+        if (frozen) {
+            count = A.snoi[k];
+        } else {
+            const double4 own = A.sxm[k];
+            const double hi2 = hi * hi;
+            const double grow = hi * (1.0 + 1e-9);
+            nn_direct(L, A, own.x - grow, own.x + grow, own.y - grow, own.y + grow, own.z - grow,
+                                          own.z + grow, nn_point(own.x, own.y, own.z, hi), 0, 1,
+                                          [&](bool v, int j, const double4 &p, double h) {
+                if (v) {
+                    const double dx = own.x - p.x;
+                    const double dy = own.y - p.y;
+                    const double dz = own.z - p.z;
+                    const double d = nn_d2(dx, dy, dz);
+                    count += (d < hi2 && d < h * h && j != k) ? 1 : 0;
+                }
+            });
+            count = wave_sum(count);
+            wave_sync();
+        }
+        done++;
+        h_tail_update(A, k, count, hi, stay, changed);
+    }
+    stay.flush(A);
+    if (lane == 0 && done != 0) atomicAdd(&cnt_slot(A.counters)[CNT_H_COUNTS], (unsigned long long)done);
+    if (lane == 0 && changed) *A.changed = 1u;
+}
+
 // Start table of the current tree: a particle alone in its level-l prefix for every
 // l >= its leaf level, and every cell of level <= kmax, written at their Lebesgue prefix.
 __global__ __launch_bounds__(256) void k_nn_start_table(int64_t n, int kmax, const uint8_t *__restrict__ lcp,
@@ -1324,7 +1419,7 @@ __global__ __launch_bounds__(256) void k_hmax_raise(const int32_t *__restrict__ 
 }
 
 static void launch_hmax_raise(mhpc_ctx *c, const int32_t *list, const uint32_t *count) {
-    hipLaunchKernelGGL(k_hmax_raise, dim3(64), dim3(256), 0, c->stream, list, count, c->sh, c->ppar, c->cpar,
+    hipLaunchKernelGGL(k_hmax_raise, dim3((unsigned)std::min<int64_t>(ceil_div(c->n, 1024), 512)), dim3(256), 0, c->stream, list, count, c->sh, c->ppar, c->cpar,
                        c->chmax, c->cap_cells);
 }
 
@@ -1387,6 +1482,7 @@ void launch_h_iterate(mhpc_ctx *c, int passes, bool speculative, hipEvent_t *wal
     // the particles still iterating are the ones whose h changed
     launch_hmax_raise(c, c->hlist[2], c->hlist_count + 0);
     // passes 1.., per-particle mode over the list of the previous pass
+    const bool few = c->n <= NN_DIRECT_MAX;
     for (int pass = 1; pass < passes; pass++) {
         a.pass = pass;
         a.h = c->sh;
@@ -1398,6 +1494,16 @@ void launch_h_iterate(mhpc_ctx *c, int passes, bool speculative, hipEvent_t *wal
         a.cnt_slot = c->hcnt;
         a.changed = c->dstatus->hchanged + pass;   // zeroed by k_h_init
         a.prev_changed = pass >= 2 ? c->dstatus->hchanged + (pass - 1) : nullptr;
+        if (few) {
+            NNArgs f = a;
+            f.h_next = c->sh2;
+            f.chmax_raise = c->chmax;
+            f.ppar = c->ppar;
+            f.cpar = c->cpar;
+            hipLaunchKernelGGL(k_h_pass, dim3(g1), dim3(64 * NN1_WAVES), 0, c->stream, f);
+            std::swap(c->sh, c->sh2);
+            continue;
+        }
         // direct counts; the particles they cannot take go to the split walk
         uint32_t *hard_count = c->hlist_count + MHPC_MAX_PASSES + 1 + pass;   // zeroed by k_h_init
         NNArgs d = a;
