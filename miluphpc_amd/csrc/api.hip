@@ -122,8 +122,6 @@ static void free_all(mhpc_ctx *c) {
     for (int f = 0; f < MHPC_F_NOI; f++)
         if (c->f_own[f]) (void)hipFree(c->f_own[f]);
     if (c->h_status) (void)hipHostFree(c->h_status);
-    if (c->h_status1) (void)hipHostFree(c->h_status1);
-    if (c->h_diag) (void)hipHostFree(c->h_diag);
     for (int e = 0; e < MHPC_NUM_EVENTS; e++)
         if (c->ev[e]) (void)hipEventDestroy(c->ev[e]);
     if (c->sync_ev) (void)hipEventDestroy(c->sync_ev);
@@ -137,11 +135,11 @@ static int create_impl(mhpc_ctx *c, int64_t cap, int64_t cap_cells) {
     HIPC(hipEventCreateWithFlags(&c->sync_ev, hipEventDisableTiming));
     HIPC(hipMalloc((void **)&c->dstatus, sizeof(DevStatus)));
     HIPC(hipMemset(c->dstatus, 0, sizeof(DevStatus)));
-    HIPC(hipHostMalloc((void **)&c->h_status, sizeof(DevStatus), hipHostMallocDefault));
-    memset(c->h_status, 0, sizeof(DevStatus));
-    HIPC(hipHostMalloc((void **)&c->h_status1, sizeof(DevStatus), hipHostMallocDefault));
-    memset(c->h_status1, 0, sizeof(DevStatus));
-    HIPC(hipHostMalloc((void **)&c->h_diag, sizeof(mhpc_diagnostics), hipHostMallocDefault));
+    // one pinned block: the two status mirrors and the global sums' record
+    HIPC(hipHostMalloc((void **)&c->h_status, 2 * sizeof(DevStatus) + sizeof(mhpc_diagnostics), hipHostMallocDefault));
+    memset(c->h_status, 0, 2 * sizeof(DevStatus));
+    c->h_status1 = c->h_status + 1;
+    c->h_diag = reinterpret_cast<mhpc_diagnostics *>(c->h_status + 2);
     c->err = &c->dstatus->err;
     c->counters = c->dstatus->counters;
     c->sort_check = &c->dstatus->sort_check;
@@ -967,7 +965,8 @@ static int rhs_plan(mhpc_ctx *c, uint32_t flags, RhsPlan &P) {
     P.feats = P.hiter && (flags & (MHPC_RHS_LEARNED_H | MHPC_RHS_FEATURES));
     // speculative lists: pass 0 of the h-iteration writes the lists, and only particles
     // whose list can differ from the final one are re-listed (same neighbour sets)
-    P.spec = P.hiter && (P.learned || (flags & MHPC_RHS_SPECULATIVE_NN));
+    // (few particles are iterated per particle and listed once, by the same two calls)
+    P.spec = P.hiter && (P.learned || (flags & MHPC_RHS_SPECULATIVE_NN) || nn_few(c));
     P.timing = flags & MHPC_RHS_TIMING;
     if (P.sph) {
         int st = ensure_nbr(c);
@@ -990,16 +989,13 @@ static void rhs_launch(mhpc_ctx *c, const RhsPlan &P, hipEvent_t *ev) {
     auto mark = [&](int idx) {
         if (P.timing || idx >= 9) (void)hipEventRecord(ev[idx], c->stream);
     };
-    reset_flags(c);
     mark(13);
     if (P.feats) {
         launch_mlp_features(c, c->last_dt);
         if (P.predict) launch_mlp_predict(c);
     }
     mark(0);
-    launch_bbox(c);
-    mark(1);
-    launch_keys(c);
+    launch_bbox_keys(c, [&] { mark(1); });
     mark(2);
     launch_sort(c);
     mark(3);

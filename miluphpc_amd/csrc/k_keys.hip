@@ -45,7 +45,13 @@ void launch_fill_u64(mhpc_ctx *c, unsigned long long *p, unsigned long long v, i
 __global__ __launch_bounds__(256) void k_bbox_partial(const double *__restrict__ x,
                                                       const double *__restrict__ y,
                                                       const double *__restrict__ z, int64_t n,
-                                                      double *__restrict__ partial) {
+                                                      double *__restrict__ partial, uint32_t *err,
+                                                      unsigned long long *counters) {
+    // the first kernel of an RHS also clears the error word and the counters
+    if (err && blockIdx.x == 0) {
+        if (threadIdx.x == 0) *err = 0u;
+        for (int t = threadIdx.x; t < CNT_SLOTS * CNT_LINE; t += 256) counters[t] = 0ull;
+    }
     double lo = 0.0, hi = 0.0;
     int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     int64_t stride = (int64_t)gridDim.x * blockDim.x;
@@ -73,10 +79,11 @@ __global__ __launch_bounds__(256) void k_bbox_partial(const double *__restrict__
     }
 }
 
-__global__ __launch_bounds__(256) void k_bbox_final(const double *__restrict__ partial, int nb,
-                                                    double *__restrict__ box) {
-    double lo = 0.0, hi = 0.0;
-    for (int b = threadIdx.x; b < nb; b += blockDim.x) {
+// folds nb <= 1024 block partials by one 256-thread block (every thread receives the result)
+__device__ __forceinline__ void bbox_fold(const double *__restrict__ partial, int nb, double &lo, double &hi) {
+    lo = 0.0;
+    hi = 0.0;
+    for (int b = threadIdx.x; b < nb; b += 256) {
         lo = fmin(lo, partial[2 * b]);
         hi = fmax(hi, partial[2 * b + 1]);
     }
@@ -89,23 +96,37 @@ __global__ __launch_bounds__(256) void k_bbox_final(const double *__restrict__ p
         shi[w] = hi;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int k = 0; k < (int)(blockDim.x / 64); k++) {
-            lo = fmin(lo, slo[k]);
-            hi = fmax(hi, shi[k]);
-        }
-        box[0] = lo; box[1] = hi;
-        box[2] = lo; box[3] = hi;
-        box[4] = lo; box[5] = hi;
+    for (int k = 0; k < 4; k++) {
+        lo = fmin(lo, slo[k]);
+        hi = fmax(hi, shi[k]);
     }
 }
 
-void launch_bbox(mhpc_ctx *c) {
+__device__ __forceinline__ void bbox_store(double *__restrict__ box, double lo, double hi) {
+    box[0] = lo; box[1] = hi;
+    box[2] = lo; box[3] = hi;
+    box[4] = lo; box[5] = hi;
+}
+
+__global__ __launch_bounds__(256) void k_bbox_final(const double *__restrict__ partial, int nb,
+                                                    double *__restrict__ box) {
+    double lo, hi;
+    bbox_fold(partial, nb, lo, hi);
+    if (threadIdx.x == 0) bbox_store(box, lo, hi);
+}
+
+// fold: also fold the partials into the box; otherwise the next key kernel does (launch_keys with
+// box partials), which saves the fold's launch.  reset: also clear the error word and counters.
+// Returns the number of partials.
+static int bbox_queue(mhpc_ctx *c, bool fold, bool reset) {
     int nb = grid_for(c->n, 256 * 8, BBOX_BLOCKS_MAX);
     hipLaunchKernelGGL(k_bbox_partial, dim3(nb), dim3(256), 0, c->stream, c->f[MHPC_F_X],
-                       c->f[MHPC_F_Y], c->f[MHPC_F_Z], c->n, c->bbox_partial);
-    hipLaunchKernelGGL(k_bbox_final, dim3(1), dim3(256), 0, c->stream, c->bbox_partial, nb, c->box);
+                       c->f[MHPC_F_Y], c->f[MHPC_F_Z], c->n, c->bbox_partial, reset ? c->err : nullptr, c->counters);
+    if (fold) hipLaunchKernelGGL(k_bbox_final, dim3(1), dim3(256), 0, c->stream, c->bbox_partial, nb, c->box);
+    return nb;
 }
+
+void launch_bbox(mhpc_ctx *c) { bbox_queue(c, true, false); }
 
 // ------------------------------------------------------------------------------------
 // a2 keys: Tree::getParticleKey (tree.cu:157-240), 21 levels of FP64 bisection, the lower
@@ -123,9 +144,9 @@ __constant__ unsigned char c_hilbert_table[12][8] = {
     {2, 3, 5, 4, 1, 0, 6, 7}, {4, 5, 3, 2, 7, 6, 0, 1}, {0, 3, 1, 2, 7, 4, 6, 5},
     {2, 1, 3, 0, 5, 6, 4, 7}, {4, 7, 5, 6, 3, 0, 2, 1}, {6, 5, 7, 4, 1, 2, 0, 3}};
 
-__device__ __forceinline__ uint64_t lebesgue_key(double x, double y, double z,
-                                                 const double *__restrict__ box) {
-    double mnx = box[0], mxx = box[1], mny = box[2], mxy = box[3], mnz = box[4], mxz = box[5];
+// the box is the same cube on all axes, [lo, hi]
+__device__ __forceinline__ uint64_t lebesgue_key(double x, double y, double z, double lo, double hi) {
+    double mnx = lo, mxx = hi, mny = lo, mxy = hi, mnz = lo, mxz = hi;
     uint64_t key = 0;
 #pragma unroll
     for (int level = 0; level < MHPC_LEVELS; level++) {
@@ -143,24 +164,35 @@ __device__ __forceinline__ uint64_t lebesgue_key(double x, double y, double z,
 
 // Also writes each particle's {x,y,z,m} as one 32-byte record in caller order, so that the
 // gather into key order reads one record per particle instead of four scattered doubles.
+// partial: every block folds the bounding box's nb partials itself and the first one stores the
+// box (a launch and its gap less; 256 partials are one load per thread).
+#define KEYS_FOLD_MAX 256
 __global__ __launch_bounds__(256) void k_keys(const double *__restrict__ x,
                                               const double *__restrict__ y,
                                               const double *__restrict__ z,
                                               const double *__restrict__ m, int64_t n,
-                                              const double *__restrict__ box, int curve,
-                                              uint64_t *__restrict__ key,
+                                              double *__restrict__ box, const double *__restrict__ partial,
+                                              int nb, int curve, uint64_t *__restrict__ key,
                                               uint64_t *__restrict__ lkey,
                                               double4 *__restrict__ xyzm) {
     __shared__ unsigned char fsm[96];
     if (threadIdx.x < 96)
         fsm[threadIdx.x] = (unsigned char)((&c_hilbert_table[0][0])[threadIdx.x] |
                                            ((&c_dir_table[0][0])[threadIdx.x] << 3));
+    double lo = 0.0, hi = 0.0;
+    if (partial) {
+        bbox_fold(partial, nb, lo, hi);
+        if (blockIdx.x == 0 && threadIdx.x == 0) bbox_store(box, lo, hi);
+    } else {
+        lo = box[0];
+        hi = box[1];
+    }
     __syncthreads();
     int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (i >= n) return;
     const double xi = x[i], yi = y[i], zi = z[i];
     xyzm[i] = make_double4(xi, yi, zi, m[i]);
-    uint64_t leb = lebesgue_key(xi, yi, zi, box);
+    uint64_t leb = lebesgue_key(xi, yi, zi, lo, hi);
     if (curve == MHPC_CURVE_HILBERT) {
         uint64_t h = 0;
         int dir = 0;
@@ -178,11 +210,21 @@ __global__ __launch_bounds__(256) void k_keys(const double *__restrict__ x,
     }
 }
 
-void launch_keys(mhpc_ctx *c) {
+static void keys_queue(mhpc_ctx *c, int nb) {
     if (c->n <= 0) return;
     hipLaunchKernelGGL(k_keys, dim3((unsigned)ceil_div(c->n, 256)), dim3(256), 0, c->stream,
                        c->f[MHPC_F_X], c->f[MHPC_F_Y], c->f[MHPC_F_Z], c->f[MHPC_F_MASS], c->n, c->box,
-                       c->p.curve, c->key, c->lkey, c->xyzm);
+                       nb > 0 ? c->bbox_partial : nullptr, nb, c->p.curve, c->key, c->lkey, c->xyzm);
+}
+
+void launch_keys(mhpc_ctx *c) { keys_queue(c, 0); }
+
+// the RHS's first two phases; mark(1) is called between them
+void launch_bbox_keys(mhpc_ctx *c, const std::function<void()> &between) {
+    const bool fold = c->n <= 0 || grid_for(c->n, 256 * 8, BBOX_BLOCKS_MAX) > KEYS_FOLD_MAX;
+    const int nb = bbox_queue(c, fold, true);
+    between();
+    keys_queue(c, fold ? 0 : nb);
 }
 
 // ------------------------------------------------------------------------------------

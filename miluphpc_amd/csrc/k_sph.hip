@@ -41,6 +41,12 @@ static_assert(64 / NN_SPLIT_MIN <= MHPC_NN_PARTS_PER_GROUP, "the part list holds
 #define NN_DRANGES 256       // direct form: candidate ranges per wavefront
 #define NN_DSPAN 5           // direct form: start cells per axis - 1 (<= 216 cells)
 #define NN_DIRECT_MAX 32768  // direct form: candidates per wavefront
+// Up to this many particles every search is per particle: a group walk of 64 takes 65 us or more
+// however few groups there are, a particle's direct search about 12 us (RHS with group walks and
+// per particle: 21^3 520 / 308 us, 25^3 530 / 341 us, 31^3 558 / 450 us in Lebesgue and 430 / 462 us
+// in Hilbert order).
+#define NN_FEW 32768
+static_assert(NN_FEW <= NN_DIRECT_MAX, "the direct form declines no box of so few particles");
 #define NN_DU 8              // direct form: candidates per lane and round (loads in flight)
 
 // per-wave LDS of the walker; TCAP = 128 gives the filtered walk room to compact the
@@ -674,7 +680,7 @@ __device__ __forceinline__ bool nn_split_wanted(const NNArgs &A, const NNBox &B,
 // Splits a group's active particles into runs that need no further split, cutting at the
 // boundaries of the largest cells first (the smallest shared key prefix between consecutive
 // particles; of several, the last).  Runs of at least NN_SPLIT_MIN particles are listed for
-// k_nn_walk_parts, one wavefront each; the others go to the per-particle mode, where lanes are
+// k_nn_rest, one wavefront each; the others go to the per-particle mode, where lanes are
 // candidates.  Every active particle ends up in exactly one of the two lists.
 __device__ __forceinline__ void nn_split_group(const NNArgs &A, int64_t group, int64_t k, bool active, double x,
                                                double y, double z, double h) {
@@ -945,19 +951,6 @@ __global__ __launch_bounds__(64 * NN_WAVES) void k_nn_walk(NNArgs A) {
     nn_group<MODE, false>(lds_all[w], A, group, 0ull);
 }
 
-// the parts of groups that k_nn_walk<MODE> split off, one wavefront each
-template <int MODE>
-__global__ __launch_bounds__(64 * NN_WAVES) void k_nn_walk_parts(NNArgs A) {
-    __shared__ NNWaveLdsF lds_all[NN_WAVES];
-    const int w = threadIdx.x / 64;
-    const uint32_t cnt = *A.seg_count;
-    for (int64_t t = (int64_t)blockIdx.x * NN_WAVES + w; t < cnt; t += (int64_t)gridDim.x * NN_WAVES) {
-        const ulonglong2 s = A.seg_list[t];
-        nn_group<MODE, true>(lds_all[w], A, (int64_t)s.x, s.y);
-        wave_sync();
-    }
-}
-
 // Per-particle mode: one wavefront per listed particle, searching the particle's own box
 // x +- h with the 64 lanes testing 64 candidates at a time.  Used for the outliers of the
 // group mode (particles whose h is far above the rest of their group) and for list fix-ups.
@@ -966,17 +959,16 @@ __global__ __launch_bounds__(64 * NN_WAVES) void k_nn_walk_parts(NNArgs A) {
 // order, one 4-byte entry per lane.
 #define NN1_WAVES 4
 #define NN1_MAX_BLOCKS 1024   // about one resident round: 4096 wavefronts loop over the list
+// Workgroups [first, first + blocks) of the launch.
 template <int MODE>
-__global__ __launch_bounds__(64 * NN1_WAVES) void k_nn_one(NNArgs A) {
-    __shared__ NNWaveLds lds_all[NN1_WAVES];
+__device__ __forceinline__ void nn_one(NNWaveLds &L, const NNArgs &A, unsigned first, unsigned blocks) {
     const int w = threadIdx.x / 64, lane = wave_lane();
-    NNWaveLds &L = lds_all[w];
-    const uint32_t cnt = *A.count_in;
-    const int64_t nwaves = (int64_t)gridDim.x * NN1_WAVES;
+    const int64_t cnt = A.list_in ? (int64_t)*A.count_in : A.n;   // no list: every particle
+    const int64_t nwaves = (int64_t)blocks * NN1_WAVES;
     const uint64_t lt = lanemask_lt();
     int32_t *nbr32 = reinterpret_cast<int32_t *>(A.nbr4);
-    for (int64_t t = (int64_t)blockIdx.x * NN1_WAVES + w; t < cnt; t += nwaves) {
-        const int64_t k = A.list_in[t];
+    for (int64_t t = (int64_t)(blockIdx.x - first) * NN1_WAVES + w; t < cnt; t += nwaves) {
+        const int64_t k = A.list_in ? A.list_in[t] : t;
         const double4 own = A.sxm[k];
         const double hi = A.h[k];
         const double hi2 = hi * hi;
@@ -1041,6 +1033,34 @@ __global__ __launch_bounds__(64 * NN1_WAVES) void k_nn_one(NNArgs A) {
             }
         }
         wave_sync();
+    }
+}
+
+template <int MODE>
+__global__ __launch_bounds__(64 * NN1_WAVES) void k_nn_one(NNArgs A) {
+    __shared__ NNWaveLds lds_all[NN1_WAVES];
+    nn_one<MODE>(lds_all[threadIdx.x / 64], A, 0, gridDim.x);
+}
+
+// What a group walk left to others, in one launch: workgroups [0, part_blocks) take the parts of
+// the groups it split (one wavefront each), the others the particles it deferred (k_nn_one).
+template <int MODE>
+__global__ __launch_bounds__(64 * NN1_WAVES) void k_nn_rest(NNArgs A, unsigned part_blocks) {
+    __shared__ union Lds {
+        NNWaveLds one;
+        NNWaveLdsF group;
+    } lds_all[NN1_WAVES];
+    Lds &L = lds_all[threadIdx.x / 64];
+    if (blockIdx.x < part_blocks) {
+        const uint32_t cnt = *A.seg_count;
+        for (int64_t t = (int64_t)blockIdx.x * NN1_WAVES + threadIdx.x / 64; t < cnt;
+             t += (int64_t)part_blocks * NN1_WAVES) {
+            const ulonglong2 s = A.seg_list[t];
+            nn_group<MODE, true>(L.group, A, (int64_t)s.x, s.y);
+            wave_sync();
+        }
+    } else {
+        nn_one<MODE>(L.one, A, part_blocks, gridDim.x - part_blocks);
     }
 }
 
@@ -1216,98 +1236,81 @@ __global__ __launch_bounds__(256) void k_h_finish(NNArgs A) {
     }
 }
 
-// Particles that keep iterating, collected by one wavefront of a tail pass (lane i holds the i-th)
-// and appended to the next pass's list together: one atomic per 64 instead of one each (atomics
-// on one address serialise), and their cells' bounds raised by 64 lanes at once.
-struct HStay {
-    int32_t k = 0;
-    double h = 0.0;
-    bool raise = false;
-    int n = 0;
-    __device__ __forceinline__ void flush(const NNArgs &A) {
-        if (n == 0) return;
-        const int lane = wave_lane();
-        uint32_t b = 0;
-        if (lane == 0) b = atomicAdd(A.count_out, (uint32_t)n);
-        b = __shfl(b, 0);
-        if (lane < n) {
-            A.list_out[b + lane] = k;
-            if (raise) hmax_raise(A.chmax_raise, A.ppar, A.cpar, A.cap_cells, k, h);
-        }
-        n = 0;
-    }
-};
-
-// the h update of particle k after a count N in a tail pass (all lanes, the same values); the new
-// h goes to the other h array, so every count of the pass sees the h from its start
-__device__ __forceinline__ void h_tail_update(const NNArgs &A, int32_t k, int N, double hi, HStay &stay,
-                                              bool &changed) {
-    double hn;
-    const bool fin = h_update(A, N, hi, hn);
-    if (wave_lane() == 0) {
-        A.iters[k] = A.pass + 1;
-        A.snoi[k] = N;
-        A.h_next[k] = hn;
-        if (fin) A.done[k] = 1;
-    }
-    if (fin) return;
-    // the next pass counts with hn: the cell bounds must cover it (they cover hi)
-    if (wave_lane() == stay.n) {
-        stay.k = k;
-        stay.h = hn;
-        stay.raise = hn != hi;
-    }
-    changed = changed || hn != hi;
-    if (++stay.n == 64) stay.flush(A);
-}
-
-// A whole tail pass in one launch, for sets of at most NN_DIRECT_MAX particles (whose boxes the
-// direct form never declines): k_nn_count_direct's counts with the h update applied at once.  The
+// A whole pass of the h-iteration in one launch, for few particles (NN_FEW): one wavefront per
+// particle that has not finished tests every particle of the start cells of its box x +- h, with
+// no tree walk (nn_direct; it declines no box of so few), and applies the h update at once.  The
 // pass reads one h array and writes the other: a particle that finished holds the same h in both
-// (its last count left it unchanged), so only the listed ones are written.  On small sets the
-// launches are the time (16^3: RHS 397 us with three per pass, 378 us with this one).  On larger
-// ones every wavefront's append to the one list counter serialises with the others' (47^3: 26 us
-// per pass against 11 + 6 us of counts and their wave-aggregated update), and they keep three.
+// (its last count left it unchanged), so only the unfinished ones are written.  No lists: with a
+// few particles per wavefront, looking at a flag costs less than appending to one counter, whose
+// atomics serialise (47^3: 26 us per pass with lists appended here, 11 + 6 us with counts and a
+// wave-aggregated update, so larger sets keep those).
 __global__ __launch_bounds__(64 * NN1_WAVES) void k_h_pass(NNArgs A) {
     __shared__ NNWaveLds lds_all[NN1_WAVES];
     const int w = threadIdx.x / 64, lane = wave_lane();
     NNWaveLds &L = lds_all[w];
     const bool frozen = h_pass_frozen(A);
-    const uint32_t cnt = *A.count_in;
     const int64_t nwaves = (int64_t)gridDim.x * NN1_WAVES;
-    HStay stay;
-    bool changed = false;
-    unsigned done = 0;
-    for (int64_t t = (int64_t)blockIdx.x * NN1_WAVES + w; t < cnt; t += nwaves) {
-        const int32_t k = A.list_in[t];
+    bool changed = false, stays = false;
+    unsigned counted = 0;
+    // the wavefront's particles whose h changed (lane i holds the i-th): their cells' bounds are
+    // raised together
+    int32_t rk = 0;
+    double rh = 0.0;
+    int rn = 0;
+    auto raise = [&]() {
+        if (lane < rn) hmax_raise(A.chmax_raise, A.ppar, A.cpar, A.cap_cells, rk, rh);
+        rn = 0;
+    };
+    for (int64_t t = (int64_t)blockIdx.x * NN1_WAVES + w; t < A.n; t += nwaves) {
+        const int32_t k = (int32_t)t;
+        if (A.done[k]) continue;
         const double hi = A.h[k];
-        int count = 0;
+        int N = 0;
         if (frozen) {
-            count = A.snoi[k];
+            N = A.snoi[k];
         } else {
             const double4 own = A.sxm[k];
             const double hi2 = hi * hi;
             const double grow = hi * (1.0 + 1e-9);
-            nn_direct(L, A, own.x - grow, own.x + grow, own.y - grow, own.y + grow, own.z - grow,
-                                          own.z + grow, nn_point(own.x, own.y, own.z, hi), 0, 1,
-                                          [&](bool v, int j, const double4 &p, double h) {
+            nn_direct(L, A, own.x - grow, own.x + grow, own.y - grow, own.y + grow, own.z - grow, own.z + grow,
+                      nn_point(own.x, own.y, own.z, hi), 0, 1, [&](bool v, int j, const double4 &p, double h) {
                 if (v) {
                     const double dx = own.x - p.x;
                     const double dy = own.y - p.y;
                     const double dz = own.z - p.z;
                     const double d = nn_d2(dx, dy, dz);
-                    count += (d < hi2 && d < h * h && j != k) ? 1 : 0;
+                    N += (d < hi2 && d < h * h && j != k) ? 1 : 0;
                 }
             });
-            count = wave_sum(count);
+            N = wave_sum(N);
             wave_sync();
         }
-        done++;
-        h_tail_update(A, k, count, hi, stay, changed);
+        counted++;
+        double hn;
+        const bool fin = h_update(A, N, hi, hn);
+        if (lane == 0) {
+            A.iters[k] = A.pass + 1;
+            A.snoi[k] = N;
+            A.h_next[k] = hn;
+            if (fin) A.done[k] = 1;
+        }
+        if (fin) continue;
+        stays = true;
+        if (hn != hi) {   // the next pass counts with hn: the cell bounds must cover it
+            changed = true;
+            if (lane == rn) {
+                rk = k;
+                rh = hn;
+            }
+            if (++rn == 64) raise();
+        }
     }
-    stay.flush(A);
-    if (lane == 0 && done != 0) atomicAdd(&cnt_slot(A.counters)[CNT_H_COUNTS], (unsigned long long)done);
-    if (lane == 0 && changed) *A.changed = 1u;
+    raise();
+    if (lane == 0) {
+        if (counted != 0) atomicAdd(&cnt_slot(A.counters)[CNT_H_COUNTS], (unsigned long long)counted);
+        if (stays) *A.count_out = 1u;   // not a length here: some particle goes on
+        if (changed) *A.changed = 1u;
+    }
 }
 
 // Start table of the current tree: a particle alone in its level-l prefix for every
@@ -1349,9 +1352,11 @@ __global__ __launch_bounds__(256) void k_nn_start_table(int64_t n, int kmax, con
     }
 }
 
-static void ensure_nn_start(mhpc_ctx *c) {
+// cleared: the table was just emptied (with the h-iteration's flags, k_h_init)
+static void ensure_nn_start(mhpc_ctx *c, bool cleared = false) {
     if (c->nn_start_valid || c->n <= 0) return;
-    launch_fill_u32(c, reinterpret_cast<uint32_t *>(c->nn_start), 0xffffffffu, nn_tab_off(c->nn_kmax + 1));
+    if (!cleared)
+        launch_fill_u32(c, reinterpret_cast<uint32_t *>(c->nn_start), 0xffffffffu, nn_tab_off(c->nn_kmax + 1));
     const uint64_t *slkey = (c->p.curve == MHPC_CURVE_HILBERT) ? c->slkey : c->skey;
     const int64_t items = c->n + c->cap_cells;
     hipLaunchKernelGGL(k_nn_start_table, dim3((unsigned)std::min<int64_t>(ceil_div(items, 256), 8192)), dim3(256),
@@ -1382,19 +1387,25 @@ static NNArgs nn_common(mhpc_ctx *c) {
     return a;
 }
 
-// parts of split groups: at most about one resident round of wavefronts, looping over the list
-static unsigned nn_parts_grid(mhpc_ctx *c) {
-    return (unsigned)std::min<int64_t>(ceil_div(nn_parts_max(c->n), NN_WAVES), 2048);
+// the split parts and the deferred particles of the group walk queued before, with its arguments:
+// about one resident round of wavefronts each, looping over their lists
+template <int MODE>
+static void launch_nn_rest(mhpc_ctx *c, const NNArgs &a) {
+    const unsigned parts = (unsigned)std::min<int64_t>(ceil_div(nn_parts_max(c->n), NN1_WAVES), NN1_MAX_BLOCKS);
+    const unsigned ones = (unsigned)std::min<int64_t>(ceil_div(c->n, NN1_WAVES), NN1_MAX_BLOCKS);
+    hipLaunchKernelGGL(k_nn_rest<MODE>, dim3(parts + ones), dim3(64 * NN1_WAVES), 0, c->stream, a, parts);
 }
+bool nn_few(const mhpc_ctx *c) { return c->n <= NN_FEW; }
 static unsigned nn_grid(mhpc_ctx *c) { return (unsigned)ceil_div(ceil_div(c->n, 64), NN_WAVES); }
 
-// done flags, iteration counts and dirty flags to zero; the per-pass list counters, the
-// per-pass changed flags and the outlier counters (pass 0, list fix-up) to zero
+// done flags, iteration counts and dirty flags to zero, the walks' start table empty; the per-pass
+// list counters, the per-pass changed flags and the outlier counters (pass 0, list fix-up) to zero
 static_assert(offsetof(DevStatus, hchanged) == offsetof(DevStatus, hlist_count) + sizeof(DevStatus::hlist_count),
               "k_h_init zeroes the list counters and the changed flags as one range");
 __global__ void k_h_init(int64_t n, uint8_t *done, int32_t *iters, uint8_t *dirty, uint32_t *list_counts,
-                         int nlc, uint32_t *ocount, uint32_t *cnt_slot) {
+                         int nlc, uint32_t *ocount, uint32_t *cnt_slot, uint32_t *tab, int64_t ntab) {
     int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    for (int64_t e = k; e < ntab; e += (int64_t)gridDim.x * blockDim.x) tab[e] = 0xffffffffu;   // empty start table
     if (k < n) {
         done[k] = 0;
         iters[k] = 0;
@@ -1430,7 +1441,9 @@ void launch_h_iterate(mhpc_ctx *c, int passes, bool speculative, hipEvent_t *wal
     if (c->n <= 0) return;
     hipLaunchKernelGGL(k_h_init, dim3((unsigned)ceil_div(c->n > 64 ? c->n : 64, 256)), dim3(256), 0, c->stream,
                        c->n, c->sdone, c->siters, c->sdirty, c->hlist_count, 3 * (MHPC_MAX_PASSES + 1), c->ocount,
-                       c->hcnt);
+                       c->hcnt, reinterpret_cast<uint32_t *>(c->nn_start),
+                       c->nn_start_valid ? (int64_t)0 : nn_tab_off(c->nn_kmax + 1));
+    ensure_nn_start(c, true);
     NNArgs a = nn_common(c);
     a.done = c->sdone;
     a.iters = c->siters;
@@ -1441,6 +1454,27 @@ void launch_h_iterate(mhpc_ctx *c, int passes, bool speculative, hipEvent_t *wal
     a.band_lo = c->p.band_lo;
     a.band_hi = c->p.band_hi;
     a.sml_max = c->p.sml_max;
+    const unsigned g1 = (unsigned)std::min<int64_t>(ceil_div(c->n, NN1_WAVES), NN1_MAX_BLOCKS);
+    if (nn_few(c)) {
+        // every pass in the per-particle mode, from one h array to the other; the lists are built
+        // once from the final h (launch_neighbours_fixup)
+        a.chmax_raise = c->chmax;
+        a.ppar = c->ppar;
+        a.cpar = c->cpar;
+        for (int pass = 0; pass < passes; pass++) {
+            a.pass = pass;
+            a.h = c->sh;
+            a.h_next = c->sh2;
+            a.count_out = c->hlist_count + pass;
+            a.changed = c->dstatus->hchanged + pass;   // zeroed by k_h_init
+            a.prev_changed = pass >= 1 ? c->dstatus->hchanged + (pass - 1) : nullptr;
+            if (walk_events && pass == 0) (void)hipEventRecord(walk_events[0], c->stream);
+            hipLaunchKernelGGL(k_h_pass, dim3(g1), dim3(64 * NN1_WAVES), 0, c->stream, a);
+            if (walk_events && pass == 0) (void)hipEventRecord(walk_events[1], c->stream);
+            std::swap(c->sh, c->sh2);
+        }
+        return;
+    }
     // pass 0, group mode; its list of unconverged particles (hlist[2]) is also the list
     // of particles whose h changed after pass 0
     a.pass = 0;
@@ -1449,32 +1483,24 @@ void launch_h_iterate(mhpc_ctx *c, int passes, bool speculative, hipEvent_t *wal
     a.list_out = c->hlist[2];
     a.count_out = c->hlist_count + 0;
     a.h0_slot = c->h0slot;
-    const unsigned g1 = (unsigned)std::min<int64_t>(ceil_div(c->n, NN1_WAVES), NN1_MAX_BLOCKS);
     a.out_list = c->olist;
     a.out_count = c->ocount;   // zeroed by k_h_init
     a.seg_list = c->seglist;
     a.seg_count = c->ocount + 2;
-    const unsigned gs = nn_parts_grid(c);
     if (walk_events) (void)hipEventRecord(walk_events[0], c->stream);
     if (speculative) {
         a.nbr4 = reinterpret_cast<int4 *>(c->nbr);
         a.stride = c->cap_pad;
         hipLaunchKernelGGL(k_nn_walk<2>, dim3(nn_grid(c)), dim3(64 * NN_WAVES), 0, c->stream, a);
-        hipLaunchKernelGGL(k_nn_walk_parts<2>, dim3(gs), dim3(64 * NN_WAVES), 0, c->stream, a);
     } else {
         hipLaunchKernelGGL(k_nn_walk<1>, dim3(nn_grid(c)), dim3(64 * NN_WAVES), 0, c->stream, a);
-        hipLaunchKernelGGL(k_nn_walk_parts<1>, dim3(gs), dim3(64 * NN_WAVES), 0, c->stream, a);
     }
     if (walk_events) (void)hipEventRecord(walk_events[1], c->stream);
-    // the group mode's outliers, same pass, per-particle mode
-    {
-        NNArgs o = a;
-        o.out_list = nullptr;
-        o.list_in = c->olist;
-        o.count_in = c->ocount;
-        if (speculative) hipLaunchKernelGGL(k_nn_one<2>, dim3(g1), dim3(64 * NN1_WAVES), 0, c->stream, o);
-        else hipLaunchKernelGGL(k_nn_one<1>, dim3(g1), dim3(64 * NN1_WAVES), 0, c->stream, o);
-    }
+    // the group mode's split parts and outliers, same pass
+    a.list_in = c->olist;
+    a.count_in = c->ocount;
+    if (speculative) launch_nn_rest<2>(c, a);
+    else launch_nn_rest<1>(c, a);
     a.nbr4 = nullptr;
     a.out_list = nullptr;
     a.h0_slot = nullptr;   // the pass-0 slots stay for the dirty marking
@@ -1482,7 +1508,6 @@ void launch_h_iterate(mhpc_ctx *c, int passes, bool speculative, hipEvent_t *wal
     // the particles still iterating are the ones whose h changed
     launch_hmax_raise(c, c->hlist[2], c->hlist_count + 0);
     // passes 1.., per-particle mode over the list of the previous pass
-    const bool few = c->n <= NN_DIRECT_MAX;
     for (int pass = 1; pass < passes; pass++) {
         a.pass = pass;
         a.h = c->sh;
@@ -1494,16 +1519,6 @@ void launch_h_iterate(mhpc_ctx *c, int passes, bool speculative, hipEvent_t *wal
         a.cnt_slot = c->hcnt;
         a.changed = c->dstatus->hchanged + pass;   // zeroed by k_h_init
         a.prev_changed = pass >= 2 ? c->dstatus->hchanged + (pass - 1) : nullptr;
-        if (few) {
-            NNArgs f = a;
-            f.h_next = c->sh2;
-            f.chmax_raise = c->chmax;
-            f.ppar = c->ppar;
-            f.cpar = c->cpar;
-            hipLaunchKernelGGL(k_h_pass, dim3(g1), dim3(64 * NN1_WAVES), 0, c->stream, f);
-            std::swap(c->sh, c->sh2);
-            continue;
-        }
         // direct counts; the particles they cannot take go to the split walk
         uint32_t *hard_count = c->hlist_count + MHPC_MAX_PASSES + 1 + pass;   // zeroed by k_h_init
         NNArgs d = a;
@@ -1527,10 +1542,20 @@ void launch_h_iterate(mhpc_ctx *c, int passes, bool speculative, hipEvent_t *wal
 // pass-0 list may differ from the list with the final h (the changed particles and every
 // particle within its own h of one).  The lists then equal those of a full list walk with the
 // final h as sets (order may differ); the density kernel publishes the counts.
+// For few particles the iteration built no lists: all are listed, one wavefront each.
 void launch_neighbours_fixup(mhpc_ctx *c) {
     if (c->n <= 0) return;
     NNArgs a = nn_common(c);
     a.h = c->sh;
+    if (nn_few(c)) {
+        a.nbr4 = reinterpret_cast<int4 *>(c->nbr);
+        a.stride = c->cap_pad;
+        a.snoi = c->snoi;
+        a.counters = nullptr;   // the density kernel counts every particle
+        hipLaunchKernelGGL(k_nn_one<0>, dim3((unsigned)std::min<int64_t>(ceil_div(c->n, NN1_WAVES), NN1_MAX_BLOCKS)),
+                           dim3(64 * NN1_WAVES), 0, c->stream, a);
+        return;
+    }
     a.list_in = c->hlist[2];
     a.count_in = c->hlist_count + 0;
     a.dirty = c->sdirty;
@@ -1549,13 +1574,11 @@ void launch_neighbours_fixup(mhpc_ctx *c) {
     b.seg_list = c->seglist;
     b.seg_count = c->ocount + 3;
     hipLaunchKernelGGL(k_nn_walk<0>, dim3(nn_grid(c)), dim3(64 * NN_WAVES), 0, c->stream, b);
-    hipLaunchKernelGGL(k_nn_walk_parts<0>, dim3(nn_parts_grid(c)), dim3(64 * NN_WAVES), 0, c->stream, b);
-    b.out_list = nullptr;
     b.list_in = c->olist;
     b.count_in = c->ocount + 1;
     b.counters = nullptr;   // the density kernel counts every particle
     b.noi_out = nullptr;
-    hipLaunchKernelGGL(k_nn_one<0>, dim3(g1), dim3(64 * NN1_WAVES), 0, c->stream, b);
+    launch_nn_rest<0>(c, b);
     // h, counts and the neighbour sums go to caller order with the density kernel
     // (launch_density_eos(c, true)), which runs next and visits every particle
 }
@@ -1571,18 +1594,20 @@ void launch_neighbours(mhpc_ctx *c) {
     a.sml_out = nullptr;
     a.siters = c->siters;
     a.iters_out = nullptr;
+    const unsigned g1 = (unsigned)std::min<int64_t>(ceil_div(c->n, NN1_WAVES), NN1_MAX_BLOCKS);
+    if (nn_few(c)) {
+        hipLaunchKernelGGL(k_nn_one<0>, dim3(g1), dim3(64 * NN1_WAVES), 0, c->stream, a);
+        return;
+    }
     launch_fill_u32(c, c->ocount, 0u, 4);
     a.out_list = c->olist;
     a.out_count = c->ocount;
     a.seg_list = c->seglist;
     a.seg_count = c->ocount + 2;
     hipLaunchKernelGGL(k_nn_walk<0>, dim3(nn_grid(c)), dim3(64 * NN_WAVES), 0, c->stream, a);
-    hipLaunchKernelGGL(k_nn_walk_parts<0>, dim3(nn_parts_grid(c)), dim3(64 * NN_WAVES), 0, c->stream, a);
-    a.out_list = nullptr;
     a.list_in = c->olist;
     a.count_in = c->ocount;
-    const unsigned g1 = (unsigned)std::min<int64_t>(ceil_div(c->n, NN1_WAVES), NN1_MAX_BLOCKS);
-    hipLaunchKernelGGL(k_nn_one<0>, dim3(g1), dim3(64 * NN1_WAVES), 0, c->stream, a);
+    launch_nn_rest<0>(c, a);
 }
 
 // ------------------------------------------------------------------------------------
@@ -1828,6 +1853,10 @@ struct DensPub {
 // address path sees).  On a lattice 67 % of the pairs fall in a 512-particle window and 58 %
 // in a 256-particle one.  Same arithmetic and order as a pure gather.
 #define DENS_WIN 512
+// Up to this many particles a list is shared by 16 lanes instead (k_density_split,
+// k_forces_split): RHS of 31^3 598 -> 558 us, of 36^3 625 -> 605 us, but of 45^3 712 -> 738 us,
+// where the windows' saved gathers count more than idle lanes
+#define SPLIT_MAX 49152
 
 // EOS: the sound speed / pressure of the particle follow in the same kernel (the RHS path)
 template <bool FP64, bool EOS, bool CUBIC>
@@ -1929,18 +1958,86 @@ __global__ __launch_bounds__(DENS_WIN) void k_density(int64_t n, const double4 *
     }
 }
 
+// The same for few particles: 16 lanes per particle, each taking every 16th list row (four
+// neighbours), their sums added across the lanes; neighbours are gathered (no window).  With one
+// lane per particle, 4096 particles are eight workgroups whose lanes walk their lists alone
+// (30 us; this 7 us).
+#define SPLIT_LANES 16
+template <bool FP64, bool EOS, bool CUBIC>
+__global__ __launch_bounds__(256) void k_density_split(int64_t n, const double4 *__restrict__ sxm,
+                                                       const double *__restrict__ sh,
+                                                       const int32_t *__restrict__ snoi,
+                                                       const int32_t *__restrict__ nbr, int64_t stride, int max_nb,
+                                                       int sml_avg, int kind, const int32_t *__restrict__ perm,
+                                                       double *__restrict__ srho, double *__restrict__ rho,
+                                                       uint32_t *err, EosArgs E, DensPub P) {
+    const int64_t k = xcd_block(blockIdx.x, gridDim.x) * (256 / SPLIT_LANES) + threadIdx.x / SPLIT_LANES;
+    const int sub = threadIdx.x % SPLIT_LANES;
+    double sum = 0.0, hi = 0.0;
+    double4 pi = make_double4(0.0, 0.0, 0.0, 0.0);
+    int noi = 0;
+    if (k < n) {
+        pi = sxm[k];
+        hi = sh[k];
+        noi = snoi[k];
+        const int cnt = noi > max_nb ? max_nb : noi;
+        const int4 *nrow = reinterpret_cast<const int4 *>(nbr) + k;
+        double acc = 0.0;
+        Kahan acc32;
+        for (int r = sub; 4 * r < cnt; r += SPLIT_LANES) {
+            const int4 q = nrow[(int64_t)r * stride];
+            const int m = cnt - 4 * r;
+            const int32_t jj[4] = {q.x, q.y, q.z, q.w};
+            double4 pj[4];
+            double hj[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int32_t j = e < m ? jj[e] : (int32_t)k;
+                pj[e] = sxm[j];
+                hj[e] = sh[j];
+            }
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if (e < m) density_pair<FP64, CUBIC>(pi, hi, pj[e], hj[e], sml_avg, kind, acc, acc32);
+        }
+        sum = FP64 ? acc : acc32.value();
+    }
+    sum = row_sum(sum);
+    if (k < n && sub == 0) {
+        const double self = CUBIC ? K8PI / (hi * hi * hi) : kernel_sigma(kind) / (hi * hi * hi);   // W(0)
+        const double r = pi.w * self + sum;
+        srho[k] = r;
+        const int32_t i = perm[k];
+        rho[i] = r;
+        if (!(r > 0.0)) set_err(err, ERRF_RHO);
+        if (EOS) eos_particle(E, k, i, r, pi.w, hi);
+        if (P.noi) {
+            P.noi[i] = noi;
+            P.sml[i] = hi;
+            P.iters[i] = P.siters[k];
+        }
+    }
+    if (P.noi) {
+        const unsigned long long tot = wave_sum((unsigned long long)(sub == 0 ? noi : 0));
+        const int mx = wave_max(noi);
+        if (wave_lane() == 0) {
+            atomicAdd(&cnt_slot(P.counters)[CNT_NEIGHBOURS], tot);
+            atomicMax(&cnt_slot(P.counters)[CNT_MAX_NOI], (unsigned long long)mx);
+        }
+    }
+}
+
 template <bool FP64, bool EOS>
 static void launch_density_p(mhpc_ctx *c, const EosArgs &E, const DensPub &P) {
-    const unsigned g = (unsigned)ceil_div(c->n, DENS_WIN);
-    const int kind = c->p.smoothing_kernel;
-    if (kind == MHPC_KERNEL_CUBIC_SPLINE)
-        hipLaunchKernelGGL((k_density<FP64, EOS, true>), dim3(g), dim3(DENS_WIN), 0, c->stream, c->n, c->sxm, c->sh,
-                           c->snoi, c->nbr, c->cap_pad, c->p.max_nb, c->p.sml_avg, kind, c->perm, c->srho,
-                           c->f[MHPC_F_RHO], c->err, E, P);
-    else
-        hipLaunchKernelGGL((k_density<FP64, EOS, false>), dim3(g), dim3(DENS_WIN), 0, c->stream, c->n, c->sxm,
-                           c->sh, c->snoi, c->nbr, c->cap_pad, c->p.max_nb, c->p.sml_avg, kind, c->perm, c->srho,
-                           c->f[MHPC_F_RHO], c->err, E, P);
+    const bool cubic = c->p.smoothing_kernel == MHPC_KERNEL_CUBIC_SPLINE;
+    const bool split = c->n <= SPLIT_MAX;
+    auto kernel = split ? (cubic ? k_density_split<FP64, EOS, true> : k_density_split<FP64, EOS, false>)
+                        : (cubic ? k_density<FP64, EOS, true> : k_density<FP64, EOS, false>);
+    const unsigned threads = split ? 256 : DENS_WIN;
+    const unsigned g = (unsigned)ceil_div(c->n * (split ? SPLIT_LANES : 1), threads);
+    hipLaunchKernelGGL(kernel, dim3(g), dim3(threads), 0, c->stream, c->n, c->sxm, c->sh, c->snoi, c->nbr, c->cap_pad,
+                       c->p.max_nb, c->p.sml_avg, c->p.smoothing_kernel, c->perm, c->srho, c->f[MHPC_F_RHO], c->err, E,
+                       P);
 }
 
 template <bool EOS>
@@ -2122,6 +2219,43 @@ __device__ __forceinline__ void force_pair(const ForceI &I, const double4 &pj, c
     }
 }
 
+// a particle's accumulated sums (drho and dsml share one sum in FP64)
+struct ForceSums {
+    double a[3], drho, dsml, de, mumax, feat[6];
+    __device__ __forceinline__ void take(const ForceAcc<true> &s, double mu, const double *f) {
+        a[0] = s.a0; a[1] = s.a1; a[2] = s.a2;
+        drho = dsml = s.dvv;
+        de = s.de;
+        mumax = mu;
+        for (int q = 0; q < 6; q++) feat[q] = f[q];
+    }
+    __device__ __forceinline__ void take(const ForceAcc<false> &s, double mu, const double *f) {
+        a[0] = s.a0.value(); a[1] = s.a1.value(); a[2] = s.a2.value();
+        drho = s.drho.value();
+        dsml = s.dsml.value();
+        de = s.de.value();
+        mumax = mu;
+        for (int q = 0; q < 6; q++) feat[q] = f[q];
+    }
+};
+
+template <bool FEAT>
+__device__ __forceinline__ void force_store(const ForceArgs &A, int64_t k, const ForceI &I, const ForceSums &S) {
+    const int32_t i = A.perm[k];
+    A.ax[i] = S.a[0];
+    A.ay[i] = S.a[1];
+    A.az[i] = S.a[2];
+    A.drhodt[i] = I.r.x * S.drho;
+    A.dedt[i] = 0.5 * S.de;
+    A.dsmldt[i] = -(1.0 / 3.0) * I.h * S.dsml;
+    A.muijmax[i] = S.mumax;
+    if (FEAT) {
+        const double *f = S.feat;
+        A.curlv[i] = sqrt(f[0] * f[0] + f[1] * f[1] + f[2] * f[2]);
+        A.gradrho[i] = sqrt(f[3] * f[3] + f[4] * f[4] + f[5] * f[5]);
+    }
+}
+
 // One block per window of FORCE_WIN consecutive sorted particles, their records staged in
 // LDS (see the density kernel): in-window neighbours are read there, the others gathered.
 #define FORCE_WIN 512
@@ -2188,39 +2322,75 @@ __global__ __launch_bounds__(FORCE_WIN) void k_forces(ForceArgs A) {
                 if (h + e < m) force_pair<FP64, FEAT, CUBIC>(I, pj[e], vj[e], rj[e], acc, mumax, feat);
         }
     }
-    double out[6];
-    if constexpr (FP64) {
-        out[0] = acc.a0; out[1] = acc.a1; out[2] = acc.a2;
-        out[3] = I.r.x * acc.dvv;
-        out[4] = 0.5 * acc.de;
-        out[5] = -(1.0 / 3.0) * I.h * acc.dvv;
-    } else {
-        out[0] = acc.a0.value(); out[1] = acc.a1.value(); out[2] = acc.a2.value();
-        out[3] = I.r.x * acc.drho.value();
-        out[4] = 0.5 * acc.de.value();
-        out[5] = -(1.0 / 3.0) * I.h * acc.dsml.value();
+    ForceSums S;
+    S.take(acc, mumax, feat);
+    force_store<FEAT>(A, k, I, S);
+}
+
+// the same for few particles, 16 lanes per particle (see k_density_split; 4096 particles: 49 -> 6 us)
+template <bool FP64, bool FEAT, bool CUBIC>
+__global__ __launch_bounds__(256) void k_forces_split(ForceArgs A) {
+    const int64_t k = xcd_block(blockIdx.x, gridDim.x) * (256 / SPLIT_LANES) + threadIdx.x / SPLIT_LANES;
+    const int sub = threadIdx.x % SPLIT_LANES;
+    ForceAcc<FP64> acc;
+    double mumax = 0.0;
+    double feat[6] = {0, 0, 0, 0, 0, 0};
+    ForceI I = {};
+    if (k < A.n) {
+        I.p = A.sxm[k];
+        I.v = A.sv4[k];
+        I.r = A.sr4[k];
+        I.h = A.sh[k];
+        I.sml_avg = A.sml_avg;
+        I.kind = A.kind;
+        I.alpha = A.alpha;
+        I.beta = A.beta;
+        int cnt = A.snoi[k];
+        cnt = cnt > A.max_nb ? A.max_nb : cnt;
+        const int4 *nrow = reinterpret_cast<const int4 *>(A.nbr) + k;
+        for (int r = sub; 4 * r < cnt; r += SPLIT_LANES) {
+            const int4 q = nrow[(int64_t)r * A.stride];
+            const int m = cnt - 4 * r;
+            const int32_t jj[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+            for (int h = 0; h < 4; h += 2) {
+                double4 pj[2], vj[2], rj[2];
+#pragma unroll
+                for (int e = 0; e < 2; e++) {
+                    const int32_t j = h + e < m ? jj[h + e] : (int32_t)k;
+                    pj[e] = A.sxm[j];
+                    vj[e] = A.sv4[j];
+                    rj[e] = A.sr4[j];
+                }
+#pragma unroll
+                for (int e = 0; e < 2; e++)
+                    if (h + e < m) force_pair<FP64, FEAT, CUBIC>(I, pj[e], vj[e], rj[e], acc, mumax, feat);
+            }
+        }
     }
-    const int32_t i = A.perm[k];
-    A.ax[i] = out[0];
-    A.ay[i] = out[1];
-    A.az[i] = out[2];
-    A.drhodt[i] = out[3];
-    A.dedt[i] = out[4];
-    A.dsmldt[i] = out[5];
-    A.muijmax[i] = mumax;
-    if (FEAT) {
-        A.curlv[i] = sqrt(feat[0] * feat[0] + feat[1] * feat[1] + feat[2] * feat[2]);
-        A.gradrho[i] = sqrt(feat[3] * feat[3] + feat[4] * feat[4] + feat[5] * feat[5]);
-    }
+    ForceSums S;
+    S.take(acc, mumax, feat);
+#pragma unroll
+    for (int q = 0; q < 3; q++) S.a[q] = row_sum(S.a[q]);
+    S.drho = row_sum(S.drho);
+    S.dsml = FP64 ? S.drho : row_sum(S.dsml);
+    S.de = row_sum(S.de);
+    S.mumax = row_max(S.mumax);
+    if (FEAT)
+#pragma unroll
+        for (int q = 0; q < 6; q++) S.feat[q] = row_sum(S.feat[q]);
+    if (k < A.n && sub == 0) force_store<FEAT>(A, k, I, S);
 }
 
 template <bool FP64, bool FEAT>
 static void launch_forces_p(mhpc_ctx *c, const ForceArgs &a) {
-    const unsigned g = (unsigned)ceil_div(c->n, FORCE_WIN);
-    if (a.kind == MHPC_KERNEL_CUBIC_SPLINE)
-        hipLaunchKernelGGL((k_forces<FP64, FEAT, true>), dim3(g), dim3(FORCE_WIN), 0, c->stream, a);
-    else
-        hipLaunchKernelGGL((k_forces<FP64, FEAT, false>), dim3(g), dim3(FORCE_WIN), 0, c->stream, a);
+    const bool cubic = a.kind == MHPC_KERNEL_CUBIC_SPLINE;
+    const bool split = c->n <= SPLIT_MAX;
+    auto kernel = split ? (cubic ? k_forces_split<FP64, FEAT, true> : k_forces_split<FP64, FEAT, false>)
+                        : (cubic ? k_forces<FP64, FEAT, true> : k_forces<FP64, FEAT, false>);
+    const unsigned threads = split ? 256 : FORCE_WIN;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)ceil_div(c->n * (split ? SPLIT_LANES : 1), threads)), dim3(threads), 0,
+                       c->stream, a);
 }
 
 void launch_forces(mhpc_ctx *c, bool features) {

@@ -16,6 +16,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <functional>
 #include <string>
 
 #include "../../include/mhpc.h"
@@ -201,6 +202,9 @@ void fill_u32_on(hipStream_t stream, uint32_t *p, uint32_t v, int64_t n);
 void launch_fill_u64(mhpc_ctx *c, unsigned long long *p, unsigned long long v, int64_t n);
 void launch_bbox(mhpc_ctx *c);
 void launch_keys(mhpc_ctx *c);
+// both, and the error word and counters cleared, as an RHS starts; `between` is called after the
+// bounding box's launch
+void launch_bbox_keys(mhpc_ctx *c, const std::function<void()> &between);
 void launch_sort(mhpc_ctx *c);
 void launch_gather(mhpc_ctx *c, bool gravity, bool sph, bool rhs);
 void launch_tree(mhpc_ctx *c);
@@ -210,6 +214,7 @@ void launch_gravity(mhpc_ctx *c, bool potential);
 // walk_events (may be null): two events recorded around the pass-0 group walk kernel
 void launch_h_iterate(mhpc_ctx *c, int passes, bool speculative, hipEvent_t *walk_events = nullptr);
 void launch_neighbours(mhpc_ctx *c);
+bool nn_few(const mhpc_ctx *c);   // the h-iteration's per-particle form, which builds no lists
 void launch_neighbours_fixup(mhpc_ctx *c);
 void launch_density(mhpc_ctx *c);
 void launch_eos(mhpc_ctx *c);
@@ -358,6 +363,18 @@ __device__ __forceinline__ T wave_max(T v) {
 template <typename T>
 __device__ __forceinline__ T wave_sum(T v) {
     return wave_reduce(v, [](T a, T b) { return a + b; });
+}
+
+// over each row of 16 lanes
+template <typename T>
+__device__ __forceinline__ T row_sum(T v) {
+    auto op = [](T a, T b) { return a + b; };
+    return wave_step<3>(wave_step<2>(wave_step<1>(wave_step<0>(v, op), op), op), op);
+}
+template <typename T>
+__device__ __forceinline__ T row_max(T v) {
+    auto op = [](T a, T b) { return b > a ? b : a; };
+    return wave_step<3>(wave_step<2>(wave_step<1>(wave_step<0>(v, op), op), op), op);
 }
 
 // inclusive prefix sum over the wave: within rows of 16 by shifts, then the rows' totals
