@@ -115,7 +115,7 @@ static void free_all(mhpc_ctx *c) {
                     c->mlp_grad, c->mlp_norm, c->mlp_x, c->mlp_t, c->mlp_hprev,
                     c->mlp_partial, c->mlp_frag, c->mlp_loss, c->mlp_io_x, c->mlp_io_y,
                     c->hlist[0], c->hlist[1], c->hlist[2], c->sdirty,
-                    c->h0slot, c->olist, c->ocount, c->seglist, c->hcnt, c->nn_start, c->nn_start_rng, c->hhard,
+                    c->h0slot, c->olist, c->ocount, c->hcnt, c->nn_start, c->nn_start_rng, c->hhard,
                     c->xyzm, c->ppar, c->cpar};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
@@ -185,10 +185,11 @@ static int create_impl(mhpc_ctx *c, int64_t cap, int64_t cap_cells) {
     HIPC(dalloc(&c->hlist[2], cap));
     HIPC(dalloc(&c->sdirty, cap));
     HIPC(dalloc(&c->h0slot, cap));
-    HIPC(dalloc(&c->hhard, cap));
+    // also the list of split parts, which is read before the tail passes use it
+    HIPC(dalloc(&c->hhard, std::max<int64_t>(cap, nn_parts_max(cap) * (int64_t)(sizeof(ulonglong2) / sizeof(int32_t)))));
+    c->seglist = reinterpret_cast<ulonglong2 *>(c->hhard);
     HIPC(dalloc(&c->olist, cap));
     HIPC(dalloc(&c->ocount, 4));
-    HIPC(dalloc(&c->seglist, nn_parts_max(cap)));
     HIPC(dalloc(&c->hcnt, cap));
     // start table levels: the smallest K with 8^K >= cap (one geometric cell per particle on
     // average at the deepest level), 1 <= K <= MHPC_NN_KMAX

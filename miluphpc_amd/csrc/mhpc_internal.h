@@ -146,7 +146,7 @@ struct mhpc_ctx {
     int32_t *olist = nullptr;                    // neighbour search: group-mode outliers
     uint32_t *ocount = nullptr;                  // [4] outliers of pass 0 / of the list fix-up, then
                                                  // the parts of the same two walks
-    ulonglong2 *seglist = nullptr;               // neighbour search: parts of split groups
+    ulonglong2 *seglist = nullptr;               // neighbour search: parts of split groups (in hhard)
     double *h0slot = nullptr;                    // pass-0 h of the unconverged particles (list slot)
     int32_t *hhard = nullptr;                    // tail passes: slots left to the split counts
     uint32_t *hlist_count = nullptr;             // = dstatus->hlist_count: list lengths of the
