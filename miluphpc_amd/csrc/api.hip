@@ -167,10 +167,10 @@ static int create_impl(mhpc_ctx *c, int64_t cap, int64_t cap_cells) {
     HIPC(dalloc(&c->perm, cap));
     HIPC(dalloc(&c->valB, cap));
     HIPC(dalloc(&c->xyzm, cap));
-    c->sort_tiles_cap = ceil_div(cap, MHPC_SORT_TILE);
+    c->sort_tiles_cap = sort_tiles_cap(cap);
     HIPC(dalloc(&c->tile_hist, MHPC_SORT_BUCKETS * c->sort_tiles_cap));
     HIPC(dalloc(&c->tile_off, MHPC_SORT_BUCKETS * c->sort_tiles_cap));
-    HIPC(dalloc(&c->digit_hist, MHPC_SORT_PASSES * MHPC_SORT_BUCKETS));
+    HIPC(dalloc(&c->digit_hist, MHPC_SORT_BUCKETS));
     double **sorted[] = {&c->sh, &c->sh2, &c->se, &c->srho, &c->sp, &c->scs};
     for (double **p : sorted) HIPC(dalloc(p, cap));
     HIPC(dalloc(&c->sxm, cap));

@@ -3,60 +3,63 @@
 // Replaces TreeNS::prepareSorting + HelperNS::sortArray = cub::DeviceRadixSort::SortPairs
 // (tree.cu:1404-1413, helper.cu:150-167): same result, a stable sort by key in which
 // ties keep ascending index order.  Eight passes of 8-bit digits.  Per pass:
-//   count   -- digit histogram of each 2048-key tile (LDS atomics);
-//   scan    -- one workgroup per digit scans the tile histograms (digit-major), adding
-//              the digit's global offset from the one-read histogram of all passes;
-//   scatter -- each wave ranks its 8 slots of 64 keys with a ballot multisplit (peers
+//   count   -- digit histogram of each tile (LDS atomics);
+//   scan    -- one workgroup per digit scans the tile histograms (digit-major) and writes the
+//              digit's total;
+//   scatter -- each wave ranks its slots of 64 keys with a ballot multisplit (peers
 //              = lanes holding the same digit), the block stages the tile in LDS in
-//              digit order and writes each digit run contiguously.
+//              digit order and writes each digit run contiguously, behind the keys of smaller
+//              digits (a scan of the 256 totals in every block: a separate pass over all keys for
+//              the digit totals took 13 us at 1M keys and 122 us at 16.7M).
+// Tiles of 2048 keys, of 1024 while these are at most SORT_SMALL_TILES: a tile's chain of ranking
+// steps is then the pass's time (sorts of 300,007 keys 107 us, 500,009 keys 121 us; 1,000,003 keys take
+// 172 us with the small tiles, 151 us with the large ones, 186 us before these two changes).
 // HBM bytes per pass: count reads 8 B/key, scatter reads 12 and writes 12.
 //
 // Small sets are sorted by rank instead (k_sort_rank, k_sort_merge): a key's place is the number
 // of keys before it, counted directly, which is one or two launches and no host wait.
+#include <algorithm>
 #include <mutex>
 
 #include "mhpc_internal.h"
 
 #define SORT_BLOCK 256
-#define SORT_ITEMS (MHPC_SORT_TILE / SORT_BLOCK)   // 16
 #define SORT_WAVES (SORT_BLOCK / 64)
+#define SORT_ITEMS_LARGE (MHPC_SORT_TILE / SORT_BLOCK)   // 8
+#define SORT_ITEMS_SMALL 4
+#define SORT_SMALL_TILES 512
 
-// digit histograms of passes [p_lo, p_hi) over all keys (one read of the keys)
-__global__ __launch_bounds__(SORT_BLOCK) void k_sort_hist_all(const uint64_t *__restrict__ keys,
-                                                              int64_t n,
-                                                              uint32_t *__restrict__ hist,
-                                                              uint32_t *__restrict__ check_flag, int p_lo,
-                                                              int p_hi) {
-    __shared__ uint32_t h[MHPC_SORT_PASSES * MHPC_SORT_BUCKETS];
-    if (blockIdx.x == 0 && threadIdx.x == 0) *check_flag = 0u;
-    for (int t = threadIdx.x; t < MHPC_SORT_PASSES * MHPC_SORT_BUCKETS; t += SORT_BLOCK) h[t] = 0;
-    __syncthreads();
-    int64_t i = blockIdx.x * (int64_t)SORT_BLOCK + threadIdx.x;
-    const int64_t stride = (int64_t)gridDim.x * SORT_BLOCK;
-    for (; i < n; i += stride) {
-        const uint64_t k = keys[i];
-#pragma unroll
-        for (int p = 0; p < MHPC_SORT_PASSES; p++)
-            if (p >= p_lo && p < p_hi)
-                atomicAdd(&h[p * MHPC_SORT_BUCKETS + (int)((k >> (MHPC_SORT_BITS * p)) & 255u)], 1u);
-    }
-    __syncthreads();
-    for (int t = threadIdx.x; t < MHPC_SORT_PASSES * MHPC_SORT_BUCKETS; t += SORT_BLOCK)
-        if (h[t]) atomicAdd(&hist[t], h[t]);
-}
-
+// check_flag (may be null): cleared for k_sort_check
+template <int ITEMS>
 __global__ __launch_bounds__(SORT_BLOCK) void k_sort_count(const uint64_t *__restrict__ keys,
                                                            int64_t n, int shift,
                                                            uint32_t *__restrict__ tile_hist,
-                                                           int64_t ntiles) {
+                                                           int64_t ntiles, uint32_t *check_flag) {
     __shared__ uint32_t h[MHPC_SORT_BUCKETS];
     h[threadIdx.x] = 0;
+    if (check_flag && blockIdx.x == 0 && threadIdx.x == 0) *check_flag = 0u;
     __syncthreads();
-    const int64_t base = (int64_t)blockIdx.x * MHPC_SORT_TILE;
-#pragma unroll 4
-    for (int s = 0; s < SORT_ITEMS; s++) {
-        int64_t idx = base + s * SORT_BLOCK + threadIdx.x;
-        if (idx < n) atomicAdd(&h[(int)((keys[idx] >> shift) & 255u)], 1u);
+    const int64_t base = (int64_t)blockIdx.x * (SORT_BLOCK * ITEMS);
+    uint64_t k[ITEMS];
+#pragma unroll
+    for (int s = 0; s < ITEMS; s++) {
+        const int64_t idx = base + s * SORT_BLOCK + threadIdx.x;
+        k[s] = idx < n ? keys[idx] : 0ull;
+    }
+#pragma unroll
+    for (int s = 0; s < ITEMS; s++) {
+        const bool valid = base + s * SORT_BLOCK + threadIdx.x < n;
+        const uint32_t d = (uint32_t)((k[s] >> shift) & 255u);
+        // a wave whose keys share the digit (the high digits of sorted or clustered keys) adds
+        // once: 64 LDS atomics on one word would serialise
+        const uint64_t m = wave_ballot(valid);
+        if (m == 0) continue;
+        const uint32_t d0 = __builtin_amdgcn_readfirstlane(d);
+        if (wave_ballot(valid && d != d0) == 0 && (m & 1ull)) {
+            if (wave_lane() == 0) atomicAdd(&h[d0], (uint32_t)popc64(m));
+        } else if (valid) {
+            atomicAdd(&h[d], 1u);
+        }
     }
     __syncthreads();
     tile_hist[(int64_t)threadIdx.x * ntiles + blockIdx.x] = h[threadIdx.x];
@@ -64,49 +67,59 @@ __global__ __launch_bounds__(SORT_BLOCK) void k_sort_count(const uint64_t *__res
 
 __global__ __launch_bounds__(SORT_BLOCK) void k_sort_scan(const uint32_t *__restrict__ tile_hist,
                                                           uint32_t *__restrict__ tile_off,
-                                                          int64_t ntiles,
-                                                          const uint32_t *__restrict__ digit_hist) {
+                                                          int64_t ntiles, uint32_t *__restrict__ digit_total) {
     __shared__ uint32_t lds4[SORT_WAVES];
     const int d = blockIdx.x;
-    // global offset of digit d = number of keys with a smaller digit in this pass
-    uint32_t part = (threadIdx.x < (unsigned)d) ? digit_hist[threadIdx.x] : 0u;
-    uint32_t dummy;
-    uint32_t carry = block_excl_scan256(part, &dummy, lds4);
-    block_scan_row(tile_hist + (int64_t)d * ntiles, tile_off + (int64_t)d * ntiles, ntiles, carry,
-                   lds4);
+    const uint32_t tot = block_scan_row(tile_hist + (int64_t)d * ntiles, tile_off + (int64_t)d * ntiles, ntiles, 0u,
+                                        lds4);
+    if (threadIdx.x == 0) digit_total[d] = tot;
 }
 
+template <int ITEMS>
 __global__ __launch_bounds__(SORT_BLOCK) void k_sort_scatter(const uint64_t *__restrict__ kin,
                                                              const int32_t *__restrict__ vin,
                                                              uint64_t *__restrict__ kout,
                                                              int32_t *__restrict__ vout, int64_t n,
                                                              int shift,
                                                              const uint32_t *__restrict__ tile_off,
-                                                             int64_t ntiles) {
-    __shared__ uint64_t skeys[MHPC_SORT_TILE];
-    __shared__ int32_t svals[MHPC_SORT_TILE];
+                                                             int64_t ntiles,
+                                                             const uint32_t *__restrict__ digit_total) {
+    constexpr int TILE = SORT_BLOCK * ITEMS;
+    __shared__ uint64_t skeys[TILE];
+    __shared__ int32_t svals[TILE];
     __shared__ uint32_t wcnt[SORT_WAVES][MHPC_SORT_BUCKETS];
     __shared__ uint32_t dstart[MHPC_SORT_BUCKETS];
     __shared__ uint32_t goff[MHPC_SORT_BUCKETS];
     __shared__ uint32_t lds4[SORT_WAVES];
 
     const int tid = threadIdx.x, w = tid / 64, lane = wave_lane();
-    const int64_t base = (int64_t)blockIdx.x * MHPC_SORT_TILE;
+    const int64_t base = (int64_t)blockIdx.x * TILE;
+    // the tile's keys and values are requested before the digit offsets' scan
+    uint64_t kr[ITEMS];
+    int32_t vr[ITEMS];
+    uint32_t rank[ITEMS];
+#pragma unroll
+    for (int s = 0; s < ITEMS; s++) {
+        const int64_t idx = base + (int64_t)w * (64 * ITEMS) + s * 64 + lane;
+        kr[s] = idx < n ? kin[idx] : 0ull;
+        vr[s] = idx < n ? (vin ? vin[idx] : (int32_t)idx) : 0;
+    }
 #pragma unroll
     for (int k = 0; k < SORT_WAVES; k++) wcnt[k][tid] = 0;
-    goff[tid] = tile_off[(int64_t)tid * ntiles + blockIdx.x];
+    {
+        const uint32_t off = tile_off[(int64_t)tid * ntiles + blockIdx.x];
+        uint32_t smaller;   // keys with a smaller digit
+        block_excl_scan256(digit_total[tid], &smaller, lds4);
+        goff[tid] = smaller + off;
+    }
     __syncthreads();
 
-    uint64_t kr[SORT_ITEMS];
-    int32_t vr[SORT_ITEMS];
-    uint32_t rank[SORT_ITEMS];
     const uint64_t lt = lanemask_lt();
 #pragma unroll
-    for (int s = 0; s < SORT_ITEMS; s++) {
-        const int64_t idx = base + (int64_t)w * (64 * SORT_ITEMS) + s * 64 + lane;
+    for (int s = 0; s < ITEMS; s++) {
+        const int64_t idx = base + (int64_t)w * (64 * ITEMS) + s * 64 + lane;
         const bool valid = idx < n;
-        const uint64_t key = valid ? kin[idx] : 0ull;
-        const int32_t val = valid ? (vin ? vin[idx] : (int32_t)idx) : 0;
+        const uint64_t key = kr[s];
         const uint32_t d = (uint32_t)((key >> shift) & 255u);
         uint64_t peers = wave_ballot(valid);
 #pragma unroll
@@ -121,8 +134,6 @@ __global__ __launch_bounds__(SORT_BLOCK) void k_sort_scatter(const uint64_t *__r
         wave_sync();
         if (valid && r == 0) wcnt[w][d] = prior + (uint32_t)popc64(peers);
         wave_sync();
-        kr[s] = key;
-        vr[s] = val;
         rank[s] = prior + r;
     }
     __syncthreads();
@@ -140,8 +151,8 @@ __global__ __launch_bounds__(SORT_BLOCK) void k_sort_scatter(const uint64_t *__r
     }
     __syncthreads();
 #pragma unroll
-    for (int s = 0; s < SORT_ITEMS; s++) {
-        const int64_t idx = base + (int64_t)w * (64 * SORT_ITEMS) + s * 64 + lane;
+    for (int s = 0; s < ITEMS; s++) {
+        const int64_t idx = base + (int64_t)w * (64 * ITEMS) + s * 64 + lane;
         if (idx < n) {
             const uint32_t d = (uint32_t)((kr[s] >> shift) & 255u);
             const uint32_t pos = dstart[d] + wcnt[w][d] + rank[s];
@@ -151,7 +162,7 @@ __global__ __launch_bounds__(SORT_BLOCK) void k_sort_scatter(const uint64_t *__r
     }
     __syncthreads();
     const int64_t rem = n - base;
-    const int cnt = rem < MHPC_SORT_TILE ? (int)rem : MHPC_SORT_TILE;
+    const int cnt = rem < TILE ? (int)rem : TILE;
     for (int t = tid; t < cnt; t += SORT_BLOCK) {
         const uint64_t key = skeys[t];
         const uint32_t d = (uint32_t)((key >> shift) & 255u);
@@ -274,11 +285,19 @@ struct SortBufs {
     int32_t *valB;
     uint64_t *kout;
     int32_t *vout;
-    uint32_t *tile_hist, *tile_off, *digit_hist;
+    uint32_t *tile_hist, *tile_off, *digit_total;
 };
-static void sort_passes(hipStream_t stream, int64_t n, int first, int64_t ntiles, const SortBufs &b);
+static void sort_passes(hipStream_t stream, int64_t n, int first, const SortBufs &b, uint32_t *check_flag);
 static SortBufs ctx_bufs(mhpc_ctx *c) {
     return SortBufs{c->key, c->keyB, c->valB, c->skey, c->perm, c->tile_hist, c->tile_off, c->digit_hist};
+}
+
+static bool sort_small_tiles(int64_t n) { return ceil_div(n, SORT_BLOCK * SORT_ITEMS_SMALL) <= SORT_SMALL_TILES; }
+
+// tiles of the largest sort up to cap keys
+int64_t sort_tiles_cap(int64_t cap) {
+    return std::max<int64_t>(ceil_div(cap, MHPC_SORT_TILE),
+                             std::min<int64_t>(ceil_div(cap, SORT_BLOCK * SORT_ITEMS_SMALL), SORT_SMALL_TILES));
 }
 
 // Adjacent sorted keys equal in the bits the passes sorted (>= shift): their order in the low
@@ -302,62 +321,60 @@ void launch_sort(mhpc_ctx *c) {
         sort_by_rank(c->stream, c->key, n, c->keyB, c->valB, c->skey, c->perm, false);
         return;
     }
-    const int64_t ntiles = ceil_div(n, MHPC_SORT_TILE);
-    launch_fill_u32(c, c->digit_hist, 0u, MHPC_SORT_PASSES * MHPC_SORT_BUCKETS);
-    int hb = (int)(ceil_div(n, SORT_BLOCK * 16) < 1024 ? ceil_div(n, SORT_BLOCK * 16) : 1024);
     const int levels = c->com_depth_hint + 2;
     const int first = levels < MHPC_LEVELS ? 3 * (MHPC_LEVELS - levels) / MHPC_SORT_BITS : 0;
-    hipLaunchKernelGGL(k_sort_hist_all, dim3(hb), dim3(SORT_BLOCK), 0, c->stream, c->key, n,
-                       c->digit_hist, c->sort_check, first, MHPC_SORT_PASSES);
     if (first > 0) {
-        sort_passes(c->stream, n, first, ntiles, ctx_bufs(c));
+        sort_passes(c->stream, n, first, ctx_bufs(c), c->sort_check);
         hipLaunchKernelGGL(k_sort_check, dim3((unsigned)ceil_div(n, 256)), dim3(256), 0, c->stream, c->skey, n,
                            MHPC_SORT_BITS * first, c->sort_check);
         if (ctx_fetch_status(c) == hipSuccess && c->h_status->sort_check == 0u) return;
-        // the full sort also needs the low passes' histograms
-        hipLaunchKernelGGL(k_sort_hist_all, dim3(hb), dim3(SORT_BLOCK), 0, c->stream, c->key, n,
-                           c->digit_hist, c->sort_check, 0, first);
     }
-    sort_passes(c->stream, n, 0, ntiles, ctx_bufs(c));
+    sort_passes(c->stream, n, 0, ctx_bufs(c), nullptr);
 }
 
 // LSD passes first .. MHPC_SORT_PASSES - 1 from the input keys; the last (odd) pass writes
 // kout / vout
-static void sort_passes(hipStream_t stream, int64_t n, int first, int64_t ntiles, const SortBufs &b) {
+template <int ITEMS>
+static void sort_passes_t(hipStream_t stream, int64_t n, int first, const SortBufs &b, uint32_t *check_flag) {
+    const unsigned ntiles = (unsigned)ceil_div(n, SORT_BLOCK * ITEMS);
     const uint64_t *kin = b.kin;
     const int32_t *vin = nullptr;
     for (int pass = first; pass < MHPC_SORT_PASSES; pass++) {
         uint64_t *kout = (pass & 1) ? b.kout : b.keyB;
         int32_t *vout = (pass & 1) ? b.vout : b.valB;
         const int shift = MHPC_SORT_BITS * pass;
-        hipLaunchKernelGGL(k_sort_count, dim3((unsigned)ntiles), dim3(SORT_BLOCK), 0, stream, kin, n, shift,
-                           b.tile_hist, ntiles);
+        hipLaunchKernelGGL(k_sort_count<ITEMS>, dim3(ntiles), dim3(SORT_BLOCK), 0, stream, kin, n, shift, b.tile_hist,
+                           (int64_t)ntiles, pass == first ? check_flag : nullptr);
         hipLaunchKernelGGL(k_sort_scan, dim3(MHPC_SORT_BUCKETS), dim3(SORT_BLOCK), 0, stream, b.tile_hist,
-                           b.tile_off, ntiles, b.digit_hist + pass * MHPC_SORT_BUCKETS);
-        hipLaunchKernelGGL(k_sort_scatter, dim3((unsigned)ntiles), dim3(SORT_BLOCK), 0, stream, kin, vin, kout,
-                           vout, n, shift, b.tile_off, ntiles);
+                           b.tile_off, (int64_t)ntiles, b.digit_total);
+        hipLaunchKernelGGL(k_sort_scatter<ITEMS>, dim3(ntiles), dim3(SORT_BLOCK), 0, stream, kin, vin, kout, vout, n,
+                           shift, b.tile_off, (int64_t)ntiles, b.digit_total);
         kin = kout;
         vin = vout;
     }
+}
+
+static void sort_passes(hipStream_t stream, int64_t n, int first, const SortBufs &b, uint32_t *check_flag) {
+    if (sort_small_tiles(n)) sort_passes_t<SORT_ITEMS_SMALL>(stream, n, first, b, check_flag);
+    else sort_passes_t<SORT_ITEMS_LARGE>(stream, n, first, b, check_flag);
 }
 
 // ------------------------------------------------------------------------------------
 // The key sort without allocation (mhpc_sort_keys_noalloc): the same passes on caller-owned
 // device arrays, with every buffer beyond the inputs and outputs carved from `scratch`, one
 // static array per GPU that lives until the process ends.  Layout (byte offsets, each
-// 256-aligned): even passes' keys and values, per-tile histograms and offsets, the all-pass
-// digit histogram, the check word k_sort_hist_all clears.
+// 256-aligned): even passes' keys and values, per-tile histograms and offsets, the digit totals.
 #define NA_TILES (MHPC_NOALLOC_SORT_MAX / MHPC_SORT_TILE)
 #define NA_KEYB 0
 #define NA_VALB (NA_KEYB + 8 * (size_t)MHPC_NOALLOC_SORT_MAX)
 #define NA_THIST (NA_VALB + 4 * (size_t)MHPC_NOALLOC_SORT_MAX)
 #define NA_TOFF (NA_THIST + 4 * (size_t)MHPC_SORT_BUCKETS * NA_TILES)
 #define NA_DHIST (NA_TOFF + 4 * (size_t)MHPC_SORT_BUCKETS * NA_TILES)
-#define NA_CHECK (NA_DHIST + 4 * (size_t)MHPC_SORT_PASSES * MHPC_SORT_BUCKETS)
-#define NA_BYTES (NA_CHECK + 256)
+#define NA_BYTES (NA_DHIST + 4 * (size_t)MHPC_SORT_BUCKETS)
 static_assert(MHPC_NOALLOC_SORT_MAX % MHPC_SORT_TILE == 0, "whole tiles");
 static_assert(NA_VALB % 256 == 0 && NA_THIST % 256 == 0 && NA_TOFF % 256 == 0 && NA_DHIST % 256 == 0 &&
-                  NA_CHECK % 256 == 0, "256-aligned parts");
+                  NA_BYTES % 256 == 0, "256-aligned parts");
+static_assert(NA_TILES >= SORT_SMALL_TILES, "the tables hold the small tiles too");
 
 static __device__ __align__(256) unsigned char scratch[NA_BYTES];
 
@@ -400,15 +417,6 @@ extern "C" int mhpc_sort_keys_noalloc(const uint64_t *keys, int64_t n, uint64_t 
                      overlaps(sorted_keys, sizeof(uint64_t) * (size_t)n) || overlaps(sorted, sizeof(int32_t) * (size_t)n));
         return hipGetLastError() == hipSuccess ? MHPC_OK : MHPC_E_HIP;
     }
-    uint32_t *digit_hist = reinterpret_cast<uint32_t *>(ptr + NA_DHIST);
-    uint32_t *check = reinterpret_cast<uint32_t *>(ptr + NA_CHECK);
-    // the digit histogram accumulates with atomics: cleared first (the previous call's counts
-    // are still there)
-    fill_u32_on(s, digit_hist, 0u, MHPC_SORT_PASSES * MHPC_SORT_BUCKETS);
-    const int64_t ntiles = ceil_div(n, MHPC_SORT_TILE);
-    const int hb = (int)(ceil_div(n, SORT_BLOCK * 16) < 1024 ? ceil_div(n, SORT_BLOCK * 16) : 1024);
-    hipLaunchKernelGGL(k_sort_hist_all, dim3(hb), dim3(SORT_BLOCK), 0, s, keys, n, digit_hist, check, 0,
-                       MHPC_SORT_PASSES);
     const SortBufs b{keys,
                      reinterpret_cast<uint64_t *>(ptr + NA_KEYB),
                      reinterpret_cast<int32_t *>(ptr + NA_VALB),
@@ -416,7 +424,7 @@ extern "C" int mhpc_sort_keys_noalloc(const uint64_t *keys, int64_t n, uint64_t 
                      sorted,
                      reinterpret_cast<uint32_t *>(ptr + NA_THIST),
                      reinterpret_cast<uint32_t *>(ptr + NA_TOFF),
-                     digit_hist};
-    sort_passes(s, n, 0, ntiles, b);
+                     reinterpret_cast<uint32_t *>(ptr + NA_DHIST)};
+    sort_passes(s, n, 0, b, nullptr);
     return hipGetLastError() == hipSuccess ? MHPC_OK : MHPC_E_HIP;
 }

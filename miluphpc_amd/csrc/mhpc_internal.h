@@ -29,7 +29,7 @@
 #define MHPC_SORT_BITS 8
 #define MHPC_SORT_BUCKETS 256
 #define MHPC_SORT_PASSES 8
-#define MHPC_SORT_TILE 2048    // keys per scatter block (256 threads x 8)
+#define MHPC_SORT_TILE 2048    // keys per scatter block (256 threads x 8; small sorts 256 x 4)
 #define MHPC_TREE_TILE 1024     // positions per tree block (256 threads x 4)
 #define MHPC_TREE_SMALL_TILES 1024   // up to this many tiles of 256 positions (256 threads x 1) instead
 #define MHPC_HTABLE_MAX 4096    // h-iteration factor table size
@@ -102,7 +102,7 @@ struct mhpc_ctx {
     uint32_t *sort_check = nullptr;              // = &dstatus->sort_check
     int32_t *cpar = nullptr;                     // cell -> parent cell (tree build)
     uint32_t *tile_hist = nullptr, *tile_off = nullptr;
-    uint32_t *digit_hist = nullptr;              // [passes][256]
+    uint32_t *digit_hist = nullptr;              // [256] digit totals of the current pass
     int64_t sort_tiles_cap = 0;
     uint64_t *slkey = nullptr;                   // Lebesgue keys in sorted order
 
@@ -206,6 +206,7 @@ void launch_keys(mhpc_ctx *c);
 // bounding box's launch
 void launch_bbox_keys(mhpc_ctx *c, const std::function<void()> &between);
 void launch_sort(mhpc_ctx *c);
+int64_t sort_tiles_cap(int64_t cap);
 void launch_gather(mhpc_ctx *c, bool gravity, bool sph, bool rhs);
 void launch_tree(mhpc_ctx *c);
 // sph: also the cells' largest h from the key-sorted h (sh must hold the gathered h)
