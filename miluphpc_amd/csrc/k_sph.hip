@@ -1611,51 +1611,48 @@ void launch_neighbours(mhpc_ctx *c) {
 }
 
 // ------------------------------------------------------------------------------------
-// a10 cubic spline (kernel.cu:50-83), support radius h.  FP64 form: the reference's
-// expressions in the same order; FP32 form: the same formula in float.
-#define MHPC_8_OVER_PI_F 2.546479089470325f
-
-__device__ __forceinline__ void cubic32(float r, float h, float &W, float &dWdr) {
-    const float hinv = 1.0f / h;
-    const float q = r * hinv;
-    const float f = MHPC_8_OVER_PI_F * hinv * hinv * hinv;
-    const float omq = 1.0f - q;
-    if (q > 1.0f) {
-        W = 0.f;
-        dWdr = 0.f;
-    } else if (q > 0.5f) {
-        W = 2.f * f * omq * omq * omq;
-        dWdr = -6.f * f * hinv * omq * omq;
-    } else {
-        W = f * __builtin_fmaf(6.f * q * q, q - 1.0f, 1.0f);
-        dWdr = 6.f * f * hinv * q * __builtin_fmaf(3.f, q, -2.f);
-    }
-}
-
-// ------------------------------------------------------------------------------------
 // a11 density (density.cu:8-72): rho_i = m_i W(0, h_i) + sum_j m_j W(r_ij, h_ij).
 // Neighbour records are read as one 32-byte {x,y,z,m} plus h; the loop is unrolled so a
 // wave keeps several independent gathers in flight.
 #define K8PI 2.5464790894703255   // 8 / pi
 
-// 1/x and 1/sqrt(x) from the hardware estimates (v_rcp_f64, v_rsq_f64) refined by two
-// Newton-Raphson steps each, for positive normal x: a few FP64 ulp, several instructions
-// fewer than a correctly rounded division / square root
-__device__ __forceinline__ double rcp_nr(double x) {
-    double y = __builtin_amdgcn_rcp(x);
-    double e = fma(-x, y, 1.0);
-    y = fma(y, e, y);
-    e = fma(-x, y, 1.0);
-    return fma(y, e, y);
+// a10 cubic spline (kernel.cu:50-83), support radius h, q = r / h: W = 8/pi h^-3 w(q) with
+// w = 1 + 6 q^2 (q - 1) up to q = 1/2, 2 (1 - q)^3 up to 1, and 0 beyond.  The pair loops evaluate
+// both branches and select: their lanes take different ones, so a wavefront pays for both anyway,
+// and a NaN q (coincident particles) selects 0.
+template <typename T>
+__device__ __forceinline__ T cubic_w(T q) {
+    const T t = T(1) - q;
+    const T a = fma(T(6) * q * q, q - T(1), T(1)), b = (t + t) * (t * t);
+    const T w = q <= T(0.5) ? a : b;
+    return q <= T(1) ? w : T(0);
+}
+// (dW/dr) / r without its factor 6 * 8/pi h^-4: (3 q - 2) / h up to q = 1/2 (q / r = 1 / h), else
+// -(1 - q)^2 / r
+template <typename T>
+__device__ __forceinline__ T cubic_grad(T q, T ih, T rinv) {
+    const T t = T(1) - q;
+    const T a = ih * fma(T(3), q, T(-2)), b = -(rinv * (t * t));
+    const T s = q <= T(0.5) ? a : b;
+    return q <= T(1) ? s : T(0);
 }
 
-__device__ __forceinline__ double rsq_nr(double x) {
-    double y = __builtin_amdgcn_rsq(x);
-    const double hx = 0.5 * x;
-    double e = fma(-hx, y * y, 0.5);
-    y = fma(y, e, y);
-    e = fma(-hx, y * y, 0.5);
-    return fma(y, e, y);
+// 1/x of a positive normal x from the hardware estimate (2^-23 at least) and one third-order step
+// y (1 + e + e^2), e = 1 - x y: the error of a correctly rounded division (0.998 x 2^-53 largest
+// over 2^20 arguments), in three instructions after the estimate.  1/sqrt(x): rsq_f64.
+__device__ __forceinline__ double rcp_f64(double x) {
+    const double y = __builtin_amdgcn_rcp(x);
+    const double e = fma(-x, y, 1.0);
+    return fma(y, fma(e, e, e), y);
+}
+// the same in FP32, one Newton step from the estimates (1 ulp)
+__device__ __forceinline__ float rcp_f32(float x) {
+    const float y = __builtin_amdgcn_rcpf(x);
+    return __builtin_fmaf(y, __builtin_fmaf(-x, y, 1.f), y);
+}
+__device__ __forceinline__ float rsq_f32(float x) {
+    const float y = __builtin_amdgcn_rsqf(x);
+    return __builtin_fmaf(0.5f * y, __builtin_fmaf(-(x * y), y, 1.f), y);
 }
 
 // a10, the five kernels of SPH::SmoothingKernel (kernel.cu:14-183, 3D branches; Dehnen & Aly
@@ -1790,49 +1787,33 @@ static EosArgs eos_args(mhpc_ctx *c) {
 template <bool FP64, bool CUBIC>
 __device__ __forceinline__ void density_pair(const double4 &pi, double hi, const double4 &pj, double hj,
                                              int sml_avg, int kind, double &acc, Kahan &acc32) {
-    if constexpr (!CUBIC) {
-        if constexpr (FP64) {
-            const double hb = sml_avg ? 0.5 * (hi + hj) : hi;
-            const double dx = pi.x - pj.x, dy = pi.y - pj.y, dz = pi.z - pj.z;
-            const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
-            const double ih = rcp_nr(hb);
-            const double q = r2 * rsq_nr(r2) * ih;
-            if (q <= 1.0) {
-                double w, dw;
-                kernel_shape<double>(kind, q, w, dw);
-                acc = fma(pj.w, kernel_sigma(kind) * (ih * ih * ih) * w, acc);
-            }
-        } else {
-            const float hb = (float)(sml_avg ? 0.5 * (hi + hj) : hi);
-            const float dx = (float)(pi.x - pj.x), dy = (float)(pi.y - pj.y), dz = (float)(pi.z - pj.z);
-            const float ih = 1.0f / hb;
-            const float q = sqrtf(__builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz))) * ih;
-            if (q <= 1.0f) {
-                float w, dw;
-                kernel_shape<float>(kind, q, w, dw);
-                acc32.add((float)pj.w * ((float)kernel_sigma(kind) * ih * ih * ih * w));
-            }
-        }
-        return;
-    }
+    const double hb = sml_avg ? 0.5 * (hi + hj) : hi;
     if constexpr (FP64) {
-        const double hb = sml_avg ? 0.5 * (hi + hj) : hi;
         const double dx = pi.x - pj.x, dy = pi.y - pj.y, dz = pi.z - pj.z;
         const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
-        const double ih = rcp_nr(hb);
-        const double q = r2 * rsq_nr(r2) * ih;
-        const double f = K8PI * (ih * ih * ih);
-        double W = 0.0;
-        if (q <= 0.5) W = f * fma(6.0 * q * q, q - 1.0, 1.0);
-        else if (q <= 1.0) { const double t = 1.0 - q; W = 2.0 * f * (t * t * t); }
-        acc = fma(pj.w, W, acc);
+        const double ih = rcp_f64(hb);
+        const double q = r2 * rsq_f64(r2) * ih;
+        const double ih3 = ih * ih * ih;
+        if constexpr (CUBIC) {
+            acc = fma(pj.w * (K8PI * ih3), cubic_w(q), acc);
+        } else if (q <= 1.0) {
+            double w, dw;
+            kernel_shape<double>(kind, q, w, dw);
+            acc = fma(pj.w, kernel_sigma(kind) * ih3 * w, acc);
+        }
     } else {
-        const float hb = (float)(sml_avg ? 0.5 * (hi + hj) : hi);
         const float dx = (float)(pi.x - pj.x), dy = (float)(pi.y - pj.y), dz = (float)(pi.z - pj.z);
-        const float rr = sqrtf(__builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz)));
-        float W, dW;
-        cubic32(rr, hb, W, dW);
-        acc32.add((float)pj.w * W);
+        const float r2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
+        const float ih = rcp_f32((float)hb);
+        const float q = r2 * rsq_f32(r2) * ih;
+        const float ih3 = ih * ih * ih;
+        if constexpr (CUBIC) {
+            acc32.add((float)pj.w * ((float)K8PI * ih3) * cubic_w(q));
+        } else if (q <= 1.0f) {
+            float w, dw;
+            kernel_shape<float>(kind, q, w, dw);
+            acc32.add((float)pj.w * ((float)kernel_sigma(kind) * ih3 * w));
+        }
     }
 }
 
@@ -1905,8 +1886,8 @@ __global__ __launch_bounds__(DENS_WIN) void k_density(int64_t n, const double4 *
     #pragma unroll
             for (int e = 0; e < 8; e++) {
                 const int32_t j = e < m ? jj[e] : (int32_t)k;
-                const uint64_t o = (uint64_t)((int64_t)j - base);
-                const bool in = o < (uint64_t)DENS_WIN;
+                const uint32_t o = (uint32_t)(j - (int32_t)base);
+                const bool in = o < (uint32_t)DENS_WIN;
                 const int oc = in ? (int)o : 0;
                 pj[e] = wp[oc];
                 hj[e] = wh[oc];
@@ -2099,7 +2080,7 @@ struct ForceAcc<true> {
 };
 template <>
 struct ForceAcc<false> {
-    Kahan a0, a1, a2, drho, de, dsml;
+    Kahan a0, a1, a2, dvv, de;
 };
 
 struct ForceI {   // particle i's data and the constants of the pair loop
@@ -2110,131 +2091,100 @@ struct ForceI {   // particle i's data and the constants of the pair loop
 };
 
 // one pair (i, j) of the force loop; j's records {x,y,z,m}, {vx,vy,vz,cs},
-// {rho, p/rho^2, m/rho, h}
+// {rho, p/rho^2, m/rho, h}.  The loop is bound by its instructions as much as by its gathers, so
+// every shared factor is taken out: with grad W = gs r_ij, v.grad W = gs (v.r_ij) and the
+// acceleration is (fa gs) r_ij; the viscosity Pi_ij = (beta mu - alpha c) mu / rho with
+// mu = h v.r / D, D = r^2 + 0.01 h^2, is taken as one quotient over D^2 rho (two reciprocals fewer
+// instructions than dividing by D and by rho).  112 -> 96 vector instructions per FP64 pair (256^3 RHS 18.1 ->
+// 17.9 ms).
+// mu is negative wherever it is used, so the largest mu_ij, which starts at 0
+// (internal_forces.cu:135, :383-385), is always 0.
 template <bool FP64, bool FEAT, bool CUBIC>
 __device__ __forceinline__ void force_pair(const ForceI &I, const double4 &pj, const double4 &vj, const double4 &rj,
-                                           ForceAcc<FP64> &acc, double &mumax, double *feat) {
+                                           ForceAcc<FP64> &acc, double *feat) {
+    typedef typename std::conditional<FP64, double, float>::type T;
     const double4 pi = I.p, vi = I.v, ri = I.r;
+    const T hi = (T)I.h, hj = (T)rj.w;
+    const T hs = hi + hj;
+    const T hb = T(0.5) * hs;
+    const T sml = I.sml_avg ? hb : hi;
+    const T d0 = (T)(pi.x - pj.x), d1 = (T)(pi.y - pj.y), d2 = (T)(pi.z - pj.z);
+    const T v0 = (T)(vi.x - vj.x), v1 = (T)(vi.y - vj.y), v2 = (T)(vi.z - vj.z);
+    const T r2 = fma(d0, d0, fma(d1, d1, d2 * d2));
+    T rinv, ih;
     if constexpr (FP64) {
-        const double hi = I.h;
-        const double hj = rj.w;
-        const double hb = 0.5 * (hi + hj);
-        const double sml = I.sml_avg ? hb : hi;
-        const double d0 = pi.x - pj.x, d1 = pi.y - pj.y, d2 = pi.z - pj.z;
-        const double r2 = fma(d0, d0, fma(d1, d1, d2 * d2));
-        const double rinv = rsq_nr(r2);
-        const double ih = rcp_nr(sml);
-        const double q = r2 * rinv * ih;
-        const double ih2 = ih * ih;
-        // grad W = (dW/dr / r) r_ij
-        double gs = 0.0;
-        if constexpr (CUBIC) {
-            // for q <= 1/2, dW/dr / r = 6 f/h (3q - 2) q / r with q / r = 1/h
-            const double fih = K8PI * (ih2 * ih2);
-            if (q <= 0.5) gs = fih * ih * fma(18.0, q, -12.0);
-            else if (q <= 1.0) { const double t = 1.0 - q; gs = -6.0 * fih * (t * t) * rinv; }
-        } else if (q <= 1.0) {
-            double w, dw;
-            kernel_shape<double>(I.kind, q, w, dw);
-            gs = kernel_sigma(I.kind) * (ih2 * ih2) * dw * rinv;
-        }
-        const double g0 = gs * d0, g1 = gs * d1, g2 = gs * d2;
-        const double v0 = vi.x - vj.x, v1 = vi.y - vj.y, v2 = vi.z - vj.z;
-        const double vv = fma(v0, g0, fma(v1, g1, v2 * g2));
-        const double vr = fma(v0, d0, fma(v1, d1, v2 * d2));
-        double mpij = 0.0;
-        if (vr < 0) {
-            const double csbar = 0.5 * (vi.w + vj.w);
-            const double mu = hb * vr * rcp_nr(fma(hb * hb, 1e-2, r2));
-            mumax = fmax(mumax, mu);
-            const double rhobar = 0.5 * (ri.x + rj.x);
-            mpij = pj.w * fma(I.beta, mu, -I.alpha * csbar) * mu * rcp_nr(rhobar);
-        }
-        const double pf = -pj.w * (ri.y + rj.y);
-        const double fa = pf - mpij;
-        acc.a0 = fma(fa, g0, acc.a0);
-        acc.a1 = fma(fa, g1, acc.a1);
-        acc.a2 = fma(fa, g2, acc.a2);
+        rinv = rsq_f64(r2);
+        ih = rcp_f64(sml);
+    } else {
+        rinv = rsq_f32(r2);
+        ih = rcp_f32(sml);
+    }
+    const T q = r2 * rinv * ih;
+    const T ih2 = ih * ih;
+    // grad W = gs r_ij, gs = (dW/dr) / r
+    T gs = T(0);
+    if constexpr (CUBIC) {
+        gs = T(6 * K8PI) * (ih2 * ih2) * cubic_grad(q, ih, rinv);
+    } else if (q <= T(1)) {
+        T w, dw;
+        kernel_shape<T>(I.kind, q, w, dw);
+        gs = (T)kernel_sigma(I.kind) * (ih2 * ih2) * dw * rinv;
+    }
+    const T vr = fma(v0, d0, fma(v1, d1, v2 * d2));
+    const T vv = gs * vr;   // v.grad W
+    const T mj = (T)pj.w;
+    // m_j Pi_ij = m (2 h v.r) (beta/2 (2 h v.r) - alpha c D) / (D^2 (rho_i + rho_j)), c the mean
+    // sound speed
+    const T D = fma(hb * hb, T(1e-2), r2);
+    const T x = hs * vr;
+    const T cD = T(0.5) * ((T)vi.w + (T)vj.w) * D;
+    const T num = mj * x * fma(T(0.5) * (T)I.beta, x, -(T)I.alpha * cD);
+    const T den = D * D * ((T)ri.x + (T)rj.x);
+    T mpij;
+    if constexpr (FP64) mpij = num * rcp_f64(den);
+    else mpij = num * rcp_f32(den);
+    mpij = vr < T(0) ? mpij : T(0);
+    const T pf = -mj * ((T)ri.y + (T)rj.y);
+    const T fa = (pf - mpij) * gs;
+    const T rv = (T)rj.z * vv;
+    const T ev = (mpij - pf) * vv;
+    if constexpr (FP64) {
+        acc.a0 = fma(fa, d0, acc.a0);
+        acc.a1 = fma(fa, d1, acc.a1);
+        acc.a2 = fma(fa, d2, acc.a2);
         acc.dvv = fma(rj.z, vv, acc.dvv);   // the drho/dt and dh/dt sums are the same sum
         acc.de = fma(mpij - pf, vv, acc.de);
-        if (FEAT) {
-            feat[0] += rj.z * (v1 * g2 - v2 * g1);
-            feat[1] += rj.z * (v2 * g0 - v0 * g2);
-            feat[2] += rj.z * (v0 * g1 - v1 * g0);
-            feat[3] += pj.w * g0;
-            feat[4] += pj.w * g1;
-            feat[5] += pj.w * g2;
-        }
     } else {
-        const float hif = (float)I.h, rhoif = (float)ri.x, csif = (float)vi.w, prif = (float)ri.y;
-        const float alpha = (float)I.alpha, beta = (float)I.beta;
-        const float hj = (float)rj.w;
-        const float hb = 0.5f * (hif + hj);
-        const float sml = I.sml_avg ? hb : hif;
-        const float d0 = (float)(pi.x - pj.x), d1 = (float)(pi.y - pj.y), d2 = (float)(pi.z - pj.z);
-        const float v0 = (float)(vi.x - vj.x), v1 = (float)(vi.y - vj.y), v2 = (float)(vi.z - vj.z);
-        const float r2 = __builtin_fmaf(d0, d0, __builtin_fmaf(d1, d1, d2 * d2));
-        const float r = sqrtf(r2);
-        float W, dWdr;
-        if constexpr (CUBIC) {
-            cubic32(r, sml, W, dWdr);
-        } else {
-            const float ih = 1.0f / sml;
-            const float q = r * ih;
-            float w = 0.f, dw = 0.f;
-            if (q <= 1.0f) kernel_shape<float>(I.kind, q, w, dw);
-            dWdr = (float)kernel_sigma(I.kind) * (ih * ih) * (ih * ih) * dw;
-        }
-        const float gs = dWdr / r;
-        const float g0 = gs * d0, g1 = gs * d1, g2 = gs * d2;
-        const float vv = __builtin_fmaf(v0, g0, __builtin_fmaf(v1, g1, v2 * g2));
-        const float vr = __builtin_fmaf(v0, d0, __builtin_fmaf(v1, d1, v2 * d2));
-        const float mj = (float)pj.w;
-        float mpij = 0.f;
-        if (vr < 0.f) {
-            const float csbar = 0.5f * (csif + (float)vj.w);
-            const float mu = hb * vr / __builtin_fmaf(hb * hb, 1e-2f, r2);
-            mumax = fmax(mumax, (double)mu);
-            const float rhobar = 0.5f * (rhoif + (float)rj.x);
-            mpij = mj * (beta * mu - alpha * csbar) * mu / rhobar;
-        }
-        const float pf = -mj * (prif + (float)rj.y);
-        const float fa = pf - mpij;
-        acc.a0.add(fa * g0);
-        acc.a1.add(fa * g1);
-        acc.a2.add(fa * g2);
-        const float mr_vv = (float)rj.z * vv;
-        acc.drho.add(mr_vv);
-        acc.dsml.add(mr_vv);
-        acc.de.add((mpij - pf) * vv);
-        if (FEAT) {
-            const float vjr = (float)rj.z;
-            feat[0] += vjr * (v1 * g2 - v2 * g1);
-            feat[1] += vjr * (v2 * g0 - v0 * g2);
-            feat[2] += vjr * (v0 * g1 - v1 * g0);
-            feat[3] += mj * g0;
-            feat[4] += mj * g1;
-            feat[5] += mj * g2;
-        }
+        acc.a0.add(fa * d0);
+        acc.a1.add(fa * d1);
+        acc.a2.add(fa * d2);
+        acc.dvv.add(rv);
+        acc.de.add(ev);
+    }
+    if (FEAT) {
+        const T rg = (T)rj.z * gs, mg = mj * gs;
+        feat[0] += rg * (v1 * d2 - v2 * d1);
+        feat[1] += rg * (v2 * d0 - v0 * d2);
+        feat[2] += rg * (v0 * d1 - v1 * d0);
+        feat[3] += mg * d0;
+        feat[4] += mg * d1;
+        feat[5] += mg * d2;
     }
 }
 
-// a particle's accumulated sums (drho and dsml share one sum in FP64)
+// a particle's accumulated sums (drho/dt and dh/dt share one)
 struct ForceSums {
-    double a[3], drho, dsml, de, mumax, feat[6];
-    __device__ __forceinline__ void take(const ForceAcc<true> &s, double mu, const double *f) {
+    double a[3], dvv, de, feat[6];
+    __device__ __forceinline__ void take(const ForceAcc<true> &s, const double *f) {
         a[0] = s.a0; a[1] = s.a1; a[2] = s.a2;
-        drho = dsml = s.dvv;
+        dvv = s.dvv;
         de = s.de;
-        mumax = mu;
         for (int q = 0; q < 6; q++) feat[q] = f[q];
     }
-    __device__ __forceinline__ void take(const ForceAcc<false> &s, double mu, const double *f) {
+    __device__ __forceinline__ void take(const ForceAcc<false> &s, const double *f) {
         a[0] = s.a0.value(); a[1] = s.a1.value(); a[2] = s.a2.value();
-        drho = s.drho.value();
-        dsml = s.dsml.value();
+        dvv = s.dvv.value();
         de = s.de.value();
-        mumax = mu;
         for (int q = 0; q < 6; q++) feat[q] = f[q];
     }
 };
@@ -2245,10 +2195,10 @@ __device__ __forceinline__ void force_store(const ForceArgs &A, int64_t k, const
     A.ax[i] = S.a[0];
     A.ay[i] = S.a[1];
     A.az[i] = S.a[2];
-    A.drhodt[i] = I.r.x * S.drho;
+    A.drhodt[i] = I.r.x * S.dvv;
     A.dedt[i] = 0.5 * S.de;
-    A.dsmldt[i] = -(1.0 / 3.0) * I.h * S.dsml;
-    A.muijmax[i] = S.mumax;
+    A.dsmldt[i] = -(1.0 / 3.0) * I.h * S.dvv;
+    A.muijmax[i] = 0.0;   // see force_pair
     if (FEAT) {
         const double *f = S.feat;
         A.curlv[i] = sqrt(f[0] * f[0] + f[1] * f[1] + f[2] * f[2]);
@@ -2286,7 +2236,6 @@ __global__ __launch_bounds__(FORCE_WIN) void k_forces(ForceArgs A) {
     int cnt = A.snoi[k];
     cnt = cnt > A.max_nb ? A.max_nb : cnt;
     ForceAcc<FP64> acc;
-    double mumax = 0.0;
     double feat[6] = {0, 0, 0, 0, 0, 0};
     const int4 *nrow = reinterpret_cast<const int4 *>(A.nbr) + k;   // row r at nrow[r * stride]
     const int64_t stride = A.stride;
@@ -2305,8 +2254,8 @@ __global__ __launch_bounds__(FORCE_WIN) void k_forces(ForceArgs A) {
 #pragma unroll
             for (int e = 0; e < 2; e++) {
                 const int32_t j = h + e < m ? jj[h + e] : (int32_t)k;
-                const uint64_t o = (uint64_t)((int64_t)j - base);
-                const bool in = o < (uint64_t)FORCE_WIN;
+                const uint32_t o = (uint32_t)(j - (int32_t)base);
+                const bool in = o < (uint32_t)FORCE_WIN;
                 const int oc = in ? (int)o : 0;
                 pj[e] = wp[oc];
                 vj[e] = wv[oc];
@@ -2319,11 +2268,11 @@ __global__ __launch_bounds__(FORCE_WIN) void k_forces(ForceArgs A) {
             }
 #pragma unroll
             for (int e = 0; e < 2; e++)
-                if (h + e < m) force_pair<FP64, FEAT, CUBIC>(I, pj[e], vj[e], rj[e], acc, mumax, feat);
+                if (h + e < m) force_pair<FP64, FEAT, CUBIC>(I, pj[e], vj[e], rj[e], acc, feat);
         }
     }
     ForceSums S;
-    S.take(acc, mumax, feat);
+    S.take(acc, feat);
     force_store<FEAT>(A, k, I, S);
 }
 
@@ -2333,7 +2282,6 @@ __global__ __launch_bounds__(256) void k_forces_split(ForceArgs A) {
     const int64_t k = xcd_block(blockIdx.x, gridDim.x) * (256 / SPLIT_LANES) + threadIdx.x / SPLIT_LANES;
     const int sub = threadIdx.x % SPLIT_LANES;
     ForceAcc<FP64> acc;
-    double mumax = 0.0;
     double feat[6] = {0, 0, 0, 0, 0, 0};
     ForceI I = {};
     if (k < A.n) {
@@ -2364,18 +2312,16 @@ __global__ __launch_bounds__(256) void k_forces_split(ForceArgs A) {
                 }
 #pragma unroll
                 for (int e = 0; e < 2; e++)
-                    if (h + e < m) force_pair<FP64, FEAT, CUBIC>(I, pj[e], vj[e], rj[e], acc, mumax, feat);
+                    if (h + e < m) force_pair<FP64, FEAT, CUBIC>(I, pj[e], vj[e], rj[e], acc, feat);
             }
         }
     }
     ForceSums S;
-    S.take(acc, mumax, feat);
+    S.take(acc, feat);
 #pragma unroll
     for (int q = 0; q < 3; q++) S.a[q] = row_sum(S.a[q]);
-    S.drho = row_sum(S.drho);
-    S.dsml = FP64 ? S.drho : row_sum(S.dsml);
+    S.dvv = row_sum(S.dvv);
     S.de = row_sum(S.de);
-    S.mumax = row_max(S.mumax);
     if (FEAT)
 #pragma unroll
         for (int q = 0; q < 6; q++) S.feat[q] = row_sum(S.feat[q]);
