@@ -47,11 +47,19 @@ static_assert(64 / NN_SPLIT_MIN <= MHPC_NN_PARTS_PER_GROUP, "the part list holds
 // in Hilbert order).
 #define NN_FEW 32768
 static_assert(NN_FEW <= NN_DIRECT_MAX, "the direct form declines no box of so few particles");
-#define NN_DU 8              // direct form: candidates per lane and round (loads in flight)
+#define NN_DU 4              // direct form: candidates per lane and round (loads in flight; 2 / 4 / 8 alike)
+
+// per-wave LDS of the direct form: its candidate ranges (first particle less the number of
+// candidates before the range) and where ranges begin among the candidates of a round
+struct NNDirectLds {
+    int off[NN_DRANGES];
+    unsigned long long head[NN_DU];
+};
+struct NNNoDirect {};
 
 // per-wave LDS of the walker; TCAP = 128 gives the filtered walk room to compact the
 // candidates of two 64-particle loads before a full tile of 64 is handed on
-template <int TCAP, int DR>
+template <int TCAP, typename Direct>
 struct NNWaveLdsT {
     int stack[NN_STACK_PHYS];
     int rstart[NN_RANGES];
@@ -59,10 +67,10 @@ struct NNWaveLdsT {
     int rpre[64];
     double tx[TCAP], ty[TCAP], tz[TCAP], th2[TCAP];
     int tj[TCAP];
-    int drs[DR], drp[DR];   // direct form: candidate ranges (first particle, exclusive prefix)
+    Direct direct;
 };
-using NNWaveLds = NNWaveLdsT<64, NN_DRANGES>;
-using NNWaveLdsF = NNWaveLdsT<128, 1>;
+using NNWaveLds = NNWaveLdsT<64, NNDirectLds>;
+using NNWaveLdsF = NNWaveLdsT<128, NNNoDirect>;
 
 // candidate filter that keeps everything (per-particle walks test each candidate once)
 struct KeepAll {
@@ -210,6 +218,8 @@ struct NNStart {
     int ilx, ihx, ily, ihy, ilz, ihz;  // the box corners' cell indices at level kmax
 };
 
+// Called by all lanes together with the same box.  The six bisections run side by side, one per
+// lane (one after the other they are a sixth of a direct search's instructions).
 template <int SPAN = 3>
 __device__ __forceinline__ NNStart nn_start_level(const NNArgs &A, double lox, double hix, double loy,
                                                   double hiy, double loz, double hiz) {
@@ -217,13 +227,16 @@ __device__ __forceinline__ NNStart nn_start_level(const NNArgs &A, double lox, d
     const int K0 = A.stab ? A.kmax : 0;
     S.s = K0;
     if (K0 > 0) {
-        const double b0 = A.box[0], b1 = A.box[1], b2 = A.box[2], b3 = A.box[3], b4 = A.box[4], b5 = A.box[5];
-        S.ilx = nn_axis_index(lox, b0, b1, K0);
-        S.ihx = nn_axis_index(hix, b0, b1, K0);
-        S.ily = nn_axis_index(loy, b2, b3, K0);
-        S.ihy = nn_axis_index(hiy, b2, b3, K0);
-        S.ilz = nn_axis_index(loz, b4, b5, K0);
-        S.ihz = nn_axis_index(hiz, b4, b5, K0);
+        const int side = wave_lane() & 7;   // {lo, hi} of x, y, z
+        const double vx = side & 1 ? hix : lox, vy = side & 1 ? hiy : loy, vz = side & 1 ? hiz : loz;
+        const int axis = side < 6 ? side >> 1 : 0;
+        const int idx = nn_axis_index(axis == 0 ? vx : axis == 1 ? vy : vz, A.box[2 * axis], A.box[2 * axis + 1], K0);
+        S.ilx = __builtin_amdgcn_readlane(idx, 0);
+        S.ihx = __builtin_amdgcn_readlane(idx, 1);
+        S.ily = __builtin_amdgcn_readlane(idx, 2);
+        S.ihy = __builtin_amdgcn_readlane(idx, 3);
+        S.ilz = __builtin_amdgcn_readlane(idx, 4);
+        S.ihz = __builtin_amdgcn_readlane(idx, 5);
         int s = 0;
         while (s < K0 && ((S.ihx >> s) - (S.ilx >> s) > SPAN || (S.ihy >> s) - (S.ily >> s) > SPAN ||
                           (S.ihz >> s) - (S.ilz >> s) > SPAN))
@@ -253,14 +266,16 @@ __device__ __forceinline__ bool nn_win_clip(int w0, int w1, int &rs, int &rc, in
 
 // Lebesgue prefix of the level-K cell with the per-axis indices (ix, iy, iz) (the lower half of
 // an axis sets its key bit, so the indices' bits enter inverted).
-__device__ __forceinline__ uint64_t nn_cell_prefix(int ix, int iy, int iz, int K) {
-    uint64_t P = 0;
-    for (int l = K - 1; l >= 0; l--) {
-        const uint64_t d = (uint64_t)(((ix >> l) & 1) ^ 1) | ((uint64_t)(((iy >> l) & 1) ^ 1) << 1) |
-                           ((uint64_t)(((iz >> l) & 1) ^ 1) << 2);
-        P = (P << 3) | d;
-    }
-    return P;
+static_assert(MHPC_NN_KMAX <= 10, "a prefix of the start table has at most 30 bits");
+__device__ __forceinline__ uint32_t nn_spread3(uint32_t v) {   // bit b of ten to bit 3 b
+    v = (v | v << 16) & 0x030000ffu;
+    v = (v | v << 8) & 0x0300f00fu;
+    v = (v | v << 4) & 0x030c30c3u;
+    return (v | v << 2) & 0x09249249u;
+}
+__device__ __forceinline__ uint32_t nn_cell_prefix(int ix, int iy, int iz, int K) {
+    const uint32_t m = (1u << K) - 1u;
+    return nn_spread3(~(uint32_t)ix & m) | nn_spread3(~(uint32_t)iy & m) << 1 | nn_spread3(~(uint32_t)iz & m) << 2;
 }
 
 // Particles in the start cells a walk for the box [lo, hi] would begin from (see nn_start_push):
@@ -309,7 +324,7 @@ __device__ __forceinline__ int nn_start_push(LdsT &L, const NNArgs &A, double lo
         const int nx = (ihx >> s) - bx + 1, ny = (ihy >> s) - by + 1, nz = (ihz >> s) - bz + 1;
         if (lane < nx * ny * nz && lane % nparts == part) {
             const int ix = bx + lane % nx, iy = by + (lane / nx) % ny, iz = bz + lane / (nx * ny);
-            const uint64_t P = nn_cell_prefix(ix, iy, iz, K);
+            const uint32_t P = nn_cell_prefix(ix, iy, iz, K);
             node = A.stab[nn_tab_off(K) + (int64_t)P];
             if (node >= 0) rng = A.srng[nn_tab_off(K) + (int64_t)P];
         }
@@ -354,15 +369,17 @@ __device__ __forceinline__ int nn_start_push(LdsT &L, const NNArgs &A, double lo
 // particle ranges -- no tree walk -- and every particle of them is handed to
 // visit(valid, j, {x,y,z,m}_j, h_j), NN_DU candidates per lane and round with all their loads
 // issued first; candidates come in ascending order of (round, slot, lane), and visit is called
-// by all lanes together (it may use ballots).  With nparts > 1 only the start cells of index =
-// part (mod nparts).  Returns false, before any visit, when the box is too large for the
-// table, has more than NN_DRANGES non-empty cells or more than NN_DIRECT_MAX candidates
-// (counted over the whole box, so every part of a split search decides alike).
-static_assert(NN_DRANGES >= (NN_DSPAN + 1) * (NN_DSPAN + 1) * (NN_DSPAN + 1), "boxes are declined by candidates only");
-template <typename LdsT, typename VisitFn>
-__device__ __forceinline__ bool nn_direct(LdsT &L, const NNArgs &A, double lox, double hix, double loy,
-                                          double hiy, double loz, double hiz, const NNCore &q, int part,
-                                          int nparts, VisitFn &&visit) {
+// by all lanes together (it may use ballots).  Returns false, before any visit, when the box is
+// too large for the table or has more than NN_DIRECT_MAX candidates.
+// A search is a chain of waits, so each link is kept short: table entry, range and cell bounds of
+// 128 cells are requested at once, and a candidate's range follows from one bit per range start
+// (set in LDS) by counting bits, where a binary search would be eight dependent LDS reads per
+// candidate (1M cloud: the first tail pass 320 -> 206 us, the re-list marking 311 -> 207 us).
+#define NN_DROUNDS ((NN_DSPAN + 1) * (NN_DSPAN + 1) * (NN_DSPAN + 1) + 63) / 64
+static_assert(NN_DRANGES >= (NN_DSPAN + 1) * (NN_DSPAN + 1) * (NN_DSPAN + 1), "every cell's range has room");
+template <typename VisitFn>
+__device__ __forceinline__ bool nn_direct(NNDirectLds &L, const NNArgs &A, double lox, double hix, double loy,
+                                          double hiy, double loz, double hiz, const NNCore &q, VisitFn &&visit) {
     const int lane = wave_lane();
     const uint64_t lt = lanemask_lt();
     const NNStart S = nn_start_level<NN_DSPAN>(A, lox, hix, loy, hiy, loz, hiz);
@@ -371,52 +388,66 @@ __device__ __forceinline__ bool nn_direct(LdsT &L, const NNArgs &A, double lox, 
     const int bx = S.ilx >> s, by = S.ily >> s, bz = S.ilz >> s;
     const int nx = (S.ihx >> s) - bx + 1, ny = (S.ihy >> s) - by + 1, nz = (S.ihz >> s) - bz + 1;
     const int ncell = nx * ny * nz;
-    int nr = 0, total = 0, nr_all = 0, total_all = 0;
-    for (int c0 = 0; c0 < ncell; c0 += 64) {
-        const int idx = c0 + lane;
-        int first = 0, num = 0;
-        if (idx < ncell) {
-            const int ix = bx + idx % nx, iy = by + (idx / nx) % ny, iz = bz + idx / (nx * ny);
-            const uint64_t P = nn_cell_prefix(ix, iy, iz, K);
-            const int64_t e = nn_tab_off(K) + (int64_t)P;
+    // quotients of an index below 256 by nx, ny <= 6: exact with a 16-bit reciprocal rounded up
+    const uint32_t rx = 65536u / (uint32_t)nx + 1u, ry = 65536u / (uint32_t)ny + 1u;
+    const int64_t tab = nn_tab_off(K);
+    constexpr int ROUNDS = NN_DROUNDS;
+    int pre[ROUNDS];   // candidates before this lane's range of the round (-1: none)
+    int nr = 0, total = 0;
+#pragma unroll
+    for (int r = 0; r < ROUNDS; r += 2) {
+        pre[r] = -1;
+        if (r + 1 < ROUNDS) pre[r + 1] = -1;
+        if (64 * r >= ncell) continue;
+        int first[2], num[2];
+#pragma unroll
+        for (int v = 0; v < 2; v++) {
+            const uint32_t idx = 64 * (r + v) + lane;
+            const bool in = idx < (uint32_t)ncell;
+            const uint32_t iyz = (idx * rx) >> 16, iz = (iyz * ry) >> 16;
+            const uint32_t P = nn_cell_prefix(bx + (int)(idx - iyz * nx), by + (int)(iyz - iz * ny), bz + (int)iz, K);
+            const int64_t e = tab + (in ? (int64_t)P : 0);
             const int node = A.stab[e];
-            if (node >= 0 && (node < A.n || nn_cell_reaches(A, q, node - A.n))) {
-                const int2 r = A.srng[e];
-                first = r.x;
-                num = r.y;
+            const int2 rg = A.srng[e];   // read beside the node; unused where there is none
+            // (cell 0 is read for particles and empty entries, and not looked at)
+            const bool reach = nn_cell_reaches(A, q, node >= A.n ? node - A.n : 0);
+            const bool keep = in && node >= 0 && (node < A.n || reach);
+            first[v] = rg.x;
+            num[v] = keep ? rg.y : 0;
+        }
+#pragma unroll
+        for (int v = 0; v < 2; v++) {
+            if (r + v >= ROUNDS) break;
+            const uint64_t m = wave_ballot(num[v] > 0);
+            const int incl = wave_incl_scan(num[v]);
+            if (num[v] > 0) {
+                pre[r + v] = total + incl - num[v];
+                L.off[nr + popc64(m & lt)] = first[v] - pre[r + v];
             }
+            nr += popc64(m);
+            total += __builtin_amdgcn_readlane(incl, 63);
+            if (total > NN_DIRECT_MAX) return false;
         }
-        // the decision to decline is taken on the whole box, so all parts agree
-        nr_all += popc64(wave_ballot(num > 0));
-        total_all += wave_sum(num);
-        if (nr_all > NN_DRANGES || total_all > NN_DIRECT_MAX) return false;
-        if (idx % nparts != part) num = 0;
-        const uint64_t m = wave_ballot(num > 0);
-        const int incl = wave_incl_scan(num);
-        const int tot = __shfl(incl, 63);
-        if (num > 0) {
-            const int pos = nr + popc64(m & lt);
-            L.drs[pos] = first;
-            L.drp[pos] = total + incl - num;
-        }
-        nr += popc64(m);
-        total += tot;
     }
-    wave_sync();
+    int before = 0;   // ranges that begin before the round's candidates
     for (int base = 0; base < total; base += 64 * NN_DU) {
+        if (lane < NN_DU) L.head[lane] = 0ull;
+        wave_sync();
+#pragma unroll
+        for (int r = 0; r < ROUNDS; r++) {
+            const uint32_t o = (uint32_t)(pre[r] - base);
+            if (pre[r] >= 0 && o < 64u * NN_DU) atomicOr(&L.head[o >> 6], 1ull << (o & 63u));
+        }
+        wave_sync();
         int jj[NN_DU];
 #pragma unroll
         for (int u = 0; u < NN_DU; u++) {
+            const unsigned long long w = L.head[u];
             const int c = base + 64 * u + lane;
-            jj[u] = -1;
-            if (c < total) {
-                int lo = 0, hi_ = nr - 1;
-                while (lo < hi_) {
-                    const int mid = (lo + hi_ + 1) >> 1;
-                    if (L.drp[mid] <= c) lo = mid; else hi_ = mid - 1;
-                }
-                jj[u] = L.drs[lo] + (c - L.drp[lo]);
-            }
+            // a candidate's range is the last one beginning at or before it
+            const int own = before + popc64(w & (lt | 1ull << lane)) - 1;
+            before += popc64(w);
+            jj[u] = c < total ? L.off[own] + c : -1;
         }
         double4 pj[NN_DU];
         double hj[NN_DU];
@@ -959,6 +990,9 @@ __global__ __launch_bounds__(64 * NN_WAVES) void k_nn_walk(NNArgs A) {
 // order, one 4-byte entry per lane.
 #define NN1_WAVES 4
 #define NN1_MAX_BLOCKS 1024   // about one resident round: 4096 wavefronts loop over the list
+// the same for the kernels that search in the direct form only: little LDS, five wavefronts a SIMD
+#define NN_DIRECT_BLOCKS 1280
+inline unsigned nn_direct_grid(int64_t n) { return (unsigned)std::min<int64_t>(ceil_div(n, NN1_WAVES), NN_DIRECT_BLOCKS); }
 // Workgroups [first, first + blocks) of the launch.
 template <int MODE>
 __device__ __forceinline__ void nn_one(NNWaveLds &L, const NNArgs &A, unsigned first, unsigned blocks) {
@@ -993,7 +1027,7 @@ __device__ __forceinline__ void nn_one(NNWaveLds &L, const NNArgs &A, unsigned f
         };
         const double lox = own.x - grow, hix = own.x + grow, loy = own.y - grow, hiy = own.y + grow;
         const double loz = own.z - grow, hiz = own.z + grow;
-        const bool direct = nn_direct(L, A, lox, hix, loy, hiy, loz, hiz, nn_point(own.x, own.y, own.z, hi), 0, 1,
+        const bool direct = nn_direct(L.direct, A, lox, hix, loy, hiy, loz, hiz, nn_point(own.x, own.y, own.z, hi),
                                       [&](bool v, int j, const double4 &p, double h) { take(v, j, p.x, p.y, p.z, h * h); });
         if (!direct) {
             const bool ok = nn_walk_box<false>(L, A, lox, hix, loy, hiy, loz, hiz, nn_point(own.x, own.y, own.z, hi), NN_START_ALL, 0, 0, -1, KeepAll(), [&](int m) {
@@ -1069,21 +1103,26 @@ __global__ __launch_bounds__(64 * NN1_WAVES) void k_nn_rest(NNArgs A, unsigned p
 // membership with j changed, (d < min(h_i, h_j0)) != (d < min(h_i, h_j1)) with h_j1 the final
 // h: the only pairs whose membership d < h_i and d < h_j can differ from pass 0 (an unflagged
 // particle keeps its pass-0 h).  Such an i lies within max(h_j0, h_j1) of x_j.  One wavefront
-// per changed particle; lanes are candidates; d is the pair test's (symmetric) value.
+// per changed particle; lanes are candidates; d is the pair test's (symmetric) value.  The boxes
+// the direct form declines (DIRECT) go to a second launch that walks the tree for them: the
+// walk's LDS would keep half of the direct searches off the chip.
+template <bool DIRECT>
 __global__ __launch_bounds__(64 * NN1_WAVES) void k_nn_mark_dirty(NNArgs A) {
-    __shared__ NNWaveLds lds_all[NN1_WAVES];
+    using Lds = std::conditional_t<DIRECT, NNDirectLds, NNWaveLds>;
+    __shared__ Lds lds_all[NN1_WAVES];
     const int w = threadIdx.x / 64, lane = wave_lane();
-    NNWaveLds &L = lds_all[w];
-    const uint32_t cnt = *A.count_in;
+    Lds &L = lds_all[w];
+    const uint32_t cnt = DIRECT ? *A.count_in : *A.slot_count;
     const int64_t nwaves = (int64_t)gridDim.x * NN1_WAVES;
-    for (int64_t t = (int64_t)blockIdx.x * NN1_WAVES + w; t < cnt; t += nwaves) {
+    for (int64_t tt = (int64_t)blockIdx.x * NN1_WAVES + w; tt < cnt; tt += nwaves) {
+        const int64_t t = DIRECT ? tt : A.slot_list[tt];
         const int64_t jc = A.list_in[t];
         const double4 own = A.sxm[jc];
         const double h0 = A.h0_slot[t], h1 = A.h[jc];
         const double h02 = h0 * h0, h12 = h1 * h1;
         const double hq = h0 > h1 ? h0 : h1;
         const double grow = hq * (1.0 + 1e-9);
-        if (lane == 0) A.dirty[jc] = 1;
+        if (DIRECT && lane == 0) A.dirty[jc] = 1;
         auto mark = [&](bool v, int i, double x, double y, double z, double hi2) {
             if (v) {
                 const double dx = own.x - x;
@@ -1095,9 +1134,11 @@ __global__ __launch_bounds__(64 * NN1_WAVES) void k_nn_mark_dirty(NNArgs A) {
         };
         const double lox = own.x - grow, hix = own.x + grow, loy = own.y - grow, hiy = own.y + grow;
         const double loz = own.z - grow, hiz = own.z + grow;
-        const bool direct = nn_direct(L, A, lox, hix, loy, hiy, loz, hiz, nn_point(own.x, own.y, own.z, hq), 0, 1,
-                                      [&](bool v, int i, const double4 &p, double h) { mark(v, i, p.x, p.y, p.z, h * h); });
-        if (!direct) {
+        if constexpr (DIRECT) {
+            const bool direct = nn_direct(L, A, lox, hix, loy, hiy, loz, hiz, nn_point(own.x, own.y, own.z, hq),
+                                          [&](bool v, int i, const double4 &p, double h) { mark(v, i, p.x, p.y, p.z, h * h); });
+            if (!direct && lane == 0) A.list_out[atomicAdd(A.count_out, 1u)] = (int32_t)t;
+        } else {
             const bool ok = nn_walk_box<false>(L, A, lox, hix, loy, hiy, loz, hiz, nn_point(own.x, own.y, own.z, hq), NN_START_ALL, 0, 0, -1, KeepAll(), [&](int m) {
                 if (lane < m) mark(true, L.tj[lane], L.tx[lane], L.ty[lane], L.tz[lane], L.th2[lane]);
             });
@@ -1117,9 +1158,9 @@ __global__ __launch_bounds__(64 * NN1_WAVES) void k_nn_mark_dirty(NNArgs A) {
 // direct form declines (too large for the table, too many cells or candidates) is appended to
 // hard_list for k_nn_count_split.  The count goes to cnt_slot[t] (integer, exact).
 __global__ __launch_bounds__(64 * NN1_WAVES) void k_nn_count_direct(NNArgs A) {
-    __shared__ NNWaveLds lds_all[NN1_WAVES];
+    __shared__ NNDirectLds lds_all[NN1_WAVES];
     const int w = threadIdx.x / 64, lane = wave_lane();
-    NNWaveLds &L = lds_all[w];
+    NNDirectLds &L = lds_all[w];
     if (h_pass_frozen(A)) return;
     const uint32_t cnt = *A.count_in;
     const int64_t nwaves = (int64_t)gridDim.x * NN1_WAVES;
@@ -1131,7 +1172,7 @@ __global__ __launch_bounds__(64 * NN1_WAVES) void k_nn_count_direct(NNArgs A) {
         const double grow = hi * (1.0 + 1e-9);
         int count = 0;
         const bool direct = nn_direct(L, A, own.x - grow, own.x + grow, own.y - grow, own.y + grow, own.z - grow,
-                                      own.z + grow, nn_point(own.x, own.y, own.z, hi), 0, 1,
+                                      own.z + grow, nn_point(own.x, own.y, own.z, hi),
                                       [&](bool v, int j, const double4 &p, double h) {
             if (v) {
                 const double dx = own.x - p.x;
@@ -1245,9 +1286,9 @@ __global__ __launch_bounds__(256) void k_h_finish(NNArgs A) {
 // atomics serialise (47^3: 26 us per pass with lists appended here, 11 + 6 us with counts and a
 // wave-aggregated update, so larger sets keep those).
 __global__ __launch_bounds__(64 * NN1_WAVES) void k_h_pass(NNArgs A) {
-    __shared__ NNWaveLds lds_all[NN1_WAVES];
+    __shared__ NNDirectLds lds_all[NN1_WAVES];
     const int w = threadIdx.x / 64, lane = wave_lane();
-    NNWaveLds &L = lds_all[w];
+    NNDirectLds &L = lds_all[w];
     const bool frozen = h_pass_frozen(A);
     const int64_t nwaves = (int64_t)gridDim.x * NN1_WAVES;
     bool changed = false, stays = false;
@@ -1273,7 +1314,7 @@ __global__ __launch_bounds__(64 * NN1_WAVES) void k_h_pass(NNArgs A) {
             const double hi2 = hi * hi;
             const double grow = hi * (1.0 + 1e-9);
             nn_direct(L, A, own.x - grow, own.x + grow, own.y - grow, own.y + grow, own.z - grow, own.z + grow,
-                      nn_point(own.x, own.y, own.z, hi), 0, 1, [&](bool v, int j, const double4 &p, double h) {
+                      nn_point(own.x, own.y, own.z, hi), [&](bool v, int j, const double4 &p, double h) {
                 if (v) {
                     const double dx = own.x - p.x;
                     const double dy = own.y - p.y;
@@ -1469,7 +1510,7 @@ void launch_h_iterate(mhpc_ctx *c, int passes, bool speculative, hipEvent_t *wal
             a.changed = c->dstatus->hchanged + pass;   // zeroed by k_h_init
             a.prev_changed = pass >= 1 ? c->dstatus->hchanged + (pass - 1) : nullptr;
             if (walk_events && pass == 0) (void)hipEventRecord(walk_events[0], c->stream);
-            hipLaunchKernelGGL(k_h_pass, dim3(g1), dim3(64 * NN1_WAVES), 0, c->stream, a);
+            hipLaunchKernelGGL(k_h_pass, dim3(nn_direct_grid(c->n)), dim3(64 * NN1_WAVES), 0, c->stream, a);
             if (walk_events && pass == 0) (void)hipEventRecord(walk_events[1], c->stream);
             std::swap(c->sh, c->sh2);
         }
@@ -1524,7 +1565,7 @@ void launch_h_iterate(mhpc_ctx *c, int passes, bool speculative, hipEvent_t *wal
         NNArgs d = a;
         d.list_out = c->hhard;
         d.count_out = hard_count;
-        hipLaunchKernelGGL(k_nn_count_direct, dim3(g1), dim3(64 * NN1_WAVES), 0, c->stream, d);
+        hipLaunchKernelGGL(k_nn_count_direct, dim3(nn_direct_grid(c->n)), dim3(64 * NN1_WAVES), 0, c->stream, d);
         a.slot_list = c->hhard;
         a.slot_count = hard_count;
         // the split work is 8 wavefronts per particle the direct form declined: usually none
@@ -1561,7 +1602,13 @@ void launch_neighbours_fixup(mhpc_ctx *c) {
     a.dirty = c->sdirty;
     a.h0_slot = c->h0slot;
     const unsigned g1 = (unsigned)std::min<int64_t>(ceil_div(c->n, NN1_WAVES), NN1_MAX_BLOCKS);
-    hipLaunchKernelGGL(k_nn_mark_dirty, dim3(g1), dim3(64 * NN1_WAVES), 0, c->stream, a);
+    // declined boxes: the list the counting passes used, its length in the entry pass 0 leaves unused
+    a.list_out = c->hhard;
+    a.count_out = c->hlist_count + MHPC_MAX_PASSES + 1;   // zeroed by k_h_init
+    hipLaunchKernelGGL(k_nn_mark_dirty<true>, dim3(nn_direct_grid(c->n)), dim3(64 * NN1_WAVES), 0, c->stream, a);
+    a.slot_list = c->hhard;
+    a.slot_count = a.count_out;
+    hipLaunchKernelGGL(k_nn_mark_dirty<false>, dim3(std::min(g1, 256u)), dim3(64 * NN1_WAVES), 0, c->stream, a);
     NNArgs b = nn_common(c);
     b.h = c->sh;
     b.nbr4 = reinterpret_cast<int4 *>(c->nbr);

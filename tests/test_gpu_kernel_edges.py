@@ -236,3 +236,35 @@ def test_tree_and_com_at_the_tile_and_launch_splits(gpu_lib, orc, n):
     a = np.array(sorted(zip(t["level"], t["mass"], t["x"], t["y"], t["z"])))
     b = np.array(sorted(zip(lev, nm, nx, ny, nz)))
     assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("curve", [0, 1])
+def test_relists_around_boxes_the_direct_search_declines(gpu_lib, orc, curve):
+    """A jittered 33^3 lattice (35,937 particles: group walks, an odd last group) where some h are
+    several times and a few are hundreds of times the others', so that their search boxes hold more
+    particles than the direct search takes: h, iteration counts and neighbour sets of the speculative
+    lists equal the plain iteration's and the oracle's."""
+    print_case(f"declined boxes, 33^3 curve={curve}")
+    s = ics.sedov_lattice(33)
+    rng = np.random.default_rng(91)
+    n = len(s["x"])
+    for a in "xyz":
+        s[a] = s[a] + rng.uniform(-0.2, 0.2, n) / 33
+    u = rng.uniform(size=n)
+    h0 = s["sml"] * rng.uniform(0.9, 1.25, n) * np.where(u < 0.05, 6.0, 1.0)
+    h0[rng.choice(n, 12, replace=False)] = 3.0 * (s["x"].max() - s["x"].min())
+    base = gpu_lib.RHS_SPH | gpu_lib.RHS_VARIABLE_SML
+    out = {}
+    for name, flags in (("plain", base), ("spec", base | gpu_lib.RHS_SPECULATIVE_NN)):
+        with load_ctx(gpu_lib, {**s, "sml": h0}, gpu_lib.default_params(curve=curve)) as ctx:
+            ctx.rhs(flags)
+            out[name] = {k: ctx.download(k) for k in ("sml", "h_iters", "noi", "rho")}
+            nnl, noi = ctx.neighbour_lists(180)
+        out[name]["sets"] = [frozenset(nnl[i, :noi[i]].tolist()) for i in range(n)]
+    a, b = out["plain"], out["spec"]
+    st, oh, oiters, _ = orc.h_iterate(s["x"], s["y"], s["z"], h0)
+    assert np.array_equal(b["h_iters"], oiters) and np.array_equal(b["sml"], oh)
+    for k in ("sml", "h_iters", "noi"):
+        assert np.array_equal(a[k], b[k]), k
+    assert a["sets"] == b["sets"]
+    assert np.max(np.abs(a["rho"] - b["rho"])) <= 1e-12 * a["rho"].max()   # order of 180 terms at most
