@@ -6,9 +6,9 @@
 // consecutive key-sorted particles: it walks the tree once with the group's bounding box
 // grown by the group's largest h, collecting the particle ranges of small cells (each
 // cell is a contiguous range of sorted positions), then streams the candidates through
-// LDS in tiles of 64 with coalesced SoA loads; every lane tests every candidate of the
-// tile against its own particle with the reference criterion d^2 < h_i^2 and
-// d^2 < h_j^2 (FP64, exact), so the neighbour sets equal a brute-force search.
+// LDS in tiles of 64 with coalesced SoA loads; every particle is tested against every candidate of
+// the tile with the reference criterion d^2 < h_i^2 and d^2 < h_j^2, on the matrix cores where the
+// result is clear and in FP64 otherwise, so the neighbour sets equal a brute-force search.
 #include <algorithm>
 #include <type_traits>
 
@@ -16,9 +16,8 @@
 
 #define NN_WAVES 2
 #define NN_CWIN 512   // group walk, list modes: the consumers' LDS window (in-window neighbours first)
-#define NN_PB 4      // group walk, list modes: candidates read from LDS per batch
-#define NN_STACK 512
-#define NN_STACK_PHYS (NN_STACK + 192)
+#define NN_PB 4      // group walk, FP64 tests: candidates read from LDS per batch
+#define NN_STACK_SLACK 192   // hard stack capacity above the soft one: a node a level opens
 #define NN_RANGES 128
 #define NN_LEAF 16           // per-particle walks: cells of at most this many particles are taken whole
 #define NN_LEAF_GROUP 64     // group walks: the same for the 64-particle groups' boxes
@@ -48,29 +47,6 @@ static_assert(64 / NN_SPLIT_MIN <= MHPC_NN_PARTS_PER_GROUP, "the part list holds
 #define NN_FEW 32768
 static_assert(NN_FEW <= NN_DIRECT_MAX, "the direct form declines no box of so few particles");
 #define NN_DU 4              // direct form: candidates per lane and round (loads in flight; 2 / 4 / 8 alike)
-
-// per-wave LDS of the direct form: its candidate ranges (first particle less the number of
-// candidates before the range) and where ranges begin among the candidates of a round
-struct NNDirectLds {
-    int off[NN_DRANGES];
-    unsigned long long head[NN_DU];
-};
-struct NNNoDirect {};
-
-// per-wave LDS of the walker; TCAP = 128 gives the filtered walk room to compact the
-// candidates of two 64-particle loads before a full tile of 64 is handed on
-template <int TCAP, typename Direct>
-struct NNWaveLdsT {
-    int stack[NN_STACK_PHYS];
-    int rstart[NN_RANGES];
-    int rcnt[NN_RANGES];
-    int rpre[64];
-    double tx[TCAP], ty[TCAP], tz[TCAP], th2[TCAP];
-    int tj[TCAP];
-    Direct direct;
-};
-using NNWaveLds = NNWaveLdsT<64, NNDirectLds>;
-using NNWaveLdsF = NNWaveLdsT<128, NNNoDirect>;
 
 // candidate filter that keeps everything (per-particle walks test each candidate once)
 struct KeepAll {
@@ -153,11 +129,57 @@ struct NNCore {
     double h;
 };
 
+// What a walk searches: the box [lo, hi] (the core grown by the search radius) and the core.
+struct NNBounds {
+    double lox, hix, loy, hiy, loz, hiz;
+    NNCore core;
+};
+
+// per-wave LDS of the direct form: its candidate ranges (first particle less the number of
+// candidates before the range) and where ranges begin among the candidates of a round
+struct NNDirectLds {
+    int off[NN_DRANGES];
+    unsigned long long head[NN_DU];
+};
+// per-wave LDS of the group walks' matrix tests (nn_tile): one axis of a tile's 64 candidates in
+// 16-bit parts, and the parts of their second norms
+struct NNTileLds {
+    uint2 part[3][64];
+    uint16_t norm2[3][64];
+    NNBounds bounds;                          // the group's
+    double cx, cy, cz, scale, hm2s;           // middle of its box, scale and scaled largest h^2 (nn_tile)
+};
+
+// per-wave LDS of the walker; the filtered walk's tiles (TCAP = 128) have room to compact the
+// candidates of two 64-particle loads before a full tile of 64 is handed on
+template <int TCAP, int STACK, typename Extra>
+struct NNWaveLdsT {
+    static constexpr int soft = STACK;   // soft stack capacity (see nn_walk_box)
+    int stack[STACK + NN_STACK_SLACK];
+    int rstart[NN_RANGES];
+    int rcnt[NN_RANGES];
+    int rpre[64];
+    double tx[TCAP], ty[TCAP], tz[TCAP], th2[TCAP];
+    int tj[TCAP];
+    Extra extra;
+};
+using NNWaveLds = NNWaveLdsT<64, 512, NNDirectLds>;
+// 10 KB, so that 16 wavefronts fit a CU; the stack takes what is left, since it bounds the nodes opened
+// per round (208 / 376 entries: 128^3 blast step 7.76 / 7.51 ms, 1M cloud RHS 4.94 / 4.82 ms)
+using NNWaveLdsF = NNWaveLdsT<128, 376, NNTileLds>;
+static_assert(sizeof(NNWaveLdsF) <= 163840 / 16, "16 wavefronts per CU");
+
 // the squared distance of every neighbour test (and of the bounds that prune them):
 // fma(dx, dx, fma(dy, dy, dz^2)), the oracle's form (two fused multiply-adds per test)
 __device__ __forceinline__ double nn_d2(double dx, double dy, double dz) { return fma(dx, dx, fma(dy, dy, dz * dz)); }
 __device__ __forceinline__ NNCore nn_point(double x, double y, double z, double h) {
     return NNCore{x, x, y, y, z, z, h};
+}
+
+// one particle's bounds: its search radius plus a relative margin far above FP64 rounding
+__device__ __forceinline__ NNBounds nn_ball(const double4 &p, double h) {
+    const double grow = h * (1.0 + 1e-9);
+    return NNBounds{p.x - grow, p.x + grow, p.y - grow, p.y + grow, p.z - grow, p.z + grow, nn_point(p.x, p.y, p.z, h)};
 }
 
 // Can cell c hold a neighbour j of some particle i of the core?  A pair needs d < h_i^2 and
@@ -378,11 +400,11 @@ __device__ __forceinline__ int nn_start_push(LdsT &L, const NNArgs &A, double lo
 #define NN_DROUNDS ((NN_DSPAN + 1) * (NN_DSPAN + 1) * (NN_DSPAN + 1) + 63) / 64
 static_assert(NN_DRANGES >= (NN_DSPAN + 1) * (NN_DSPAN + 1) * (NN_DSPAN + 1), "every cell's range has room");
 template <typename VisitFn>
-__device__ __forceinline__ bool nn_direct(NNDirectLds &L, const NNArgs &A, double lox, double hix, double loy,
-                                          double hiy, double loz, double hiz, const NNCore &q, VisitFn &&visit) {
+__device__ __forceinline__ bool nn_direct(NNDirectLds &L, const NNArgs &A, const NNBounds &B, VisitFn &&visit) {
     const int lane = wave_lane();
     const uint64_t lt = lanemask_lt();
-    const NNStart S = nn_start_level<NN_DSPAN>(A, lox, hix, loy, hiy, loz, hiz);
+    const NNCore &q = B.core;
+    const NNStart S = nn_start_level<NN_DSPAN>(A, B.lox, B.hix, B.loy, B.hiy, B.loz, B.hiz);
     if (S.K < 1) return false;
     const int K = S.K, s = S.s;
     const int bx = S.ilx >> s, by = S.ily >> s, bz = S.ilz >> s;
@@ -476,10 +498,11 @@ __device__ __forceinline__ bool nn_direct(NNDirectLds &L, const NNArgs &A, doubl
 // with keep(x, y, z, h^2) true reach the tiles (compacted in walk order, so the tile sequence
 // is the unfiltered one minus the dropped candidates).  Returns false on stack overflow.
 // Wave-uniform control flow.
-template <bool FILTER, typename LdsT, typename KeepFn, typename TileFn>
-__device__ __forceinline__ bool nn_walk_box(LdsT &L, const NNArgs &A, double lox, double hix, double loy,
-                                            double hiy, double loz, double hiz, const NNCore &q, int start,
-                                            int w0, int w1, int g0, KeepFn &&keep, TileFn &&tile) {
+// `bounds()` gives the box and the core: a group's are read from LDS where they are needed (they
+// are the same in all lanes and would take 38 registers throughout).
+template <bool FILTER, typename LdsT, typename BoundsFn, typename KeepFn, typename TileFn>
+__device__ __forceinline__ bool nn_walk_box(LdsT &L, const NNArgs &A, BoundsFn &&bounds, int start, int w0, int w1,
+                                            int g0, KeepFn &&keep, TileFn &&tile) {
     const int lane = wave_lane();
     const int64_t n = A.n;
     // a group's box spans a few 64-particle cells per axis: taken whole, their candidates come
@@ -490,8 +513,10 @@ __device__ __forceinline__ bool nn_walk_box(LdsT &L, const NNArgs &A, double lox
     if (start >= 0) {
         if (lane == 0) L.stack[0] = start;
     } else {
-        top = nn_start_push(L, A, lox, hix, loy, hiy, loz, hiz, q, start == NN_START_ALL ? 0 : NN_START_PART0 - start,
-                            start == NN_START_ALL ? 1 : 8, w0, w1, g0, nr, leaf);
+        const NNBounds B = bounds();
+        top = nn_start_push(L, A, B.lox, B.hix, B.loy, B.hiy, B.loz, B.hiz, B.core,
+                            start == NN_START_ALL ? 0 : NN_START_PART0 - start, start == NN_START_ALL ? 1 : 8, w0, w1,
+                            g0, nr, leaf);
     }
     wave_sync();
     const uint64_t lt = lanemask_lt();
@@ -499,7 +524,7 @@ __device__ __forceinline__ bool nn_walk_box(LdsT &L, const NNArgs &A, double lox
     for (;;) {
         // walk until 64 ranges are pending or the stack is empty
         while (top > 0 && nr < 64) {
-            int kpop = (NN_STACK - top) / 7;
+            int kpop = (LdsT::soft - top) / 7;
             kpop = kpop < 1 ? 1 : kpop;
             kpop = kpop > 64 ? 64 : kpop;
             kpop = kpop > top ? top : kpop;
@@ -512,17 +537,19 @@ __device__ __forceinline__ bool nn_walk_box(LdsT &L, const NNArgs &A, double lox
             if (node >= 0 && node < n) {
                 const double4 r = A.sxm[node];
                 const double px = r.x, py = r.y, pz = r.z;
-                take = px >= lox && px <= hix && py >= loy && py <= hiy && pz >= loz && pz <= hiz;
+                const NNBounds B = bounds();
+                take = px >= B.lox && px <= B.hix && py >= B.loy && py <= B.hiy && pz >= B.loz && pz <= B.hiz;
                 rs = node;
                 rc = 1;
                 take = take && nn_win_clip(w0, w1, rs, rc, leaf);
             } else if (node >= n) {
                 c = node - n;
                 const int64_t cc = A.cap_cells;
-                const bool overlap = A.cbmin[c] <= hix && A.cbmax[c] >= lox &&
-                                     A.cbmin[cc + c] <= hiy && A.cbmax[cc + c] >= loy &&
-                                     A.cbmin[2 * cc + c] <= hiz && A.cbmax[2 * cc + c] >= loz &&
-                                     nn_cell_reaches(A, q, c);
+                const NNBounds B = bounds();
+                const bool overlap = A.cbmin[c] <= B.hix && A.cbmax[c] >= B.lox &&
+                                     A.cbmin[cc + c] <= B.hiy && A.cbmax[cc + c] >= B.loy &&
+                                     A.cbmin[2 * cc + c] <= B.hiz && A.cbmax[2 * cc + c] >= B.loz &&
+                                     nn_cell_reaches(A, B.core, c);
                 if (overlap) {
                     rs = A.cstart[c];
                     rc = A.cend[c] - rs + 1;
@@ -550,7 +577,7 @@ __device__ __forceinline__ bool nn_walk_box(LdsT &L, const NNArgs &A, double lox
             }
             const int incl = wave_incl_scan(nc);
             const int tot = __shfl(incl, 63);
-            if (top + tot > NN_STACK_PHYS) return false;
+            if (top + tot > LdsT::soft + NN_STACK_SLACK) return false;
             if (open) {
                 int pos = top + incl - nc;
 #pragma unroll
@@ -560,10 +587,9 @@ __device__ __forceinline__ bool nn_walk_box(LdsT &L, const NNArgs &A, double lox
             top += tot;
             wave_sync();
         }
-        if (nr == 0 && top == 0) {
-            if (FILTER && fill > 0) tile(fill);
-            return true;
-        }
+        // nothing left: one more step hands on the candidates still waiting
+        const bool last = nr == 0 && top == 0;
+        if (last && fill == 0) return true;
         // stream the candidates of up to 64 ranges through LDS
         const int np = nr < 64 ? nr : 64;
         const int v = lane < np ? L.rcnt[lane] : 0;
@@ -572,7 +598,7 @@ __device__ __forceinline__ bool nn_walk_box(LdsT &L, const NNArgs &A, double lox
         const int pre = incl - v;
         L.rpre[lane] = pre;
         wave_sync();
-        for (int base = 0; base < total; base += 64) {
+        for (int base = 0; base < total || (FILTER && last); base += 64) {
             const int t = base + lane;
             // the ranges holding this chunk's first and last candidates bound every lane's
             // search (prefixes are non-decreasing): usually one or two ranges apart
@@ -627,8 +653,9 @@ __device__ __forceinline__ bool nn_walk_box(LdsT &L, const NNArgs &A, double lox
                 }
                 fill += popc64(mk);
                 wave_sync();
-                if (fill >= 64) {
-                    tile(64);
+                if (fill >= 64 || last) {
+                    tile(fill < 64 ? fill : 64);
+                    if (last) return true;
                     wave_sync();
                     // move the overflow [64, fill) to the front (disjoint ranges)
                     const int rest = fill - 64;
@@ -690,6 +717,205 @@ __device__ __forceinline__ NNBox nn_box(bool active, double x, double y, double 
     B.y0 = wave_min(active ? y : 1e300); B.y1 = wave_max(active ? y : -1e300);
     B.z0 = wave_min(active ? z : 1e300); B.z1 = wave_max(active ? z : -1e300);
     return B;
+}
+
+// The neighbour tests of a group walk on the matrix cores.  For a particle i and a candidate j, both
+// relative to the middle of the group's box and scaled by a power of two so that the largest h is
+// below 2, (h_i^2 - d) / 2 = x_i . x_j + (h_i^2 - |x_i|^2) / 2 - |x_j|^2 / 2 is a row of six products
+// per axis (each coordinate split exactly into three bfloat16 parts, the products of the parts but
+// the smallest three) and three parts of each norm: 24 of the 32 products of one
+// v_mfma_f32_16x16x32_bf16 element.  Its sign decides the test unless it is within `eps` of zero;
+// then the pair is tested as in every other walk (FP64), so that the sets are the same.
+// The error of an element, with M = (box half-diagonal + largest h)^2 bounding the terms' sum by
+// 2.5 M: 32 FP32 additions, even truncated one after another, 32 2^-23 2.5 M = 2^-16.7 M; the dropped products
+// 2^-20 M; the rounding of coordinates and norms to FP32 2^-22 M.  eps = 2^-16 M.  (Largest error
+// measured over 67 million random pairs: 2^-21.2 M.)
+// The FP64 tests were most of a walk that is bound by its instructions: 6 operations, 2
+// comparisons and a bit per pair, against 1.5 to 2.5 instructions here (256^3 list walk 6.4 -> 5.2 ms,
+// 47^3 RHS in two walks 884 -> 668 us, 1M cloud RHS 5.05 -> 4.80 ms, 128^3 blast step 7.69 -> 7.50 ms).
+#define NN_MFMA_REACH 64.0   // largest M (h is 1 to 2): above, most tiles hold a pair too close to zero
+typedef unsigned nn_u32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 nn_bf16x8 __attribute__((ext_vector_type(8)));
+typedef float nn_f32x4 __attribute__((ext_vector_type(4)));
+
+// x = parts a + b + c of eight significant bits each (exact), as FP32
+struct NNParts {
+    uint32_t a, b, c;
+};
+__device__ __forceinline__ NNParts nn_parts(float x) {
+    NNParts p;
+    p.a = __float_as_uint(x) & 0xffff0000u;
+    const float r = x - __uint_as_float(p.a);
+    p.b = __float_as_uint(r) & 0xffff0000u;
+    p.c = __float_as_uint(r - __uint_as_float(p.b));
+    return p;
+}
+// the upper halves of two words: lo's below hi's
+__device__ __forceinline__ uint32_t nn_pack_hi(uint32_t hi, uint32_t lo) {
+    return __builtin_amdgcn_perm(hi, lo, 0x07060302u);
+}
+
+// A group's particles as the matrix test needs them: lane (q, c) = 16 q + c holds axis q (none for
+// q = 3) of the particles 16 a + c in `xy` {part b, part a} and `zn` {norm part q, part c}, and the second
+// norm's part q in n2.
+struct NNTileI {
+    bool on;
+    float eps;
+    uint32_t ab[4], cn[4], n2[4], one;
+};
+
+__device__ __forceinline__ void nn_tile_write(NNTileLds &T, int e, double X, double Y, double Z, float n1, float n2) {
+    const NNParts x = nn_parts((float)X), y = nn_parts((float)Y), z = nn_parts((float)Z);
+    const NNParts p = nn_parts(n1), r = nn_parts(n2);
+    T.part[0][e] = make_uint2(nn_pack_hi(x.b, x.a), nn_pack_hi(p.a, x.c));
+    T.part[1][e] = make_uint2(nn_pack_hi(y.b, y.a), nn_pack_hi(p.b, y.c));
+    T.part[2][e] = make_uint2(nn_pack_hi(z.b, z.a), nn_pack_hi(p.c, z.c));
+    T.norm2[0][e] = (uint16_t)(r.a >> 16);
+    T.norm2[1][e] = (uint16_t)(r.b >> 16);
+    T.norm2[2][e] = (uint16_t)(r.c >> 16);
+}
+
+// live: the lane's particle takes part (its position is finite then)
+__device__ __forceinline__ NNTileI nn_tile_group(NNTileLds &T, bool live, double x, double y, double z, double h2,
+                                                 const NNBox &B) {
+    NNTileI I;
+    const double cx = 0.5 * (B.x0 + B.x1), cy = 0.5 * (B.y0 + B.y1), cz = 0.5 * (B.z0 + B.z1);
+    const double scale = ldexp(1.0, -ilogb(B.h));   // largest h in [1, 2)
+    const double hs = B.h * scale;
+    const double reach =
+        0.5 * sqrt(nn_d2((B.x1 - B.x0) * scale, (B.y1 - B.y0) * scale, (B.z1 - B.z0) * scale)) + hs;
+    const double M = reach * reach;
+    I.on = M <= NN_MFMA_REACH && B.h > 0.0;   // false for boxes that are not finite
+    I.eps = (float)(M * 1.52587890625e-05);
+    if (!I.on) return I;
+    const double X = live ? (x - cx) * scale : 0.0, Y = live ? (y - cy) * scale : 0.0,
+                 Z = live ? (z - cz) * scale : 0.0;
+    const double r2 = nn_d2(X, Y, Z);
+    // a lane that takes no part is far from everything
+    nn_tile_write(T, wave_lane(), X, Y, Z, live ? (float)(0.5 * (h2 * (scale * scale) - r2)) : -1e30f,
+                  live ? (float)(-0.5 * r2) : -1e30f);
+    if (wave_lane() == 0) {
+        T.cx = cx;
+        T.cy = cy;
+        T.cz = cz;
+        T.scale = scale;
+        T.hm2s = hs * hs;
+    }
+    wave_sync();
+    const int q = wave_lane() >> 4, c = wave_lane() & 15, ax = q < 3 ? q : 0;
+    I.one = q < 3 ? 0x3f80u : 0u;
+#pragma unroll
+    for (int a = 0; a < 4; a++) {
+        const uint2 v = T.part[ax][16 * a + c];
+        I.ab[a] = q < 3 ? v.x : 0u;
+        I.cn[a] = q < 3 ? v.y : 0u;
+        I.n2[a] = q < 3 ? 0x3f800000u | T.norm2[ax][16 * a + c] : 0u;
+    }
+    wave_sync();
+    return I;
+}
+
+// lane 16 q' + c gathers its particle's bits from the four rows of lanes: candidate 0 first
+__device__ __forceinline__ void nn_tile_bits(const uint32_t w[4], uint32_t &lo, uint32_t &hi) {
+    const auto s02 = __builtin_amdgcn_permlane32_swap(w[0], w[2], false, false);
+    const auto s13 = __builtin_amdgcn_permlane32_swap(w[1], w[3], false, false);
+    const auto r01 = __builtin_amdgcn_permlane16_swap(s02[0], s13[0], false, false);
+    const auto r23 = __builtin_amdgcn_permlane16_swap(s02[1], s13[1], false, false);
+    lo = __builtin_bitreverse32(r01[0] << 16 | r01[1]);
+    hi = __builtin_bitreverse32(r23[0] << 16 | r23[1]);
+}
+
+// The tests of the tile's m candidates (bit e of lo, e - 32 of hi: candidate e; bits past m are any)
+// for every lane's particle; `exact(e)` is the lane's test of candidate e in FP64.  SAME: every
+// candidate's h^2 is at least the largest of the group, so h_i^2 alone decides.
+template <bool SAME, typename LdsT, typename ExactFn>
+__device__ __forceinline__ void nn_tile(LdsT &L, const NNTileI &I, int m, uint32_t &lo, uint32_t &hi,
+                                        ExactFn &&exact) {
+    const int lane = wave_lane(), q = lane >> 4, ax = q < 3 ? q : 0;
+    NNTileLds &T = L.extra;
+    {
+        const bool in = lane < m;   // past the tile: far from everything
+        const double sc = T.scale;
+        const double X = in ? (L.tx[lane] - T.cx) * sc : 0.0, Y = in ? (L.ty[lane] - T.cy) * sc : 0.0,
+                     Z = in ? (L.tz[lane] - T.cz) * sc : 0.0;
+        const double r2 = nn_d2(X, Y, Z);
+        // beyond the largest h^2 the candidate's own never decides (and may be any size)
+        const double h2 = SAME ? 0.0 : fmin(L.th2[lane] * (sc * sc), T.hm2s);
+        nn_tile_write(T, lane, X, Y, Z, in ? (float)(-0.5 * r2) : -1e30f,
+                      !SAME && in ? (float)(0.5 * (h2 - r2)) : SAME ? 0.f : -1e30f);
+    }
+    wave_sync();
+    uint32_t w[4] = {0, 0, 0, 0}, close[4] = {0, 0, 0, 0};
+    bool any_close = false;
+    // row 4 q + r of step t is candidate 16 q + 4 t + r, so that a lane's bits of one q are in order
+    const int row = 16 * ((lane & 15) >> 2) + (lane & 3);
+    auto mfma = [](uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3, uint32_t p0, uint32_t p1, uint32_t p2,
+                   uint32_t p3) {
+        const nn_u32x4 c = {c0, c1, c2, c3}, p = {p0, p1, p2, p3};
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(nn_bf16x8, c),
+                                                       __builtin_bit_cast(nn_bf16x8, p),
+                                                       nn_f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+    };
+    // take(a, r, v): v is the element of row r and the particles 16 a + c
+    auto step = [&](int t, auto &&take) {
+        // candidate slots {a b, a c, a b, 1 n}, particle slots {a a, b a, c b, n 1}
+        const uint2 v = T.part[ax][row + 4 * t];
+        const uint32_t ac = __builtin_amdgcn_perm(v.y, v.x, 0x05040100u);
+        const uint32_t n = __builtin_amdgcn_perm(v.y, 0x3f80u, 0x07060100u);
+        uint32_t n2 = 0;
+        if constexpr (!SAME) n2 = (uint32_t)T.norm2[ax][row + 4 * t] << 16 | 0x3f80u;
+#pragma unroll
+        for (int a = 0; a < 4; a += 2) {
+            nn_f32x4 d[2], d2[2];
+#pragma unroll
+            for (int g = 0; g < 2; g++) {
+                uint32_t ab = I.ab[a + g], cn = I.cn[a + g];
+                asm("" : "+v"(ab), "+v"(cn));   // unpacked in every step: kept unpacked, they cost registers
+                const uint32_t p0 = __builtin_amdgcn_perm(ab, ab, 0x01000100u);
+                const uint32_t p1 = __builtin_amdgcn_alignbit(ab, ab, 16);
+                const uint32_t p2 = __builtin_amdgcn_perm(ab, cn, 0x07060100u);
+                const uint32_t p3 = __builtin_amdgcn_alignbit(I.one, cn, 16);
+                d[g] = mfma(v.x, ac, v.x, n, p0, p1, p2, p3);
+                if constexpr (!SAME) d2[g] = mfma(v.x, ac, v.x, n2, p0, p1, p2, I.n2[a + g]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            // the smaller of two floats is the smaller integer, but that of two negative ones it is
+            // the one nearer zero, which at most tests a pair again
+#pragma unroll
+            for (int g = 0; g < 2; g++)
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    take(a + g, r, SAME ? d[g][r] : __int_as_float(min(__float_as_int(d[g][r]), __float_as_int(d2[g][r]))));
+        }
+    };
+#pragma unroll 1
+    for (int t = 0; t < 4; t++) {
+        float least = 3.0e38f;
+        step(t, [&](int a, int, float v) {
+            least = fminf(least, fabsf(v));
+            w[a] = __builtin_amdgcn_alignbit(w[a], __float_as_uint(v), 31);   // the sign: no neighbour
+        });
+        if (wave_ballot(least <= I.eps) != 0) {   // once more, for where
+            any_close = true;
+            step(t, [&](int a, int r, float v) { close[a] |= (fabsf(v) <= I.eps ? 0x8000u : 0u) >> (4 * t + r); });
+        }
+    }
+    wave_sync();
+    nn_tile_bits(w, lo, hi);
+    lo = ~lo;
+    hi = ~hi;
+    if (any_close) {
+        uint32_t cl, ch;
+        nn_tile_bits(close, cl, ch);
+        for (; cl != 0; cl &= cl - 1) {
+            const int e = __builtin_ctz(cl);
+            lo = exact(e) ? lo | 1u << e : lo & ~(1u << e);
+        }
+        for (; ch != 0; ch &= ch - 1) {
+            const int e = __builtin_ctz(ch);
+            hi = exact(32 + e) ? hi | 1u << e : hi & ~(1u << e);
+        }
+    }
 }
 
 // A run of 64 keys can cross a boundary of a large cell.  The Lebesgue curve jumps there, so the
@@ -804,23 +1030,26 @@ __device__ __forceinline__ void nn_group(NNWaveLdsF &L, const NNArgs &A, int64_t
         if (MODE >= 1 && valid && !active && !outlier) A.h_next[k] = hi;
         return;
     }
-    const double hmax = B.h, bx0 = B.x0, bx1 = B.x1, by0 = B.y0, by1 = B.y1, bz0 = B.z0, bz1 = B.z1;
-    const double grow = hmax * (1.0 + 1e-9);
-    const double lox = bx0 - grow, hix = bx1 + grow;
-    const double loy = by0 - grow, hiy = by1 + grow;
-    const double loz = bz0 - grow, hiz = bz1 + grow;
+    if (lane == 0) {
+        const double grow = B.h * (1.0 + 1e-9);
+        L.extra.bounds = NNBounds{B.x0 - grow, B.x1 + grow, B.y0 - grow, B.y1 + grow, B.z0 - grow, B.z1 + grow,
+                                  NNCore{B.x0, B.x1, B.y0, B.y1, B.z0, B.z1, B.h}};
+    }
+    const bool live = active && nn_d2(xi - xi, yi - yi, zi - zi) == 0.0;   // not for positions that are not finite
+    const NNTileI I = nn_tile_group(L.extra, live, xi, yi, zi, hi2, B);
+    wave_sync();
     // candidate filter: squared distance from the box of the active positions, below both
     // hmax^2 and h_j^2.  Per axis fl(b0 - x) <= fl(x_i - x) for every x_i >= b0 (rounding is
     // monotone), and nn_d2 is monotone in each |axis distance|, so this distance never exceeds
     // the pair test's d for any active i, and every
     // pair with d < h_i^2 <= hmax^2 and d < h_j^2 passes: the tiles lose only non-pairs.
-    const double hm2 = hmax * hmax;
     auto keep = [&](double x, double y, double z, double h2) {
-        const double ex = fmax(fmax(bx0 - x, x - bx1), 0.0);
-        const double ey = fmax(fmax(by0 - y, y - by1), 0.0);
-        const double ez = fmax(fmax(bz0 - z, z - bz1), 0.0);
+        const NNCore &q = L.extra.bounds.core;
+        const double ex = fmax(fmax(q.x0 - x, x - q.x1), 0.0);
+        const double ey = fmax(fmax(q.y0 - y, y - q.y1), 0.0);
+        const double ez = fmax(fmax(q.z0 - z, z - q.z1), 0.0);
         const double d = nn_d2(ex, ey, ez);
-        return d < hm2 && d < h2;
+        return d < q.h * q.h && d < h2;
     };
 
     int count = 0;
@@ -842,59 +1071,86 @@ __device__ __forceinline__ void nn_group(NNWaveLdsF &L, const NNArgs &A, int64_t
         if (w1 - w0 < NN_LEAF_GROUP) w0 = w1 = 0;
     }
     // with the window on, the group's own particles are the first candidates streamed, so all of
-    // them that pass the filter are in the first tile: only its pair tests must skip j == k
+    // them that pass the filter are in the first tile: only its hits must skip j == k
     bool first_tile = true;
-    const NNCore core = {bx0, bx1, by0, by1, bz0, bz1, hmax};
-    const bool ok = nn_walk_box<true>(L, A, lox, hix, loy, hiy, loz, hiz, core, NN_START_ALL, w0, w1,
+    const bool ok = nn_walk_box<true>(L, A, [&]() { return L.extra.bounds; }, NN_START_ALL, w0, w1,
                                       (int)(group * 64), keep, [&](int m) {
-        if (!active) return;
-        if (MODE == 1) {
-            for (int e = 0; e < m; e++) {
-                const double dx = xi - L.tx[e];
-                const double dy = yi - L.ty[e];
-                const double dz = zi - L.tz[e];
-                const double d = nn_d2(dx, dy, dz);
-                count += (d < hi2 && d < L.th2[e] && L.tj[e] != (int)k) ? 1 : 0;
-            }
-            return;
-        }
-        // list modes: candidates come as LDS broadcasts, NN_PB per batch with all their reads
-        // issued first (the appends below are branches, across which the compiler does not
-        // move loads).  The append is predicated (three selects shift the pending entries);
-        // only the 16-byte store of every fourth entry is a branch.  The capacity check of
-        // the stores is needed only when some lane could reach max_nb within this tile.
-        auto pairs = [&](auto check_cap, auto check_self) {
-            for (int e = 0; e < m; e += NN_PB) {
-                int js[NN_PB];
-                double xs[NN_PB], ys[NN_PB], zs[NN_PB], h2s[NN_PB];
+        uint32_t bits[2];
+        if (I.on) {
+            const double hm = L.extra.bounds.core.h;
+            auto exact = [&](int e) {
+                const double4 own = A.sxm[k];   // k < n: only live lanes have candidates that are close
+                const double hk = A.h[k];
+                const double d = nn_d2(own.x - L.tx[e], own.y - L.ty[e], own.z - L.tz[e]);
+                return (d < hk * hk) & (d < L.th2[e]);
+            };
+            if (wave_ballot(lane < m && L.th2[lane] < hm * hm) == 0) nn_tile<true>(L, I, m, bits[0], bits[1], exact);
+            else nn_tile<false>(L, I, m, bits[0], bits[1], exact);
+        } else {
+            // FP64: candidates come as LDS broadcasts, NN_PB per batch with all their reads issued
+            // first; one bit per test, the last candidate's lowest.  (The lane's own particle is read
+            // again: kept, it would cost the matrix form its registers.)
+            const int64_t ko = valid ? k : n - 1;
+            const double4 own = A.sxm[ko];
+            const double xi = own.x, yi = own.y, zi = own.z, hi2 = A.h[ko] * A.h[ko];
 #pragma unroll
-                for (int u = 0; u < NN_PB; u++) {
-                    const int eu = e + u < m ? e + u : m - 1;   // m >= 1: a tile is never empty
-                    xs[u] = L.tx[eu];
-                    ys[u] = L.ty[eu];
-                    zs[u] = L.tz[eu];
-                    h2s[u] = L.th2[eu];
-                    js[u] = L.tj[eu];
-                }
+            for (int s = 0; s < 2; s++) {
+                uint32_t b = 0;
+                for (int e = 32 * s; e < 32 * s + 32; e += NN_PB) {   // past the tile's end: any of its slots
+                    double xs[NN_PB], ys[NN_PB], zs[NN_PB], h2s[NN_PB];
 #pragma unroll
-                for (int u = 0; u < NN_PB; u++) {
-                    if (e + u < m) {
-                        const int j = js[u];
+                    for (int u = 0; u < NN_PB; u++) {
+                        xs[u] = L.tx[e + u];
+                        ys[u] = L.ty[e + u];
+                        zs[u] = L.tz[e + u];
+                        h2s[u] = L.th2[e + u];
+                    }
+                    uint32_t hits = 0;
+#pragma unroll
+                    for (int u = 0; u < NN_PB; u++) {
                         const double dx = xi - xs[u];
                         const double dy = yi - ys[u];
                         const double dz = zi - zs[u];
                         const double d = nn_d2(dx, dy, dz);
-                        const bool hit =
-                            (d < hi2) & (d < h2s[u]) & (!decltype(check_self)::value || j != (int)k);
-                        if (hit && (count & 3) == 3) {
-                            if (!decltype(check_cap)::value || count < A.max_nb) *wp = make_int4(p0, p1, p2, j);
-                            wp += A.stride;
-                        }
-                        p0 = hit ? p1 : p0;
-                        p1 = hit ? p2 : p1;
-                        p2 = hit ? j : p2;
-                        count += hit ? 1 : 0;
+                        hits |= ((d < hi2) & (d < h2s[u])) ? 1u << (NN_PB - 1 - u) : 0u;
                     }
+                    b = b << NN_PB | hits;
+                }
+                bits[s] = __builtin_bitreverse32(b);
+            }
+        }
+        if (m < 64) {
+            bits[0] &= m < 32 ? (1u << m) - 1u : ~0u;
+            bits[1] &= m < 32 ? 0u : (1u << (m - 32)) - 1u;
+        }
+        if (!active) return;
+        if (MODE == 1) {   // the particle itself is taken off at the end
+            count += __popc(bits[0]) + __popc(bits[1]);
+            return;
+        }
+        // list modes: only the hits pass through the append code, bit by bit: every lane appends its
+        // own next hit, so a wavefront runs it as often as its busiest lane has hits.  Every fourth
+        // hit's 16-byte store is a branch; its capacity check is needed only when some lane could
+        // reach max_nb within this tile.
+        auto pairs = [&](auto check_cap, auto check_self) {
+            auto append = [&](int j) {
+                if (decltype(check_self)::value && j == (int)k) return;
+                if ((count & 3) == 3) {
+                    if (!decltype(check_cap)::value || count < A.max_nb) *wp = make_int4(p0, p1, p2, j);
+                    wp += A.stride;
+                }
+                p0 = p1;
+                p1 = p2;
+                p2 = j;
+                count++;
+            };
+#pragma unroll
+            for (int s = 0; s < 2; s++) {
+                uint32_t b = bits[s];
+                while (b != 0) {
+                    const int e = __builtin_ctz(b);
+                    b &= b - 1;
+                    append(L.tj[32 * s + e]);
                 }
             }
         };
@@ -912,6 +1168,8 @@ __device__ __forceinline__ void nn_group(NNWaveLdsF &L, const NNArgs &A, int64_t
         if (lane == 0) set_err(A.err, ERRF_STACK);
         return;
     }
+    // every active particle is one of its own candidates
+    if (MODE == 1 && active && nn_d2(xi - xi, yi - yi, zi - zi) < hi2) count--;
     if (MODE == 2 && active && (count & 3) != 0 && count < A.max_nb)
         A.nbr4[(int64_t)(count >> 2) * A.stride + k] = tail4();
     if (MODE == 0 && A.only) {
@@ -973,8 +1231,9 @@ __device__ __forceinline__ void nn_group(NNWaveLdsF &L, const NNArgs &A, int64_t
     }
 }
 
+// Four wavefronts per SIMD (128 registers): free, the matrix tests would take 140 and run at two.
 template <int MODE>
-__global__ __launch_bounds__(64 * NN_WAVES) void k_nn_walk(NNArgs A) {
+__global__ __launch_bounds__(64 * NN_WAVES, 4) void k_nn_walk(NNArgs A) {
     __shared__ NNWaveLdsF lds_all[NN_WAVES];
     const int w = threadIdx.x / 64;
     const int64_t group = xcd_block(blockIdx.x, gridDim.x) * NN_WAVES + w;
@@ -1006,7 +1265,6 @@ __device__ __forceinline__ void nn_one(NNWaveLds &L, const NNArgs &A, unsigned f
         const double4 own = A.sxm[k];
         const double hi = A.h[k];
         const double hi2 = hi * hi;
-        const double grow = hi * (1.0 + 1e-9);
         int count = 0;
         // one candidate per lane: pair test, then the hits appended in lane order
         auto take = [&](bool v, int j, double x, double y, double z, double h2) {
@@ -1025,12 +1283,10 @@ __device__ __forceinline__ void nn_one(NNWaveLds &L, const NNArgs &A, unsigned f
             }
             count += popc64(mh);
         };
-        const double lox = own.x - grow, hix = own.x + grow, loy = own.y - grow, hiy = own.y + grow;
-        const double loz = own.z - grow, hiz = own.z + grow;
-        const bool direct = nn_direct(L.direct, A, lox, hix, loy, hiy, loz, hiz, nn_point(own.x, own.y, own.z, hi),
+        const bool direct = nn_direct(L.extra, A, nn_ball(own, hi),
                                       [&](bool v, int j, const double4 &p, double h) { take(v, j, p.x, p.y, p.z, h * h); });
         if (!direct) {
-            const bool ok = nn_walk_box<false>(L, A, lox, hix, loy, hiy, loz, hiz, nn_point(own.x, own.y, own.z, hi), NN_START_ALL, 0, 0, -1, KeepAll(), [&](int m) {
+            const bool ok = nn_walk_box<false>(L, A, [&]() { return nn_ball(own, hi); }, NN_START_ALL, 0, 0, -1, KeepAll(), [&](int m) {
                 const bool v = lane < m;
                 take(v, v ? L.tj[lane] : -1, v ? L.tx[lane] : 0.0, v ? L.ty[lane] : 0.0, v ? L.tz[lane] : 0.0,
                      v ? L.th2[lane] : 0.0);
@@ -1121,7 +1377,6 @@ __global__ __launch_bounds__(64 * NN1_WAVES) void k_nn_mark_dirty(NNArgs A) {
         const double h0 = A.h0_slot[t], h1 = A.h[jc];
         const double h02 = h0 * h0, h12 = h1 * h1;
         const double hq = h0 > h1 ? h0 : h1;
-        const double grow = hq * (1.0 + 1e-9);
         if (DIRECT && lane == 0) A.dirty[jc] = 1;
         auto mark = [&](bool v, int i, double x, double y, double z, double hi2) {
             if (v) {
@@ -1132,14 +1387,12 @@ __global__ __launch_bounds__(64 * NN1_WAVES) void k_nn_mark_dirty(NNArgs A) {
                 if (((d < hi2) & (d < h02)) != ((d < hi2) & (d < h12))) A.dirty[i] = 1;
             }
         };
-        const double lox = own.x - grow, hix = own.x + grow, loy = own.y - grow, hiy = own.y + grow;
-        const double loz = own.z - grow, hiz = own.z + grow;
         if constexpr (DIRECT) {
-            const bool direct = nn_direct(L, A, lox, hix, loy, hiy, loz, hiz, nn_point(own.x, own.y, own.z, hq),
+            const bool direct = nn_direct(L, A, nn_ball(own, hq),
                                           [&](bool v, int i, const double4 &p, double h) { mark(v, i, p.x, p.y, p.z, h * h); });
             if (!direct && lane == 0) A.list_out[atomicAdd(A.count_out, 1u)] = (int32_t)t;
         } else {
-            const bool ok = nn_walk_box<false>(L, A, lox, hix, loy, hiy, loz, hiz, nn_point(own.x, own.y, own.z, hq), NN_START_ALL, 0, 0, -1, KeepAll(), [&](int m) {
+            const bool ok = nn_walk_box<false>(L, A, [&]() { return nn_ball(own, hq); }, NN_START_ALL, 0, 0, -1, KeepAll(), [&](int m) {
                 if (lane < m) mark(true, L.tj[lane], L.tx[lane], L.ty[lane], L.tz[lane], L.th2[lane]);
             });
             if (!ok) {
@@ -1169,10 +1422,8 @@ __global__ __launch_bounds__(64 * NN1_WAVES) void k_nn_count_direct(NNArgs A) {
         const double4 own = A.sxm[k];
         const double hi = A.h[k];
         const double hi2 = hi * hi;
-        const double grow = hi * (1.0 + 1e-9);
         int count = 0;
-        const bool direct = nn_direct(L, A, own.x - grow, own.x + grow, own.y - grow, own.y + grow, own.z - grow,
-                                      own.z + grow, nn_point(own.x, own.y, own.z, hi),
+        const bool direct = nn_direct(L, A, nn_ball(own, hi),
                                       [&](bool v, int j, const double4 &p, double h) {
             if (v) {
                 const double dx = own.x - p.x;
@@ -1212,11 +1463,9 @@ __global__ __launch_bounds__(64 * NN1_WAVES) void k_nn_count_split(NNArgs A) {
         const double4 own = A.sxm[k];
         const double hi = A.h[k];
         const double hi2 = hi * hi;
-        const double grow = hi * (1.0 + 1e-9);
         const int start = NN_START_PART0 - o;   // eighth o of the start cells
         int count = 0;
-        const bool ok = nn_walk_box<false>(L, A, own.x - grow, own.x + grow, own.y - grow, own.y + grow, own.z - grow,
-                                    own.z + grow, nn_point(own.x, own.y, own.z, hi), start, 0, 0, -1, KeepAll(), [&](int m) {
+        const bool ok = nn_walk_box<false>(L, A, [&]() { return nn_ball(own, hi); }, start, 0, 0, -1, KeepAll(), [&](int m) {
             bool hit = false;
             if (lane < m) {
                 const double dx = own.x - L.tx[lane];
@@ -1326,9 +1575,7 @@ __global__ __launch_bounds__(64 * NN1_WAVES) void k_h_pass(NNArgs A) {
         } else {
             const double4 own = A.sxm[k];
             const double hi2 = hi * hi;
-            const double grow = hi * (1.0 + 1e-9);
-            nn_direct(L, A, own.x - grow, own.x + grow, own.y - grow, own.y + grow, own.z - grow, own.z + grow,
-                      nn_point(own.x, own.y, own.z, hi), [&](bool v, int j, const double4 &p, double h) {
+                nn_direct(L, A, nn_ball(own, hi), [&](bool v, int j, const double4 &p, double h) {
                 if (v) {
                     const double dx = own.x - p.x;
                     const double dy = own.y - p.y;

@@ -268,3 +268,47 @@ def test_relists_around_boxes_the_direct_search_declines(gpu_lib, orc, curve):
         assert np.array_equal(a[k], b[k]), k
     assert a["sets"] == b["sets"]
     assert np.max(np.abs(a["rho"] - b["rho"])) <= 1e-12 * a["rho"].max()   # order of 180 terms at most
+
+
+@pytest.mark.parametrize("scale,offset,mixed", [(1.0, 0.0, True), (1.0, 0.0, False), (2.0 ** 60, 0.0, True),
+                                                (2.0 ** -60, 0.0, True), (1.0, 2.0 ** 20, True),
+                                                (1.0, 0.0, "far"), (1.0, 0.0, "random")])
+def test_group_walks_decide_pairs_at_the_radius_exactly(gpu_lib, orc, scale, offset, mixed):
+    """Lattice distances are whole, and the radii are whole or one rounding to either side: a pair's
+    squared distance equals, just misses or just meets h^2, in both particles' h.  The walks' matrix
+    tests cannot tell these apart and must leave them to the FP64 test: neighbour sets and counts are
+    the oracle's, at scales whose squares leave FP32, far from the origin, and (`far`) in groups whose
+    box is too large against h for the matrix tests."""
+    print_case(f"pairs at the radius scale={scale} offset={offset} mixed={mixed}")
+    side = 33
+    n = side ** 3
+    rng = np.random.default_rng(3)
+    g = np.stack(np.meshgrid(*[np.arange(side, dtype=np.float64)] * 3, indexing="ij")).reshape(3, n)
+    r = np.array([2.0, 3.0, 2.5, 2.0])
+    r = np.concatenate([r, np.nextafter(r, 9.0), np.nextafter(r, 0.0)])
+    h = rng.choice(r, n) if mixed else np.full(n, np.nextafter(3.0, 9.0))
+    if mixed == "far":
+        h = np.where(rng.uniform(size=n) < 0.5, 1.0, np.nextafter(1.0, 2.0))
+        g = g * np.where(np.arange(3) < 2, 1.0, 40.0)[:, None]
+    if mixed == "random":
+        g = rng.uniform(0.0, side, (3, n))
+        h = rng.uniform(1.5, 2.6, n)
+    p = (g + offset) * scale
+    h = h * scale
+    s = dict(x=p[0], y=p[1], z=p[2], mass=np.full(n, 1.0 / n), sml=h)
+    st, onnl, onoi = orc.nn_grid(p[0], p[1], p[2], h, 180)
+    assert st == 0
+    with load_ctx(gpu_lib, s, gpu_lib.default_params(curve=0)) as ctx:
+        ctx.bbox(); ctx.keys(); ctx.sort(); ctx.build_tree()
+        ctx.neighbours()
+        nnl, noi = ctx.neighbour_lists(180)
+    assert np.array_equal(noi, onoi)
+    used = np.arange(180) < noi[:, None]
+    assert np.array_equal(np.sort(np.where(used, nnl, -1), 1), np.sort(np.where(used, onnl, -1), 1))
+    # the counting and the list-writing passes of the h-iteration, from the same h
+    oh, oiters = orc.h_iterate(p[0], p[1], p[2], h)[1:3]
+    for spec in (0, gpu_lib.RHS_SPECULATIVE_NN):
+        with load_ctx(gpu_lib, s, gpu_lib.default_params(curve=0)) as ctx:
+            ctx.rhs(gpu_lib.RHS_SPH | gpu_lib.RHS_VARIABLE_SML | spec)
+            assert np.array_equal(ctx.download("sml"), oh)
+            assert np.array_equal(ctx.download("h_iters"), oiters)
