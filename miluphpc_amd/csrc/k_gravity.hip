@@ -230,13 +230,15 @@ __global__ __launch_bounds__(64 * (MULTI ? BH_MULTI_MAX : BH_WAVES)) void k_bh_w
     const double glo_x = wave_min(valid ? px : 1e300), ghi_x = wave_max(valid ? px : -1e300);
     const double glo_y = wave_min(valid ? py : 1e300), ghi_y = wave_max(valid ? py : -1e300);
     const double glo_z = wave_min(valid ? pz : 1e300), ghi_z = wave_max(valid ? pz : -1e300);
-    const int nvalid = popc64(wave_ballot(valid));
+    const uint64_t mInvalid = ~wave_ballot(valid);
+    const int nvalid = 64 - popc64(mInvalid);
     // acceptance constants, same expressions as the oracle
     const double R = 0.5 * (A.box[1] - A.box[0]);
     const double s2_0 = 4.0 * R * R;
     const double dp_1 = R * R / A.theta;
     const double theta2 = A.theta * A.theta;
     const double eps2 = A.eps2;
+    const bool classic = A.mac == MHPC_MAC_CLASSIC;
     // FP32 mode: positions relative to the group's centre
     const double refx = 0.5 * (glo_x + ghi_x), refy = 0.5 * (glo_y + ghi_y), refz = 0.5 * (glo_z + ghi_z);
     const T tx = FP64 ? (T)px : (T)(px - refx), ty = FP64 ? (T)py : (T)(py - refy),
@@ -297,13 +299,13 @@ __global__ __launch_bounds__(64 * (MULTI ? BH_MULTI_MAX : BH_WAVES)) void k_bh_w
         bool accept = false, open = false;
         double ccx = 0, ccy = 0, ccz = 0;
         int64_t c = 0;
-        int lev = 0;
-        // the acceptance test of distance^2 d2 for a cell of level L (same expressions as the
+        double size = 0.0;
+        // the acceptance test of distance^2 d2 for a cell of size term S (same expressions as the
         // oracle)
-        auto mac_ok = [&](double d2, int L) {
-            if (A.mac == MHPC_MAC_CLASSIC) return (d2 + eps2) * theta2 > s2_0 * ldexp(1.0, -2 * L);
-            return dp_1 * ldexp(1.0, -2 * (L - 1)) <= d2 + eps2;
+        auto mac_size = [&](int L) {
+            return classic ? s2_0 * ldexp(1.0, -2 * L) : dp_1 * ldexp(1.0, -2 * (L - 1));
         };
+        auto mac_ok = [&](double d2, double S) { return classic ? (d2 + eps2) * theta2 > S : S <= d2 + eps2; };
         // everything the round may need of its node is requested together, before the test
         // decides which of it is used: one memory round trip per round instead of one for the
         // test and one more for the children or the list entries
@@ -325,12 +327,11 @@ __global__ __launch_bounds__(64 * (MULTI ? BH_MULTI_MAX : BH_WAVES)) void k_bh_w
             ccx = A.cx[c];
             ccy = A.cy[c];
             ccz = A.cz[c];
-            lev = A.clevel[c];
-            double dx = 0.0, dy = 0.0, dz = 0.0;
-            if (ccx < glo_x) dx = glo_x - ccx; else if (ccx > ghi_x) dx = ccx - ghi_x;
-            if (ccy < glo_y) dy = glo_y - ccy; else if (ccy > ghi_y) dy = ccy - ghi_y;
-            if (ccz < glo_z) dz = glo_z - ccz; else if (ccz > ghi_z) dz = ccz - ghi_z;
-            accept = mac_ok(dx * dx + dy * dy + dz * dz, lev);
+            size = mac_size(A.clevel[c]);
+            const double dx = fmax(fmax(glo_x - ccx, ccx - ghi_x), 0.0);
+            const double dy = fmax(fmax(glo_y - ccy, ccy - ghi_y), 0.0);
+            const double dz = fmax(fmax(glo_z - ccz, ccz - ghi_z), 0.0);
+            accept = mac_ok(dx * dx + dy * dy + dz * dz, size);
         }
         if constexpr (VOTE) {
             // cells the box test rejects: one member's rejection settles the vote, and the
@@ -339,7 +340,7 @@ __global__ __launch_bounds__(64 * (MULTI ? BH_MULTI_MAX : BH_WAVES)) void k_bh_w
             if (amb) {
                 const int o = (ccx > refx ? 1 : 0) | (ccy > refy ? 2 : 0) | (ccz > refz ? 4 : 0);
                 const double dx = ccx - ends[o], dy = ccy - ends[8 + o], dz = ccz - ends[16 + o];
-                amb = mac_ok(dx * dx + dy * dy + dz * dz, lev);
+                amb = mac_ok(dx * dx + dy * dy + dz * dz, size);
             }
             // the others: every member tests each with its own distance
             uint64_t mAmb = wave_ballot(amb);
@@ -348,10 +349,10 @@ __global__ __launch_bounds__(64 * (MULTI ? BH_MULTI_MAX : BH_WAVES)) void k_bh_w
                 const int b = __builtin_ctzll(mAmb);
                 mAmb &= mAmb - 1;
                 const double bx = readlane_d(ccx, b), by = readlane_d(ccy, b), bz = readlane_d(ccz, b);
-                const int bl = __builtin_amdgcn_readlane(lev, b);
+                const double bs = readlane_d(size, b);
                 const double dx = bx - px, dy = by - py, dz = bz - pz;
-                const bool ok = !valid || mac_ok(dx * dx + dy * dy + dz * dz, bl);
-                if (wave_ballot(ok) == ~0ull) mVote |= 1ull << b;
+                const bool ok = mac_ok(dx * dx + dy * dy + dz * dz, bs);
+                if ((wave_ballot(ok) | mInvalid) == ~0ull) mVote |= 1ull << b;
             }
             accept = accept || ((mVote >> lane) & 1ull);
         }
