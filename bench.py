@@ -292,9 +292,9 @@ def run_sedov(args, lib, ics, result):
         gbs = bpp * n / (med[k] * 1e-3) / 1e9
         kernels[k[3:]] = {"kernel": name, "ms": round(med[k], 4), "alg_bytes_per_particle": round(bpp, 1),
                           "GB/s": round(gbs, 1), "frac": round(gbs / HBM_PEAK_GBS, 4)}
-    kernels["nn_fixup"] = {"kernel": "k_nn_mark_dirty + k_nn_walk<0> + k_nn_one<0> (re-lists)",
+    kernels["nn_fixup"] = {"kernel": "k_nn_mark_dirty + k_nn_walk<0> + k_nn_rest<0> (re-lists)",
                            "ms": round(phase_med["ms_nn"], 4), "note": "re-lists only the changed neighbourhoods"}
-    kernels["hiter_rest"] = {"kernel": "pass-0 outliers + tail passes (k_nn_one, k_nn_count_direct, k_h_finish)",
+    kernels["hiter_rest"] = {"kernel": "pass-0 parts and outliers + tail passes (k_nn_rest, k_nn_count_direct, k_h_finish)",
                              "ms": round(phase_med["ms_hiter"] - phase_med["ms_nn_walk"], 4)}
     # the roofline is quoted on the kernel with the largest time per RHS
     dom = max(table, key=lambda k: med[k])

@@ -372,11 +372,6 @@ __device__ __forceinline__ T row_sum(T v) {
     auto op = [](T a, T b) { return a + b; };
     return wave_step<3>(wave_step<2>(wave_step<1>(wave_step<0>(v, op), op), op), op);
 }
-template <typename T>
-__device__ __forceinline__ T row_max(T v) {
-    auto op = [](T a, T b) { return b > a ? b : a; };
-    return wave_step<3>(wave_step<2>(wave_step<1>(wave_step<0>(v, op), op), op), op);
-}
 
 // inclusive prefix sum over the wave: within rows of 16 by shifts, then the rows' totals
 __device__ __forceinline__ int wave_incl_scan(int v) {
