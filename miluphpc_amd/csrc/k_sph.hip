@@ -785,7 +785,8 @@ __device__ __forceinline__ NNTileI nn_tile_group(NNTileLds &T, bool live, double
     const double reach =
         0.5 * sqrt(nn_d2((B.x1 - B.x0) * scale, (B.y1 - B.y0) * scale, (B.z1 - B.z0) * scale)) + hs;
     const double M = reach * reach;
-    I.on = M <= NN_MFMA_REACH && B.h > 0.0;   // false for boxes that are not finite
+    // false for boxes that are not finite; beyond these h the squares leave the normal numbers
+    I.on = M <= NN_MFMA_REACH && B.h > 1e-140 && B.h < 1e140;
     I.eps = (float)(M * 1.52587890625e-05);
     if (!I.on) return I;
     const double X = live ? (x - cx) * scale : 0.0, Y = live ? (y - cy) * scale : 0.0,
@@ -1035,7 +1036,8 @@ __device__ __forceinline__ void nn_group(NNWaveLdsF &L, const NNArgs &A, int64_t
         L.extra.bounds = NNBounds{B.x0 - grow, B.x1 + grow, B.y0 - grow, B.y1 + grow, B.z0 - grow, B.z1 + grow,
                                   NNCore{B.x0, B.x1, B.y0, B.y1, B.z0, B.z1, B.h}};
     }
-    const bool live = active && nn_d2(xi - xi, yi - yi, zi - zi) == 0.0;   // not for positions that are not finite
+    // not for positions that are not finite, nor for an h that is no number: they have no neighbours
+    const bool live = active && nn_d2(xi - xi, yi - yi, zi - zi) == 0.0 && hi2 >= 0.0;
     const NNTileI I = nn_tile_group(L.extra, live, xi, yi, zi, hi2, B);
     wave_sync();
     // candidate filter: squared distance from the box of the active positions, below both

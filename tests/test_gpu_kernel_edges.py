@@ -312,3 +312,25 @@ def test_group_walks_decide_pairs_at_the_radius_exactly(gpu_lib, orc, scale, off
             ctx.rhs(gpu_lib.RHS_SPH | gpu_lib.RHS_VARIABLE_SML | spec)
             assert np.array_equal(ctx.download("sml"), oh)
             assert np.array_equal(ctx.download("h_iters"), oiters)
+
+
+@pytest.mark.parametrize("scale", [2.0 ** 500, 2.0 ** -500, 2.0 ** -520])
+def test_group_walks_where_squares_leave_the_normal_numbers(gpu_lib, orc, scale):
+    """Radii whose squares come close to the largest FP64 number, or are denormal (exact multiples of
+    the lattice's, so the comparison still has one answer): neighbour sets are the oracle's."""
+    print_case(f"extreme scales scale={scale}")
+    side = 33
+    n = side ** 3
+    rng = np.random.default_rng(4)
+    p = np.stack(np.meshgrid(*[np.arange(side, dtype=np.float64)] * 3, indexing="ij")).reshape(3, n)
+    h = rng.choice([2.0, 2.5, 3.0], n)
+    st, onnl, onoi = orc.nn_grid(p[0], p[1], p[2], h, 180)   # scaling by a power of two changes nothing
+    assert st == 0
+    s = dict(x=p[0] * scale, y=p[1] * scale, z=p[2] * scale, mass=np.full(n, 1.0 / n), sml=h * scale)
+    with load_ctx(gpu_lib, s, gpu_lib.default_params(curve=0)) as ctx:
+        ctx.bbox(); ctx.keys(); ctx.sort(); ctx.build_tree()
+        ctx.neighbours()
+        nnl, noi = ctx.neighbour_lists(180)
+    assert np.array_equal(noi, onoi)
+    used = np.arange(180) < noi[:, None]
+    assert np.array_equal(np.sort(np.where(used, nnl, -1), 1), np.sort(np.where(used, onnl, -1), 1))
