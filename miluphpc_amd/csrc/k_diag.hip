@@ -25,31 +25,61 @@ struct Neu {
         add(o.c);
     }
     __device__ __forceinline__ double value() const { return s + c; }
-    // the wave's sum in every lane: a butterfly of compensated merges (each step adds a lane's
-    // sum and correction into its partner's, lower lane first, so both hold the same bits)
+    // merges over each row of 16 lanes, the row's sum in its first lane (the other lanes hold it
+    // with its terms in another order)
+    template <int CTRL>
+    __device__ __forceinline__ void merge_dpp() {
+        auto moved = [](double v) {
+            const uint64_t u = __builtin_bit_cast(uint64_t, v);
+            const uint32_t lo = (uint32_t)dpp_mov<CTRL>((int)u), hi = (uint32_t)dpp_mov<CTRL>((int)(u >> 32));
+            return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+        };
+        Neu o;
+        o.s = moved(s);
+        o.c = moved(c);
+        add(o);
+    }
+    __device__ __forceinline__ void row_fold() {
+        merge_dpp<DPP_XOR1>();
+        merge_dpp<DPP_XOR2>();
+        merge_dpp<DPP_HALF_MIRROR>();
+        merge_dpp<DPP_MIRROR>();
+    }
+    // a merged over the wave's halves (ROWS 2) or over its rows pairwise (ROWS 1) in the lower half /
+    // the even rows, b in the upper half / the odd rows: one merge for two quantities
+    template <int ROWS>
+    static __device__ __forceinline__ Neu merge_rows(const Neu &a, const Neu &b) {
+        Neu r, o;
+        auto swap = [](double x, double y, double &first, double &second) {
+            const uint64_t u = __builtin_bit_cast(uint64_t, x), v = __builtin_bit_cast(uint64_t, y);
+            const auto lo = ROWS == 2 ? __builtin_amdgcn_permlane32_swap((uint32_t)u, (uint32_t)v, false, false)
+                                      : __builtin_amdgcn_permlane16_swap((uint32_t)u, (uint32_t)v, false, false);
+            const auto hi = ROWS == 2
+                                ? __builtin_amdgcn_permlane32_swap((uint32_t)(u >> 32), (uint32_t)(v >> 32), false, false)
+                                : __builtin_amdgcn_permlane16_swap((uint32_t)(u >> 32), (uint32_t)(v >> 32), false, false);
+            first = __builtin_bit_cast(double, (uint64_t)hi[0] << 32 | lo[0]);
+            second = __builtin_bit_cast(double, (uint64_t)hi[1] << 32 | lo[1]);
+        };
+        swap(a.s, b.s, r.s, o.s);
+        swap(a.c, b.c, r.c, o.c);
+        r.add(o);
+        return r;
+    }
+    // the wave's sum in lane 0
     __device__ __forceinline__ void wave_fold() {
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            Neu a, b;
-            const double ps = __shfl_xor(s, o), pc = __shfl_xor(c, o);
-            const bool upper = wave_lane() & o;
-            a.s = upper ? ps : s;
-            a.c = upper ? pc : c;
-            b.s = upper ? s : ps;
-            b.c = upper ? c : pc;
-            a.add(b);
-            *this = a;
-        }
+        row_fold();
+        *this = merge_rows<1>(*this, *this);
+        *this = merge_rows<2>(*this, *this);
     }
 };
 
 // quantities: 0 kinetic, 1 potential (sum u), 2 internal (sum m e), 3-5 momentum,
 // 6-8 angular momentum sum m x cross v, 9 mass, 10-12 sum m x
 //
-// Bound by the nine field reads (72 B per particle).  A block's 256 partial sums are merged by
-// wavefront butterflies: one thread per quantity adding them in turn was a chain of 512 dependent
-// compensated additions (68 us for 2,097,152 particles; 42 us as butterflies, 40 us = 3.8 TB/s with
-// the next particle's fields requested ahead).
+// Bound by the nine field reads (72 B per particle).  One thread per quantity adding a block's 256
+// partial sums in turn was a chain of 512 dependent compensated additions (68 us for 2,097,152
+// particles); a butterfly per quantity through LDS 40 us, with the next particle's fields requested
+// ahead; lane-row swaps that merge two quantities at once 28.7 us = 5.3 TB/s, a large copy's rate.
 __global__ __launch_bounds__(256) void k_diag_partial(int64_t n, const double *__restrict__ x,
                                                       const double *__restrict__ y,
                                                       const double *__restrict__ z,
@@ -90,12 +120,18 @@ __global__ __launch_bounds__(256) void k_diag_partial(int64_t n, const double *_
         q[12].add(mi * zi);
     }
     __shared__ double ws[DIAG_Q][4], wc[DIAG_Q][4];
+    // sixteen quantities to eight per half wave, four per row, then over the rows: 28 merges where
+    // a butterfly per quantity is 78.  Row r's first lane ends with quantities 4 r .. 4 r + 3.
 #pragma unroll
-    for (int k = 0; k < DIAG_Q; k++) {
-        q[k].wave_fold();
-        if (wave_lane() == 0) {
-            ws[k][threadIdx.x / 64] = q[k].s;
-            wc[k][threadIdx.x / 64] = q[k].c;
+    for (int k = 0; k < 8; k++) q[k] = Neu::merge_rows<2>(q[k], k + 8 < DIAG_Q ? q[k + 8 < DIAG_Q ? k + 8 : 0] : Neu());
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        q[k] = Neu::merge_rows<1>(q[k], q[k + 4]);
+        q[k].row_fold();
+        const int at = 4 * (wave_lane() >> 4) + k;
+        if ((wave_lane() & 15) == 0 && at < DIAG_Q) {
+            ws[at][threadIdx.x / 64] = q[k].s;
+            wc[at][threadIdx.x / 64] = q[k].c;
         }
     }
     __syncthreads();
