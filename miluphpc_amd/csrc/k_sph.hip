@@ -1960,6 +1960,13 @@ __device__ __forceinline__ float rcp_f32(float x) {
     const float y = __builtin_amdgcn_rcpf(x);
     return __builtin_fmaf(y, __builtin_fmaf(-x, y, 1.f), y);
 }
+// n/d from the estimate of 1/d, corrected by the quotient's exact residual: 0.5 ulp and a little, in
+// four instructions (a correctly rounded division takes about ten)
+__device__ __forceinline__ float div_f32(float n, float d) {
+    const float y = __builtin_amdgcn_rcpf(d);
+    const float q = n * y;
+    return __builtin_fmaf(__builtin_fmaf(-d, q, n), y, q);
+}
 __device__ __forceinline__ float rsq_f32(float x) {
     const float y = __builtin_amdgcn_rsqf(x);
     return __builtin_fmaf(0.5f * y, __builtin_fmaf(-(x * y), y, 1.f), y);
@@ -2404,9 +2411,11 @@ struct ForceI {   // particle i's data and the constants of the pair loop
 // {rho, p/rho^2, m/rho, h}.  The loop is bound by its instructions as much as by its gathers, so
 // every shared factor is taken out: with grad W = gs r_ij, v.grad W = gs (v.r_ij) and the
 // acceleration is (fa gs) r_ij; the viscosity Pi_ij = (beta mu - alpha c) mu / rho with
-// mu = h v.r / D, D = r^2 + 0.01 h^2, is taken as one quotient over D^2 rho (two reciprocals fewer
-// instructions than dividing by D and by rho).  112 -> 96 vector instructions per FP64 pair (256^3 RHS 18.1 ->
-// 17.9 ms).
+// mu = h v.r / D, D = r^2 + 0.01 h^2, is taken in FP64 as one quotient over D^2 rho (two reciprocals
+// fewer instructions than dividing by D and by rho).  112 -> 96 vector instructions per FP64 pair
+// (256^3 RHS 18.1 -> 17.9 ms).  In FP32 numerator and D^2, which grow like h^4, would leave the
+// range in which every other term of the pair stays (h of 50 km in metres): there mu, of the size of
+// v, is formed first.
 // mu is negative wherever it is used, so the largest mu_ij, which starts at 0
 // (internal_forces.cu:135, :383-385), is always 0.
 template <bool FP64, bool FEAT, bool CUBIC>
@@ -2443,16 +2452,20 @@ __device__ __forceinline__ void force_pair(const ForceI &I, const double4 &pj, c
     const T vr = fma(v0, d0, fma(v1, d1, v2 * d2));
     const T vv = gs * vr;   // v.grad W
     const T mj = (T)pj.w;
-    // m_j Pi_ij = m (2 h v.r) (beta/2 (2 h v.r) - alpha c D) / (D^2 (rho_i + rho_j)), c the mean
-    // sound speed
+    // Pi_ij = (beta mu - alpha c) mu / rho, mu = h v.r / D, c and rho the pair's means
     const T D = fma(hb * hb, T(1e-2), r2);
-    const T x = hs * vr;
-    const T cD = T(0.5) * ((T)vi.w + (T)vj.w) * D;
-    const T num = mj * x * fma(T(0.5) * (T)I.beta, x, -(T)I.alpha * cD);
-    const T den = D * D * ((T)ri.x + (T)rj.x);
     T mpij;
-    if constexpr (FP64) mpij = num * rcp_f64(den);
-    else mpij = num * rcp_f32(den);
+    if constexpr (FP64) {
+        // m (2 h v.r) (beta/2 (2 h v.r) - alpha c D) / (D^2 (rho_i + rho_j))
+        const T x = hs * vr;
+        const T cD = T(0.5) * (vi.w + vj.w) * D;
+        const T num = mj * x * fma(T(0.5) * I.beta, x, -I.alpha * cD);
+        mpij = num * rcp_f64(D * D * (ri.x + rj.x));
+    } else {
+        const T mu = div_f32(hb * vr, D);
+        const T c = T(0.5) * ((T)vi.w + (T)vj.w), rho = T(0.5) * ((T)ri.x + (T)rj.x);
+        mpij = div_f32(mj * fma((T)I.beta, mu, -(T)I.alpha * c) * mu, rho);
+    }
     mpij = vr < T(0) ? mpij : T(0);
     const T pf = -mj * ((T)ri.y + (T)rj.y);
     const T fa = (pf - mpij) * gs;

@@ -334,3 +334,46 @@ def test_group_walks_where_squares_leave_the_normal_numbers(gpu_lib, orc, scale)
     assert np.array_equal(noi, onoi)
     used = np.arange(180) < noi[:, None]
     assert np.array_equal(np.sort(np.where(used, nnl, -1), 1), np.sort(np.where(used, onnl, -1), 1))
+
+
+def gas_in_units(side, h, v, rho, cs, seed=17):
+    """A jittered lattice of gas with smoothing length h and random velocities of size v, density rho
+    and sound speed cs, in whatever units these are."""
+    s = ics.sedov_lattice(side)
+    rng = np.random.default_rng(seed)
+    n = side ** 3
+    L = h / float(s["sml"][0])
+    for a in "xyz":
+        s[a] = L * (s[a] + 0.1 / side * rng.uniform(-1, 1, n))
+        s["v" + a] = v * rng.normal(size=n)
+    s["sml"] = L * s["sml"]
+    s["mass"] = np.full(n, rho * L ** 3 / n)
+    s["e"] = cs ** 2 / (5.0 / 3.0 * 2.0 / 3.0) * rng.uniform(0.9, 1.1, n)
+    s["p"] = 2.0 / 3.0 * rho * s["e"]
+    s["rho"] = np.full(n, rho)
+    return s
+
+
+def compare_fp32_rhs(gpu_lib, orc, s):
+    """The FP32 SPH RHS against the FP64 oracle.  A pair term carries about a dozen roundings
+    (7e-7) and a sum's terms add up to some 30 times the field's RMS."""
+    p = gpu_lib.default_params(precision=gpu_lib.PREC_FP32_KAHAN)
+    with load_ctx(gpu_lib, s, p) as ctx:
+        ctx.rhs(gpu_lib.RHS_SPH | gpu_lib.RHS_VARIABLE_SML)
+        g = {k: ctx.download(k) for k in ("sml", "rho", "ax", "ay", "az", "drhodt", "dedt", "dsmldt")}
+    o = orc.sph_rhs(s)
+    assert np.array_equal(g["sml"], o["sml"])
+    assert np.max(np.abs(g["rho"] / o["rho"] - 1.0)) < 5e-6
+    for k in ("ax", "ay", "az", "drhodt", "dedt", "dsmldt"):
+        scale = np.maximum(np.abs(o[k]), np.sqrt(np.mean(o[k] ** 2)))
+        assert np.all(np.isfinite(g[k])), k
+        assert np.max(np.abs(g[k] - o[k]) / scale) < 5e-5, k
+
+
+@pytest.mark.parametrize("side", [16, 37])   # shared lists; windows
+@pytest.mark.parametrize("h,v,rho,cs", [(1e5, 1e4, 3e3, 5e3), (5e4, 3e3, 3e3, 5e3), (1e6, 1e6, 3.0, 5e5),
+                                        (1e-5, 1.0, 1e-18, 0.5), (1.0, 1.0, 1.0, 0.5)])
+def test_fp32_forces_in_physical_units(gpu_lib, orc, side, h, v, rho, cs):
+    """FP32 pair sums where lengths are far from one: rock in SI and cgs units, thin gas at small h."""
+    print_case(f"fp32 forces side={side} h={h} v={v} rho={rho}")
+    compare_fp32_rhs(gpu_lib, orc, gas_in_units(side, h, v, rho, cs))
