@@ -26,7 +26,8 @@ static_assert(NN_LEAF_GROUP < NN_CWIN, "a clipped range crosses at most one end 
 #define NN_OUTLIER_MAX 32    // at most this many outliers per group are split off
 #define NN_SPLIT_VOL 8.0     // group walks: a box of more than this many search cubes (2 h)^3 ...
 #define NN_SPLIT_CAND 3072   // ... whose start cells hold more than this many particles is split
-#define NN_SPLIT_MIN 16      // split-off parts of fewer particles go to the per-particle mode
+#define NN_PART_CAND 12288   // split-off parts of more candidates than this, and ...
+#define NN_SPLIT_MIN 16      // ... of fewer particles go to the per-particle mode
 static_assert(64 / NN_SPLIT_MIN <= MHPC_NN_PARTS_PER_GROUP, "the part list holds every group's parts");
 // Re-lists: groups with at most this many flagged particles go per particle (lanes are
 // candidates), the others are walked again.  A group walk costs as much as about ten
@@ -733,6 +734,12 @@ __device__ __forceinline__ NNBox nn_box(bool active, double x, double y, double 
 // The FP64 tests were most of a walk that is bound by its instructions: 6 operations, 2
 // comparisons and a bit per pair, against 1.5 to 2.5 instructions here (256^3 list walk 6.4 -> 5.2 ms,
 // 47^3 RHS in two walks 884 -> 668 us, 1M cloud RHS 5.05 -> 4.80 ms, 128^3 blast step 7.69 -> 7.50 ms).
+// Sets with a dense clump (40,000 particles, half of them in a ball of 1/1000 of the box): of a group
+// that also holds particles from outside, those inside find every particle of the clump within eps,
+// and the tests one by one cost more than the tile's by broadcast (k_nn_walk<1> 3.7 ms; 2.0 with such
+// tiles tested by broadcast, 1.7 also without the matrix tests in the rest of such a group's walk).
+#define NN_CLOSE_MAX 16      // a lane's candidates tested one by one in a tile
+#define NN_CLOSE_OFF 48      // with more than these, no matrix tests in the group's further tiles
 #define NN_MFMA_REACH 64.0   // largest M (h is 1 to 2): above, most tiles hold a pair too close to zero
 typedef unsigned nn_u32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 nn_bf16x8 __attribute__((ext_vector_type(8)));
@@ -829,8 +836,10 @@ __device__ __forceinline__ void nn_tile_bits(const uint32_t w[4], uint32_t &lo, 
 // The tests of the tile's m candidates (bit e of lo, e - 32 of hi: candidate e; bits past m are any)
 // for every lane's particle; `exact(e)` is the lane's test of candidate e in FP64.  SAME: every
 // candidate's h^2 is at least the largest of the group, so h_i^2 alone decides.
+// Returns false, with the bits of the candidates left to FP64, where some lane has more than
+// NN_CLOSE_MAX of them: the caller tests the whole tile then.
 template <bool SAME, typename LdsT, typename ExactFn>
-__device__ __forceinline__ void nn_tile(LdsT &L, const NNTileI &I, int m, uint32_t &lo, uint32_t &hi,
+__device__ __forceinline__ bool nn_tile(LdsT &L, const NNTileI &I, int m, uint32_t &lo, uint32_t &hi,
                                         ExactFn &&exact) {
     const int lane = wave_lane(), q = lane >> 4, ax = q < 3 ? q : 0;
     NNTileLds &T = L.extra;
@@ -908,6 +917,11 @@ __device__ __forceinline__ void nn_tile(LdsT &L, const NNTileI &I, int m, uint32
     if (any_close) {
         uint32_t cl, ch;
         nn_tile_bits(close, cl, ch);
+        if (wave_ballot(__popc(cl) + __popc(ch) > NN_CLOSE_MAX) != 0) {
+            lo = cl;
+            hi = ch;
+            return false;
+        }
         for (; cl != 0; cl &= cl - 1) {
             const int e = __builtin_ctz(cl);
             lo = exact(e) ? lo | 1u << e : lo & ~(1u << e);
@@ -917,6 +931,12 @@ __device__ __forceinline__ void nn_tile(LdsT &L, const NNTileI &I, int m, uint32
             hi = exact(32 + e) ? hi | 1u << e : hi & ~(1u << e);
         }
     }
+    return true;
+}
+
+// does the box, grown by its largest h, hold more than `most` particles?
+__device__ __forceinline__ bool nn_crowded(const NNArgs &A, const NNBox &B, int most) {
+    return nn_box_particles(A, B.x0 - B.h, B.x1 + B.h, B.y0 - B.h, B.y1 + B.h, B.z0 - B.h, B.z1 + B.h) > most;
 }
 
 // A run of 64 keys can cross a boundary of a large cell.  The Lebesgue curve jumps there, so the
@@ -931,23 +951,26 @@ __device__ __forceinline__ void nn_tile(LdsT &L, const NNTileI &I, int m, uint32
 __device__ __forceinline__ bool nn_split_wanted(const NNArgs &A, const NNBox &B, uint64_t m) {
     if ((m & (m - 1)) == 0) return false;   // one particle
     const double w = 2.0 * B.h, ex = B.x1 - B.x0, ey = B.y1 - B.y0, ez = B.z1 - B.z0;
-    if (!((w + ex) * (w + ey) * (w + ez) > NN_SPLIT_VOL * (w * w * w))) return false;
-    return nn_box_particles(A, B.x0 - B.h, B.x1 + B.h, B.y0 - B.h, B.y1 + B.h, B.z0 - B.h, B.z1 + B.h) > NN_SPLIT_CAND;
+    return (w + ex) * (w + ey) * (w + ez) > NN_SPLIT_VOL * (w * w * w) && nn_crowded(A, B, NN_SPLIT_CAND);
 }
 
 // Splits a group's active particles into runs that need no further split, cutting at the
 // boundaries of the largest cells first (the smallest shared key prefix between consecutive
 // particles; of several, the last).  Runs of at least NN_SPLIT_MIN particles are listed for
 // k_nn_rest, one wavefront each; the others go to the per-particle mode, where lanes are
-// candidates.  Every active particle ends up in exactly one of the two lists.
+// candidates, and so do runs whose box holds a dense clump (NN_PART_CAND): the one wavefront streaming
+// it would be all that the launch waits for (the clump of NN_CLOSE_MAX, RHS in two walks 10.4 -> 7.4 ms;
+// a bound of NN_SPLIT_CAND: the same there, 4 to 5 % slower where a fifth of the particles around a
+// wider clump meet it).  Every active particle ends up in exactly one of the two lists.
 __device__ __forceinline__ void nn_split_group(const NNArgs &A, int64_t group, int64_t k, bool active, double x,
                                                double y, double z, double h) {
     const int lane = wave_lane();
     uint64_t todo = wave_ballot(active);
     while (todo != 0) {
         uint64_t m = todo;
+        NNBox B;
         for (;;) {
-            const NNBox B = nn_box((m >> lane) & 1ull, x, y, z, h);
+            B = nn_box((m >> lane) & 1ull, x, y, z, h);
             if (!nn_split_wanted(A, B, m)) break;
             // lanes first .. last - 1 of the run own the boundary to their successor
             const int first = __builtin_ctzll(m), last = 63 - __builtin_clzll(m);
@@ -957,7 +980,7 @@ __device__ __forceinline__ void nn_split_group(const NNArgs &A, int64_t group, i
         }
         todo &= ~m;
         const int num = popc64(m);
-        const bool part = num >= NN_SPLIT_MIN;
+        const bool part = num >= NN_SPLIT_MIN && !nn_crowded(A, B, NN_PART_CAND);
         uint32_t b = 0;
         if (lane == 0) b = part ? atomicAdd(A.seg_count, 1u) : atomicAdd(A.out_count, (uint32_t)num);
         b = __shfl(b, 0);
@@ -1038,7 +1061,7 @@ __device__ __forceinline__ void nn_group(NNWaveLdsF &L, const NNArgs &A, int64_t
     }
     // not for positions that are not finite, nor for an h that is no number: they have no neighbours
     const bool live = active && nn_d2(xi - xi, yi - yi, zi - zi) == 0.0 && hi2 >= 0.0;
-    const NNTileI I = nn_tile_group(L.extra, live, xi, yi, zi, hi2, B);
+    NNTileI I = nn_tile_group(L.extra, live, xi, yi, zi, hi2, B);
     wave_sync();
     // candidate filter: squared distance from the box of the active positions, below both
     // hmax^2 and h_j^2.  Per axis fl(b0 - x) <= fl(x_i - x) for every x_i >= b0 (rounding is
@@ -1078,6 +1101,7 @@ __device__ __forceinline__ void nn_group(NNWaveLdsF &L, const NNArgs &A, int64_t
     const bool ok = nn_walk_box<true>(L, A, [&]() { return L.extra.bounds; }, NN_START_ALL, w0, w1,
                                       (int)(group * 64), keep, [&](int m) {
         uint32_t bits[2];
+        bool done = false;
         if (I.on) {
             const double hm = L.extra.bounds.core.h;
             auto exact = [&](int e) {
@@ -1086,9 +1110,11 @@ __device__ __forceinline__ void nn_group(NNWaveLdsF &L, const NNArgs &A, int64_t
                 const double d = nn_d2(own.x - L.tx[e], own.y - L.ty[e], own.z - L.tz[e]);
                 return (d < hk * hk) & (d < L.th2[e]);
             };
-            if (wave_ballot(lane < m && L.th2[lane] < hm * hm) == 0) nn_tile<true>(L, I, m, bits[0], bits[1], exact);
-            else nn_tile<false>(L, I, m, bits[0], bits[1], exact);
-        } else {
+            if (wave_ballot(lane < m && L.th2[lane] < hm * hm) == 0) done = nn_tile<true>(L, I, m, bits[0], bits[1], exact);
+            else done = nn_tile<false>(L, I, m, bits[0], bits[1], exact);
+            if (!done && wave_ballot(__popc(bits[0]) + __popc(bits[1]) > NN_CLOSE_OFF) != 0) I.on = false;
+        }
+        if (!done) {
             // FP64: candidates come as LDS broadcasts, NN_PB per batch with all their reads issued
             // first; one bit per test, the last candidate's lowest.  (The lane's own particle is read
             // again: kept, it would cost the matrix form its registers.)

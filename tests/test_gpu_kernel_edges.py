@@ -377,3 +377,30 @@ def test_fp32_forces_in_physical_units(gpu_lib, orc, side, h, v, rho, cs):
     """FP32 pair sums where lengths are far from one: rock in SI and cgs units, thin gas at small h."""
     print_case(f"fp32 forces side={side} h={h} v={v} rho={rho}")
     compare_fp32_rhs(gpu_lib, orc, gas_in_units(side, h, v, rho, cs))
+
+
+@pytest.mark.parametrize("sigma", [2e-2, 3e-4])
+@pytest.mark.parametrize("curve", [0, 1])
+def test_groups_that_straddle_a_dense_clump(gpu_lib, orc, curve, sigma):
+    """Half of 40,000 particles in a small ball, the others spread around it with h hundreds of times
+    as large: groups that hold both test the clump in FP64, and split parts whose box holds it go to
+    the per-particle searches.  h, iteration counts, counts and neighbour sets are the oracle's."""
+    print_case(f"dense clump sigma={sigma} curve={curve}")
+    n, k = 40000, 20000
+    rng = np.random.default_rng(2)
+    p = np.concatenate([sigma * rng.normal(size=(k, 3)) + 0.3, rng.uniform(-1, 1, (n - k, 3))])
+    h = np.concatenate([np.full(k, 1.2 * sigma * (64 / (4.19 * k / 15.75)) ** (1 / 3)),
+                        np.full(n - k, (64 * 8 / (4.19 * (n - k))) ** (1 / 3))])
+    s = dict(x=p[:, 0].copy(), y=p[:, 1].copy(), z=p[:, 2].copy(), mass=np.full(n, 1.0 / n), sml=h)
+    st, oh, oiters, _ = orc.h_iterate(s["x"], s["y"], s["z"], h, max_nb=400)
+    assert st == 0
+    st, onnl, onoi = orc.nn_grid(s["x"], s["y"], s["z"], oh, 400)
+    assert st == 0
+    used = np.arange(400) < onoi[:, None]
+    for spec in (0, gpu_lib.RHS_SPECULATIVE_NN):
+        with load_ctx(gpu_lib, s, gpu_lib.default_params(curve=curve, max_nb=400)) as ctx:
+            ctx.rhs(gpu_lib.RHS_SPH | gpu_lib.RHS_VARIABLE_SML | spec)
+            nnl, noi = ctx.neighbour_lists(400)
+            assert np.array_equal(ctx.download("sml"), oh) and np.array_equal(ctx.download("h_iters"), oiters)
+        assert np.array_equal(noi, onoi)
+        assert np.array_equal(np.sort(np.where(used, nnl, -1), 1), np.sort(np.where(used, onnl, -1), 1))
