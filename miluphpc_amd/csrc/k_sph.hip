@@ -782,7 +782,7 @@ __device__ __forceinline__ void nn_tile_write(NNTileLds &T, int e, double X, dou
     T.norm2[2][e] = (uint16_t)(r.c >> 16);
 }
 
-// live: the lane's particle takes part (its position is finite then)
+// live: the lane's particle takes part
 __device__ __forceinline__ NNTileI nn_tile_group(NNTileLds &T, bool live, double x, double y, double z, double h2,
                                                  const NNBox &B) {
     NNTileI I;
@@ -792,7 +792,7 @@ __device__ __forceinline__ NNTileI nn_tile_group(NNTileLds &T, bool live, double
     const double reach =
         0.5 * sqrt(nn_d2((B.x1 - B.x0) * scale, (B.y1 - B.y0) * scale, (B.z1 - B.z0) * scale)) + hs;
     const double M = reach * reach;
-    // false for boxes that are not finite; beyond these h the squares leave the normal numbers
+    // false where h is infinite; beyond these h the squares leave the normal numbers
     I.on = M <= NN_MFMA_REACH && B.h > 1e-140 && B.h < 1e140;
     I.eps = (float)(M * 1.52587890625e-05);
     if (!I.on) return I;
@@ -844,11 +844,12 @@ __device__ __forceinline__ bool nn_tile(LdsT &L, const NNTileI &I, int m, uint32
     const int lane = wave_lane(), q = lane >> 4, ax = q < 3 ? q : 0;
     NNTileLds &T = L.extra;
     {
-        const bool in = lane < m;   // past the tile: far from everything
         const double sc = T.scale;
-        const double X = in ? (L.tx[lane] - T.cx) * sc : 0.0, Y = in ? (L.ty[lane] - T.cy) * sc : 0.0,
-                     Z = in ? (L.tz[lane] - T.cz) * sc : 0.0;
-        const double r2 = nn_d2(X, Y, Z);
+        const double dx = (L.tx[lane] - T.cx) * sc, dy = (L.ty[lane] - T.cy) * sc, dz = (L.tz[lane] - T.cz) * sc;
+        const double r2 = nn_d2(dx, dy, dz);
+        // past the tile, or no position (the filter lets a NaN pass): far from everything
+        const bool in = lane < m && r2 == r2;
+        const double X = in ? dx : 0.0, Y = in ? dy : 0.0, Z = in ? dz : 0.0;
         // beyond the largest h^2 the candidate's own never decides (and may be any size)
         const double h2 = SAME ? 0.0 : fmin(L.th2[lane] * (sc * sc), T.hm2s);
         nn_tile_write(T, lane, X, Y, Z, in ? (float)(-0.5 * r2) : -1e30f,
@@ -1030,20 +1031,28 @@ __device__ __forceinline__ void nn_group(NNWaveLdsF &L, const NNArgs &A, int64_t
     const double hi = valid ? A.h[k] : 0.0;
     const double hi2 = hi * hi;
     // outliers: a few active particles with h above NN_OUTLIER x the group's smallest would
-    // grow the search box of all 64; they go to the per-particle mode instead
+    // grow the search box of all 64; they go to the per-particle mode instead.  So do particles whose
+    // position is not finite or whose h is no number: a NaN would make the box, and with it every
+    // branch below, differ between the lanes.
     bool outlier = SEG && !active;   // a part's other lanes belong to other waves
-    if (!SEG && A.out_list) {
-        const double hmin = wave_min(active ? hi : 1e300);
-        const bool big = active && hi > NN_OUTLIER * hmin;
-        const uint64_t mO = wave_ballot(big);
-        if (mO != 0 && popc64(mO) <= NN_OUTLIER_MAX) {
-            outlier = big;
+    if (!SEG) {
+        const bool live = active && nn_d2(xi - xi, yi - yi, zi - zi) == 0.0 && hi2 >= 0.0;
+        const double hmin = wave_min(live ? hi : 1e300);
+        const bool big = live && hi > NN_OUTLIER * hmin;
+        const bool few = popc64(wave_ballot(big)) <= NN_OUTLIER_MAX;
+        outlier = (active && !live) || (big && few);
+        const uint64_t mO = wave_ballot(outlier);
+        if (mO != 0) {
             uint32_t b = 0;
             if (lane == 0) b = atomicAdd(A.out_count, (uint32_t)popc64(mO));
             b = __shfl(b, 0);
             if (outlier) A.out_list[b + popc64(mO & lanemask_lt())] = (int32_t)k;
             active = active && !outlier;
             mActive = wave_ballot(active);
+            if (mActive == 0) {
+                if (MODE >= 1 && valid && !outlier) A.h_next[k] = hi;
+                return;
+            }
         }
     }
     // search box: bounding box of the active lanes grown by their largest h (plus a
@@ -1059,9 +1068,7 @@ __device__ __forceinline__ void nn_group(NNWaveLdsF &L, const NNArgs &A, int64_t
         L.extra.bounds = NNBounds{B.x0 - grow, B.x1 + grow, B.y0 - grow, B.y1 + grow, B.z0 - grow, B.z1 + grow,
                                   NNCore{B.x0, B.x1, B.y0, B.y1, B.z0, B.z1, B.h}};
     }
-    // not for positions that are not finite, nor for an h that is no number: they have no neighbours
-    const bool live = active && nn_d2(xi - xi, yi - yi, zi - zi) == 0.0 && hi2 >= 0.0;
-    NNTileI I = nn_tile_group(L.extra, live, xi, yi, zi, hi2, B);
+    NNTileI I = nn_tile_group(L.extra, active, xi, yi, zi, hi2, B);
     wave_sync();
     // candidate filter: squared distance from the box of the active positions, below both
     // hmax^2 and h_j^2.  Per axis fl(b0 - x) <= fl(x_i - x) for every x_i >= b0 (rounding is
@@ -1196,8 +1203,8 @@ __device__ __forceinline__ void nn_group(NNWaveLdsF &L, const NNArgs &A, int64_t
         if (lane == 0) set_err(A.err, ERRF_STACK);
         return;
     }
-    // every active particle is one of its own candidates
-    if (MODE == 1 && active && nn_d2(xi - xi, yi - yi, zi - zi) < hi2) count--;
+    // every active particle is one of its own candidates, at distance 0
+    if (MODE == 1 && active && hi2 > 0.0) count--;
     if (MODE == 2 && active && (count & 3) != 0 && count < A.max_nb)
         A.nbr4[(int64_t)(count >> 2) * A.stride + k] = tail4();
     if (MODE == 0 && A.only) {

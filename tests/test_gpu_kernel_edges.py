@@ -404,3 +404,56 @@ def test_groups_that_straddle_a_dense_clump(gpu_lib, orc, curve, sigma):
             assert np.array_equal(ctx.download("sml"), oh) and np.array_equal(ctx.download("h_iters"), oiters)
         assert np.array_equal(noi, onoi)
         assert np.array_equal(np.sort(np.where(used, nnl, -1), 1), np.sort(np.where(used, onnl, -1), 1))
+
+
+@pytest.mark.parametrize("side", [20, 33])   # per particle; groups
+@pytest.mark.parametrize("curve", [0, 1])
+def test_neighbours_beside_particles_that_are_no_numbers(gpu_lib, orc, side, curve):
+    """Particles with a NaN coordinate or a NaN h, alone and side by side in a group, have no neighbours
+    and are nobody's; every other particle's list, h and iteration count is that of a set without
+    them."""
+    print_case(f"nan particles side={side} curve={curve}")
+    s = ics.sedov_lattice(side)
+    n = side ** 3
+    rng = np.random.default_rng(side)
+    for a in "xyz":
+        s[a] = s[a] + rng.uniform(-0.1, 0.1, n) / side
+    s["sml"] = s["sml"] * rng.uniform(0.85, 1.15, n)
+    bad = np.array([n // 3, n // 2, n // 2 + 1, 2 * n // 3])
+    ok = np.setdiff1d(np.arange(n), bad)
+    st, oh, oiters, _ = orc.h_iterate(s["x"][ok], s["y"][ok], s["z"][ok], s["sml"][ok])
+    assert st == 0
+    s["x"][bad[0]] = np.nan
+    s["z"][bad[1]] = np.nan
+    s["sml"][bad[2]] = np.nan
+    s["sml"][bad[3]] = np.nan
+
+    def listed(h):
+        st, nnl, noi = orc.nn_grid(s["x"][ok], s["y"][ok], s["z"][ok], h, 180)
+        assert st == 0
+        return nnl, noi
+
+    p = gpu_lib.default_params(curve=curve)
+    with load_ctx(gpu_lib, s, p) as ctx:
+        ctx.bbox(); ctx.keys(); ctx.sort(); ctx.build_tree()
+        ctx.neighbours()
+        nnl, noi = ctx.neighbour_lists(180)
+    onnl, onoi = listed(s["sml"][ok])
+    assert np.all(noi[bad] == 0)
+    assert np.array_equal(noi[ok], onoi)
+    used = np.arange(180) < onoi[:, None]
+    want = np.sort(np.where(used, ok[onnl.clip(0, len(ok) - 1)], -1), 1)
+    assert np.array_equal(np.sort(np.where(used, nnl[ok], -1), 1), want)
+
+    onnl, onoi = listed(oh)
+    st, orho = orc.density(*(s[k][ok] for k in ("x", "y", "z", "mass")), oh, onnl, onoi)
+    assert st == 0
+    for spec in (0, gpu_lib.RHS_SPECULATIVE_NN):
+        with load_ctx(gpu_lib, s, p) as ctx:
+            with pytest.raises(gpu_lib.MhpcError):   # particles without neighbours or density
+                ctx.rhs(gpu_lib.RHS_SPH | gpu_lib.RHS_VARIABLE_SML | spec)
+            assert np.array_equal(ctx.download("sml")[ok], oh)
+            assert np.array_equal(ctx.download("h_iters")[ok], oiters)
+            noi, rho = ctx.download("noi"), ctx.download("rho")
+        assert np.array_equal(noi[ok], onoi) and np.all(noi[bad] == 0)
+        assert np.max(np.abs(rho[ok] / orho - 1.0)) <= 1e-12
