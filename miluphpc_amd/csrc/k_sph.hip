@@ -1961,8 +1961,8 @@ void launch_neighbours(mhpc_ctx *c) {
 
 // a10 cubic spline (kernel.cu:50-83), support radius h, q = r / h: W = 8/pi h^-3 w(q) with
 // w = 1 + 6 q^2 (q - 1) up to q = 1/2, 2 (1 - q)^3 up to 1, and 0 beyond.  The pair loops evaluate
-// both branches and select: their lanes take different ones, so a wavefront pays for both anyway,
-// and a NaN q (coincident particles) selects 0.
+// both branches and select: their lanes take different ones, so a wavefront pays for both anyway.
+// A NaN q selects 0 (the forces of coincident particles).
 template <typename T>
 __device__ __forceinline__ T cubic_w(T q) {
     const T t = T(1) - q;
@@ -1999,6 +1999,13 @@ __device__ __forceinline__ float div_f32(float n, float d) {
     const float y = __builtin_amdgcn_rcpf(d);
     const float q = n * y;
     return __builtin_fmaf(__builtin_fmaf(-d, q, n), y, q);
+}
+// sqrt(x), x >= 0, from the estimate of 1/sqrt(x) and its square's exact residual: 0.5 ulp and a
+// little, 0 for 0.  Below the normal numbers (separations under 1e-19) the result is only of that size.
+__device__ __forceinline__ float sqrt_f32(float x) {
+    const float y = __builtin_amdgcn_rsqf(fmaxf(x, 1.17549435e-38f));
+    const float r = x * y;
+    return __builtin_fmaf(__builtin_fmaf(-r, r, x), 0.5f * y, r);
 }
 __device__ __forceinline__ float rsq_f32(float x) {
     const float y = __builtin_amdgcn_rsqf(x);
@@ -2142,7 +2149,7 @@ __device__ __forceinline__ void density_pair(const double4 &pi, double hi, const
         const double dx = pi.x - pj.x, dy = pi.y - pj.y, dz = pi.z - pj.z;
         const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
         const double ih = rcp_f64(hb);
-        const double q = r2 * rsq_f64(r2) * ih;
+        const double q = fmax(r2 * rsq_f64(r2) * ih, 0.0);   // r = 0: 0 inf, no number, to 0
         const double ih3 = ih * ih * ih;
         if constexpr (CUBIC) {
             acc = fma(pj.w * (K8PI * ih3), cubic_w(q), acc);
@@ -2155,7 +2162,7 @@ __device__ __forceinline__ void density_pair(const double4 &pi, double hi, const
         const float dx = (float)(pi.x - pj.x), dy = (float)(pi.y - pj.y), dz = (float)(pi.z - pj.z);
         const float r2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
         const float ih = rcp_f32((float)hb);
-        const float q = r2 * rsq_f32(r2) * ih;
+        const float q = sqrt_f32(r2) * ih;
         const float ih3 = ih * ih * ih;
         if constexpr (CUBIC) {
             acc32.add((float)pj.w * ((float)K8PI * ih3) * cubic_w(q));

@@ -457,3 +457,35 @@ def test_neighbours_beside_particles_that_are_no_numbers(gpu_lib, orc, side, cur
             noi, rho = ctx.download("noi"), ctx.download("rho")
         assert np.array_equal(noi[ok], onoi) and np.all(noi[bad] == 0)
         assert np.max(np.abs(rho[ok] / orho - 1.0)) <= 1e-12
+
+
+@pytest.mark.parametrize("side", [16, 37])   # shared lists; windows
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("kernel", [1, 2])
+def test_density_of_coincident_particles(gpu_lib, orc, side, precision, kernel):
+    """Two particles on either side of the middle of the box, so close that their squared distance is
+    zero: each counts with the kernel's value at zero in the other's density."""
+    print_case(f"coincident pair side={side} precision={precision} kernel={kernel}")
+    s = ics.sedov_lattice(side)
+    n = side ** 3
+    rng = np.random.default_rng(side)
+    for a in "xyz":
+        s[a] = s[a] + rng.uniform(-0.1, 0.1, n) / side
+    for a in "xyz":
+        s[a][0], s[a][-1] = -0.5, 0.5   # the box is [-0.5, 0.5]: its middle is 0
+    i, j = n // 2, n // 2 + 1
+    d = 1e-170 if precision == 0 else 1e-30
+    s["x"][i], s["x"][j] = -d, d
+    for a in "yz":
+        s[a][j] = s[a][i]
+    p = gpu_lib.default_params(precision=precision, smoothing_kernel=kernel)
+    with load_ctx(gpu_lib, s, p) as ctx:
+        ctx.rhs(gpu_lib.RHS_SPH)
+        g = {k: ctx.download(k) for k in ("noi", "rho", "ax", "ay", "az", "dedt")}
+    st, nnl, noi = orc.nn_grid(s["x"], s["y"], s["z"], s["sml"], 180)
+    assert st == 0 and j in nnl[i, :noi[i]]
+    st, rho = orc.density(s["x"], s["y"], s["z"], s["mass"], s["sml"], nnl, noi, kernel=kernel)
+    assert np.array_equal(g["noi"], noi)
+    assert np.max(np.abs(g["rho"] / rho - 1.0)) < (1e-12 if precision == 0 else 5e-6)
+    for k in ("ax", "ay", "az", "dedt"):
+        assert np.all(np.isfinite(g[k])), k
