@@ -1988,7 +1988,7 @@ __device__ __forceinline__ double rcp_f64(double x) {
     const double e = fma(-x, y, 1.0);
     return fma(y, fma(e, e, e), y);
 }
-// the same in FP32, one Newton step from the estimates (1 ulp)
+// the same in FP32, one Newton step from the estimate: 0.5 ulp and a little
 __device__ __forceinline__ float rcp_f32(float x) {
     const float y = __builtin_amdgcn_rcpf(x);
     return __builtin_fmaf(y, __builtin_fmaf(-x, y, 1.f), y);
@@ -2001,15 +2001,13 @@ __device__ __forceinline__ float div_f32(float n, float d) {
     return __builtin_fmaf(__builtin_fmaf(-d, q, n), y, q);
 }
 // sqrt(x), x >= 0, from the estimate of 1/sqrt(x) and its square's exact residual: 0.5 ulp and a
-// little, 0 for 0.  Below the normal numbers (separations under 1e-19) the result is only of that size.
-__device__ __forceinline__ float sqrt_f32(float x) {
+// little, 0 for 0; rinv receives 1/sqrt(x) to 1 ulp (large for 0).  Below the normal numbers
+// (separations under 1e-19) the result is only of that size.
+__device__ __forceinline__ float sqrt_f32(float x, float &rinv) {
     const float y = __builtin_amdgcn_rsqf(fmaxf(x, 1.17549435e-38f));
-    const float r = x * y;
-    return __builtin_fmaf(__builtin_fmaf(-r, r, x), 0.5f * y, r);
-}
-__device__ __forceinline__ float rsq_f32(float x) {
-    const float y = __builtin_amdgcn_rsqf(x);
-    return __builtin_fmaf(0.5f * y, __builtin_fmaf(-(x * y), y, 1.f), y);
+    const float r = x * y, half = 0.5f * y;
+    rinv = __builtin_fmaf(half, __builtin_fmaf(-r, y, 1.f), y);
+    return __builtin_fmaf(__builtin_fmaf(-r, r, x), half, r);
 }
 
 // a10, the five kernels of SPH::SmoothingKernel (kernel.cu:14-183, 3D branches; Dehnen & Aly
@@ -2139,11 +2137,13 @@ static EosArgs eos_args(mhpc_ctx *c) {
     return E;
 }
 
-// one density pair term: FP64 adds m_j W into acc; FP32 adds it (in FP32, from FP64
-// differences) into the Kahan accumulator acc32
+// one density pair term m_j W added into acc.  FP32: W in FP32 from FP64 differences, without the
+// kernel's constant (density_sum puts it in), times the FP64 mass: a rounded constant or mass is the
+// same error in every term (8/pi: -4.0e-8 of the density), and with these gone an FP64 sum costs no
+// more than a compensated one.
 template <bool FP64, bool CUBIC>
 __device__ __forceinline__ void density_pair(const double4 &pi, double hi, const double4 &pj, double hj,
-                                             int sml_avg, int kind, double &acc, Kahan &acc32) {
+                                             int sml_avg, int kind, double &acc) {
     const double hb = sml_avg ? 0.5 * (hi + hj) : hi;
     if constexpr (FP64) {
         const double dx = pi.x - pj.x, dy = pi.y - pj.y, dz = pi.z - pj.z;
@@ -2162,16 +2162,21 @@ __device__ __forceinline__ void density_pair(const double4 &pi, double hi, const
         const float dx = (float)(pi.x - pj.x), dy = (float)(pi.y - pj.y), dz = (float)(pi.z - pj.z);
         const float r2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
         const float ih = rcp_f32((float)hb);
-        const float q = sqrt_f32(r2) * ih;
+        float rinv;
+        const float q = sqrt_f32(r2, rinv) * ih;
         const float ih3 = ih * ih * ih;
         if constexpr (CUBIC) {
-            acc32.add((float)pj.w * ((float)K8PI * ih3) * cubic_w(q));
+            acc = fma(pj.w, (double)(ih3 * cubic_w(q)), acc);
         } else if (q <= 1.0f) {
             float w, dw;
             kernel_shape<float>(kind, q, w, dw);
-            acc32.add((float)pj.w * ((float)kernel_sigma(kind) * ih3 * w));
+            acc = fma(pj.w, (double)(ih3 * w), acc);
         }
     }
+}
+template <bool FP64, bool CUBIC>
+__device__ __forceinline__ double density_sum(int kind, double acc) {
+    return FP64 ? acc : acc * (CUBIC ? K8PI : kernel_sigma(kind));
 }
 
 // caller-order h, neighbour and iteration counts and the neighbour sum / maximum, published by
@@ -2224,7 +2229,6 @@ __global__ __launch_bounds__(DENS_WIN) void k_density(int64_t n, const double4 *
         cnt = cnt > max_nb ? max_nb : cnt;
         const int4 *nrow = reinterpret_cast<const int4 *>(nbr) + k;   // row r at nrow[r * stride]
         double acc = 0.0;
-        Kahan acc32;
         // two list rows (eight neighbours) per iteration: the eight records are requested
         // together, then the pairs are evaluated in list order; the next two rows are
         // requested a step ahead.  The window copy is read unconditionally (clamped index),
@@ -2255,10 +2259,10 @@ __global__ __launch_bounds__(DENS_WIN) void k_density(int64_t n, const double4 *
             }
     #pragma unroll
             for (int e = 0; e < 8; e++)
-                if (e < m) density_pair<FP64, CUBIC>(pi, hi, pj[e], hj[e], sml_avg, kind, acc, acc32);
+                if (e < m) density_pair<FP64, CUBIC>(pi, hi, pj[e], hj[e], sml_avg, kind, acc);
         }
         const double self = CUBIC ? K8PI / (hi * hi * hi) : kernel_sigma(kind) / (hi * hi * hi);   // W(0)
-        const double r = pi.w * self + (FP64 ? acc : acc32.value());
+        const double r = pi.w * self + density_sum<FP64, CUBIC>(kind, acc);
         srho[k] = r;
         const int32_t i = perm[k];
         rho[i] = r;
@@ -2321,7 +2325,6 @@ __global__ __launch_bounds__(256) void k_density_split(int64_t n, const double4 
         const int cnt = noi > max_nb ? max_nb : noi;
         const int4 *nrow = reinterpret_cast<const int4 *>(nbr) + k;
         double acc = 0.0;
-        Kahan acc32;
         for (int r = sub; 4 * r < cnt; r += SPLIT_LANES) {
             const int4 q = nrow[(int64_t)r * stride];
             const int m = cnt - 4 * r;
@@ -2336,9 +2339,9 @@ __global__ __launch_bounds__(256) void k_density_split(int64_t n, const double4 
             }
 #pragma unroll
             for (int e = 0; e < 4; e++)
-                if (e < m) density_pair<FP64, CUBIC>(pi, hi, pj[e], hj[e], sml_avg, kind, acc, acc32);
+                if (e < m) density_pair<FP64, CUBIC>(pi, hi, pj[e], hj[e], sml_avg, kind, acc);
         }
-        sum = FP64 ? acc : acc32.value();
+        sum = density_sum<FP64, CUBIC>(kind, acc);
     }
     sum = row_sum(sum);
     if (k < n && sub == 0) {
@@ -2463,34 +2466,34 @@ __device__ __forceinline__ void force_pair(const ForceI &I, const double4 &pj, c
                                            ForceAcc<FP64> &acc, double *feat) {
     typedef typename std::conditional<FP64, double, float>::type T;
     const double4 pi = I.p, vi = I.v, ri = I.r;
-    const T hi = (T)I.h, hj = (T)rj.w;
-    const T hs = hi + hj;
+    const T hs = (T)(I.h + rj.w);
     const T hb = T(0.5) * hs;
-    const T sml = I.sml_avg ? hb : hi;
+    const T sml = I.sml_avg ? hb : (T)I.h;
     const T d0 = (T)(pi.x - pj.x), d1 = (T)(pi.y - pj.y), d2 = (T)(pi.z - pj.z);
     const T v0 = (T)(vi.x - vj.x), v1 = (T)(vi.y - vj.y), v2 = (T)(vi.z - vj.z);
     const T r2 = fma(d0, d0, fma(d1, d1, d2 * d2));
-    T rinv, ih;
+    T rinv, ih, q;
     if constexpr (FP64) {
         rinv = rsq_f64(r2);
         ih = rcp_f64(sml);
+        q = r2 * rinv * ih;
     } else {
-        rinv = rsq_f32(r2);
         ih = rcp_f32(sml);
+        q = sqrt_f32(r2, rinv) * ih;
     }
-    const T q = r2 * rinv * ih;
     const T ih2 = ih * ih;
-    // grad W = gs r_ij, gs = (dW/dr) / r
+    // grad W = gs r_ij, gs = (dW/dr) / r; in FP32 without the kernel's constant, which multiplies the
+    // sums instead (ForceSums): rounded, it would be the same error in every term
     T gs = T(0);
     if constexpr (CUBIC) {
-        gs = T(6 * K8PI) * (ih2 * ih2) * cubic_grad(q, ih, rinv);
-    } else if (q <= T(1)) {
+        const T norm = FP64 ? T(6 * K8PI) * (ih2 * ih2) : ih2 * ih2;
+        gs = norm * cubic_grad(q, ih, rinv);
+    } else if (q <= T(1) && r2 > T(0)) {
         T w, dw;
         kernel_shape<T>(I.kind, q, w, dw);
-        gs = (T)kernel_sigma(I.kind) * (ih2 * ih2) * dw * rinv;
+        gs = (FP64 ? (T)kernel_sigma(I.kind) : T(1)) * (ih2 * ih2) * dw * rinv;
     }
     const T vr = fma(v0, d0, fma(v1, d1, v2 * d2));
-    const T vv = gs * vr;   // v.grad W
     const T mj = (T)pj.w;
     // Pi_ij = (beta mu - alpha c) mu / rho, mu = h v.r / D, c and rho the pair's means
     const T D = fma(hb * hb, T(1e-2), r2);
@@ -2503,26 +2506,29 @@ __device__ __forceinline__ void force_pair(const ForceI &I, const double4 &pj, c
         mpij = num * rcp_f64(D * D * (ri.x + rj.x));
     } else {
         const T mu = div_f32(hb * vr, D);
-        const T c = T(0.5) * ((T)vi.w + (T)vj.w), rho = T(0.5) * ((T)ri.x + (T)rj.x);
+        const T c = T(0.5) * (T)(vi.w + vj.w), rho = T(0.5) * (T)(ri.x + rj.x);
         mpij = div_f32(mj * fma((T)I.beta, mu, -(T)I.alpha * c) * mu, rho);
     }
     mpij = vr < T(0) ? mpij : T(0);
-    const T pf = -mj * ((T)ri.y + (T)rj.y);
-    const T fa = (pf - mpij) * gs;
-    const T rv = (T)rj.z * vv;
-    const T ev = (mpij - pf) * vv;
+    const T pf = -mj * (T)(ri.y + rj.y);
+    const T f = pf - mpij;
     if constexpr (FP64) {
+        const T vv = gs * vr, fa = f * gs;   // vv = v.grad W
         acc.a0 = fma(fa, d0, acc.a0);
         acc.a1 = fma(fa, d1, acc.a1);
         acc.a2 = fma(fa, d2, acc.a2);
         acc.dvv = fma(rj.z, vv, acc.dvv);   // the drho/dt and dh/dt sums are the same sum
-        acc.de = fma(mpij - pf, vv, acc.de);
+        acc.de = fma(-f, vv, acc.de);
     } else {
-        acc.a0.add(fa * d0);
-        acc.a1.add(fa * d1);
-        acc.a2.add(fa * d2);
-        acc.dvv.add(rv);
-        acc.de.add(ev);
+        // v.grad W from the rounded components: the roundings of the three products are independent
+        // (de/dt, rms error over 2.4e5 particles: 1.59e-7, as gs (v.r_ij) 1.66e-7)
+        const T g0 = gs * d0, g1 = gs * d1, g2 = gs * d2;
+        const T vv = fma(v0, g0, fma(v1, g1, v2 * g2));
+        acc.a0.add(f * g0);
+        acc.a1.add(f * g1);
+        acc.a2.add(f * g2);
+        acc.dvv.add((T)rj.z * vv);
+        acc.de.add(-f * vv);
     }
     if (FEAT) {
         const T rg = (T)rj.z * gs, mg = mj * gs;
@@ -2538,17 +2544,18 @@ __device__ __forceinline__ void force_pair(const ForceI &I, const double4 &pj, c
 // a particle's accumulated sums (drho/dt and dh/dt share one)
 struct ForceSums {
     double a[3], dvv, de, feat[6];
-    __device__ __forceinline__ void take(const ForceAcc<true> &s, const double *f) {
+    __device__ __forceinline__ void take(const ForceAcc<true> &s, const double *f, double) {
         a[0] = s.a0; a[1] = s.a1; a[2] = s.a2;
         dvv = s.dvv;
         de = s.de;
         for (int q = 0; q < 6; q++) feat[q] = f[q];
     }
-    __device__ __forceinline__ void take(const ForceAcc<false> &s, const double *f) {
-        a[0] = s.a0.value(); a[1] = s.a1.value(); a[2] = s.a2.value();
-        dvv = s.dvv.value();
-        de = s.de.value();
-        for (int q = 0; q < 6; q++) feat[q] = f[q];
+    // c: the kernel's constant, left out of the FP32 terms
+    __device__ __forceinline__ void take(const ForceAcc<false> &s, const double *f, double c) {
+        a[0] = c * s.a0.value(); a[1] = c * s.a1.value(); a[2] = c * s.a2.value();
+        dvv = c * s.dvv.value();
+        de = c * s.de.value();
+        for (int q = 0; q < 6; q++) feat[q] = c * f[q];
     }
 };
 
@@ -2635,7 +2642,7 @@ __global__ __launch_bounds__(FORCE_WIN) void k_forces(ForceArgs A) {
         }
     }
     ForceSums S;
-    S.take(acc, feat);
+    S.take(acc, feat, CUBIC ? 6 * K8PI : kernel_sigma(I.kind));
     force_store<FEAT>(A, k, I, S);
 }
 
@@ -2680,7 +2687,7 @@ __global__ __launch_bounds__(256) void k_forces_split(ForceArgs A) {
         }
     }
     ForceSums S;
-    S.take(acc, feat);
+    S.take(acc, feat, CUBIC ? 6 * K8PI : kernel_sigma(I.kind));
 #pragma unroll
     for (int q = 0; q < 3; q++) S.a[q] = row_sum(S.a[q]);
     S.dvv = row_sum(S.dvv);

@@ -489,3 +489,56 @@ def test_density_of_coincident_particles(gpu_lib, orc, side, precision, kernel):
     assert np.max(np.abs(g["rho"] / rho - 1.0)) < (1e-12 if precision == 0 else 5e-6)
     for k in ("ax", "ay", "az", "dedt"):
         assert np.all(np.isfinite(g[k])), k
+
+
+def fp32_pair_sums(s, rho, p, cs, nnl, noi):
+    """Density and de/dt as FP32 pair terms (cubic spline) with correctly rounded square roots and
+    quotients, added in 64 bits."""
+    f = np.float32
+    fma = lambda a, b, c: (a.astype(np.float64) * b + c).astype(f)   # the product is exact in 64 bits
+    i = np.repeat(np.arange(len(noi)), noi)
+    j = nnl[np.arange(nnl.shape[1]) < noi[:, None]]
+    d = [(s[a][i] - s[a][j]).astype(f) for a in "xyz"]
+    v = [(s["v" + a][i] - s["v" + a][j]).astype(f) for a in "xyz"]
+    h = (0.5 * (s["sml"][i] + s["sml"][j])).astype(f)
+    r2 = fma(d[0], d[0], fma(d[1], d[1], d[2] * d[2]))
+    r, ih = np.sqrt(r2), f(1) / h
+    q = r * ih
+    t, norm = f(1) - q, f(8 / np.pi) * ih * ih * ih
+    w = np.where(q <= f(0.5), norm * fma(f(6) * q * q, q - f(1), f(1)), f(2) * norm * t * t * t)
+    dw = np.where(q <= f(0.5), f(6) * norm * ih * q * fma(f(3) * np.ones_like(q), q, f(-2)), f(-6) * norm * ih * t * t)
+    inside = q <= f(1)
+    add = lambda terms: np.bincount(i, np.where(inside, terms, f(0)).astype(np.float64), len(noi))
+    m = s["mass"][j].astype(f)
+    g = [dw / r * c for c in d]
+    vv = fma(v[0], g[0], fma(v[1], g[1], v[2] * g[2]))
+    vr = fma(v[0], d[0], fma(v[1], d[1], v[2] * d[2]))
+    c = f(0.5) * (cs[i].astype(f) + cs[j].astype(f))
+    mu = h * vr / fma(h * h, f(0.01), r2)
+    visc = np.where(vr < 0, m * (f(2) * mu - f(1) * c) * mu / (f(0.5) * (rho[i].astype(f) + rho[j].astype(f))), f(0))
+    pr = p / (rho * rho)
+    press = -m * (pr[i].astype(f) + pr[j].astype(f))
+    return s["mass"] * (8 / np.pi) / s["sml"] ** 3 + add(m * w), 0.5 * add((visc - press) * vv)
+
+
+@pytest.mark.parametrize("side", [31, 37])   # shared lists; windows
+def test_fp32_pair_sums_are_as_accurate_as_rounded_roots_and_quotients(gpu_lib, orc, side):
+    """The FP32 pair terms come from hardware estimates: their RMS error against 64 bits is within
+    one per cent of that with correctly rounded square roots and divisions, on the same particles."""
+    print_case(f"fp32 accuracy side={side}")
+    s = gas_in_units(side, 1.0, 1.0, 1.0, 0.5, seed=side)
+    s["sml"] = s["sml"] * np.random.default_rng(side).uniform(0.95, 1.05, side ** 3)
+    with load_ctx(gpu_lib, s, gpu_lib.default_params(precision=gpu_lib.PREC_FP32_KAHAN)) as ctx:
+        ctx.rhs(gpu_lib.RHS_SPH)
+        g = {k: ctx.download(k) for k in ("rho", "p", "cs", "dedt")}
+    st, nnl, noi = orc.nn_grid(s["x"], s["y"], s["z"], s["sml"], 180)
+    assert st == 0
+    st, rho = orc.density(s["x"], s["y"], s["z"], s["mass"], s["sml"], nnl, noi)
+    o = orc.forces(*(s[k] for k in ("x", "y", "z", "vx", "vy", "vz", "mass", "sml")), g["rho"], g["p"], g["cs"], nnl,
+                   noi)
+    rho32, dedt32 = fp32_pair_sums(s, g["rho"], g["p"], g["cs"], nnl, noi)
+    rms = lambda a: np.sqrt(np.mean(a ** 2))
+    errs = (rms(g["rho"] - rho), rms(rho32 - rho), rms(g["dedt"] - o["dedt"]), rms(dedt32 - o["dedt"]))
+    print("rms errors: density %.4g (rounded %.4g), de/dt %.4g (rounded %.4g)" % errs)
+    assert errs[0] <= 1.01 * errs[1] < 1e-6 * rms(rho)
+    assert errs[2] <= 1.01 * errs[3] < 1e-5 * rms(o["dedt"])
