@@ -73,8 +73,8 @@ struct BHAcc<true> {
 };
 
 // 1/sqrt(x) for normal x > 0.  SOFT: x is known to be at least the softening, a normal number.
-// Otherwise x = 0 (the particle itself, unsoftened) gives 0, and smaller x are raised to the
-// smallest normal number, so that the bare hardware estimates apply (no denormal scaling).
+// Otherwise x = 0 (the particle itself, unsoftened) and x = inf give 0, and smaller x are raised to
+// the smallest normal number, so that the bare hardware estimates apply (no denormal scaling).
 template <bool SOFT>
 __device__ __forceinline__ float rsq_pos(float x) {
     if (SOFT) return __builtin_amdgcn_rsqf(x);
@@ -83,7 +83,7 @@ __device__ __forceinline__ float rsq_pos(float x) {
 template <bool SOFT>
 __device__ __forceinline__ double rsq_pos(double x) {
     const double y = rsq_f64(SOFT ? x : fmax(x, 2.2250738585072014e-308));
-    return SOFT || x > 0.0 ? y : 0.0;
+    return SOFT || (x > 0.0 && x <= 1.7976931348623157e308) ? y : 0.0;   // rsq_f64(inf) is no number
 }
 
 // Monopole batch, FP32: plain FP32 sums over the (at most 64) entries, then one compensated
@@ -244,7 +244,8 @@ __global__ __launch_bounds__(64 * (MULTI ? BH_MULTI_MAX : BH_WAVES)) void k_bh_w
     const T tx = FP64 ? (T)px : (T)(px - refx), ty = FP64 ? (T)py : (T)(py - refy),
             tz = FP64 ? (T)pz : (T)(pz - refz);
     const T teps2 = (T)eps2;
-    const bool soft = teps2 >= (FP64 ? (T)2.2250738585072014e-308 : (T)1.17549435e-38f);
+    // every squared distance a positive normal number: softened, and (FP64) no box whose square leaves FP64
+    const bool soft = teps2 >= (FP64 ? (T)2.2250738585072014e-308 : (T)1.17549435e-38f) && (!FP64 || R < 1e150);
     auto flush_p = [&](int cnt, BHAcc<FP64> &acc) {
         if (soft) eval_mono<POT, true>(L, cnt, tx, ty, tz, (int)k, teps2, acc);
         else eval_mono<POT, false>(L, cnt, tx, ty, tz, (int)k, teps2, acc);

@@ -542,3 +542,25 @@ def test_fp32_pair_sums_are_as_accurate_as_rounded_roots_and_quotients(gpu_lib, 
     print("rms errors: density %.4g (rounded %.4g), de/dt %.4g (rounded %.4g)" % errs)
     assert errs[0] <= 1.01 * errs[1] < 1e-6 * rms(rho)
     assert errs[2] <= 1.01 * errs[3] < 1e-5 * rms(o["dedt"])
+
+
+@pytest.mark.parametrize("eps2", [1e-6, 0.0])
+@pytest.mark.parametrize("vote", [0, 1])
+def test_barnes_hut_with_strays_beyond_the_square_of_fp64(gpu_lib, orc, vote, eps2):
+    """Two particles so far out that their squared distances are infinite act on nothing (1 / sqrt(inf)
+    = 0); the others, one per octant around the middle, keep the oracle's forces."""
+    print_case(f"far strays vote={vote} eps2={eps2}")
+    rng = np.random.default_rng(8)
+    corner = np.array([[i & 1, i >> 1 & 1, i >> 2 & 1] for i in range(8)]) * 2.0 - 1.0
+    p = np.concatenate([corner * rng.uniform(0.5, 1.5, (8, 3)), [[1e160] * 3, [-1e160] * 3]])
+    s = dict(x=p[:, 0].copy(), y=p[:, 1].copy(), z=p[:, 2].copy(), mass=rng.uniform(0.5, 1.5, 10))
+    with load_ctx(gpu_lib, s, gpu_lib.default_params(theta=0.5, smoothing=eps2, curve=0, bh_accept=vote,
+                                                     precision=gpu_lib.PREC_FP64)) as ctx:
+        ctx.rhs(gpu_lib.RHS_GRAVITY)
+        g = np.stack([ctx.download(k) for k in ("g_ax", "g_ay", "g_az")])
+    d = p[None, :8] - p[:8, None]
+    r2 = (d ** 2).sum(2) + eps2
+    np.fill_diagonal(r2, 1.0)
+    want = (s["mass"][None, :8, None] * d / r2[..., None] ** 1.5).sum(1).T
+    assert np.abs(g[:, :8] - want).max() <= 1e-13 * np.abs(want).max()
+    assert np.all(g[:, 8:] == 0.0)
