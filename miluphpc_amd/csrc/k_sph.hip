@@ -29,15 +29,19 @@ static_assert(NN_LEAF_GROUP < NN_CWIN, "a clipped range crosses at most one end 
 #define NN_PART_CAND 12288   // split-off parts of more candidates than this, and ...
 #define NN_SPLIT_MIN 16      // ... of fewer particles go to the per-particle mode
 static_assert(64 / NN_SPLIT_MIN <= MHPC_NN_PARTS_PER_GROUP, "the part list holds every group's parts");
-// Re-lists: groups with at most this many flagged particles go per particle (lanes are
+// Re-lists: groups with at most NN_SPARSE flagged particles go per particle (lanes are
 // candidates), the others are walked again.  A group walk costs as much as about ten
 // per-particle searches: with 64 / 32 / 16 / 8 / 4 a step of the 128^3 blast takes
 // 9.61 / 9.50 / 8.96 / 8.88 / 8.87 ms and the 1M cloud's RHS 7.45 / 7.41 / 6.91 / 6.68 / 6.63 ms.
-// With fewer groups than fill the chip the walk's latency counts instead: every flagged
-// particle gets its own wavefront (16^3: 446 us against 466).
+// While few particles changed, the one group walk that any group needs is the launch's latency, and
+// every flagged particle gets its own wavefront: the re-lists of 128^3 with 4,900 / 37,300 / 70,100
+// particles changed take 71 / 170 / 249 us by NN_SPARSE, 44 / 162 / 279 us per particle (a ball of them;
+// scattered ones cross at 150,000), those of the evolving Sedov run 130 / 42 us.  Sets of up to
+// NN_SPARSE_SMALL particles always take them: their groups are one resident round, as long as its
+// slowest group (RHS of a 40,000-particle Plummer sphere whose h all change: 2.94 / 1.57 ms).
 #define NN_SPARSE 8
-#define NN_SPARSE_FEW 64     // below NN_FEW_GROUPS groups
-#define NN_FEW_GROUPS 1024   // one wavefront per SIMD
+#define NN_SPARSE_CHANGED 32768
+#define NN_SPARSE_SMALL 65536
 #define NN_DRANGES 256       // direct form: candidate ranges per wavefront
 #define NN_DSPAN 5           // direct form: start cells per axis - 1 (<= 216 cells)
 #define NN_DIRECT_MAX 32768  // direct form: candidates per wavefront
@@ -93,8 +97,7 @@ struct NNArgs {
     uint32_t *cnt_slot;       // split counting: neighbour count of list slot t
     const int32_t *slot_list; // split counting: the list slots it takes
     const uint32_t *slot_count;
-    int sparse;               // list mode with `only`: groups with at most this many flagged particles
-                              // go to the per-particle mode
+    const uint32_t *changed_count;   // list mode with `only`: the particles whose change flagged them
     const uint8_t *only;      // list mode: when set, only particles with only[k] != 0
     uint8_t *dirty;           // dirty marking: particles whose list must be rebuilt
     double *h0_slot;          // pass 0 with lists: the pass-0 h of each unconverged particle
@@ -1017,7 +1020,8 @@ __device__ __forceinline__ void nn_group(NNWaveLdsF &L, const NNArgs &A, int64_t
         if (MODE >= 1 && valid && !SEG) A.h_next[k] = A.h[k];
         return;
     }
-    if (!SEG && MODE == 0 && A.only && A.out_list && popc64(mActive) <= A.sparse) {
+    if (!SEG && MODE == 0 && A.only &&
+        popc64(mActive) <= (n <= NN_SPARSE_SMALL || *A.changed_count <= NN_SPARSE_CHANGED ? 64 : NN_SPARSE)) {
         // a re-list of a few flagged particles: 64 lanes testing candidates for one or two of
         // them is wasted, so they go to the per-particle mode (lanes = candidates)
         uint32_t b = 0;
@@ -1911,7 +1915,7 @@ void launch_neighbours_fixup(mhpc_ctx *c) {
     b.stride = c->cap_pad;
     b.snoi = c->snoi;
     b.only = c->sdirty;
-    b.sparse = ceil_div(c->n, 64) < NN_FEW_GROUPS ? NN_SPARSE_FEW : NN_SPARSE;
+    b.changed_count = a.count_in;
     b.out_list = c->olist;
     b.out_count = c->ocount + 1;
     b.seg_list = c->seglist;

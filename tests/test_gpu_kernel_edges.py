@@ -564,3 +564,29 @@ def test_barnes_hut_with_strays_beyond_the_square_of_fp64(gpu_lib, orc, vote, ep
     want = (s["mass"][None, :8, None] * d / r2[..., None] ** 1.5).sum(1).T
     assert np.abs(g[:, :8] - want).max() <= 1e-13 * np.abs(want).max()
     assert np.all(g[:, 8:] == 0.0)
+
+
+@pytest.mark.parametrize("fraction", [0.02, 1.0])
+@pytest.mark.parametrize("curve", [0, 1])
+def test_relists_of_few_and_of_many_changed_particles(gpu_lib, orc, curve, fraction):
+    """41^3 particles of which a few or all change h after pass 0 (32,768 changes part the re-lists per
+    particle from those by groups): h, counts and neighbour sets are the oracle's."""
+    print_case(f"re-lists fraction={fraction} curve={curve}")
+    side = 41
+    n = side ** 3
+    s = ics.sedov_lattice(side)
+    rng = np.random.default_rng(12)
+    for a in "xyz":
+        s[a] = s[a] + rng.uniform(-0.1, 0.1, n) / side
+    s["sml"] = np.where(rng.uniform(size=n) < fraction, 1.15, 1.0) * s["sml"]
+    p = gpu_lib.default_params(curve=curve, sml_max=4.0 * float(s["sml"].min()))
+    o = orc.sph_rhs(s, sml_max=p.sml_max)
+    changed = int((o["h_iters"] > 1).sum())
+    assert changed > 32768 if fraction == 1.0 else 0 < changed < 32768
+    with load_ctx(gpu_lib, s, p) as ctx:
+        ctx.rhs(gpu_lib.RHS_SPH | gpu_lib.RHS_VARIABLE_SML | gpu_lib.RHS_SPECULATIVE_NN)
+        nnl, noi = ctx.neighbour_lists(180)
+        h = ctx.download("sml")
+    assert np.array_equal(h, o["sml"]) and np.array_equal(noi, o["noi"])
+    used = np.arange(180) < noi[:, None]
+    assert np.array_equal(np.sort(np.where(used, nnl, -1), 1), np.sort(np.where(used, o["nnl"], -1), 1))
