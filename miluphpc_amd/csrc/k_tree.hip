@@ -291,44 +291,55 @@ __global__ __launch_bounds__(BLOCK) void k_bottom_up(
             if (cell_base[l + 1] > cell_base[l]) d = l;
         *depth_out = (unsigned long long)d;
     }
-    // The sweep's steps, (level, first thread) from L_hi down; a step's child slots, and the
-    // particles among the children, are requested while the step before it is worked on (they do
-    // not depend on it), so that a level of a small set waits for one memory round trip, for its child
-    // cells, instead of three (2048-body step 191 -> 186 us, 16^3 RHS 212 -> 202 us).
+    // AHEAD, the whole tree by one workgroup: a step's child slots, and the particles among the children,
+    // are requested while the step before it is worked on (they do not depend on it), so that a level of
+    // a small set waits for one memory round trip, for its child cells, instead of three (2048-body step
+    // 191 -> 186 us, 16^3 RHS 212 -> 202 us).  With a launch per level this only costs registers and the
+    // wait for the table (pass of 128^3 78 / 71 us, of 2,000,000 Plummer particles with quadrupoles 219 / 206 us,
+    // ahead / not).
+    constexpr bool AHEAD = BLOCK == BU_ONE_BLOCK;
     __shared__ int base[MHPC_LEVELS + 2];
-    for (int l = L_lo + tid; l <= L_hi + 1; l += BLOCK) base[l] = cell_base[l];
-    __syncthreads();
+    if (AHEAD) {
+        for (int l = L_lo + tid; l <= L_hi + 1; l += BLOCK) base[l] = cell_base[l];
+        __syncthreads();
+    }
     auto level_threads = [&](int L) {
         const int64_t c1 = base[L + 1] < cap_cells ? base[L + 1] : cap_cells;
         return (c1 - base[L]) * 8;
     };
-    auto settle = [&](int &L, int64_t &b) {   // past the end of a level: to the next that has cells
+    // the children of step (L, b), or of the first step of the next level that has cells
+    auto request = [&](int L, int64_t b, int32_t &k, double4 &r) {
         while (L >= L_lo && b >= level_threads(L)) {
             L--;
             b = (int64_t)blockIdx.x * BLOCK;
         }
-    };
-    auto request = [&](int L, int64_t b, int32_t &k, double4 &r) {
         const int64_t t = b + tid;
         k = L >= L_lo && t < level_threads(L) ? cchild[8 * (base[L] + (t >> 3)) + sub] : -1;
         if (k >= 0 && k < n) r = sxm[k];
     };
-    int L = L_hi;
-    int64_t b = (int64_t)blockIdx.x * BLOCK;
-    settle(L, b);
-    int32_t kn;
+    int32_t kn = -1;
     double4 rn = make_double4(0.0, 0.0, 0.0, 0.0);
-    request(L, b, kn, rn);
-    while (L >= L_lo) {
+    int L = L_hi;
+    if (AHEAD) {
+        while (L > L_lo && base[L + 1] == base[L]) L--;   // past the levels below the deepest cells
+        request(L, (int64_t)blockIdx.x * BLOCK, kn, rn);
+    }
+    for (; L >= L_lo; L--) {
+    const int64_t c0 = AHEAD ? base[L] : cell_base[L], c1a = AHEAD ? base[L + 1] : cell_base[L + 1];
+    const int64_t c1 = c1a < cap_cells ? c1a : cap_cells;
+    const int64_t nthreads = (c1 - c0) * 8;
+    for (int64_t b = (int64_t)blockIdx.x * BLOCK; b < nthreads; b += (int64_t)gridDim.x * BLOCK) {
         const int64_t t = b + tid;
-        const bool valid = t < level_threads(L);   // the eight lanes of a cell agree
-        const int64_t c = base[L] + (t >> 3);
-        const int32_t k = kn;
-        const double4 r = rn;
-        int Ln = L;
-        int64_t bn = b + (int64_t)gridDim.x * BLOCK;
-        settle(Ln, bn);
-        request(Ln, bn, kn, rn);
+        const bool valid = t < nthreads;   // the eight lanes of a cell agree
+        const int64_t c = c0 + (t >> 3);
+        int32_t k = kn;
+        double4 r = rn;
+        if (AHEAD) {
+            request(L, b + (int64_t)gridDim.x * BLOCK, kn, rn);
+        } else {
+            k = valid ? cchild[8 * c + sub] : -1;
+            if (k >= 0 && k < n) r = sxm[k];
+        }
         double px = 0.0, py = 0.0, pz = 0.0, pm = 0.0;
         double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
         double q[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
@@ -426,10 +437,9 @@ __global__ __launch_bounds__(BLOCK) void k_bottom_up(
                 }
             }
         }
-        wave_sync();   // the terms are read before the next step overwrites them
-        if (Ln != L) __syncthreads();   // a level's cells are written before the next one reads them
-        L = Ln;
-        b = bn;
+        wave_sync();   // the terms are read before the next iteration overwrites them
+    }
+    if (L != L_lo) __syncthreads();   // a level's cells are written before the next one reads them
     }
 }
 void launch_bottom_up(mhpc_ctx *c, bool gravity, bool sph) {
