@@ -50,7 +50,7 @@ static_assert(64 / NN_SPLIT_MIN <= MHPC_NN_PARTS_PER_GROUP, "the part list holds
 // per particle: 21^3 520 / 308 us, 25^3 530 / 341 us, 31^3 558 / 450 us in Lebesgue and 430 / 462 us
 // in Hilbert order).
 #define NN_FEW 32768
-static_assert(NN_FEW <= NN_DIRECT_MAX, "the direct form declines no box of so few particles");
+static_assert(NN_FEW <= NN_DIRECT_MAX && NN_DSPAN >= 1, "the direct form declines no box of so few particles");
 #define NN_DU 4              // direct form: candidates per lane and round (loads in flight; 2 / 4 / 8 alike)
 
 // candidate filter that keeps everything (per-particle walks test each candidate once)
@@ -1614,15 +1614,19 @@ __global__ __launch_bounds__(64 * NN1_WAVES) void k_h_pass(NNArgs A) {
         } else {
             const double4 own = A.sxm[k];
             const double hi2 = hi * hi;
+            const bool direct =
                 nn_direct(L, A, nn_ball(own, hi), [&](bool v, int j, const double4 &p, double h) {
-                if (v) {
-                    const double dx = own.x - p.x;
-                    const double dy = own.y - p.y;
-                    const double dz = own.z - p.z;
-                    const double d = nn_d2(dx, dy, dz);
-                    N += (d < hi2 && d < h * h && j != k) ? 1 : 0;
-                }
-            });
+                    if (v) {
+                        const double dx = own.x - p.x;
+                        const double dy = own.y - p.y;
+                        const double dz = own.z - p.z;
+                        const double d = nn_d2(dx, dy, dz);
+                        N += (d < hi2 && d < h * h && j != k) ? 1 : 0;
+                    }
+                });
+            // cannot happen: no more candidates than particles, and a box spans at most the two cells
+            // per axis of level 1; a count of zero instead would pass for a result
+            if (!direct && lane == 0) set_err(A.err, ERRF_STACK);
             N = wave_sum(N);
             wave_sync();
         }
