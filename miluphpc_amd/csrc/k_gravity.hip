@@ -92,7 +92,7 @@ __device__ __forceinline__ double rsq_pos(double x) {
 template <bool POT, bool SOFT, typename ListT>
 __device__ __forceinline__ void eval_mono(const ListT &L, int cnt, float px, float py, float pz, int self,
                                           float eps2, BHAcc<false> &acc) {
-    float bx = 0.f, by = 0.f, bz = 0.f, bp = 0.f;
+    float bx = 0.f, by = 0.f, bz = 0.f, bp[2] = {0.f, 0.f};
 #pragma unroll 4
     for (int e = 0; e < cnt; e++) {
         const float4 q = L.p[e];
@@ -104,12 +104,17 @@ __device__ __forceinline__ void eval_mono(const ListT &L, int cnt, float px, flo
         bx = __builtin_fmaf(mr3, dx, bx);
         by = __builtin_fmaf(mr3, dy, by);
         bz = __builtin_fmaf(mr3, dz, bz);
-        if (POT && L.id[e] != self) bp -= mr;
+        // two chains: all terms have one sign, so that a chain's roundings grow with its length
+        if (POT && L.id[e] != self) {
+            if (e & 1) bp[1] -= mr;
+            else bp[0] -= mr;
+        }
     }
     acc.x.add(bx);
     acc.y.add(by);
     acc.z.add(bz);
-    if (POT) acc.phi.add(bp);
+    if (POT) acc.phi.add(bp[0]);
+    if (POT) acc.phi.add(bp[1]);
 }
 
 // The same in FP64, summed as it comes.
