@@ -362,7 +362,7 @@ __global__ __launch_bounds__(64 * MLP_TR_WAVES, 1) void k_mlp_train_grad(int64_t
     const float b3 = params[P_B3];
     f32x4 gw2[4][4] = {}, gw1[4] = {};
     float gw3[4] = {}, gb2[4] = {}, gb1[4] = {}, gb3 = 0.f, loss = 0.f;
-    const float inv_nb = 1.f / (float)nb;
+    const float fnb = (float)nb, inv_nb = 1.f / fnb;
 
     while (wave_ballot(s < nb) != 0) {
         const bool valid = s < nb;
@@ -420,7 +420,10 @@ __global__ __launch_bounds__(64 * MLP_TR_WAVES, 1) void k_mlp_train_grad(int64_t
         y += __shfl_xor(y, 32);
         y += b3;
         const float e = valid ? y - t : 0.f;
-        const float dy = e * inv_nb;
+        // e / nb, the product corrected by its exact residual: the rounding of 1/nb alone would be the
+        // same error in every gradient
+        float dy = e * inv_nb;
+        dy = __builtin_fmaf(__builtin_fmaf(-fnb, dy, e), inv_nb, dy);
         if (q == 0) {
             loss += 0.5f * e * e;
             gb3 += dy;

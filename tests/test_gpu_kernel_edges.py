@@ -605,3 +605,23 @@ def test_fp32_potential_rounding(gpu_lib, vote):
             ctx.rhs(gpu_lib.RHS_GRAVITY | gpu_lib.RHS_POTENTIAL)
             u.append(ctx.download("u"))
     assert np.sqrt(np.mean((u[1] / u[0] - 1.0) ** 2)) < 2.0 ** -25
+
+
+def test_mlp_gradient_divides_by_the_sample_count(gpu_lib):
+    """db3 is the mean of y - t.  For these counts the FP32 rounding of 1/n is 5e-8 to 6e-8: scaled by
+    it, every gradient would be off by that; divided, the roundings of the terms average out (a few
+    2^-24 / sqrt(1000) and those of the sums, over eight counts)."""
+    print_case("mlp gradient scale")
+    off = []
+    for n in (1020, 1008, 1013, 976, 953, 951, 943, 933):
+        p, X, T = mlp_inputs(n, n)
+        T -= np.float32(6.0)   # every y - t positive
+        with gpu_lib.Context(64) as ctx:
+            ctx.mlp_set_params(p)
+            g, _ = ctx.mlp_gradient(X, T)
+            y = ctx.mlp_forward(X).astype(np.float64).ravel()
+        assert np.all(y - T > 0)
+        scale = float(np.float32(1) / np.float32(n)) * n - 1.0
+        assert abs(scale) > 5e-8
+        off.append((g[-1] / np.mean(y - T) - 1.0) * np.sign(scale))
+    assert abs(np.mean(off)) < 2.0 ** -25
