@@ -18,8 +18,8 @@
 //   * each time a list holds 64 entries all 64 lanes evaluate it, every lane reading
 //     the same LDS entry (broadcast) for its own particle.  FP32 mode: entries are
 //     staged as FP32 positions relative to the group's centre (each rounded once from the
-//     FP64 difference), each batch of up to 64 entries is summed in FP32 and the batch
-//     sums are added with Kahan compensation.  FP64 mode: plain FP64 throughout.
+//     FP64 difference), each batch of up to 64 entries is summed in FP32 (potentials in two
+//     chains) and the batch sums are added with Kahan compensation.  FP64 mode: plain FP64 throughout.
 // The stack lives in LDS; the number of nodes popped per round shrinks as the stack
 // fills so it cannot overflow (a hard bound still sets ERRF_STACK).
 //

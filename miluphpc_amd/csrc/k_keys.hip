@@ -219,7 +219,7 @@ static void keys_queue(mhpc_ctx *c, int nb) {
 
 void launch_keys(mhpc_ctx *c) { keys_queue(c, 0); }
 
-// the RHS's first two phases; mark(1) is called between them
+// the RHS's first two phases; `between` is called after the first one's launch
 void launch_bbox_keys(mhpc_ctx *c, const std::function<void()> &between) {
     const bool fold = c->n <= 0 || grid_for(c->n, 256 * 8, BBOX_BLOCKS_MAX) > KEYS_FOLD_MAX;
     const int nb = bbox_queue(c, fold, true);

@@ -46,9 +46,12 @@ static_assert(64 / NN_SPLIT_MIN <= MHPC_NN_PARTS_PER_GROUP, "the part list holds
 #define NN_DSPAN 5           // direct form: start cells per axis - 1 (<= 216 cells)
 #define NN_DIRECT_MAX 32768  // direct form: candidates per wavefront
 // Up to this many particles every search is per particle: a group walk of 64 takes 65 us or more
-// however few groups there are, a particle's direct search about 12 us (RHS with group walks and
-// per particle: 21^3 520 / 308 us, 25^3 530 / 341 us, 31^3 558 / 450 us in Lebesgue and 430 / 462 us
-// in Hilbert order).
+// however few groups there are, a particle's direct search about 12 us.  RHS by group walks / per
+// particle, us, lists from pass 0: lattices in Lebesgue order 25^3 423 / 269, 31^3 462 / 357, in
+// Hilbert order 340 / 283 and 367 / 365; a lattice whose side is a power of two has no group that
+// spans the domain (32^3 340 / 423).  Clustered sets gain most, although a search tests every
+// particle of its start cells: Plummer spheres of 20,000 1568 / 636, of 32,768 1400 / 812, two clumps
+// of 13,107 in a thin background 3147 / 2843, 28,500 of 30,000 in one start cell 9352 / 7479.
 #define NN_FEW 32768
 static_assert(NN_FEW <= NN_DIRECT_MAX && NN_DSPAN >= 1, "the direct form declines no box of so few particles");
 #define NN_DU 4              // direct form: candidates per lane and round (loads in flight; 2 / 4 / 8 alike)
@@ -765,9 +768,9 @@ __device__ __forceinline__ uint32_t nn_pack_hi(uint32_t hi, uint32_t lo) {
     return __builtin_amdgcn_perm(hi, lo, 0x07060302u);
 }
 
-// A group's particles as the matrix test needs them: lane (q, c) = 16 q + c holds axis q (none for
-// q = 3) of the particles 16 a + c in `xy` {part b, part a} and `zn` {norm part q, part c}, and the second
-// norm's part q in n2.
+// A group's particles as the matrix test needs them: lane (q, c) = 16 q + c holds, of axis q (none
+// for q = 3) of the particles 16 a + c, the coordinate's parts {a, b} in ab, its part c and the first
+// norm's part q in cn, and the second norm's part q with a one in n2.
 struct NNTileI {
     bool on;
     float eps;
@@ -1779,9 +1782,10 @@ static void launch_hmax_raise(mhpc_ctx *c, const int32_t *list, const uint32_t *
                        c->chmax, c->cap_cells);
 }
 
-// a9: the plain h-iteration as Jacobi passes; sh holds the final h afterwards.  Pass 0
-// runs in group mode over all particles and lists the unconverged ones; later passes run
-// in per-particle mode over that list only.
+// a9: the plain h-iteration as Jacobi passes; sh holds the final h afterwards.  Sets of up to NN_FEW
+// particles take every pass per particle and write no lists (k_h_pass).  Larger ones take pass 0 in
+// group mode over all particles, with the outliers and split parts behind it, and list the
+// unconverged ones; later passes search per particle over that list only.
 void launch_h_iterate(mhpc_ctx *c, int passes, bool speculative, hipEvent_t *walk_events) {
     if (c->n <= 0) return;
     hipLaunchKernelGGL(k_h_init, dim3((unsigned)ceil_div(c->n > 64 ? c->n : 64, 256)), dim3(256), 0, c->stream,
