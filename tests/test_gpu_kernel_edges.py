@@ -625,3 +625,28 @@ def test_mlp_gradient_divides_by_the_sample_count(gpu_lib):
         assert abs(scale) > 5e-8
         off.append((g[-1] / np.mean(y - T) - 1.0) * np.sign(scale))
     assert abs(np.mean(off)) < 2.0 ** -25
+
+
+@pytest.mark.parametrize("side", [20, 33])   # per particle; groups
+@pytest.mark.parametrize("curve", [0, 1])
+def test_neighbours_with_infinite_h(gpu_lib, orc, side, curve):
+    """Particles with an infinite h, a few scattered and a compact block of them: their lists hold every
+    particle whose own h reaches them, the others' lists are limited by their own h."""
+    print_case(f"infinite h side={side} curve={curve}")
+    s = ics.sedov_lattice(side)
+    n = side ** 3
+    rng = np.random.default_rng(side + 1)
+    for a in "xyz":
+        s[a] = s[a] + rng.uniform(-0.1, 0.1, n) / side
+    r2 = sum((s[a] - 0.1) ** 2 for a in "xyz")
+    s["sml"][np.argsort(r2)[:90]] = np.inf
+    s["sml"][[5, n // 3, n - 9]] = np.inf
+    with load_ctx(gpu_lib, s, gpu_lib.default_params(curve=curve, max_nb=400)) as ctx:
+        ctx.bbox(); ctx.keys(); ctx.sort(); ctx.build_tree()
+        ctx.neighbours()
+        nnl, noi = ctx.neighbour_lists(400)
+    st, onnl, onoi = orc.nn_brute(s["x"], s["y"], s["z"], s["sml"], 400)
+    assert st == 0
+    assert np.array_equal(noi, onoi)
+    used = np.arange(400) < noi[:, None]
+    assert np.array_equal(np.sort(np.where(used, nnl, -1), 1), np.sort(np.where(used, onnl, -1), 1))
